@@ -176,7 +176,7 @@ def bscan_line(args, traces):
         'device_ratio': round(plain_dev / (ms * 1e-3), 3),
         'batched_mcells_per_s': round(cells * args.bscan_its / (ms * 1e-3) / 1e6, 1),
         'tuned_shape': {'tile_cells': tile, 'xchunk': xchunk, 'ms_per_iteration': round(ms_tune, 4)},
-        'plain_step_form': 'fused' if args.fused else ('two-pass' if args.passes else 'default (timed choice)'),
+        'plain_step_form': 'fused' if args.fused else ('two-pass' if args.passes else 'default (chosen by rule)'),
         'receivers_identical': same,
     }
     return line
@@ -320,15 +320,14 @@ def adjoint_line(args):
 
 def step_form_label(fused, form, choice, default_form):
     """The step form that ran, and how it was chosen."""
-    name = ('fused, {} cells per block'.format(fused) if fused else
-            {3: 'split', 5: 'split, H boundary beside the interior kernel',
-             2: 'two-pass side by side', 6: 'two-pass merged, one launch per pass',
-             7: 'split, H boundary in the interior launch'}.get(form, 'two-pass'))
+    name = ('one-launch step, {} cells per block'.format(fused) if fused else
+            {2: 'passes with interior and boundary side by side',
+             6: 'two row passes'}.get(form, 'row kernels by rule'))
     if not default_form:
         return name + ' (set on the command line)'
     if choice == -1:
-        return name + ' (default form, not timed: the run was too short to time the forms)'
-    return name + ' (default form: timed against the others and kept)'
+        return name + ' (default form, the run too short for a choice)'
+    return name + ' (default form: chosen by rule)'
 
 
 def calibrate(args):
@@ -357,19 +356,13 @@ def main():
     ap.add_argument('--xchunk', type=int, default=0)
     ap.add_argument('--block', type=int, default=0)
     ap.add_argument('--tile', type=int, default=0, help='cells per fused block (0 = auto)')
-    ap.add_argument('--fused', action='store_true', help='one fused kernel per step instead of the H and E passes')
-    ap.add_argument('--overlap', action='store_true', help='H and E passes with interior and boundary kernels side by side')
+    ap.add_argument('--fused', action='store_true', help='the whole step in one launch (form 1)')
+    ap.add_argument('--overlap', action='store_true', help='the general passes with interior and boundary side by side (form 2)')
     ap.add_argument('--passes', action='store_true', help='the H and E passes (step form 0)')
-    ap.add_argument('--merged', action='store_true',
-                    help='the passes as one launch each over every cell (form 6)')
-    ap.add_argument('--split-merged', action='store_true',
-                    help='the split step with the H boundary pass inside the interior launch (form 7)')
-    ap.add_argument('--split', action='store_true',
-                    help='the split step (form 3): one kernel doing H and E for the interior, boundary passes '
-                         'around it; by default the library times forms 7, 6, 2, 5, the split step and the passes '
-                         '(forms 6, 2 and the passes where the split step does not apply) and keeps the fastest')
-    ap.add_argument('--split-beside', action='store_true',
-                    help='the split step with the H boundary pass beside the interior kernel (form 5)')
+    ap.add_argument('--merged', action='store_true', help='the two row passes (form 6)')
+    ap.add_argument('--split', action='store_true', help='form 3: the row kernels by rule')
+    ap.add_argument('--split-beside', action='store_true', help='form 5, as form 3')
+    ap.add_argument('--split-merged', action='store_true', help='form 7, as form 3')
     ap.add_argument('--traces', type=int, default=8, help='B-scan traces (workload bscan)')
     ap.add_argument('--forms', type=int, default=1,
                     help='headline workload: also run the B-scan and adjoint workloads and report them (1) or not (0)')
@@ -424,8 +417,8 @@ def main():
         s.synchronize()
         ms, _, _ = s.run_timed(W, K, per_kernel=False)
         s.synchronize()
-        form = s.step_form()       # after the runs: the default form times six forms on its first long run
-        choice = s.step_choice()   # -1: the default form has not timed them (a run shorter than 26 iterations)
+        form = s.step_form()       # after the runs: the default form chooses on its first run of 26 iterations
+        choice = s.step_choice()   # -1: not yet
         # Per-kernel durations (HIP events around every launch on the solver's
         # stream), in a separate run after the timed region.
         n_prof = min(50, G.iterations - W - K)
@@ -435,25 +428,14 @@ def main():
         mem = s.memory_bytes()
     cells = G.nx * G.ny * G.nz
     mcells = cells * K / (ms * 1e-3) / 1e6
-    if fused:
-        kernels = {'step': (algorithmic_bytes_per_step(G), ms4[0])}
-    elif form in (3, 5, 7):
-        # the fused box is the interior box less its first plane, row and column
-        box3 = (box[0] + 1, box[1], box[2] + 1, box[3], box[4] + 1, box[5])
-        bh, be = kernel_bytes(G, 1, box3), kernel_bytes(G, 0, box3)
-        kernels = {'interior': (bh[0] + be[0], ms4[0]), 'h_boundary': (bh[1], ms4[1]),
-                   'e_boundary': (be[1], ms4[3])}
-        if form == 7:
-            # the H boundary pass runs inside the interior kernel's launch
-            kernels = {'interior_and_h_boundary': (bh[0] + be[0] + bh[1], ms4[0]), 'e_boundary': (be[1], ms4[3])}
-    elif form == 6:
-        # one launch per pass over every cell
-        bh, be = kernel_bytes(G, 1, box), kernel_bytes(G, 0, box)
-        kernels = {'h_pass': (bh[0] + bh[1], ms4[0]), 'e_pass': (be[0] + be[1], ms4[2])}
-    else:
-        bh, be = kernel_bytes(G, 1, box), kernel_bytes(G, 0, box)
+    bh, be = kernel_bytes(G, 1, box), kernel_bytes(G, 0, box)
+    if ms4[1] > 0 or ms4[3] > 0:       # the general passes, interior and boundary apart
         kernels = {'h_interior': (bh[0], ms4[0]), 'h_boundary': (bh[1], ms4[1]),
                    'e_interior': (be[0], ms4[2]), 'e_boundary': (be[1], ms4[3])}
+    elif ms4[2] > 0:                   # the row passes, each one launch over every cell
+        kernels = {'h_pass': (bh[0] + bh[1], ms4[0]), 'e_pass': (be[0] + be[1], ms4[2])}
+    else:
+        kernels = {'step': (algorithmic_bytes_per_step(G), ms4[0])}
     dom = max(kernels, key=lambda k: kernels[k][1])
     dbytes, dms = kernels[dom]
     achieved = dbytes / (dms * 1e-3) / 1e9 if dms > 0 else 0.0

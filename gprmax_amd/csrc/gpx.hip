@@ -36,16 +36,15 @@
 
 #include "gpx.h"
 #include "gpx_step.h"
-#include "gpx_interior.h"
+#include "gpx_rows.h"
 
 namespace gpx {
 
 struct StepArgs {
     int nx, ny, nz;
-    int plane;           // (ny+1)*(nz+1)
+    int kp, plane;       // floats per row of a field array; (ny+1)*kp
     int nseg, nitems, per_xcd, xc;  // work items: nseg plane segments x x-chunks of xc planes
     float *Ex, *Ey, *Ez, *Hx, *Hy, *Hz;
-    float *So[3];        // where the pass writes its own field (the same arrays, or the next state)
     const void *ID;      // [6][ntot] of the compact index type
     long long ntot;
     const float *coef;   // [nmat][5]
@@ -73,15 +72,11 @@ struct StepArgs {
     // PML slab; the interior kernel covers it.  The boundary kernel covers
     // the rest: full planes for x outside [ix0, ix1) (items_a1 items below
     // ix0, items_a2 above), and for x inside, the plane cells of the frame
-    // list (plane offsets j*(nz+1)+k outside the interior rectangle).
+    // list (plane offsets j*kp+k outside the interior rectangle).
     int box[6];
     int nseg_a, nseg_b, items_a1, items_a2;
     const int *frame;
     int nframe;
-    // One launch over every cell (k_h_merged, k_e_merged): the chunks of the
-    // interior box's x range (m_nchunk, the interior and the frame items share
-    // the chunk length xc) and the number of items of both kinds (m_items).
-    int m_nchunk, m_items;
 };
 
 
@@ -111,7 +106,6 @@ __device__ __forceinline__ Cell item_cell(const StepArgs &a, int item)
 {
     Cell c;
     const int lane = threadIdx.x, B = blockDim.x;
-    const int NZ1 = a.nz + 1;
     if (!BND) {
         const int Kin = a.box[5] - a.box[4];
         const int ncell = (a.box[3] - a.box[2]) * Kin;
@@ -144,8 +138,12 @@ __device__ __forceinline__ Cell item_cell(const StepArgs &a, int item)
         c.live = q < a.nframe;
         t = c.live ? a.frame[q] : 0;
     }
-    c.j = t / NZ1;
-    c.k = t - c.j * NZ1;
+    c.j = t / a.kp;
+    c.k = t - c.j * a.kp;
+    if (c.k > a.nz) {  // padding of the row
+        c.live = false;
+        c.k = a.nz;
+    }
     return c;
 }
 
@@ -185,13 +183,12 @@ __device__ __forceinline__ void h_pass_run(const StepArgs &a, int first, int str
     __syncthreads();
 
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int NZ1 = nz + 1;
+    const int NZ1 = a.kp;
     const size_t N = a.ntot;
     const int flags = a.flags;
     const IDT *ID = static_cast<const IDT *>(a.ID);
     const rsrc_t rEx = rsrc(a.Ex), rEy = rsrc(a.Ey), rEz = rsrc(a.Ez);
     const rsrc_t rHx = rsrc(a.Hx), rHy = rsrc(a.Hy), rHz = rsrc(a.Hz);
-    const rsrc_t wHx = rsrc(a.So[0]), wHy = rsrc(a.So[1]), wHz = rsrc(a.So[2]);
     const rsrc_t rI3 = rsrc(ID + 3 * N), rI4 = rsrc(ID + 4 * N), rI5 = rsrc(ID + 5 * N);
     const uint32_t P4 = (uint32_t)a.plane * 4u, Pid = (uint32_t)a.plane * (uint32_t)sizeof(IDT);
 
@@ -273,19 +270,19 @@ __device__ __forceinline__ void h_pass_run(const StepArgs &a, int first, int str
                         if (!(smask & (1u << s))) continue;
                         const SlabArgs &sl = lslab[s];
                         int p;
-                        uint32_t q1, q2, o1, o2;
+                        uint32_t q;
                         float a1, b1, a2, b2;
-                        phi_get(sl, s, pre, i, j, k, p, q1, q2, o1, o2, a1, b1, a2, b2);
+                        phi_get(sl, s, pre, i, j, k, p, q, a1, b1, a2, b2);
                         const float *R = lR + sl.roff;
                         if (sl.axis == 0) {
-                            hy = pml_correct_pre(a.form, sl, R, p, hy, true, ls[m4], dEz_x / sl.d, a1, b1, sl.phi1, q1, o1);
-                            hz = pml_correct_pre(a.form, sl, R, p, hz, false, ls[m5], dEy_x / sl.d, a2, b2, sl.phi2, q2, o2);
+                            hy = pml_correct_pre(a.form, sl, R, p, hy, true, ls[m4], dEz_x / sl.d, a1, b1, sl.phi1, q, sl.ostep);
+                            hz = pml_correct_pre(a.form, sl, R, p, hz, false, ls[m5], dEy_x / sl.d, a2, b2, sl.phi2, q, sl.ostep);
                         } else if (sl.axis == 1) {
-                            hx = pml_correct_pre(a.form, sl, R, p, hx, false, ls[m3], dEz_y / sl.d, a1, b1, sl.phi1, q1, o1);
-                            hz = pml_correct_pre(a.form, sl, R, p, hz, true, ls[m5], dEx_y / sl.d, a2, b2, sl.phi2, q2, o2);
+                            hx = pml_correct_pre(a.form, sl, R, p, hx, false, ls[m3], dEz_y / sl.d, a1, b1, sl.phi1, q, sl.ostep);
+                            hz = pml_correct_pre(a.form, sl, R, p, hz, true, ls[m5], dEx_y / sl.d, a2, b2, sl.phi2, q, sl.ostep);
                         } else {
-                            hx = pml_correct_pre(a.form, sl, R, p, hx, true, ls[m3], dEy_z / sl.d, a1, b1, sl.phi1, q1, o1);
-                            hy = pml_correct_pre(a.form, sl, R, p, hy, false, ls[m4], dEx_z / sl.d, a2, b2, sl.phi2, q2, o2);
+                            hx = pml_correct_pre(a.form, sl, R, p, hx, true, ls[m3], dEy_z / sl.d, a1, b1, sl.phi1, q, sl.ostep);
+                            hy = pml_correct_pre(a.form, sl, R, p, hy, false, ls[m4], dEx_z / sl.d, a2, b2, sl.phi2, q, sl.ostep);
                         }
                     }
                 }
@@ -308,9 +305,9 @@ __device__ __forceinline__ void h_pass_run(const StepArgs &a, int first, int str
             }
 
             if (flags & (F_MAIN | F_PML_ALL | F_SRC)) {
-                bst(wHx, to, so, hx);
-                bst(wHy, to, so, hy);
-                bst(wHz, to, so, hz);
+                bst(rHx, to, so, hx);
+                bst(rHy, to, so, hy);
+                bst(rHz, to, so, hz);
             }
 
             if ((flags & F_RX) && (pf & PF_RX)) {  // the state at the start of the iteration
@@ -392,13 +389,12 @@ __device__ __forceinline__ void e_pass_run(const StepArgs &a, int first, int str
     __syncthreads();
 
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int NZ1 = nz + 1;
+    const int NZ1 = a.kp;
     const size_t Pl = a.plane, N = a.ntot;
     const int flags = a.flags;
     const IDT *ID = static_cast<const IDT *>(a.ID);
     const rsrc_t rEx = rsrc(a.Ex), rEy = rsrc(a.Ey), rEz = rsrc(a.Ez);
     const rsrc_t rHx = rsrc(a.Hx), rHy = rsrc(a.Hy), rHz = rsrc(a.Hz);
-    const rsrc_t wEx = rsrc(a.So[0]), wEy = rsrc(a.So[1]), wEz = rsrc(a.So[2]);
     const rsrc_t rI0 = rsrc(ID), rI1 = rsrc(ID + N), rI2 = rsrc(ID + 2 * N);
     const uint32_t P4 = (uint32_t)Pl * 4u, Pid = (uint32_t)Pl * (uint32_t)sizeof(IDT);
 
@@ -515,19 +511,19 @@ __device__ __forceinline__ void e_pass_run(const StepArgs &a, int first, int str
                         if (!(smask & (1u << s))) continue;
                         const SlabArgs &sl = lslab[s];
                         int p;
-                        uint32_t q1, q2, o1, o2;
+                        uint32_t q;
                         float a1, b1, a2, b2;
-                        phi_get(sl, s, pre, i, j, k, p, q1, q2, o1, o2, a1, b1, a2, b2);
+                        phi_get(sl, s, pre, i, j, k, p, q, a1, b1, a2, b2);
                         const float *R = lR + sl.roff;
                         if (sl.axis == 0) {
-                            ey = pml_correct_pre(a.form, sl, R, p, ey, false, ls[m1], dHz_x / sl.d, a1, b1, sl.phi1, q1, o1);
-                            ez = pml_correct_pre(a.form, sl, R, p, ez, true, ls[m2], dHy_x / sl.d, a2, b2, sl.phi2, q2, o2);
+                            ey = pml_correct_pre(a.form, sl, R, p, ey, false, ls[m1], dHz_x / sl.d, a1, b1, sl.phi1, q, sl.ostep);
+                            ez = pml_correct_pre(a.form, sl, R, p, ez, true, ls[m2], dHy_x / sl.d, a2, b2, sl.phi2, q, sl.ostep);
                         } else if (sl.axis == 1) {
-                            ex = pml_correct_pre(a.form, sl, R, p, ex, true, ls[m0], dHz_y / sl.d, a1, b1, sl.phi1, q1, o1);
-                            ez = pml_correct_pre(a.form, sl, R, p, ez, false, ls[m2], dHx_y / sl.d, a2, b2, sl.phi2, q2, o2);
+                            ex = pml_correct_pre(a.form, sl, R, p, ex, true, ls[m0], dHz_y / sl.d, a1, b1, sl.phi1, q, sl.ostep);
+                            ez = pml_correct_pre(a.form, sl, R, p, ez, false, ls[m2], dHx_y / sl.d, a2, b2, sl.phi2, q, sl.ostep);
                         } else {
-                            ex = pml_correct_pre(a.form, sl, R, p, ex, false, ls[m0], dHy_z / sl.d, a1, b1, sl.phi1, q1, o1);
-                            ey = pml_correct_pre(a.form, sl, R, p, ey, true, ls[m1], dHx_z / sl.d, a2, b2, sl.phi2, q2, o2);
+                            ex = pml_correct_pre(a.form, sl, R, p, ex, false, ls[m0], dHy_z / sl.d, a1, b1, sl.phi1, q, sl.ostep);
+                            ey = pml_correct_pre(a.form, sl, R, p, ey, true, ls[m1], dHx_z / sl.d, a2, b2, sl.phi2, q, sl.ostep);
                         }
                     }
                 }
@@ -574,9 +570,9 @@ __device__ __forceinline__ void e_pass_run(const StepArgs &a, int first, int str
                 if (dz_) t_store<P, CPLX>(a.T, 2, sz, tzr, tzi);
             }
             if (flags & (F_MAIN | F_PML_ALL | F_SRC)) {
-                bst(wEx, to, so, ex);
-                bst(wEy, to, so, ey);
-                bst(wEz, to, so, ez);
+                bst(rEx, to, so, ex);
+                bst(rEy, to, so, ey);
+                bst(rEz, to, so, ez);
             }
             hy_m = hy;
             hz_m = hz;
@@ -603,85 +599,10 @@ __global__ void k_e_pass_many(const StepArgs *__restrict__ args, PassMany m)
 }
 
 
-// ---------------------------------------------------------------- merged passes
-// One launch per pass over every cell.  Block order (before the per-XCD
-// remap): the boundary planes below the interior box, then per x chunk of the
-// box its interior items followed by its frame items, then the boundary planes
-// above.  The frame rows' short z runs share their first and last 64-byte
-// sectors with the interior rows next to them; with the items of one chunk
-// adjacent in one launch on one XCD, the second reader of such a sector finds
-// it in L2 instead of fetching it again from HBM, as it does when the frame
-// waits for a kernel of its own.  Returns true for a boundary item and sets
-// `item` to its index in the interior or the boundary numbering.
-__device__ __forceinline__ bool merged_item(const StepArgs &a, int L, int &item)
-{
-    if (L < a.items_a1) {
-        item = L;
-        return true;
-    }
-    L -= a.items_a1;
-    const int per = a.nseg + a.nseg_b;
-    const int mid = a.m_nchunk * per;
-    if (L < mid) {
-        // within a chunk, the frame items spread evenly among the interior
-        // items: position r is a frame item when floor((r+1) nb / per) >
-        // floor(r nb / per), so frame and interior rows advance together
-        const int c = L / per, r = L - c * per;
-        const long long nb = a.nseg_b;
-        const int f0 = (int)(r * nb / per), f1 = (int)((r + 1) * nb / per);
-        if (f1 == f0) {
-            item = c * a.nseg + (r - f1);
-            return false;
-        }
-        item = a.items_a1 + a.items_a2 + c * a.nseg_b + f0;
-        return true;
-    }
-    item = a.items_a1 + (L - mid);
-    return true;
-}
-
-// One item per block; the pass bodies' item loop runs once (a.nitems = 2^30).
-template <class IDT>
-__global__ void k_h_merged(StepArgs a)
-{
-    const int L = logical_block(a.per_xcd);
-    if (L >= a.m_items) return;
-    int item;
-    if (merged_item(a, L, item)) h_pass_run<IDT, true>(a, item, 1 << 30, a.it);
-    else h_pass_run<IDT, false>(a, item, 1 << 30, a.it);
-}
-
-template <class IDT, int P, bool CPLX>
-__global__ void k_e_merged(StepArgs a)
-{
-    const int L = logical_block(a.per_xcd);
-    if (L >= a.m_items) return;
-    int item;
-    if (merged_item(a, L, item)) e_pass_run<IDT, P, CPLX, true>(a, item, 1 << 30, a.it);
-    else e_pass_run<IDT, P, CPLX, false>(a, item, 1 << 30, a.it);
-}
-
-
-// Form 7: the split step's interior items (interior_run) and its H boundary
-// items in one launch of INT_BLOCK threads, in merged_item's order.  `hb` is
-// the H boundary pass of the split step (current state in, next state out)
-// with hb.nseg set to the interior's segment count.  Neither kind of item
-// reads what the other writes (form 5 runs the same two on two streams).
-template <class IDT>
-__global__ void __launch_bounds__(INT_BLOCK) k_interior_hb(IntArgs ai, StepArgs hb)
-{
-    const int L = logical_block(hb.per_xcd);
-    if (L >= hb.m_items) return;
-    int item;
-    if (merged_item(hb, L, item)) h_pass_run<IDT, true>(hb, item, 1 << 30, hb.it);
-    else interior_run<IDT>(ai, item);
-}
-
-
 // ---------------------------------------------------------------- snapshots
 // Cell averages of gprMax/snapshots_ext.pyx:58-71 over the slices of
 // gprMax/snapshots.py:78-80; one thread per output cell.
-__global__ void k_snapshot(int ny, int nz, int xs, int ys, int zs, int sdx, int sdy, int sdz,
+__global__ void k_snapshot(int ny, int kp, int xs, int ys, int zs, int sdx, int sdy, int sdz,
                            int snx, int sny, int snz, const float *Ex, const float *Ey,
                            const float *Ez, const float *Hx, const float *Hy, const float *Hz,
                            float *out)
@@ -692,7 +613,7 @@ __global__ void k_snapshot(int ny, int nz, int xs, int ys, int zs, int sdx, int 
     const int k = (int)(o % snz);
     const int j = (int)((o / snz) % sny);
     const int i = (int)(o / ((long long)snz * sny));
-    const long long NY1 = ny + 1, NZ1 = nz + 1;
+    const long long NY1 = ny + 1, NZ1 = kp;
     auto at = [&](int a, int b, int c) {
         return ((long long)(xs + a * sdx) * NY1 + (ys + b * sdy)) * NZ1 + (zs + c * sdz);
     };
@@ -726,7 +647,7 @@ struct TLDev {
 // current is updated and its antenna end takes the current of the H loop
 // around the edge (update_magnetic, gprMax/sources.py:428-451, and
 // Ix/Iy/Iz, gprMax/grid.py:413-461).  One thread per line.
-__global__ void k_tl_h(const TLDev *tl, int n, int it, int ny, int nz, const float *Hx, const float *Hy,
+__global__ void k_tl_h(const TLDev *tl, int n, int it, int ny, int kp, const float *Hx, const float *Hy,
                        const float *Hz)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -740,7 +661,7 @@ __global__ void k_tl_h(const TLDev *tl, int n, int it, int ny, int nz, const flo
         L.I[m] = (float)((double)L.I[m] - L.cI * (double)d);
     }
     L.I[L.srcpos - 1] = (float)((double)L.I[L.srcpos - 1] + L.cI * (double)L.half[it]);
-    const long long NY1 = ny + 1, NZ1 = nz + 1;
+    const long long NY1 = ny + 1, NZ1 = kp;
     auto at = [&](int a, int b, int c) { return ((long long)a * NY1 + b) * NZ1 + c; };
     const int x = L.i, y = L.j, z = L.k;
     float cur = 0.f;
@@ -760,7 +681,7 @@ __global__ void k_tl_h(const TLDev *tl, int n, int it, int ny, int nz, const flo
 // After the E pass, in the active window: line voltage, the one-way
 // injector, the absorbing end, then the edge's E from the antenna voltage
 // (update_electric, gprMax/sources.py:361-426).
-__global__ void k_tl_e(const TLDev *tl, int n, int it, int ny, int nz, float *Ex, float *Ey, float *Ez)
+__global__ void k_tl_e(const TLDev *tl, int n, int it, int ny, int kp, float *Ex, float *Ey, float *Ez)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
@@ -775,7 +696,7 @@ __global__ void k_tl_e(const TLDev *tl, int n, int it, int ny, int nz, float *Ex
     L.V[0] = (float)(L.h * (double)(L.V[1] - a0) + (double)a1);
     L.abc[0] = L.V[0];
     L.abc[1] = L.V[1];
-    const long long at = ((long long)L.i * (ny + 1) + L.j) * (nz + 1) + L.k;
+    const long long at = ((long long)L.i * (ny + 1) + L.j) * kp + L.k;
     float *E = L.pol == 0 ? Ex : (L.pol == 1 ? Ey : Ez);
     E[at] = -L.V[L.antpos] / L.dpol;
 }
@@ -788,10 +709,14 @@ using namespace gpx;
 struct Slab {
     int dir, xs, xf, ys, yf, zs, zf, order, t, roff = 0;
     float d;
-    float *phi[4] = {nullptr, nullptr, nullptr, nullptr};  // EPhi1, EPhi2, HPhi1, HPhi2 (current)
-    float *phin[2] = {nullptr, nullptr};                    // HPhi1, HPhi2 of the next state
-    long long dims[4][3];
-    float *eR = nullptr, *hR = nullptr;
+    long long dims[4][3];  // reference shapes of EPhi1, EPhi2, HPhi1, HPhi2, without the order axis
+    // Phi on the device: all slabs of a field in one array, per order and term
+    // (1, 2) the slabs one after the other, each [ni][nj][nkp] in ascending
+    // cell order (the reference runs the profile axis of the minus slabs
+    // backwards), rows padded so that cell k sits at k mod 4 as in the fields.
+    long long base;        // of the slab within a block of one order and term
+    int ni, nj, nkp;
+    std::vector<float> R[2];  // E, H profile tables RA, RB, RE, RF, each [order][t]
 };
 
 struct Snap {
@@ -814,16 +739,29 @@ struct SrcSet {
 struct gpx_ctx {
     gpx_desc desc;
     long long ntot = 0;
-    int plane = 0;
+    int kp = 0, plane = 0;    // floats per field row (nz + 1 rounded up to 4 where that fits); (ny + 1) kp
     hipStream_t stream = nullptr;
-    float *F[6] = {nullptr};  // Ex, Ey, Ez, Hx, Hy, Hz (current state)
-    float *Fn[6] = {nullptr}; // the next state written by the double-buffered forms (1, 3, 5)
-    float *Fmem[2] = {nullptr, nullptr};  // the two states, 6 x fstride floats each; the second is
-                                          // allocated only when a double-buffered form runs
-    size_t next_bytes = 0;    // bytes of the second state and of the second H-PML Phi copies
-    long long fstride = 0;    // floats between components: ntot rounded up to 64
-    void *ID = nullptr;       // [6][ntot] as uint8, uint16 or uint32
-    int id_bytes = 2;         // material indices are uint16 on the device (nmat < 2^16, see gpx_create)
+    // The state: fields and H Phi, twice for the double-buffered step (the
+    // second copy is allocated when it first runs), `cur` the current one; E
+    // Phi once.  ntot counts padded points.
+    float *Fmem[2] = {nullptr, nullptr};    // 6 x fstride floats: Ex, Ey, Ez, Hx, Hy, Hz
+    float *phiH[2] = {nullptr, nullptr}, *phiE = nullptr;
+    int cur = 0;
+    float *field(int c) const { return Fmem[cur] + c * fstride; }
+    long long np = 0;         // floats of one (order, term) block of Phi
+    int phi_orders = 0;       // orders the Phi arrays hold
+    bool phi_dirty = false;   // slabs were added since the Phi arrays were laid out
+    size_t next_bytes = 0;    // bytes of the second state and of the second H Phi
+    long long fstride = 0;    // floats between components: ntot rounded up to 64, and a row more
+    uint16_t *ID = nullptr;   // [6][ntot] (nmat < 2^16, see gpx_create)
+    std::vector<float> hostE, hostH, hostdisp;  // coefficients and pole tables, for the row kernels' tables
+    float *img = nullptr;     // those tables (row_stage), nimg floats
+    int nimg = 0;
+    RowModel *row = nullptr;  // the model as the row kernels see it
+    RowModel rowh;            // its host copy
+    bool row_dirty = true;    // something in it changed
+    bool hu = false;          // every material has the same H coefficients
+    int row_block = 0;        // threads per block of the one-launch step
     float *cE = nullptr, *cH = nullptr;
     float *Rall[2] = {nullptr, nullptr};  // E, H: all slabs' R tables back to back
     std::vector<float> Rhost[2];
@@ -844,26 +782,19 @@ struct gpx_ctx {
     std::vector<Snap> snaps;
     std::vector<TLine> tls;          // transmission lines
     TLDev *tldev = nullptr;          // device copy of their descriptions
-    uint32_t *planeflag = nullptr;  // [nx+1]
+    uint32_t *planeflag = nullptr;  // [2][nx+1]: slab bits by slab, by direction
     StepRare *rare = nullptr;        // device copy of the source/receiver tables for the fused step
     bool rare_dirty = true;
     int box[6] = {0, 0, 0, 0, 0, 0}; // interior box (see StepArgs)
     int *frame = nullptr;            // plane offsets outside the interior rectangle
     int nframe = 0;
-    int box3[6] = {0, 0, 0, 0, 0, 0};  // the split step's fused box: the interior box less its
-    int *frame3 = nullptr;              // first plane, row and column on the minus sides, and
-    int nframe3 = 0;                    // the plane offsets outside its rectangle
+    bool deep = false;               // the interior box has at least two cells on every axis
     int xchunk = 0, block = 0;
-    int fused = 4;                   // step form (gpx_set_step): 0 passes, 1 fused step, 2 passes side
-                                     // by side, 3 split step, 4 (default) the fastest of 7, 6, 2, 5, 3 and 0,
-                                     // 5 split step with the H boundary pass beside the interior kernel,
-                                     // 6 passes as one launch each over every cell, 7 split step with the
-                                     // H boundary pass in the interior kernel's launch
-    int split_choice = -1;           // form 4: -1 not yet timed, 0 passes, 1 split step, 2 form 5, 3 form 2,
-                                     // 4 form 6, 5 form 7
-    hipStream_t stream2 = nullptr;   // second stream of forms 2 and 5
+    int fused = 4;                   // step form, see gpx_set_step
+    int choice = -1;                 // form 4: -1 open, 4 form 6, 5 form 7
+    hipStream_t stream2 = nullptr;   // second stream of form 2
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    int tile_cells = 0;              // cells per fused block (0 = auto)
+    int tile_cells = 0;              // cells per block of the one-launch step (0 = auto)
     int cus = 0;                     // compute units of the device
     mutable std::map<std::pair<const void *, size_t>, int> occupancy;
     size_t bytes = 0;
@@ -956,7 +887,12 @@ extern "C" int gpx_create(const gpx_desc *d, gpx_ctx **out)
         }
         ctx->cus = prop.multiProcessorCount;
     }
-    ctx->plane = (d->ny + 1) * (d->nz + 1);
+    // Rows padded to four floats, so that the row kernels load and store whole
+    // lanes; unpadded where the padding alone would pass the 32-bit offsets
+    // (such a grid takes the general passes).
+    ctx->kp = (d->nz + 1 + 3) / 4 * 4;
+    if ((unsigned long long)(d->nx + 1) * (d->ny + 1) * ctx->kp * 4ull > 0xFFFFFFFFull) ctx->kp = d->nz + 1;
+    ctx->plane = (d->ny + 1) * ctx->kp;
     ctx->ntot = (long long)(d->nx + 1) * ctx->plane;
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
@@ -964,24 +900,19 @@ extern "C" int gpx_create(const gpx_desc *d, gpx_ctx **out)
         delete ctx;
         return rc;
     }
-    ctx->fstride = (ctx->ntot + 63) / 64 * 64;
+    ctx->fstride = (ctx->ntot + 16 + 63) / 64 * 64;
     e = dalloc(ctx, (void **)&ctx->Fmem[0], (size_t)6 * ctx->fstride * 4);
     if (e != hipSuccess) goto fail_alloc;
-    for (int c = 0; c < 6; ++c) {
-        ctx->F[c] = ctx->Fmem[0] + c * ctx->fstride;
-        ctx->Fn[c] = nullptr;
-    }
     // The coefficient tables must fit LDS (as the reference's must fit 64 KB
     // of constant memory, gprMax/model_build_run.py:512-516), which bounds
     // nmat far below 2^16: every material index fits 16 bits.
-    ctx->id_bytes = 2;
-    e = dalloc(ctx, (void **)&ctx->ID, 6 * (size_t)ctx->ntot * ctx->id_bytes, false);
+    e = dalloc(ctx, (void **)&ctx->ID, (6 * (size_t)ctx->ntot + 16) * 2, false);
     if (e != hipSuccess) goto fail_alloc;
     e = dalloc(ctx, (void **)&ctx->cE, (size_t)d->nmat * 5 * 4);
     if (e != hipSuccess) goto fail_alloc;
     e = dalloc(ctx, (void **)&ctx->cH, (size_t)d->nmat * 5 * 4);
     if (e != hipSuccess) goto fail_alloc;
-    e = dalloc(ctx, (void **)&ctx->planeflag, (size_t)(d->nx + 1) * 4);
+    e = dalloc(ctx, (void **)&ctx->planeflag, (size_t)(d->nx + 1) * 8);
     if (e != hipSuccess) goto fail_alloc;
     if (int rc = update_planeflags(ctx)) {
         gpx_destroy(ctx);
@@ -1010,12 +941,10 @@ extern "C" int gpx_destroy(gpx_ctx *ctx)
     for (auto &p : ctx->Rall) if (p) hipFree(p);
     if (ctx->disp) hipFree(ctx->disp);
     if (ctx->dispflag) hipFree(ctx->dispflag);
-    for (auto &s : ctx->slabs) {
-        for (auto &p : s.phi) if (p) hipFree(p);
-        for (auto &p : s.phin) if (p) hipFree(p);
-        if (s.eR) hipFree(s.eR);
-        if (s.hR) hipFree(s.hR);
-    }
+    for (auto &p : ctx->phiH) if (p) hipFree(p);
+    if (ctx->phiE) hipFree(ctx->phiE);
+    if (ctx->img) hipFree(ctx->img);
+    if (ctx->row) hipFree(ctx->row);
     for (auto &s : ctx->src) {
         if (s.info) hipFree(s.info);
         if (s.fac) hipFree(s.fac);
@@ -1026,7 +955,6 @@ extern "C" int gpx_destroy(gpx_ctx *ctx)
     if (ctx->planeflag) hipFree(ctx->planeflag);
     if (ctx->rare) hipFree(ctx->rare);
     if (ctx->frame) hipFree(ctx->frame);
-    if (ctx->frame3) hipFree(ctx->frame3);
     for (auto &s : ctx->snaps) if (s.out) hipFree(s.out);
     for (auto &t : ctx->tls) if (t.mem) hipFree(t.mem);
     if (ctx->tldev) hipFree(ctx->tldev);
@@ -1053,60 +981,80 @@ static int copy_out(gpx_ctx *ctx, void *dst, const void *src, size_t bytes)
     return 0;
 }
 
-// ---------------------------------------------------------------- second state
-// The double-buffered forms write the next state into a second copy of the
-// fields (the fused step and the split step) and the fused step also the
-// H-PML Phi into a second copy.  The copies are made on first use, equal to
-// the current state, so a model that only ever updates in place (the passes,
-// dispersive models, models with transmission lines) holds one field state.
-static int ensure_next_state(gpx_ctx *ctx, bool phi)
+// ---------------------------------------------------------------- Phi arrays
+static size_t phi_bytes(const gpx_ctx *ctx) { return (size_t)ctx->phi_orders * 2 * ctx->np * 4 + 16; }
+
+static int phi_transfer(gpx_ctx *ctx, int slab, int which, float *host, bool up);
+
+// Lays the Phi arrays out once slabs are there; slabs added later keep the
+// values of the ones before.
+static int ensure_phi(gpx_ctx *ctx)
 {
-    const size_t fb = (size_t)6 * ctx->fstride * 4;
-    if (!ctx->Fmem[1]) {
-        // Without a second state the current one is Fmem[0].
-        float *m = nullptr;
-        GPX_TRY(dalloc(ctx, (void **)&m, fb, false));
-        ctx->Fmem[1] = m;
-        ctx->next_bytes += fb;
-        for (int c = 0; c < 6; ++c) ctx->Fn[c] = m + c * ctx->fstride;
-        GPX_TRY(hipMemcpyAsync(m, ctx->Fmem[0], fb, hipMemcpyDeviceToDevice, ctx->stream));
-    }
-    if (phi) {
-        for (Slab &S : ctx->slabs)
-            for (int q = 0; q < 2; ++q) {
-                if (S.phin[q]) continue;
-                const size_t b = (size_t)S.order * S.dims[q + 2][0] * S.dims[q + 2][1] * S.dims[q + 2][2] * 4;
-                GPX_TRY(dalloc(ctx, (void **)&S.phin[q], b, false));
-                ctx->next_bytes += b;
-                GPX_TRY(hipMemcpyAsync(S.phin[q], S.phi[q + 2], b, hipMemcpyDeviceToDevice, ctx->stream));
+    if (!ctx->phi_dirty) return 0;
+    hipSetDevice(ctx->desc.device);
+    std::vector<std::vector<float>> keep;
+    std::vector<Slab> now = ctx->slabs;
+    if (ctx->phiE) {  // values of the slabs that were there, in the old layout
+        long long acc = 0;
+        size_t n = 0;
+        while (n < ctx->slabs.size() && acc < ctx->np) acc += (long long)now[n].ni * now[n].nj * now[n].nkp, ++n;
+        ctx->phi_dirty = false;
+        for (size_t s = 0; s < n; ++s)
+            for (int w = 0; w < 4; ++w) {
+                const Slab &S = ctx->slabs[s];
+                keep.emplace_back((size_t)S.order * S.dims[w][0] * S.dims[w][1] * S.dims[w][2]);
+                if (int rc = phi_transfer(ctx, (int)s, w, keep.back().data(), false)) return rc;
             }
+        GPX_TRY(hipStreamSynchronize(ctx->stream));
+        ctx->bytes -= phi_bytes(ctx) * (ctx->phiH[1] ? 3 : 2);
+        if (ctx->phiH[1]) ctx->next_bytes -= phi_bytes(ctx);
+        for (float **p : {&ctx->phiE, &ctx->phiH[0], &ctx->phiH[1]}) {
+            if (*p) hipFree(*p);
+            *p = nullptr;
+        }
     }
+    ctx->np = 0;
+    ctx->phi_orders = 0;
+    for (Slab &S : ctx->slabs) {
+        S.base = ctx->np;
+        ctx->np += (long long)S.ni * S.nj * S.nkp;
+        if (S.order > ctx->phi_orders) ctx->phi_orders = S.order;
+    }
+    GPX_TRY(dalloc(ctx, (void **)&ctx->phiE, phi_bytes(ctx)));
+    const bool two = ctx->Fmem[1] != nullptr;
+    for (int q = 0; q < (two ? 2 : 1); ++q) {
+        GPX_TRY(dalloc(ctx, (void **)&ctx->phiH[q], phi_bytes(ctx)));
+        if (q) ctx->next_bytes += phi_bytes(ctx);
+    }
+    ctx->phi_dirty = false;
+    ctx->row_dirty = true;
+    for (size_t n = 0; n < keep.size(); ++n)
+        if (int rc = phi_transfer(ctx, (int)n / 4, (int)n % 4, keep[n].data(), true)) return rc;
     return 0;
 }
 
-// Gives the second copies back (the default form settled on a form that
-// updates in place).  The current state is whichever copy F points into.
-static int release_next_state(gpx_ctx *ctx)
+// ---------------------------------------------------------------- second state
+// The one-launch step writes the next state, fields and H Phi, into second
+// copies.  They are made on first use, equal to the current ones, so a model
+// that only ever updates in place (dispersive models, models with
+// transmission lines) holds one state.
+static int ensure_next_state(gpx_ctx *ctx)
 {
-    if (!ctx->Fmem[1]) return 0;
-    GPX_TRY(hipStreamSynchronize(ctx->stream));
-    if (ctx->stream2) GPX_TRY(hipStreamSynchronize(ctx->stream2));
+    if (ctx->Fmem[1]) return 0;
+    // Without a second state the current one is Fmem[0].
     const size_t fb = (size_t)6 * ctx->fstride * 4;
-    if (ctx->F[0] == ctx->Fmem[1]) std::swap(ctx->Fmem[0], ctx->Fmem[1]);
-    GPX_TRY(hipFree(ctx->Fmem[1]));
-    ctx->Fmem[1] = nullptr;
-    for (int c = 0; c < 6; ++c) ctx->Fn[c] = nullptr;
-    ctx->bytes -= fb;
-    ctx->next_bytes -= fb;
-    for (Slab &S : ctx->slabs)
-        for (int q = 0; q < 2; ++q) {
-            if (!S.phin[q]) continue;
-            const size_t b = (size_t)S.order * S.dims[q + 2][0] * S.dims[q + 2][1] * S.dims[q + 2][2] * 4;
-            GPX_TRY(hipFree(S.phin[q]));
-            S.phin[q] = nullptr;
-            ctx->bytes -= b;
-            ctx->next_bytes -= b;
-        }
+    float *m = nullptr;
+    GPX_TRY(dalloc(ctx, (void **)&m, fb, false));
+    ctx->Fmem[1] = m;
+    ctx->next_bytes += fb;
+    GPX_TRY(hipMemcpyAsync(m, ctx->Fmem[0], fb, hipMemcpyDeviceToDevice, ctx->stream));
+    if (ctx->phiH[0]) {
+        const size_t b = phi_bytes(ctx);
+        GPX_TRY(dalloc(ctx, (void **)&ctx->phiH[1], b, false));
+        ctx->next_bytes += b;
+        GPX_TRY(hipMemcpyAsync(ctx->phiH[1], ctx->phiH[0], b, hipMemcpyDeviceToDevice, ctx->stream));
+    }
+    ctx->row_dirty = true;
     return 0;
 }
 
@@ -1180,7 +1128,7 @@ static int ensure_tslots(gpx_ctx *ctx)
             if (e != hipSuccess) { rc = fail_hip(ctx, e, "slot array"); break; }
         }
         hipLaunchKernelGGL(k_tslot_count<uint16_t>, dim3(nb), dim3(256), 0, ctx->stream,
-                           (const uint16_t *)ctx->ID + (size_t)c * N, ctx->dispflag, N, boff);
+                           ctx->ID + (size_t)c * N, ctx->dispflag, N, boff);
         if ((rc = copy_out(ctx, h.data(), boff, (size_t)nb * 4))) break;
         unsigned long long acc = 0;
         for (int b = 0; b < nb; ++b) {
@@ -1190,11 +1138,12 @@ static int ensure_tslots(gpx_ctx *ctx)
         }
         if ((rc = copy_in(ctx, boff, h.data(), (size_t)nb * 4))) break;
         hipLaunchKernelGGL(k_tslot_fill<uint16_t>, dim3(nb), dim3(1024), 0, ctx->stream,
-                           (const uint16_t *)ctx->ID + (size_t)c * N, ctx->dispflag, N, boff, ctx->tslot[c]);
+                           ctx->ID + (size_t)c * N, ctx->dispflag, N, boff, ctx->tslot[c]);
         hipError_t e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) { rc = fail_hip(ctx, e, "slot build"); break; }
         ctx->tn[c] = (long long)acc;
         if (ctx->T[c]) { hipFree(ctx->T[c]); ctx->T[c] = nullptr; }
+        ctx->row_dirty = true;
         const size_t tb = (size_t)P * (size_t)(acc > 0 ? acc : 1) * 4 * (ctx->disp_complex ? 2 : 1);
         e = dalloc(ctx, (void **)&ctx->T[c], tb);
         if (e != hipSuccess) { rc = fail_hip(ctx, e, "auxiliary values"); break; }
@@ -1211,16 +1160,23 @@ extern "C" int gpx_upload_id(gpx_ctx *ctx, const uint32_t *ID)
 {
     if (!ctx || !ID) return fail(ctx, GPX_EARG, "gpx_upload_id: null argument");
     const uint32_t nmat = (uint32_t)ctx->desc.nmat;
-    const size_t n = 6 * (size_t)ctx->ntot;
+    const gpx_desc &g = ctx->desc;
+    const size_t nk = (size_t)g.nz + 1, kp = (size_t)ctx->kp, rows = 6 * (size_t)(g.nx + 1) * (g.ny + 1);
     // Every ID indexes the coefficient tables; reject out-of-range values on the
     // host so no kernel can read outside them.
+    const size_t n = rows * nk;
     for (size_t q = 0; q < n; ++q)
         if (ID[q] >= nmat)
             return fail(ctx, GPX_EARG, "gpx_upload_id: material index " + std::to_string(ID[q]) +
                                            " >= nmat " + std::to_string(nmat));
     hipSetDevice(ctx->desc.device);
-    std::vector<uint16_t> c(ID, ID + n);   // every index < nmat < 2^16
-    int rc = copy_in(ctx, ctx->ID, c.data(), n * 2);
+    std::vector<uint16_t> c(rows * kp, 0);   // every index < nmat < 2^16; the padding takes material 0
+    for (size_t r = 0; r < rows; ++r) {
+        const uint32_t *src = ID + r * nk;
+        uint16_t *dst = c.data() + r * kp;
+        for (size_t k = 0; k < nk; ++k) dst[k] = (uint16_t)src[k];
+    }
+    int rc = copy_in(ctx, ctx->ID, c.data(), c.size() * 2);
     if (!rc) {
         ctx->have_id = true;
         ctx->tslot_dirty = true;
@@ -1237,6 +1193,16 @@ extern "C" int gpx_upload_coeffs(gpx_ctx *ctx, const float *cE, const float *cH)
     int rc = copy_in(ctx, ctx->cE, cE, b);
     if (!rc) rc = copy_in(ctx, ctx->cH, cH, b);
     if (!rc) ctx->have_coeffs = true;
+    // Non-magnetic models (mu_r and sigma* the same everywhere, the rule in
+    // ground-penetrating radar) have one row of H coefficients: the row
+    // kernels then read no H index and look nothing up, 6 bytes a cell and
+    // step less.
+    ctx->hu = true;
+    for (int m = 1; m < ctx->desc.nmat; ++m)
+        if (memcmp(cH, cH + 5 * (size_t)m, 20) != 0) ctx->hu = false;
+    ctx->hostE.assign(cE, cE + 5 * (size_t)ctx->desc.nmat);
+    ctx->hostH.assign(cH, cH + 5 * (size_t)ctx->desc.nmat);
+    ctx->row_dirty = true;
     return rc;
 }
 
@@ -1272,7 +1238,8 @@ extern "C" int gpx_upload_dispersive(gpx_ctx *ctx, const float *dc)
     if (!rc) rc = copy_in(ctx, ctx->dispflag, flag.data(), nm);
     if (!rc) {
         ctx->have_disp = true;
-        ctx->tslot_dirty = true;
+        ctx->tslot_dirty = ctx->row_dirty = true;
+        ctx->hostdisp.swap(host);
         rc = ensure_tslots(ctx);
     }
     return rc;
@@ -1319,28 +1286,25 @@ extern "C" int gpx_add_pml(gpx_ctx *ctx, int dir, int xs, int xf, int ys, int yf
     s.order = order; s.t = t; s.d = d;
     phi_dims(0, axis, xf - xs, yf - ys, zf - zs, s.dims[0], s.dims[1]);
     phi_dims(1, axis, xf - xs, yf - ys, zf - zs, s.dims[2], s.dims[3]);
-    for (int q = 0; q < 4; ++q) {
-        size_t b = (size_t)order * s.dims[q][0] * s.dims[q][1] * s.dims[q][2] * 4;
-        GPX_TRY(dalloc(ctx, (void **)&s.phi[q], b));
+    s.ni = s.nj = 0;
+    int nk = 0;
+    for (auto &q : s.dims) {
+        s.ni = s.ni > q[0] ? s.ni : (int)q[0];
+        s.nj = s.nj > q[1] ? s.nj : (int)q[1];
+        nk = nk > q[2] ? nk : (int)q[2];
     }
+    s.nkp = (nk + 3 + 3) / 4 * 4;  // up to three floats before the first cell
     const size_t rb = (size_t)4 * order * t * 4;
-    GPX_TRY(dalloc(ctx, (void **)&s.eR, rb, false));
-    GPX_TRY(dalloc(ctx, (void **)&s.hR, rb, false));
     s.roff = (int)ctx->Rhost[0].size();
     const size_t need = (size_t)g.nmat * 5 * 4 + (ctx->Rhost[0].size() + rb / 4) * 4 +
                         (size_t)g.nmat * 3 * g.maxpoles * 2 * 4 + g.nmat;
-    if (need > (size_t)MAX_LDS_BYTES) {
-        hipFree(s.eR);
-        hipFree(s.hR);
-        for (auto &p : s.phi) hipFree(p);
-        for (auto &p : s.phin) hipFree(p);
+    if (need > (size_t)MAX_LDS_BYTES)
         return fail(ctx, GPX_ELIMIT, "gpx_add_pml: coefficient tables exceed the LDS budget");
-    }
+    s.R[0].assign(eR, eR + rb / 4);
+    s.R[1].assign(hR, hR + rb / 4);
     ctx->slabs.push_back(s);
-    Slab &ref = ctx->slabs.back();
-    int rc = copy_in(ctx, ref.eR, eR, rb);
-    if (!rc) rc = copy_in(ctx, ref.hR, hR, rb);
-    if (rc) return rc;
+    ctx->phi_dirty = ctx->row_dirty = true;
+    int rc = 0;
     ctx->Rhost[0].insert(ctx->Rhost[0].end(), eR, eR + rb / 4);
     ctx->Rhost[1].insert(ctx->Rhost[1].end(), hR, hR + rb / 4);
     for (int f = 0; f < 2; ++f) {
@@ -1497,7 +1461,8 @@ extern "C" int gpx_set_step(gpx_ctx *ctx, int fused, int tile_cells)
         return fail(ctx, GPX_EARG, "gpx_set_step: bad argument");
     ctx->fused = fused;
     ctx->tile_cells = tile_cells;
-    ctx->split_choice = -1;
+    ctx->choice = -1;
+    ctx->row_dirty = true;
     return 0;
 }
 
@@ -1507,6 +1472,7 @@ extern "C" int gpx_set_launch(gpx_ctx *ctx, int xchunk, int block)
         return fail(ctx, GPX_EARG, "gpx_set_launch: bad argument");
     ctx->xchunk = xchunk;
     ctx->block = block;
+    ctx->row_dirty = true;
     return 0;
 }
 
@@ -1518,10 +1484,10 @@ extern "C" int gpx_set_launch(gpx_ctx *ctx, int xchunk, int block)
 // half-space these beat both longer chunks and a persistent grid of resident
 // blocks by 11 %, since fewer planes are streamed at once.  Grids too small
 // to fill the GPU with such items take shorter chunks.
-static long long count_items(const gpx_ctx *ctx, bool bnd, int block, int xc, StepArgs *a, bool f3 = false)
+static long long count_items(const gpx_ctx *ctx, bool bnd, int block, int xc, StepArgs *a)
 {
-    const int *b = f3 ? ctx->box3 : ctx->box;
-    const int nframe = f3 ? ctx->nframe3 : ctx->nframe;
+    const int *b = ctx->box;
+    const int nframe = ctx->nframe;
     auto ch = [&](int len) { return len > 0 ? (len + xc - 1) / xc : 0; };
     if (!bnd) {
         const long long cells = (long long)(b[3] - b[2]) * (b[5] - b[4]);
@@ -1543,8 +1509,7 @@ static long long count_items(const gpx_ctx *ctx, bool bnd, int block, int xc, St
     return a1 + a2 + bb;
 }
 
-static void plan(const gpx_ctx *ctx, bool bnd, int resident, int block, StepArgs &a, int &grid, int fill = 0,
-                 bool f3 = false)
+static void plan(const gpx_ctx *ctx, bool bnd, int block, StepArgs &a, int &grid, int fill = 0)
 {
     const int NX1 = ctx->desc.nx + 1;
     int xc = ctx->xchunk ? ctx->xchunk : (bnd ? 4 : 6);
@@ -1553,10 +1518,9 @@ static void plan(const gpx_ctx *ctx, bool bnd, int resident, int block, StepArgs
     // `fill` blocks the GPU holds at once (on the 100^3 grid 2 planes beat 1:
     // each chunk loads one neighbour plane more).
     if (!ctx->xchunk)
-        while (xc > 2 && count_items(ctx, bnd, block, xc, nullptr, f3) < fill) --xc;
+        while (xc > 2 && count_items(ctx, bnd, block, xc, nullptr) < fill) --xc;
     a.xc = xc;
-    const long long items = count_items(ctx, bnd, block, xc, &a, f3);
-    long long g = resident > 0 && resident < items ? resident : items;
+    long long g = count_items(ctx, bnd, block, xc, &a);
     g = (g + 7) / 8 * 8;
     if (g < 8) g = 8;
     a.per_xcd = (int)(g / 8);
@@ -1575,6 +1539,7 @@ static int resident_blocks(const gpx_ctx *ctx, const void *kernel, int block, si
     return r;
 }
 
+// Box of corrected cells, profile direction and Phi strides of slab s.
 static void fill_slab_args(const gpx_ctx *ctx, int field, int s, SlabArgs &a)
 {
     const Slab &S = ctx->slabs[s];
@@ -1585,7 +1550,6 @@ static void fill_slab_args(const gpx_ctx *ctx, int field, int s, SlabArgs &a)
     for (int n = 0; n < 3; ++n) {
         a.lo[n] = st[n];
         a.hi[n] = en[n];
-        a.org[n] = st[n];
     }
     if (minus) {
         if (field == 0) {  // cells f - p, p in [0, t)
@@ -1602,16 +1566,15 @@ static void fill_slab_args(const gpx_ctx *ctx, int field, int s, SlabArgs &a)
         a.hi[axis] = st[axis] + S.t;
         a.pend = st[axis];
     }
-    const int q = field == 0 ? 0 : 2;
-    for (int n = 0; n < 3; ++n) {
-        a.d1[n] = (int)S.dims[q][n];
-        a.d2[n] = (int)S.dims[q + 1][n];
-    }
+    a.sx = S.nj * S.nkp;
+    a.sy = S.nkp;
+    a.off = (int)(S.base - (long long)a.lo[0] * a.sx - (long long)a.lo[1] * a.sy - a.lo[2] + (a.lo[2] & 3));
+    a.ostep = (uint32_t)(2 * ctx->np);
     a.t = S.t;
     a.order = S.order;
     a.d = S.d;
-    a.phi1 = a.phw1 = S.phi[q];
-    a.phi2 = a.phw2 = S.phi[q + 1];
+    a.phi1 = field == 0 ? ctx->phiE : ctx->phiH[ctx->cur];
+    a.phi2 = a.phi1 ? a.phi1 + ctx->np : nullptr;
     a.roff = S.roff;
 }
 
@@ -1619,7 +1582,7 @@ static int update_planeflags(gpx_ctx *ctx)
 {
     ctx->rare_dirty = true;  // sources or receivers may have changed
     const int NX1 = ctx->desc.nx + 1;
-    std::vector<uint32_t> pf(NX1, 0);
+    std::vector<uint32_t> pf(2 * NX1, 0);
     for (int r = 0; r < ctx->nrx; ++r) pf[ctx->rxhost[3 * r]] |= PF_RX;
     for (int s = 0; s < ctx->src[GPX_SRC_MAGNETIC].n; ++s) pf[ctx->src[GPX_SRC_MAGNETIC].host[6 * s]] |= PF_SRCH;
     for (int kind : {GPX_SRC_HERTZIAN, GPX_SRC_VOLTAGE})
@@ -1628,11 +1591,13 @@ static int update_planeflags(gpx_ctx *ctx)
         SlabArgs e, h;
         fill_slab_args(ctx, 0, (int)s, e);
         fill_slab_args(ctx, 1, (int)s, h);
+        const int dir = ctx->slabs[s].dir;
         for (int i = 0; i < NX1; ++i) {
-            if (i >= e.lo[0] && i < e.hi[0]) pf[i] |= 1u << (PF_SLAB_E + s);
-            if (i >= h.lo[0] && i < h.hi[0]) pf[i] |= 1u << (PF_SLAB_H + s);
+            if (i >= e.lo[0] && i < e.hi[0]) pf[i] |= 1u << (PF_SLAB_E + s), pf[NX1 + i] |= 1u << (PF_SLAB_E + dir);
+            if (i >= h.lo[0] && i < h.hi[0]) pf[i] |= 1u << (PF_SLAB_H + s), pf[NX1 + i] |= 1u << (PF_SLAB_H + dir);
         }
     }
+    for (int i = 0; i < NX1; ++i) pf[NX1 + i] |= pf[i] & (PF_RX | PF_SRCH | PF_SRCE);
     int rc = copy_in(ctx, ctx->planeflag, pf.data(), pf.size() * 4);
     if (rc) return rc;
 
@@ -1668,7 +1633,7 @@ static int update_planeflags(gpx_ctx *ctx)
     if (!empty) {
         for (int j = 0; j <= g.ny; ++j)
             for (int k = 0; k <= g.nz; ++k)
-                if (!(j >= lo[1] && j < hi[1] && k >= lo[2] && k < hi[2])) fr.push_back(j * (g.nz + 1) + k);
+                if (!(j >= lo[1] && j < hi[1] && k >= lo[2] && k < hi[2])) fr.push_back(j * ctx->kp + k);
     }
     if (ctx->frame) { hipFree(ctx->frame); ctx->frame = nullptr; }
     ctx->nframe = (int)fr.size();
@@ -1677,45 +1642,22 @@ static int update_planeflags(gpx_ctx *ctx)
         rc = copy_in(ctx, ctx->frame, fr.data(), fr.size() * 4);
         if (rc) return rc;
     }
-    // The split step's fused box: one more plane, row and column off on the
-    // minus sides, so that the neighbours its kernel recomputes are interior
-    // cells.  Empty when the interior box is too thin.
-    {
-        const int *b = ctx->box;
-        const bool ok = !empty && b[0] + 1 < b[1] && b[2] + 1 < b[3] && b[4] + 1 < b[5];
-        const int b3[6] = {ok ? b[0] + 1 : g.nx + 1, ok ? b[1] : g.nx + 1, ok ? b[2] + 1 : 0, ok ? b[3] : 0,
-                           ok ? b[4] + 1 : 0, ok ? b[5] : 0};
-        memcpy(ctx->box3, b3, sizeof(b3));
-        std::vector<int> f3;
-        if (ok)
-            for (int j = 0; j <= g.ny; ++j)
-                for (int k = 0; k <= g.nz; ++k)
-                    if (!(j >= b3[2] && j < b3[3] && k >= b3[4] && k < b3[5])) f3.push_back(j * (g.nz + 1) + k);
-        if (ctx->frame3) { hipFree(ctx->frame3); ctx->frame3 = nullptr; }
-        ctx->nframe3 = (int)f3.size();
-        if (!f3.empty()) {
-            GPX_TRY(dalloc(ctx, (void **)&ctx->frame3, f3.size() * 4, false));
-            rc = copy_in(ctx, ctx->frame3, f3.data(), f3.size() * 4);
-        }
-    }
+    const int *b = ctx->box;
+    ctx->deep = !empty && b[0] + 1 < b[1] && b[2] + 1 < b[3] && b[4] + 1 < b[5];
+    ctx->row_dirty = true;
     return rc;
 }
 
-// f3: the boundary passes of the split step, around the fused box, from the
-// current state into the next: the H pass reads E and H from F and writes H
-// to Fn; the E pass reads E from F and the new H from Fn and writes E to Fn.
-static void base_args(const gpx_ctx *ctx, int field, StepArgs &a, int &block, size_t &lds, bool f3 = false)
+static void base_args(const gpx_ctx *ctx, int field, StepArgs &a, int &block, size_t &lds)
 {
     block = ctx->block ? ctx->block : 256;
     memset(&a, 0, sizeof(a));
     const gpx_desc &g = ctx->desc;
     a.nx = g.nx; a.ny = g.ny; a.nz = g.nz;
+    a.kp = ctx->kp;
     a.plane = ctx->plane;
-    float *const *hin = (f3 && field == 0) ? ctx->Fn : ctx->F;
-    a.Ex = ctx->F[0]; a.Ey = ctx->F[1]; a.Ez = ctx->F[2];
-    a.Hx = hin[3]; a.Hy = hin[4]; a.Hz = hin[5];
-    float *const *out = f3 ? ctx->Fn : ctx->F;
-    for (int c = 0; c < 3; ++c) a.So[c] = out[field == 0 ? c : 3 + c];
+    a.Ex = ctx->field(0); a.Ey = ctx->field(1); a.Ez = ctx->field(2);
+    a.Hx = ctx->field(3); a.Hy = ctx->field(4); a.Hz = ctx->field(5);
     a.ID = ctx->ID;
     a.ntot = ctx->ntot;
     a.nmat = g.nmat;
@@ -1724,9 +1666,9 @@ static void base_args(const gpx_ctx *ctx, int field, StepArgs &a, int &block, si
     a.nR = (int)ctx->Rhost[0].size();
     a.form = g.pml_formulation;
     a.planeflag = ctx->planeflag;
-    memcpy(a.box, f3 ? ctx->box3 : ctx->box, sizeof(a.box));
-    a.frame = f3 ? ctx->frame3 : ctx->frame;
-    a.nframe = f3 ? ctx->nframe3 : ctx->nframe;
+    memcpy(a.box, ctx->box, sizeof(a.box));
+    a.frame = ctx->frame;
+    a.nframe = ctx->nframe;
     a.iterations = g.iterations;
     a.nslab = (int)ctx->slabs.size();
     for (int s = 0; s < a.nslab; ++s) fill_slab_args(ctx, field, s, a.slab[s]);
@@ -1751,18 +1693,16 @@ static void base_args(const gpx_ctx *ctx, int field, StepArgs &a, int &block, si
 
 typedef void (*pass_kernel)(StepArgs);
 
-// `share` < 1 plans the kernel for that fraction of the resident blocks, so
-// that another kernel can run beside it.
 static hipError_t launch_kernel(const gpx_ctx *ctx, pass_kernel kernel, bool bnd, int field, int flags, int it,
-                                hipStream_t stream = nullptr, bool f3 = false)
+                                hipStream_t stream = nullptr)
 {
     StepArgs a;
     int block, grid;
     size_t lds;
-    base_args(ctx, field, a, block, lds, f3);
-    if (count_items(ctx, bnd, block, 1, nullptr, f3) <= 0) return hipSuccess;
+    base_args(ctx, field, a, block, lds);
+    if (count_items(ctx, bnd, block, 1, nullptr) <= 0) return hipSuccess;
     const int fill = resident_blocks(ctx, (const void *)kernel, block, lds);
-    plan(ctx, bnd, 0, block, a, grid, fill, f3);   // one block per item
+    plan(ctx, bnd, block, a, grid, fill);   // one block per item
     a.flags = flags;
     a.it = it;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds, stream ? stream : ctx->stream, a);
@@ -1863,78 +1803,14 @@ static hipError_t launch_pass_overlap(gpx_ctx *ctx, int field, int flags, int it
     return hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0);
 }
 
-template <class IDT>
-static pass_kernel e_merged(int P, bool C)
-{
-    switch (P) {
-    case 0: return k_e_merged<IDT, 0, false>;
-    case 1: return C ? k_e_merged<IDT, 1, true> : k_e_merged<IDT, 1, false>;
-    case 2: return C ? k_e_merged<IDT, 2, true> : k_e_merged<IDT, 2, false>;
-    case 3: return C ? k_e_merged<IDT, 3, true> : k_e_merged<IDT, 3, false>;
-    default: return C ? k_e_merged<IDT, 4, true> : k_e_merged<IDT, 4, false>;
-    }
-}
-
-static pass_kernel pick_merged(const gpx_ctx *ctx, int field)
-{
-    if (field == 1) return k_h_merged<uint16_t>;
-    const int P = ctx->desc.maxpoles;
-    const bool C = ctx->disp_complex != 0;
-    return e_merged<uint16_t>(P, C);
-}
-
-// Items of the merged pass with chunks of xc planes (both kinds), and the
-// map's fields of `a` when given.
-static long long count_merged(const gpx_ctx *ctx, int block, int xc, StepArgs *a)
-{
-    StepArgs t;
-    StepArgs &q = a ? *a : t;
-    const long long ni = count_items(ctx, false, block, xc, &q);
-    const long long nb = count_items(ctx, true, block, xc, &q);
-    const int len = ctx->box[1] - ctx->box[0];
-    q.m_nchunk = len > 0 ? (len + xc - 1) / xc : 0;
-    q.m_items = (int)(ni + nb);
-    q.nitems = 1 << 30;
-    if (ni == 0) q.nseg = 0;  // an empty box: no interior item in any chunk
-    return ni + nb;
-}
-
-// One pass as one launch over every cell (form 6).
-static hipError_t launch_merged(const gpx_ctx *ctx, int field, int flags, int it)
-{
-    StepArgs a;
-    int block;
-    size_t lds;
-    base_args(ctx, field, a, block, lds);
-    const pass_kernel kernel = pick_merged(ctx, field);
-    const int NX1 = ctx->desc.nx + 1;
-    int xc = ctx->xchunk ? ctx->xchunk : 4;
-    if (xc > NX1) xc = NX1;
-    if (!ctx->xchunk) {
-        const int fill = resident_blocks(ctx, (const void *)kernel, block, lds);
-        while (xc > 2 && count_merged(ctx, block, xc, nullptr) < fill) --xc;
-    }
-    a.xc = xc;
-    const long long items = count_merged(ctx, block, xc, &a);
-    if (items <= 0) return hipSuccess;
-    const long long g = (items + 7) / 8 * 8;
-    a.per_xcd = (int)(g / 8);
-    a.flags = flags;
-    a.it = it;
-    hipLaunchKernelGGL(kernel, dim3((unsigned int)g), dim3(block), lds, ctx->stream, a);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------- fused step
-constexpr int STEP_LDS_MAX = 64 * 1024;
-
-// The fused kernels are compiled in step_*.hip, one file per PML form.
+// ---------------------------------------------------------------- row kernels
+// The row kernels are compiled in step_*.hip, one file per PML form.
 namespace gpx {
-StepKernels step_kernel_plain(int id_bytes, int P, bool C);
-StepKernels step_kernel_hori1(int id_bytes, int P, bool C);
-StepKernels step_kernel_hori2(int id_bytes, int P, bool C);
-StepKernels step_kernel_mri1(int id_bytes, int P, bool C);
-StepKernels step_kernel_mri2(int id_bytes, int P, bool C);
+RowKernels row_kernel_plain(int P, bool C, bool hu);
+RowKernels row_kernel_hori1(int P, bool C, bool hu);
+RowKernels row_kernel_hori2(int P, bool C, bool hu);
+RowKernels row_kernel_mri1(int P, bool C, bool hu);
+RowKernels row_kernel_mri2(int P, bool C, bool hu);
 }  // namespace gpx
 
 // PML order shared by every slab, 0 without slabs, -1 when they differ.
@@ -1948,123 +1824,357 @@ static int slab_order(const gpx_ctx *ctx)
     return o;
 }
 
-static StepKernels pick_step(const gpx_ctx *ctx)
+static RowKernels row_kernels(const gpx_ctx *ctx)
 {
-    const int P = ctx->desc.maxpoles, idb = ctx->id_bytes;
-    const bool C = ctx->disp_complex != 0;
+    const int P = ctx->desc.maxpoles;
+    const bool C = ctx->disp_complex != 0, hu = ctx->hu;
     const int o = slab_order(ctx);
-    if (o == 0) return step_kernel_plain(idb, P, C);
-    if (ctx->desc.pml_formulation == 0)
-        return o == 1 ? step_kernel_hori1(idb, P, C) : step_kernel_hori2(idb, P, C);
-    return o == 1 ? step_kernel_mri1(idb, P, C) : step_kernel_mri2(idb, P, C);
+    if (o <= 0) return row_kernel_plain(P, C, hu);
+    if (ctx->desc.pml_formulation == 0) return o == 1 ? row_kernel_hori1(P, C, hu) : row_kernel_hori2(P, C, hu);
+    return o == 1 ? row_kernel_mri1(P, C, hu) : row_kernel_mri2(P, C, hu);
 }
 
-// LDS of the fused step besides the H exchange area: both coefficient
-// tables, both R tables, dispersive coefficients and flags.
-static size_t step_table_lds(const gpx_ctx *ctx)
+// Floats of dispersive coefficients and of one field's profile tables.
+static int disp_floats(const gpx_ctx *ctx)
 {
+    return ctx->desc.maxpoles > 0 ? ctx->desc.nmat * 3 * ctx->desc.maxpoles * (ctx->disp_complex ? 2 : 1) : 0;
+}
+static int profile_floats(const gpx_ctx *ctx)
+{
+    int n = 0;
+    const int o = slab_order(ctx);
+    for (const Slab &S : ctx->slabs) n += S.t * row_entry(ctx->desc.pml_formulation, o);
+    return n;
+}
+
+// Floats of a field's tables, and dynamic LDS of the one-launch step with
+// blocks of B threads and of a pass.
+static int image_floats(const gpx_ctx *ctx, int field)
+{
+    return field == 0 ? row_image(ctx->desc.nmat, profile_floats(ctx), disp_floats(ctx))
+                      : row_image(ctx->hu ? 0 : ctx->desc.nmat, profile_floats(ctx), 0);
+}
+static size_t step_lds(const gpx_ctx *ctx, int B)
+{
+    return (size_t)(image_floats(ctx, 0) + image_floats(ctx, 1)) * 4 + (size_t)B * (NC * 16 + 8);
+}
+static size_t pass_lds(const gpx_ctx *ctx, int field) { return (size_t)image_floats(ctx, field) * 4 + 16; }
+
+// Models the row kernels take: rows of whole lanes, one PML order for all
+// slabs, slabs given in the order x0, y0, z0, xmax, ymax, zmax (the kernels
+// apply them so; any may be missing) that do not overlap the one opposite, with
+// cell sizes row_quot takes, 32-bit byte offsets into a whole state, the indices
+// and the Phi arrays, and tables that leave room in LDS.  Others take the
+// general passes.
+static bool rows_ok(const gpx_ctx *ctx)
+{
+    const int o = slab_order(ctx);
+    if (ctx->kp % 4 != 0 || o < 0) return false;
+    double np = 0;
+    int before = -1, end[2][3];
+    for (auto &f : end)
+        for (int &e : f) e = -1;
+    for (size_t s = 0; s < ctx->slabs.size(); ++s) {
+        const Slab &S = ctx->slabs[s];
+        if (S.dir <= before || !(S.d > 1e-12f && S.d < 1.6e7f)) return false;
+        before = S.dir;
+        np += (double)S.ni * S.nj * S.nkp;
+        for (int f = 0; f < 2; ++f) {
+            SlabArgs a;
+            fill_slab_args(ctx, f, (int)s, a);
+            const int u = a.axis == 2 ? NC : 1;   // nor share a lane
+            int &e = end[f][a.axis];
+            if (a.lo[a.axis] / u < e) return false;
+            e = (a.hi[a.axis] + u - 1) / u;
+        }
+    }
+    if ((double)ctx->fstride * 24.0 >= 4294967295.0 || (double)ctx->ntot * 12.0 >= 4294967295.0 ||
+        np * 8.0 * (o > 0 ? o : 1) >= 2147483647.0)
+        return false;
+    return pass_lds(ctx, 0) <= (size_t)MAX_LDS_BYTES && pass_lds(ctx, 1) <= (size_t)MAX_LDS_BYTES;
+}
+
+// Threads per block of the one-launch step: 0 when it cannot run.
+static int step_block(const gpx_ctx *ctx)
+{
+    if (!rows_ok(ctx) || !ctx->tls.empty()) return 0;
+    auto ok = [&](int B) { return B >= 128 && B <= ROW_BLOCK_MAX && step_lds(ctx, B) <= (size_t)MAX_LDS_BYTES; };
+    if (ctx->fused == 1 && ctx->tile_cells) return ok(ctx->tile_cells / NC) ? ctx->tile_cells / NC : 0;
+    for (int B : {ROW_BLOCK_MAX, 256, 128})
+        if (ok(B)) return B;
+    return 0;
+}
+
+// Lanes at the start and at the end of a row with a cell in a z slab.
+static void z_lanes(const gpx_ctx *ctx, int &za, int &zb)
+{
+    const int lpr = ctx->kp / NC;
+    za = zb = 0;
+    for (size_t s = 0; s < ctx->slabs.size(); ++s)
+        for (int f = 0; f < 2; ++f) {
+            SlabArgs a;
+            fill_slab_args(ctx, f, (int)s, a);
+            if (ctx->slabs[s].dir == 2) za = std::max(za, (a.hi[2] + NC - 1) / NC);
+            if (ctx->slabs[s].dir == 5) zb = std::max(zb, lpr - a.lo[2] / NC);
+        }
+    if (za + zb > lpr) zb = lpr - za;
+}
+
+// Tiles and x chunks of the one-launch step with blocks of B threads.
+static void row_tiles(const gpx_ctx *ctx, int B, int xchunk, RowModel &m)
+{
+    const int lpr = ctx->kp / NC, ny1 = ctx->desc.ny + 1, nx1 = ctx->desc.nx + 1;
+    // Rows longer than ROW_LANES_MAX lanes are split, each part with one lane
+    // of the part before it.
+    // Short enough that two rows fit with the z lanes apart.
+    const int most = std::min((B - 63) / 2, ROW_LANES_MAX);
+    m.ntk = lpr <= most ? 1 : (lpr + most - 2) / (most - 1);
+    m.hk = m.ntk > 1;
+    m.LTo = (lpr + m.ntk - 1) / m.ntk;
+    m.LT = m.LTo + m.hk;
+    z_lanes(ctx, m.za, m.zb);
+    // in lanes of the first and of the last part, the lanes past a row's start
+    // and end among them
+    const int last = lpr - (m.ntk - 1) * m.LTo + m.hk;
+    m.za = std::min(m.za + m.hk, m.LT);
+    m.zb = std::min(m.zb, last - m.hk) + m.LT - last;
+    if (m.ntk == 1) m.zb = std::min(m.zb, m.LT - m.za);
+    // rows: as many as fit with the z lanes from a whole wave on
+    auto need = [&](int R) {
+        int most_t = 0;
+        for (int tk : {0, 1, m.ntk - 1}) {
+            if (tk >= m.ntk) continue;
+            const int z = (tk == 0 ? m.za : 0) + (tk == m.ntk - 1 ? m.zb : 0);
+            most_t = std::max(most_t, (R * (m.LT - z) + 63) / 64 * 64 + R * z);
+        }
+        return most_t;
+    };
+    m.R = B / m.LT;
+    while (m.R > 1 && need(m.R) > B) --m.R;
+    if (m.R >= ny1) {  // the plane in one row of tiles
+        m.R = m.Ro = ny1;
+        m.hj = 0;
+    } else {
+        m.hj = 1;
+        m.Ro = m.R - 1;
+    }
+    m.ntj = (ny1 + m.Ro - 1) / m.Ro;
+    m.xc = xchunk < 1 ? 1 : (xchunk > nx1 ? nx1 : xchunk);
+    m.nitems = m.ntk * m.ntj * ((nx1 + m.xc - 1) / m.xc);
+    m.threads = (need(m.R) + 63) / 64 * 64;
+}
+
+static int resident_blocks(const gpx_ctx *ctx, const void *kernel, int block, size_t lds);
+
+// The launch shape of the one-launch step.
+static void plan_step(const gpx_ctx *ctx, RowModel &m, int &B)
+{
+    B = step_block(ctx);
+    int xc = ctx->xchunk ? ctx->xchunk : 4;
+    row_tiles(ctx, B, xc, m);
+    // Small grids: shorter chunks (a chunk also computes H of the plane before
+    // it) and smaller blocks, until the items fill the GPU.
+    const int fill = 2 * (ctx->cus > 0 ? ctx->cus : 256);
+    const bool fixed = ctx->fused == 1 && ctx->tile_cells;
+    while (!fixed && B > 128 && m.nitems < fill && 2 * m.LT <= B / 2) row_tiles(ctx, B /= 2, xc, m);
+    while (!ctx->xchunk && xc > 2 && m.nitems < fill) row_tiles(ctx, B, --xc, m);
+    if (m.threads < B && !fixed) B = m.threads;  // no idle waves
+}
+
+// One slab for the row kernels, and its profile entries (row_corr's order).
+static void row_slab_args(const gpx_ctx *ctx, int field, int s, RowSlab &r)
+{
+    SlabArgs a;
+    fill_slab_args(ctx, field, s, a);
+    r.pend = a.pend;
+    r.sign = a.minus ? -1 : 1;
+    r.t = a.t;
+    memcpy(r.lo, a.lo, sizeof(r.lo));
+    memcpy(r.hi, a.hi, sizeof(r.hi));
+    r.off = a.off;
+    r.sx = a.sx;
+    r.sy = a.sy;
+    r.d = a.d;
+    r.rd = (float)(1.0 / (double)a.d);
+    r.rl = (float)(1.0 / (double)a.d - (double)r.rd);
+    r.rt = 0;
+}
+
+static void row_profile(const gpx_ctx *ctx, int field, int s, float *out)
+{
+    const Slab &S = ctx->slabs[s];
+    const int t = S.t, form = ctx->desc.pml_formulation, ne = row_entry(form, S.order), ot = S.order * t;
+    const float *R = S.R[field].data();
+    for (int p = 0; p < t; ++p) {
+        float *e = out + (size_t)p * ne;
+        for (int n = 0; n < ne; ++n) e[n] = 0.f;
+        const float A0 = R[p], B0 = R[ot + p], E0 = R[2 * ot + p], F0 = R[3 * ot + p];
+        if (S.order == 1) {
+            if (form == 0) {
+                e[0] = A0 - 1.0f; e[1] = B0; e[2] = E0; e[3] = F0;
+            } else {
+                const float IRA = 1.0f / A0;
+                e[0] = IRA - 1.0f; e[1] = IRA; e[2] = E0; e[3] = IRA * B0 * F0;
+            }
+            continue;
+        }
+        const float A1 = R[t + p], B1 = R[ot + t + p], E1 = R[2 * ot + t + p], F1 = R[3 * ot + t + p];
+        if (form == 0) {
+            e[0] = A0 * A1 - 1.0f; e[1] = A1 * B0; e[2] = B1; e[3] = A0; e[4] = B0; e[5] = E0; e[6] = F0; e[7] = E1; e[8] = F1;
+        } else {
+            const float IRA = 1.0f / (A0 + A1);
+            e[0] = IRA - 1.0f; e[1] = IRA; e[2] = B0; e[3] = B1; e[4] = E0; e[5] = E1; e[6] = IRA * F0; e[7] = IRA * F1;
+        }
+    }
+}
+
+static hipError_t upload_rare(gpx_ctx *ctx);
+
+// Threads per block of the row passes.
+static int pass_block(const gpx_ctx *ctx)
+{
+    const int b = ctx->block ? ctx->block : 256;
+    return b < ROW_PASS_MAX ? b : ROW_PASS_MAX;
+}
+
+// Items of the row passes: one lane per NC cells, blocks of B lanes of a plane,
+// chunks of xc planes.  Chunks are short: a longer one re-reads fewer planes
+// of the field it differences along x, but that plane is still in the
+// last-level cache, and the longer the chunks the fewer blocks there are and the
+// longer each one's chain of planes (300x300x200, HORIPML, us per iteration: 353
+// in chunks of 1, 349 of 2, 350 of 4, 377 of 10; 100x100x100: 23.1, 22.5, 27.7).
+// The dispersive E pass, with its auxiliary values, has more to wait for per
+// plane and gains from keeping H of the plane before in registers (240x240x180,
+// 3 poles: 360, 331, 326 in chunks of 1, 2, 4).
+static void pass_items(const gpx_ctx *ctx, int B, int xc, RowModel &m)
+{
+    const int lanes = (ctx->desc.ny + 1) * (ctx->kp / NC), nx1 = ctx->desc.nx + 1;
+    m.pxc = xc > nx1 ? nx1 : xc;
+    m.pseg = (lanes + B - 1) / B;
+    m.pitems = m.pseg * ((nx1 + m.pxc - 1) / m.pxc);
+}
+static int pass_chunk(const gpx_ctx *ctx) { return ctx->desc.maxpoles > 0 ? 4 : 2; }
+// Below this many items shorter chunks: blocks for every compute unit four times over (a
+// 120x105 2-D model: 8.6 us per iteration in chunks of 1, 11.4 of 2, 16.8 of 4).
+static int pass_fill(const gpx_ctx *ctx) { return 4 * (ctx->cus > 0 ? ctx->cus : 256); }
+
+// Brings the device's description of the model up to date (waits when it has
+// changed).
+static int ensure_row(gpx_ctx *ctx)
+{
+    if (ctx->rare_dirty || !ctx->rare) GPX_TRY(upload_rare(ctx));
+    if (!ctx->row_dirty) return 0;
     const gpx_desc &g = ctx->desc;
-    size_t b = (size_t)g.nmat * 40 + 2 * ctx->Rhost[0].size() * 4;
-    if (g.maxpoles > 0) b += (size_t)g.nmat * 3 * g.maxpoles * 4 * (ctx->disp_complex ? 2 : 1) + g.nmat;
+    const int o = slab_order(ctx);
+    // the tables as they lie in LDS, and the slabs
+    RowModel &m = ctx->rowh;
+    memset(&m, 0, sizeof(m));
+    const int nRT = profile_floats(ctx), nE = image_floats(ctx, 0), nH = image_floats(ctx, 1);
+    std::vector<float> img((size_t)nE + nH, 0.f);
+    for (int f = 0; f < 2; ++f) {
+        const std::vector<float> &c = f ? ctx->hostH : ctx->hostE;
+        const int nm = f && ctx->hu ? 0 : g.nmat;
+        float *at = img.data() + (f ? nE : 0), *rt = at + 4 * nm, *sl = rt + nRT, *c5 = sl;
+        if (nRT) c5 += 6 * sizeof(RowSlab) / 4;
+        for (int n = 0; n < nm; ++n) {
+            memcpy(at + 4 * n, &c[5 * (size_t)n], 16);
+            c5[n] = c[5 * (size_t)n + 4];
+        }
+        if (!f && g.maxpoles > 0) memcpy(c5 + nm, ctx->hostdisp.data(), ctx->hostdisp.size() * 4);
+        int first = 0;
+        for (size_t s = 0; s < ctx->slabs.size(); ++s) {
+            const int dir = ctx->slabs[s].dir;
+            RowSlab d;
+            row_slab_args(ctx, f, (int)s, d);
+            d.rt = first;
+            memcpy(sl + dir * (sizeof(RowSlab) / 4), &d, sizeof(d));
+            const RowAt w = {d.lo[1], d.hi[1], d.lo[2], d.hi[2], d.off, d.sx, d.sy, 0};
+            (f ? m.atH : m.atE)[dir] = w;
+            row_profile(ctx, f, (int)s, rt + first);
+            first += ctx->slabs[s].t * row_entry(g.pml_formulation, o);
+        }
+    }
+    if (nE + nH > ctx->nimg) {
+        if (ctx->img) hipFree(ctx->img);
+        ctx->img = nullptr;
+        ctx->nimg = 0;
+        GPX_TRY(dalloc(ctx, (void **)&ctx->img, img.size() * 4, false));
+        ctx->nimg = nE + nH;
+    }
+    if (int rc = copy_in(ctx, ctx->img, img.data(), img.size() * 4)) return rc;
+    m.nx = g.nx; m.ny = g.ny; m.nz = g.nz;
+    m.kp = ctx->kp;
+    m.plane = ctx->plane;
+    int B = 0;
+    if (step_block(ctx)) plan_step(ctx, m, B);
+    ctx->row_block = B;
+    int xc = ctx->xchunk ? ctx->xchunk : pass_chunk(ctx);
+    pass_items(ctx, pass_block(ctx), xc, m);
+    while (!ctx->xchunk && xc > 1 && m.pitems < pass_fill(ctx)) pass_items(ctx, pass_block(ctx), --xc, m);
+    m.F[0] = ctx->Fmem[0];
+    m.F[1] = ctx->Fmem[1];
+    m.cs = (uint32_t)(ctx->fstride * 4);
+    m.ci = (uint32_t)(ctx->ntot * 2);
+    m.ID = ctx->ID;
+    m.img = reinterpret_cast<const float4 *>(ctx->img);
+    m.n4E = nE / 4;
+    m.n4H = nH / 4;
+    m.nmat = g.nmat;
+    for (int n = 0; n < 5 && ctx->hu; ++n) m.h[n] = ctx->hostH[n];
+    m.nRT = nRT;
+    m.phiE = ctx->phiE;
+    m.phiH[0] = ctx->phiH[0];
+    m.phiH[1] = ctx->phiH[1];
+    m.np4 = (uint32_t)(ctx->np * 4);
+    if (g.maxpoles > 0) fill_targs(ctx, m.T);
+    m.iterations = g.iterations;
+    m.rare = ctx->rare;
+    m.planeflag = ctx->planeflag + g.nx + 1;
+    if (!ctx->row) GPX_TRY(dalloc(ctx, (void **)&ctx->row, sizeof(RowModel), false));
+    if (int rc = copy_in(ctx, ctx->row, &m, sizeof(m))) return rc;
+    ctx->row_dirty = false;
+    return 0;
+}
+
+static RowArgs row_args(const gpx_ctx *ctx, int nitems, int it)
+{
+    RowArgs b;
+    b.item0 = nullptr;
+    b.ntr = 1;
+    b.nitems = nitems;
+    b.per_xcd = (nitems + 7) / 8;
+    b.flip = ctx->cur;
+    b.it = it;
     return b;
 }
 
-static size_t step_lds(const gpx_ctx *ctx, int tc) { return step_table_lds(ctx) + (size_t)12 * tc + 16; }
-
-// Cells per fused block (threads x STEP_CELLS_PER_THREAD): the smallest of
-// 512, 1024 and 2048 whose halo of nz+1 cells is at most an eighth of it, else
-// the largest whose halo is at most half; 0 when none fits the LDS budget, and
-// then the two-pass kernels run instead.
-static int step_tile(const gpx_ctx *ctx)
+// One iteration in one launch; then the next state is the current one.
+static hipError_t launch_row_step(gpx_ctx *ctx, int it)
 {
-    if (ctx->fused != 1 || slab_order(ctx) < 0 || !ctx->tls.empty()) return 0;
-    const int NZ1 = ctx->desc.nz + 1;
-    // Streamed offsets are 32-bit: a state of six components and the six
-    // index arrays must each stay below 4 GiB.
-    if ((double)ctx->fstride * 24.0 >= 4294967295.0 || (double)ctx->ntot * 6 * ctx->id_bytes >= 4294967295.0)
-        return 0;
-    auto ok = [&](int tc) { return step_lds(ctx, tc) <= (size_t)STEP_LDS_MAX && 2 * NZ1 <= tc; };
-    if (ctx->tile_cells) return ok(ctx->tile_cells) ? ctx->tile_cells : 0;
-    int best = 0;
-    for (int tc : {256, 512, 1024}) {
-        if (!ok(tc)) continue;
-        best = tc;
-        if (8 * NZ1 <= tc) break;
-    }
-    return best;
+    const RowArgs b = row_args(ctx, ctx->rowh.nitems, it);
+    hipLaunchKernelGGL(row_kernels(ctx).step, dim3(8 * b.per_xcd), dim3(ctx->row_block), step_lds(ctx, ctx->row_block),
+                       ctx->stream, ctx->row, b);
+    ctx->cur ^= 1;
+    return hipGetLastError();
 }
 
-static void fill_step_args(const gpx_ctx *ctx, int tc, int it, FusedArgs &a)
+// The H (field 1) or E pass in one launch.
+static hipError_t launch_row_pass(const gpx_ctx *ctx, int field, int it)
 {
-    memset(&a, 0, sizeof(a));
-    const gpx_desc &g = ctx->desc;
-    a.nx = g.nx; a.ny = g.ny; a.nz = g.nz;
-    a.plane = ctx->plane;
-    a.L = tc - (g.nz + 1);
-    a.ntiles = (ctx->plane + a.L - 1) / a.L;
-    a.Fc = ctx->F[0];
-    a.Fx = ctx->Fn[0];
-    a.cs = (uint32_t)(ctx->fstride * 4);
-    a.ID = ctx->ID;
-    a.ntot = ctx->ntot;
-    a.coefE = ctx->cE;
-    a.coefH = ctx->cH;
-    a.RE = ctx->Rall[0];
-    a.RH = ctx->Rall[1];
-    a.nR = (int)ctx->Rhost[0].size();
-    if (g.maxpoles > 0) {
-        a.disp = ctx->disp;
-        a.dispflag = ctx->dispflag;
-        fill_targs(ctx, a.T);
-    }
-    a.nmat = g.nmat;
-    a.form = g.pml_formulation;
-    a.nslab = (int)ctx->slabs.size();
-    for (int s = 0; s < a.nslab; ++s) {
-        fill_slab_args(ctx, 0, s, a.slabE[s]);
-        fill_slab_args(ctx, 1, s, a.slabH[s]);
-        a.slabH[s].phw1 = ctx->slabs[s].phin[0];
-        a.slabH[s].phw2 = ctx->slabs[s].phin[1];
-    }
-    a.it = it;
-    a.iterations = g.iterations;
-    a.rare = ctx->rare;
-    a.planeflag = ctx->planeflag;
+    const RowArgs b = row_args(ctx, ctx->rowh.pitems, it);
+    const RowKernels k = row_kernels(ctx);
+    hipLaunchKernelGGL(field == 1 ? k.h : k.e, dim3(8 * b.per_xcd), dim3(pass_block(ctx)), pass_lds(ctx, field),
+                       ctx->stream, ctx->row, b);
+    return hipGetLastError();
 }
 
-// Items are (tile, x chunk); each chunk also recomputes H on the plane before
-// it.  Unless fixed by gpx_set_launch, the chunk length minimises
-// rounds x (planes per item), preferring longer chunks on ties.
-static void plan_step(const gpx_ctx *ctx, int resident, FusedArgs &a, int &grid)
-{
-    const int NX1 = ctx->desc.nx + 1;
-    int xc = ctx->xchunk;
-    if (!xc) {
-        long long best = -1;
-        for (int c = 2; c <= NX1; ++c) {
-            const long long items = (long long)a.ntiles * ((NX1 + c - 1) / c);
-            const long long cost = (items + resident - 1) / resident * (long long)(c + 1);
-            if (best < 0 || cost <= best) {
-                best = cost;
-                xc = c;
-            }
-        }
-    }
-    a.xc = xc;
-    a.nitems = a.ntiles * ((NX1 + xc - 1) / xc);
-    long long g = resident < a.nitems ? resident : a.nitems;
-    g = (g + 7) / 8 * 8;
-    a.per_xcd = (int)(g / 8);
-    grid = (int)g;
-}
-
-// One fused iteration, then the next state becomes the current one.
-// Copies the source and receiver tables of the fused step to the device.
+// Copies the source and receiver tables of the row kernels to the device.
 static hipError_t upload_rare(gpx_ctx *ctx)
 {
     if (!ctx->rare) {
         hipError_t e = dalloc(ctx, (void **)&ctx->rare, sizeof(StepRare), false);
         if (e != hipSuccess) return e;
+        ctx->row_dirty = true;
     }
     StepRare r;
     memset(&r, 0, sizeof(r));
@@ -2084,164 +2194,37 @@ static hipError_t upload_rare(gpx_ctx *ctx)
     return e;
 }
 
-static hipError_t launch_step(gpx_ctx *ctx, int tc, int it)
-{
-    if (ctx->rare_dirty || !ctx->rare) {
-        hipError_t e = upload_rare(ctx);
-        if (e != hipSuccess) return e;
-    }
-    FusedArgs a;
-    fill_step_args(ctx, tc, it, a);
-    const step_kernel k = pick_step(ctx).one;
-    const int B = tc / STEP_CELLS_PER_THREAD;
-    const size_t lds = step_lds(ctx, tc);
-    int grid;
-    plan_step(ctx, resident_blocks(ctx, (const void *)k, B, lds), a, grid);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(B), lds, ctx->stream, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    for (int c = 0; c < 6; ++c) std::swap(ctx->F[c], ctx->Fn[c]);
-    for (auto &S : ctx->slabs) {
-        std::swap(S.phi[2], S.phin[0]);
-        std::swap(S.phi[3], S.phin[1]);
-    }
-    return hipSuccess;
-}
-
-// The split step (form 3): the fused interior kernel over the fused box and
-// the boundary H and E passes around it, from the current state into the
-// next.  It needs no dispersive poles (the fused kernel has no auxiliary
-// values), a nonempty fused box and 32-bit buffer offsets.
+// ---------------------------------------------------------------- step forms
+// Models forms 3, 5 and 7 are reported for: no dispersive poles, no lines, and
+// a 3-D grid with an interior.
 static bool split_eligible(const gpx_ctx *ctx)
 {
-    if (ctx->desc.maxpoles > 0 || !ctx->tls.empty()) return false;
-    const int *b = ctx->box3;
-    if (b[0] >= b[1] || b[2] >= b[3] || b[4] >= b[5]) return false;
-    return (double)ctx->fstride * 24.0 < 4294967295.0 && (double)ctx->ntot * 6 * ctx->id_bytes < 4294967295.0;
+    return ctx->desc.maxpoles == 0 && ctx->deep && step_block(ctx) > 0;
 }
 
-static bool split_ok(const gpx_ctx *ctx)
+// The rule of form 4: models without slabs and poles take the one-launch step,
+// which reads and writes 54 bytes a cell where the two passes take 78; in the
+// slabs its chain of dependent work per plane (H, a barrier, E) costs more than
+// that saves (300x300x200: 386 us an iteration against 349 with 10 cells of PML
+// on each side, 285 against 300 without).
+static bool one_launch(const gpx_ctx *ctx)
 {
-    if (ctx->fused == 3 || ctx->fused == 5 || ctx->fused == 7) return split_eligible(ctx);
-    const int c = ctx->split_choice;
-    return ctx->fused == 4 && (c == -1 || c == 1 || c == 2 || c == 5) && split_eligible(ctx);
+    return ctx->slabs.empty() && ctx->desc.maxpoles == 0 && step_block(ctx) > 0;
 }
 
-// Form 7, or form 4 after it chose form 7 (with split_ok).
-static bool split_merged(const gpx_ctx *ctx)
-{
-    return ctx->fused == 7 || (ctx->fused == 4 && ctx->split_choice == 5);
-}
+// What gpx_run does with the model: STEP (one launch), PASSES (two row
+// passes), GENERAL (the general passes), BESIDE (form 2).
+enum RunKind { RUN_STEP, RUN_PASSES, RUN_GENERAL, RUN_BESIDE };
 
-// Form 5, or form 4 after it chose form 5 (with split_ok).
-static bool split_beside(const gpx_ctx *ctx)
+static RunKind run_kind(const gpx_ctx *ctx)
 {
-    return ctx->fused == 5 || (ctx->fused == 4 && ctx->split_choice == 2);
-}
-
-// Form 2, or form 4 after it chose form 2 (when neither the fused step nor
-// the split step runs).
-static bool passes_beside(const gpx_ctx *ctx)
-{
-    return ctx->fused == 2 || (ctx->fused == 4 && ctx->split_choice == 3);
-}
-
-// Form 6, or form 4 after it chose form 6 (when neither the fused step nor
-// the split step runs).
-static bool passes_merged(const gpx_ctx *ctx)
-{
-    return ctx->fused == 6 || (ctx->fused == 4 && ctx->split_choice == 4);
-}
-
-// The interior kernel's arguments except its chunk length and item counts.
-static void interior_args(const gpx_ctx *ctx, int it, IntArgs &a)
-{
-    memset(&a, 0, sizeof(a));
-    const gpx_desc &g = ctx->desc;
-    a.nx = g.nx; a.ny = g.ny; a.nz = g.nz;
-    a.plane = ctx->plane;
-    memcpy(a.box, ctx->box3, sizeof(a.box));
-    const long long cells = (long long)(a.box[3] - a.box[2]) * (a.box[5] - a.box[4]);
-    a.nseg = (int)((cells + INT_BLOCK - 1) / INT_BLOCK);
-    a.Fc = ctx->F[0];
-    a.Fx = ctx->Fn[0];
-    a.cs = (uint32_t)(ctx->fstride * 4);
-    a.ID = ctx->ID;
-    a.ntot = ctx->ntot;
-    a.coefE = ctx->cE;
-    a.coefH = ctx->cH;
-    a.nmat = g.nmat;
-    a.it = it;
-    a.iterations = g.iterations;
-    const SrcSet &M = ctx->src[GPX_SRC_MAGNETIC], &V = ctx->src[GPX_SRC_VOLTAGE], &D = ctx->src[GPX_SRC_HERTZIAN];
-    a.srcM = {M.n, M.info, M.fac, M.waves};
-    a.srcV = {V.n, V.info, V.fac, V.waves};
-    a.srcD = {D.n, D.info, D.fac, D.waves};
-    a.nrx = ctx->nrx;
-    a.rxc = ctx->rxc;
-    a.rxbuf = ctx->rxbuf;
-    a.planeflag = ctx->planeflag;
-}
-
-static hipError_t launch_interior(const gpx_ctx *ctx, int it)
-{
-    IntArgs a;
-    interior_args(ctx, it, a);
-    const int B = INT_BLOCK;
-    const int nxb = a.box[1] - a.box[0];
-    const void *k = (const void *)k_interior<uint16_t>;
-    const size_t lds = (size_t)ctx->desc.nmat * 40;
-    int xc = ctx->xchunk ? ctx->xchunk : 4;
-    if (!ctx->xchunk) {
-        const int fill = resident_blocks(ctx, k, B, lds);
-        while (xc > 2 && (long long)a.nseg * ((nxb + xc - 1) / xc) < fill) --xc;
+    const RunKind passes = rows_ok(ctx) ? RUN_PASSES : RUN_GENERAL;
+    switch (ctx->fused) {
+    case 1: return step_block(ctx) ? RUN_STEP : passes;
+    case 2: return RUN_BESIDE;
+    case 0: case 6: return passes;
+    default: return one_launch(ctx) ? RUN_STEP : passes;   // 3, 5, 7 and 4
     }
-    if (xc > nxb) xc = nxb;
-    a.xc = xc;
-    a.nitems = a.nseg * ((nxb + xc - 1) / xc);
-    const int grid = (a.nitems + 7) / 8 * 8;
-    a.per_xcd = grid / 8;
-    hipLaunchKernelGGL(k_interior<uint16_t>, dim3(grid), dim3(B), lds, ctx->stream, a);
-    return hipGetLastError();
-}
-
-// Form 7: the interior kernel and the H boundary pass of the split step as
-// one launch (k_interior_hb), both with chunks of xc planes.
-static hipError_t launch_interior_hb(const gpx_ctx *ctx, int hflags, int it)
-{
-    IntArgs a;
-    interior_args(ctx, it, a);
-    StepArgs hb;
-    int block;
-    size_t lds_b;
-    base_args(ctx, 1, hb, block, lds_b, true);
-    const int nxb = a.box[1] - a.box[0];
-    const void *k = (const void *)k_interior_hb<uint16_t>;
-    const size_t lds_i = (size_t)ctx->desc.nmat * 40;
-    const size_t lds = lds_i > lds_b ? lds_i : lds_b;
-    auto total = [&](int xc) {
-        return (long long)a.nseg * ((nxb + xc - 1) / xc) + count_items(ctx, true, INT_BLOCK, xc, nullptr, true);
-    };
-    int xc = ctx->xchunk ? ctx->xchunk : 4;
-    if (!ctx->xchunk) {
-        const int fill = resident_blocks(ctx, k, INT_BLOCK, lds);
-        while (xc > 2 && total(xc) < fill) --xc;
-    }
-    if (xc > nxb) xc = nxb;
-    a.xc = xc;
-    a.nitems = a.nseg * ((nxb + xc - 1) / xc);
-    const long long nb = count_items(ctx, true, INT_BLOCK, xc, &hb, true);
-    hb.xc = xc;
-    hb.nseg = a.nseg;
-    hb.m_nchunk = (nxb + xc - 1) / xc;
-    hb.m_items = (int)(a.nitems + nb);
-    hb.nitems = 1 << 30;
-    const int grid = (hb.m_items + 7) / 8 * 8;
-    hb.per_xcd = grid / 8;
-    hb.flags = hflags;
-    hb.it = it;
-    hipLaunchKernelGGL(k_interior_hb<uint16_t>, dim3(grid), dim3(INT_BLOCK), lds, ctx->stream, a, hb);
-    return hipGetLastError();
 }
 
 static hipError_t launch_snapshot(const gpx_ctx *ctx, int s)
@@ -2250,9 +2233,9 @@ static hipError_t launch_snapshot(const gpx_ctx *ctx, int s)
     const long long n = (long long)S.snx * S.sny * S.snz;
     const int block = 256;
     const int grid = (int)((n + block - 1) / block);
-    hipLaunchKernelGGL(k_snapshot, dim3(grid), dim3(block), 0, ctx->stream, ctx->desc.ny, ctx->desc.nz,
-                       S.xs, S.ys, S.zs, S.dx, S.dy, S.dz, S.snx, S.sny, S.snz, ctx->F[0], ctx->F[1],
-                       ctx->F[2], ctx->F[3], ctx->F[4], ctx->F[5], S.out);
+    hipLaunchKernelGGL(k_snapshot, dim3(grid), dim3(block), 0, ctx->stream, ctx->desc.ny, ctx->kp,
+                       S.xs, S.ys, S.zs, S.dx, S.dy, S.dz, S.snx, S.sny, S.snz, ctx->field(0),
+                       ctx->field(1), ctx->field(2), ctx->field(3), ctx->field(4), ctx->field(5), S.out);
     return hipGetLastError();
 }
 
@@ -2264,11 +2247,11 @@ static hipError_t launch_tl(const gpx_ctx *ctx, int field, int it)
     const int B = 64, grid = (n + B - 1) / B;
     const gpx_desc &g = ctx->desc;
     if (field == 1)
-        hipLaunchKernelGGL(k_tl_h, dim3(grid), dim3(B), 0, ctx->stream, ctx->tldev, n, it, g.ny, g.nz, ctx->F[3],
-                           ctx->F[4], ctx->F[5]);
+        hipLaunchKernelGGL(k_tl_h, dim3(grid), dim3(B), 0, ctx->stream, ctx->tldev, n, it, g.ny, ctx->kp,
+                           ctx->field(3), ctx->field(4), ctx->field(5));
     else
-        hipLaunchKernelGGL(k_tl_e, dim3(grid), dim3(B), 0, ctx->stream, ctx->tldev, n, it, g.ny, g.nz, ctx->F[0],
-                           ctx->F[1], ctx->F[2]);
+        hipLaunchKernelGGL(k_tl_e, dim3(grid), dim3(B), 0, ctx->stream, ctx->tldev, n, it, g.ny, ctx->kp,
+                           ctx->field(0), ctx->field(1), ctx->field(2));
     return hipGetLastError();
 }
 
@@ -2317,6 +2300,7 @@ static int check_ready(gpx_ctx *ctx)
     if (ctx->desc.maxpoles > 0 && !ctx->have_disp)
         return fail(ctx, GPX_ESTATE, "dispersive coefficients must be uploaded before stepping");
     if (int rc = ensure_tslots(ctx)) return rc;
+    if (int rc = ensure_phi(ctx)) return rc;
     return check_tls(ctx);
 }
 
@@ -2346,78 +2330,23 @@ struct EventSet {
 
 // Runs iterations [it0, it0+n) in the step form set by gpx_set_step.  With
 // `ms4`, events around every kernel give the mean duration of each kernel of
-// an iteration over the run: the fused kernel in ms4[0] (the rest 0); the
-// split step's interior, H boundary and E boundary kernels in ms4[0], [1]
-// and [3]; or H interior, H boundary, E interior and E boundary.
-static int run_steps_form(gpx_ctx *ctx, int it0, int n, float *ms4);
-
-// Form 4 picks among forms 7, 6, 2, 5, the split step and the passes (forms
-// 6, 2 and the passes only, where the split step does not apply) on the
-// first run long enough to time them: after two warm-up iterations, TUNE_ITS
-// iterations of each, timed with events; the fastest serves the rest of
-// this run and later runs.  The forms give the same bits, so the choice does
-// not change results.
-static const int TUNE_ITS = 4;
+// an iteration over the run: the one-launch step in ms4[0] (the rest 0); the
+// row passes in ms4[0] and ms4[2]; or H interior, H boundary, E interior and
+// E boundary of the general passes.  Form 4 settles on its first run of at
+// least CHOOSE_ITS iterations.
+static const int CHOOSE_ITS = 26;
 
 static int run_steps(gpx_ctx *ctx, int it0, int n, float *ms4)
 {
-    if (ms4 || ctx->fused != 4 || ctx->split_choice != -1 || step_tile(ctx) || n < 2 + 6 * TUNE_ITS)
-        return run_steps_form(ctx, it0, n, ms4);
-    // choices in the order timed: form 7, form 6, form 2, form 5, the split step, the passes
-    static const int all[6] = {5, 4, 3, 2, 1, 0}, passes_only[3] = {4, 3, 0};
-    const bool split = split_eligible(ctx);
-    const int *order = split ? all : passes_only;
-    const int nf = split ? 6 : 3;
-    // TUNE_ITS iterations per form, in two rounds over the forms, so that
-    // no form is timed only early or only late in the run.
-    const int half = TUNE_ITS / 2, rounds = 2;
-    EventSet ev;
-    ev.e.assign(rounds * nf + 1, nullptr);
-    for (auto &x : ev.e) GPX_TRY(hipEventCreate(&x));
-    ctx->split_choice = order[0];
-    int rc = run_steps_form(ctx, it0, 2, nullptr);
-    for (int q = 0; q < rounds * nf && !rc; ++q) {
-        ctx->split_choice = order[q % nf];
-        rc = check_hip(ctx, hipEventRecord(ev.e[q], ctx->stream));
-        if (!rc) rc = run_steps_form(ctx, it0 + 2 + q * half, half, nullptr);
-    }
-    if (!rc) rc = check_hip(ctx, hipEventRecord(ev.e[rounds * nf], ctx->stream));
-    if (!rc) rc = check_hip(ctx, hipEventSynchronize(ev.e[rounds * nf]));
-    int best = 0;
-    float t_best = 0;
-    for (int f = 0; f < nf && !rc; ++f) {
-        float t = 0;
-        for (int r = 0; r < rounds && !rc; ++r) {
-            float tq = 0;
-            const int q = r * nf + f;
-            rc = check_hip(ctx, hipEventElapsedTime(&tq, ev.e[q], ev.e[q + 1]));
-            t += tq;
-        }
-        if (!rc && (f == 0 || t < t_best)) {
-            best = f;
-            t_best = t;
-        }
-    }
-    if (rc) {
-        ctx->split_choice = -1;
-        return rc;
-    }
-    ctx->split_choice = order[best];
-    // the passes, alone, side by side or merged, update in place
-    if (order[best] == 0 || order[best] == 3 || order[best] == 4)
-        if ((rc = release_next_state(ctx))) return rc;
-    const int done = 2 + nf * TUNE_ITS;
-    return run_steps_form(ctx, it0 + done, n - done, nullptr);
-}
-
-
-static int run_steps_form(gpx_ctx *ctx, int it0, int n, float *ms4)
-{
+    if (!ms4 && ctx->fused == 4 && ctx->choice == -1 && n >= CHOOSE_ITS)
+        ctx->choice = one_launch(ctx) ? 5 : 4;
     const int hf = h_flags(ctx), ef = e_flags(ctx);
-    const int tc = step_tile(ctx);
-    const bool split = !tc && split_ok(ctx);
-    if (n > 0 && (tc || split))
-        if (int rc = ensure_next_state(ctx, tc != 0)) return rc;
+    const RunKind kind = run_kind(ctx);
+    const bool rows = kind == RUN_STEP || kind == RUN_PASSES;
+    if (n > 0 && kind == RUN_STEP)
+        if (int rc = ensure_next_state(ctx)) return rc;
+    if (n > 0 && rows)
+        if (int rc = ensure_row(ctx)) return rc;
     // With ms4, six events per iteration are recorded around the kernels and
     // read once at the end, so the host never waits between iterations and
     // the gaps between events are the kernels' own.
@@ -2431,66 +2360,26 @@ static int run_steps_form(gpx_ctx *ctx, int it0, int n, float *ms4)
         hipEvent_t *ev = ms4 ? &evs.e[(size_t)(it - it0) * per] : nullptr;
         for (size_t s = 0; s < ctx->snaps.size(); ++s)
             if (ctx->snaps[s].time == it + 1) GPX_TRY(launch_snapshot(ctx, (int)s));
-        if (tc) {
+        if (kind == RUN_STEP) {
             if (ev) GPX_TRY(hipEventRecord(ev[0], ctx->stream));
-            GPX_TRY(launch_step(ctx, tc, it));
+            GPX_TRY(launch_row_step(ctx, it));
             if (ev) GPX_TRY(hipEventRecord(ev[1], ctx->stream));
             continue;
         }
-        if (split && !ev && split_beside(ctx)) {
-            // Form 5: the H boundary pass reads only the current state and
-            // writes only boundary cells, Phi and receiver samples of boundary
-            // cells, so it runs beside the interior kernel on the second
-            // stream; the E boundary pass waits for both.  (Runs with timing
-            // events take the order of form 3.)
-            GPX_TRY(ensure_stream2(ctx));
-            GPX_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
-            GPX_TRY(hipStreamWaitEvent(ctx->stream2, ctx->ev_fork, 0));
-            GPX_TRY(launch_kernel(ctx, pick_kernel<true>(ctx, 1), true, 1, hf, it, ctx->stream2, true));
-            GPX_TRY(hipEventRecord(ctx->ev_join, ctx->stream2));
-            GPX_TRY(launch_interior(ctx, it));
-            GPX_TRY(hipStreamWaitEvent(ctx->stream, ctx->ev_join, 0));
-            GPX_TRY(launch_kernel(ctx, pick_kernel<true>(ctx, 0), true, 0, ef, it, nullptr, true));
-            for (int c = 0; c < 6; ++c) std::swap(ctx->F[c], ctx->Fn[c]);
-            continue;
-        }
-        if (split && split_merged(ctx)) {
-            // events: the merged launch between ev[0] and ev[1] (ev[2] right
-            // after), the E boundary pass between ev[2] and ev[3]
-            if (ev) GPX_TRY(hipEventRecord(ev[0], ctx->stream));
-            GPX_TRY(launch_interior_hb(ctx, hf, it));
-            if (ev) GPX_TRY(hipEventRecord(ev[1], ctx->stream));
-            if (ev) GPX_TRY(hipEventRecord(ev[2], ctx->stream));
-            GPX_TRY(launch_kernel(ctx, pick_kernel<true>(ctx, 0), true, 0, ef, it, nullptr, true));
-            if (ev) GPX_TRY(hipEventRecord(ev[3], ctx->stream));
-            for (int c = 0; c < 6; ++c) std::swap(ctx->F[c], ctx->Fn[c]);
-            continue;
-        }
-        if (split) {
-            if (ev) GPX_TRY(hipEventRecord(ev[0], ctx->stream));
-            GPX_TRY(launch_interior(ctx, it));
-            if (ev) GPX_TRY(hipEventRecord(ev[1], ctx->stream));
-            GPX_TRY(launch_kernel(ctx, pick_kernel<true>(ctx, 1), true, 1, hf, it, nullptr, true));
-            if (ev) GPX_TRY(hipEventRecord(ev[2], ctx->stream));
-            GPX_TRY(launch_kernel(ctx, pick_kernel<true>(ctx, 0), true, 0, ef, it, nullptr, true));
-            if (ev) GPX_TRY(hipEventRecord(ev[3], ctx->stream));
-            for (int c = 0; c < 6; ++c) std::swap(ctx->F[c], ctx->Fn[c]);
-            continue;
-        }
-        if (passes_merged(ctx)) {
+        if (kind == RUN_PASSES) {
             // events: the H pass between ev[0] and ev[1], the E pass between
             // ev[3] and ev[4]
             if (ev) GPX_TRY(hipEventRecord(ev[0], ctx->stream));
-            GPX_TRY(launch_merged(ctx, 1, hf, it));
+            GPX_TRY(launch_row_pass(ctx, 1, it));
             if (ev) GPX_TRY(hipEventRecord(ev[1], ctx->stream));
             GPX_TRY(launch_tl(ctx, 1, it));
             if (ev) GPX_TRY(hipEventRecord(ev[3], ctx->stream));
-            GPX_TRY(launch_merged(ctx, 0, ef, it));
+            GPX_TRY(launch_row_pass(ctx, 0, it));
             if (ev) GPX_TRY(hipEventRecord(ev[4], ctx->stream));
             GPX_TRY(launch_tl(ctx, 0, it));
             continue;
         }
-        if (passes_beside(ctx) && !ms4) {
+        if (kind == RUN_BESIDE && !ms4) {
             GPX_TRY(launch_pass_overlap(ctx, 1, hf, it));
             GPX_TRY(launch_tl(ctx, 1, it));
             GPX_TRY(launch_pass_overlap(ctx, 0, ef, it));
@@ -2505,14 +2394,12 @@ static int run_steps_form(gpx_ctx *ctx, int it0, int n, float *ms4)
     if (ms4) {
         double acc[4] = {0, 0, 0, 0};
         GPX_TRY(hipStreamSynchronize(ctx->stream));
-        // (begin, end) event pairs of each kernel slot: fused step; split
-        // step (interior, H boundary, -, E boundary); passes (H interior, H
-        // boundary, E interior, E boundary)
-        static const int pairs[4][4][2] = {{{0, 1}, {-1, -1}, {-1, -1}, {-1, -1}},
-                                           {{0, 1}, {1, 2}, {-1, -1}, {2, 3}},
-                                           {{0, 1}, {1, 2}, {3, 4}, {4, 5}},
-                                           {{0, 1}, {-1, -1}, {3, 4}, {-1, -1}}};
-        const int form = tc ? 0 : (split ? 1 : (passes_merged(ctx) ? 3 : 2));
+        // (begin, end) event pairs of each kernel slot: the step; the row
+        // passes; H interior, H boundary, E interior, E boundary
+        static const int pairs[3][4][2] = {{{0, 1}, {-1, -1}, {-1, -1}, {-1, -1}},
+                                           {{0, 1}, {-1, -1}, {3, 4}, {-1, -1}},
+                                           {{0, 1}, {1, 2}, {3, 4}, {4, 5}}};
+        const int form = kind == RUN_STEP ? 0 : (kind == RUN_PASSES ? 1 : 2);
         for (int i = 0; i < n; ++i) {
             hipEvent_t *ev = &evs.e[(size_t)i * per];
             for (int q = 0; q < 4; ++q) {
@@ -2530,22 +2417,25 @@ static int run_steps_form(gpx_ctx *ctx, int it0, int n, float *ms4)
 
 extern "C" int gpx_step_kind(const gpx_ctx *ctx)
 {
-    return ctx ? step_tile(ctx) : 0;
+    return ctx && ctx->fused == 1 ? step_block(ctx) * NC : 0;
 }
 
 extern "C" int gpx_step_form(const gpx_ctx *ctx)
 {
     if (!ctx) return GPX_EARG;
-    if (step_tile(ctx)) return 1;
-    if (split_ok(ctx)) return split_beside(ctx) ? 5 : (split_merged(ctx) ? 7 : 3);
-    if (passes_merged(ctx)) return 6;
-    return passes_beside(ctx) ? 2 : 0;
+    switch (ctx->fused) {
+    case 1: return step_block(ctx) ? 1 : 0;
+    case 2: case 6: return ctx->fused;
+    case 3: case 5: case 7: return split_eligible(ctx) ? ctx->fused : 0;
+    case 4: return ctx->choice == 5 ? 7 : (ctx->choice == 4 ? 6 : (split_eligible(ctx) ? 3 : 0));
+    default: return 0;
+    }
 }
 
 extern "C" int gpx_step_choice(const gpx_ctx *ctx)
 {
     if (!ctx) return GPX_EARG;
-    return ctx->split_choice;
+    return ctx->choice;
 }
 
 extern "C" int gpx_run(gpx_ctx *ctx, int it0, int n)
@@ -2639,55 +2529,101 @@ extern "C" int gpx_download_rx(gpx_ctx *ctx, float *out)
     return copy_out(ctx, out, ctx->rxbuf, (size_t)6 * ctx->desc.iterations * ctx->nrx * 4);
 }
 
+// A component between the reference's layout on the host and the padded rows
+// of the device.
+static int rows_transfer(gpx_ctx *ctx, float *dev, float *host, bool up)
+{
+    const gpx_desc &g = ctx->desc;
+    const size_t rows = (size_t)(g.nx + 1) * (g.ny + 1), nk = (size_t)g.nz + 1, kp = (size_t)ctx->kp;
+    if (nk == kp) return up ? copy_in(ctx, dev, host, rows * nk * 4) : copy_out(ctx, host, dev, rows * nk * 4);
+    std::vector<float> t(rows * kp, 0.f);
+    if (!up)
+        if (int rc = copy_out(ctx, t.data(), dev, t.size() * 4)) return rc;
+    for (size_t r = 0; r < rows; ++r) {
+        if (up) memcpy(t.data() + r * kp, host + r * nk, nk * 4);
+        else memcpy(host + r * nk, t.data() + r * kp, nk * 4);
+    }
+    return up ? copy_in(ctx, dev, t.data(), t.size() * 4) : 0;
+}
+
 extern "C" int gpx_download_fields(gpx_ctx *ctx, float *out6)
 {
     if (!ctx || !out6) return fail(ctx, GPX_EARG, "gpx_download_fields: null argument");
+    const gpx_desc &g = ctx->desc;
+    const size_t pts = (size_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
     for (int c = 0; c < 6; ++c)
-        if (int rc = copy_out(ctx, out6 + (size_t)c * ctx->ntot, ctx->F[c], (size_t)ctx->ntot * 4)) return rc;
+        if (int rc = rows_transfer(ctx, ctx->field(c), out6 + (size_t)c * pts, false)) return rc;
     return 0;
 }
 
 extern "C" int gpx_upload_fields(gpx_ctx *ctx, const float *in6)
 {
     if (!ctx || !in6) return fail(ctx, GPX_EARG, "gpx_upload_fields: null argument");
+    const gpx_desc &g = ctx->desc;
+    const size_t pts = (size_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
     // Both states, where there are two: cells that no update touches keep
     // their value in either.
-    for (int c = 0; c < 6; ++c) {
-        if (int rc = copy_in(ctx, ctx->F[c], in6 + (size_t)c * ctx->ntot, (size_t)ctx->ntot * 4)) return rc;
-        if (ctx->Fn[c])
-            if (int rc = copy_in(ctx, ctx->Fn[c], in6 + (size_t)c * ctx->ntot, (size_t)ctx->ntot * 4)) return rc;
+    for (int c = 0; c < 6; ++c)
+        for (float *m : ctx->Fmem)
+            if (m)
+                if (int rc = rows_transfer(ctx, m + c * ctx->fstride, const_cast<float *>(in6) + (size_t)c * pts, true)) return rc;
+    return 0;
+}
+
+// Phi `which` (EPhi1, EPhi2, HPhi1, HPhi2) of a slab between the reference's
+// layout on the host and the device's (see Slab); H Phi goes up into both
+// copies.
+static int phi_transfer(gpx_ctx *ctx, int slab, int which, float *host, bool up)
+{
+    const Slab &S = ctx->slabs[slab];
+    const int field = which < 2 ? 0 : 1, w = which & 1, axis = S.dir % 3;
+    SlabArgs a;
+    fill_slab_args(ctx, field, slab, a);
+    const int kofs = a.lo[2] & 3;
+    const long long *d = S.dims[which];
+    const size_t block = (size_t)S.ni * S.nj * S.nkp;
+    std::vector<float> t(block);
+    float *arrays[2] = {field == 0 ? ctx->phiE : ctx->phiH[ctx->cur], nullptr};
+    if (up && field == 1) arrays[1] = ctx->phiH[ctx->cur ^ 1];
+    for (int o = 0; o < S.order; ++o) {
+        const size_t at = (size_t)(2 * o + w) * ctx->np + S.base;
+        if (int rc = copy_out(ctx, t.data(), arrays[0] + at, block * 4)) return rc;
+        for (long long i = 0; i < d[0]; ++i)
+            for (long long j = 0; j < d[1]; ++j)
+                for (long long k = 0; k < d[2]; ++k) {
+                    long long c[3] = {i, j, k};
+                    if (S.dir < 3 && c[axis] < S.t) c[axis] = S.t - 1 - c[axis];
+                    float &v = t[((size_t)c[0] * S.nj + c[1]) * S.nkp + c[2] + kofs];
+                    float &h = host[(((size_t)o * d[0] + i) * d[1] + j) * d[2] + k];
+                    if (up) v = h;
+                    else h = v;
+                }
+        for (float *m : arrays)
+            if (up && m)
+                if (int rc = copy_in(ctx, m + at, t.data(), block * 4)) return rc;
     }
     return 0;
 }
 
-static int phi_ref(gpx_ctx *ctx, int slab, int which, float **p, size_t *bytes)
+static int phi_check(gpx_ctx *ctx, int slab, int which)
 {
     if (slab < 0 || slab >= (int)ctx->slabs.size() || which < 0 || which > 3)
         return fail(ctx, GPX_EARG, "bad slab or Phi index");
-    const Slab &s = ctx->slabs[slab];
-    *p = s.phi[which];
-    *bytes = (size_t)s.order * s.dims[which][0] * s.dims[which][1] * s.dims[which][2] * 4;
-    return 0;
+    return ensure_phi(ctx);
 }
 
 extern "C" int gpx_download_pml_phi(gpx_ctx *ctx, int slab, int which, float *out)
 {
     if (!ctx || !out) return fail(ctx, GPX_EARG, "gpx_download_pml_phi: null argument");
-    float *p;
-    size_t b;
-    if (int rc = phi_ref(ctx, slab, which, &p, &b)) return rc;
-    return copy_out(ctx, out, p, b);
+    if (int rc = phi_check(ctx, slab, which)) return rc;
+    return phi_transfer(ctx, slab, which, out, false);
 }
 
 extern "C" int gpx_upload_pml_phi(gpx_ctx *ctx, int slab, int which, const float *in)
 {
     if (!ctx || !in) return fail(ctx, GPX_EARG, "gpx_upload_pml_phi: null argument");
-    float *p;
-    size_t b;
-    if (int rc = phi_ref(ctx, slab, which, &p, &b)) return rc;
-    if (which >= 2 && ctx->slabs[slab].phin[which - 2])  // H Phi, double-buffered for the fused step
-        if (int rc = copy_in(ctx, ctx->slabs[slab].phin[which - 2], in, b)) return rc;
-    return copy_in(ctx, p, in, b);
+    if (int rc = phi_check(ctx, slab, which)) return rc;
+    return phi_transfer(ctx, slab, which, const_cast<float *>(in), true);
 }
 
 // T in the reference's layout, complex64 [3][P][ntot]; edges without poles
@@ -2700,7 +2636,8 @@ extern "C" int gpx_download_dispersive_T(gpx_ctx *ctx, float *out)
     if (int rc = ensure_tslots(ctx)) return rc;
     if (ctx->tslot_dirty || !ctx->T[0]) return fail(ctx, GPX_ESTATE, "gpx_download_dispersive_T: no dispersive state");
     const size_t N = (size_t)ctx->ntot, w = ctx->disp_complex ? 2 : 1;
-    std::fill(out, out + (size_t)3 * P * N * 2, 0.0f);
+    const size_t nk = (size_t)ctx->desc.nz + 1, kp = (size_t)ctx->kp, pts = N / kp * nk;
+    std::fill(out, out + (size_t)3 * P * pts * 2, 0.0f);
     std::vector<uint32_t> slot(N);
     for (int c = 0; c < 3; ++c) {
         const size_t n = (size_t)ctx->tn[c];
@@ -2709,9 +2646,10 @@ extern "C" int gpx_download_dispersive_T(gpx_ctx *ctx, float *out)
         if (int rc = copy_out(ctx, t.data(), ctx->T[c], t.size() * 4)) return rc;
         for (size_t e = 0; e < N; ++e) {
             const uint32_t s = slot[e];
-            if (s == 0xffffffffu) continue;
+            if (s == 0xffffffffu || e % kp >= nk) continue;  // no poles, or padding
+            const size_t h = e / kp * nk + e % kp;
             for (int p = 0; p < P; ++p) {
-                float *o = out + (((size_t)c * P + p) * N + e) * 2;
+                float *o = out + (((size_t)c * P + p) * pts + h) * 2;
                 o[0] = t[((size_t)p * n + s) * w];
                 if (w == 2) o[1] = t[((size_t)p * n + s) * w + 1];
             }
@@ -2729,6 +2667,7 @@ extern "C" int gpx_upload_dispersive_T(gpx_ctx *ctx, const float *in)
     if (ctx->tslot_dirty || !ctx->T[0])
         return fail(ctx, GPX_ESTATE, "gpx_upload_dispersive_T: upload the indices and dispersive tables first");
     const size_t N = (size_t)ctx->ntot, w = ctx->disp_complex ? 2 : 1;
+    const size_t nk = (size_t)ctx->desc.nz + 1, kp = (size_t)ctx->kp, pts = N / kp * nk;
     std::vector<uint32_t> slot(N);
     for (int c = 0; c < 3; ++c) {
         const size_t n = (size_t)ctx->tn[c];
@@ -2736,9 +2675,10 @@ extern "C" int gpx_upload_dispersive_T(gpx_ctx *ctx, const float *in)
         if (int rc = copy_out(ctx, slot.data(), ctx->tslot[c], N * 4)) return rc;
         for (size_t e = 0; e < N; ++e) {
             const uint32_t s = slot[e];
-            if (s == 0xffffffffu) continue;
+            if (s == 0xffffffffu || e % kp >= nk) continue;  // no poles, or padding
+            const size_t h = e / kp * nk + e % kp;
             for (int p = 0; p < P; ++p) {
-                const float *v = in + (((size_t)c * P + p) * N + e) * 2;
+                const float *v = in + (((size_t)c * P + p) * pts + h) * 2;
                 if (w == 1 && v[1] != 0.0f)
                     return fail(ctx, GPX_EARG, "gpx_upload_dispersive_T: imaginary part in a real-pole model");
                 t[((size_t)p * n + s) * w] = v[0];
@@ -2806,19 +2746,18 @@ extern "C" size_t gpx_memory_bytes(const gpx_ctx *ctx)
 }
 
 // ====================================================================== batch
-// Many models advanced together: one launch of the fused step per iteration
-// covers the work items of every model, optionally all iterations captured in
-// one HIP graph.  Each model keeps its own gpx_ctx (buffers, sources,
-// receivers); the batch only holds the launch tables.
+// Many models advanced together: one launch of the one-launch step per
+// iteration covers the work items of every model of a group, optionally all
+// iterations captured in one HIP graph.  Each model keeps its own gpx_ctx
+// (buffers, sources, receivers); the batch only holds the launch tables.
 struct gpx_batch {
     std::vector<gpx_ctx *> ctx;
     int device = 0;
     hipStream_t stream = nullptr;
-    int tile = 0, xchunk = 0;      // fused-step tile and chunk; tile 0 = the H and E passes
-    bool fused_ok = false;         // every model can take the same fused step
-    double group_bytes = 192.0 * 1024 * 1024;  // state bytes per group of models (passes)
-    FusedArgs *dargs = nullptr;    // [2][ntr]
-    int *ditem0 = nullptr;         // [ntr + 1]
+    int tile = 0, xchunk = 0;      // cells per block and chunk of the step; tile 0 = planned, in groups
+    double group_bytes = 192.0 * 1024 * 1024;  // state bytes per group of models
+    RowModel *dmodels = nullptr;   // [ntr]
+    int *ditem0 = nullptr;         // each group's first item per model: [ntr + groups]
     StepArgs *dpass = nullptr;     // [4][ntr]: H interior, H boundary, E interior, E boundary
     int *dpitem = nullptr;         // [4][ntr + groups]: each group's first item per model
     std::string err;
@@ -2842,17 +2781,42 @@ extern "C" const char *gpx_batch_last_error(const gpx_batch *b)
     return b ? b->err.c_str() : g_err.c_str();
 }
 
+// Whether models [g0, g0 + gn) all take the row passes with the same kernels.
+static bool batch_passes(const gpx_batch *b, int g0, int gn)
+{
+    const RowKernels k = row_kernels(b->ctx[g0]);
+    for (int t = g0; t < g0 + gn; ++t) {
+        const RowKernels q = row_kernels(b->ctx[t]);
+        if (!rows_ok(b->ctx[t]) || q.h != k.h || q.e != k.e) return false;
+    }
+    return true;
+}
+
+// Whether models [g0, g0 + gn) all take the one-launch step with one kernel.
+static bool batch_rows(const gpx_batch *b, int g0, int gn)
+{
+    for (int t = g0; t < g0 + gn; ++t)
+        if (!step_block(b->ctx[t]) || row_kernels(b->ctx[t]).step != row_kernels(b->ctx[g0]).step) return false;
+    return true;
+}
+
+// Whether form 4 would take the one-launch step for all of them.
+static bool batch_plain(const gpx_batch *b, int g0, int gn)
+{
+    for (int t = g0; t < g0 + gn; ++t)
+        if (!one_launch(b->ctx[t])) return false;
+    return true;
+}
+
 // Tile sizes every model of the batch accepts, smallest first.
 static std::vector<int> batch_tiles(const gpx_batch *b)
 {
     std::vector<int> out;
-    if (!b->fused_ok) return out;
+    if (!batch_rows(b, 0, (int)b->ctx.size())) return out;
     for (int tc : {256, 512, 1024}) {
-        bool ok = true;
-        for (const gpx_ctx *c : b->ctx) {
-            const int NZ1 = c->desc.nz + 1;
-            if (step_lds(c, tc) > (size_t)STEP_LDS_MAX || 2 * NZ1 > tc) ok = false;
-        }
+        bool ok = tc / NC <= ROW_BLOCK_MAX;
+        for (const gpx_ctx *c : b->ctx)
+            if (step_lds(c, tc / NC) > (size_t)MAX_LDS_BYTES) ok = false;
         if (ok) out.push_back(tc);
     }
     return out;
@@ -2877,25 +2841,18 @@ extern "C" int gpx_batch_create(gpx_ctx *const *ctxs, int n, gpx_batch **out)
             return bfail(nullptr, GPX_EARG, "gpx_batch_create: all models must have the same number of iterations");
         if (!c->snaps.empty())
             return bfail(nullptr, GPX_EARG, "gpx_batch_create: models with snapshots are stepped one by one");
-        if (c->id_bytes != c0->id_bytes || c->desc.maxpoles != c0->desc.maxpoles ||
+        if (c->desc.maxpoles != c0->desc.maxpoles ||
             c->disp_complex != c0->disp_complex || c->desc.pml_formulation != c0->desc.pml_formulation)
-            return bfail(nullptr, GPX_EARG, "gpx_batch_create: all models need the same kernel (index width, "
+            return bfail(nullptr, GPX_EARG, "gpx_batch_create: all models need the same kernel ("
                                             "poles and their kind, PML formulation)");
     }
     gpx_batch *b = new gpx_batch();
     b->ctx.assign(ctxs, ctxs + n);
     b->device = c0->desc.device;
-    // The fused step as a second choice: every model eligible, one kernel.
-    b->fused_ok = true;
-    for (gpx_ctx *c : b->ctx)
-        if (slab_order(c) < 0 || (double)c->fstride * 24.0 >= 4294967295.0 ||
-            (double)c->ntot * 6 * c->id_bytes >= 4294967295.0 || pick_step(c).many != pick_step(c0).many)
-            b->fused_ok = false;
-    if (b->fused_ok && batch_tiles(b).empty()) b->fused_ok = false;
     hipSetDevice(b->device);
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc((void **)&b->dargs, sizeof(FusedArgs) * 2 * n);
-    if (e == hipSuccess) e = hipMalloc((void **)&b->ditem0, sizeof(int) * (n + 1));
+    if (e == hipSuccess) e = hipMalloc((void **)&b->dmodels, sizeof(RowModel) * n);
+    if (e == hipSuccess) e = hipMalloc((void **)&b->ditem0, sizeof(int) * 2 * n);
     if (e == hipSuccess) e = hipMalloc((void **)&b->dpass, sizeof(StepArgs) * 4 * n);
     if (e == hipSuccess) e = hipMalloc((void **)&b->dpitem, sizeof(int) * 4 * (2 * n));
     if (e != hipSuccess) {
@@ -2912,7 +2869,7 @@ extern "C" int gpx_batch_destroy(gpx_batch *b)
     if (!b) return 0;
     hipSetDevice(b->device);
     if (b->stream) hipStreamSynchronize(b->stream);
-    if (b->dargs) hipFree(b->dargs);
+    if (b->dmodels) hipFree(b->dmodels);
     if (b->ditem0) hipFree(b->ditem0);
     if (b->dpass) hipFree(b->dpass);
     if (b->dpitem) hipFree(b->dpitem);
@@ -2924,7 +2881,7 @@ extern "C" int gpx_batch_destroy(gpx_batch *b)
 extern "C" int gpx_batch_set_shape(gpx_batch *b, int tile_cells, int xchunk)
 {
     if (!b || xchunk < 0) return bfail(b, GPX_EARG, "gpx_batch_set_shape: bad argument");
-    if (tile_cells) {  // 0 = the H and E passes
+    if (tile_cells) {  // 0 = planned
         const std::vector<int> ok = batch_tiles(b);
         bool found = false;
         for (int tc : ok) found = found || tc == tile_cells;
@@ -2935,149 +2892,14 @@ extern "C" int gpx_batch_set_shape(gpx_batch *b, int tile_cells, int xchunk)
     return 0;
 }
 
-// Launch tables for tile size `tc`: every model's arguments for both state
-// orders, the first item of each model, and the common x-chunk length that
-// minimises rounds x planes per item over all items.
-struct BatchPlan {
-    int tc = 0, B = 0, xc = 0, nitems = 0, grid = 0;
-    size_t lds = 0;
-    batch_kernel k = nullptr;
-};
-
-static int batch_prepare(gpx_batch *b, int tc, int xchunk, BatchPlan &p)
-{
-    const int n = (int)b->ctx.size();
-    p.tc = tc;
-    p.B = tc / STEP_CELLS_PER_THREAD;
-    p.k = pick_step(b->ctx[0]).many;
-    p.lds = 0;
-    int maxnx1 = 0;
-    for (gpx_ctx *c : b->ctx) {
-        if (c->rare_dirty || !c->rare) {
-            hipError_t e = upload_rare(c);
-            if (e != hipSuccess) return bfail(b, (int)e, std::string("gpx_batch: ") + hipGetErrorString(e));
-        }
-        if (int rc = ensure_next_state(c, true)) return bfail(b, rc, "gpx_batch: " + c->err);
-        const size_t l = step_lds(c, tc);
-        if (l > p.lds) p.lds = l;
-        if (c->desc.nx + 1 > maxnx1) maxnx1 = c->desc.nx + 1;
-    }
-    const int resident = resident_blocks(b->ctx[0], (const void *)p.k, p.B, p.lds);
-    std::vector<FusedArgs> args(2 * (size_t)n);
-    for (int t = 0; t < n; ++t) fill_step_args(b->ctx[t], tc, 0, args[t]);
-    int xc = xchunk;
-    if (!xc) {
-        long long best = -1;
-        for (int c = 2; c <= maxnx1; ++c) {
-            long long items = 0;
-            for (int t = 0; t < n; ++t) items += (long long)args[t].ntiles * ((b->ctx[t]->desc.nx + 1 + c - 1) / c);
-            const long long cost = (items + resident - 1) / resident * (long long)(c + 1);
-            if (best < 0 || cost <= best) {
-                best = cost;
-                xc = c;
-            }
-        }
-    }
-    std::vector<int> item0(n + 1, 0);
-    for (int t = 0; t < n; ++t) {
-        FusedArgs &a = args[t];
-        a.xc = xc;
-        a.nitems = a.ntiles * ((b->ctx[t]->desc.nx + 1 + xc - 1) / xc);
-        item0[t + 1] = item0[t] + a.nitems;
-        FusedArgs &s = args[n + t];  // the same model with its two states exchanged
-        s = a;
-        const float *fc = s.Fc;
-        s.Fc = s.Fx;
-        s.Fx = const_cast<float *>(fc);
-        for (int q = 0; q < s.nslab; ++q) {
-            std::swap(s.slabH[q].phi1, s.slabH[q].phw1);
-            std::swap(s.slabH[q].phi2, s.slabH[q].phw2);
-        }
-    }
-    p.xc = xc;
-    p.nitems = item0[n];
-    long long g = resident < p.nitems ? resident : p.nitems;
-    g = (g + 7) / 8 * 8;
-    p.grid = (int)g;
-    hipSetDevice(b->device);
-    GPX_BTRY(hipMemcpyAsync(b->dargs, args.data(), args.size() * sizeof(FusedArgs), hipMemcpyHostToDevice, b->stream));
-    GPX_BTRY(hipMemcpyAsync(b->ditem0, item0.data(), item0.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
-    GPX_BTRY(hipStreamSynchronize(b->stream));
-    return 0;
-}
-
-static BatchArgs batch_args(const gpx_batch *b, const BatchPlan &p, int step, int it)
-{
-    BatchArgs a;
-    a.args = b->dargs;
-    a.item0 = b->ditem0;
-    a.ntr = (int)b->ctx.size();
-    a.nitems = p.nitems;
-    a.per_xcd = p.grid / 8;
-    a.flip = step & 1;
-    a.it = it;
-    return a;
-}
-
-// After n batched iterations every model's next state is its current one
-// when n is odd.
-static void batch_swap(gpx_batch *b, int n)
-{
-    if (!(n & 1)) return;
-    for (gpx_ctx *c : b->ctx) {
-        for (int q = 0; q < 6; ++q) std::swap(c->F[q], c->Fn[q]);
-        for (auto &S : c->slabs) {
-            std::swap(S.phi[2], S.phin[0]);
-            std::swap(S.phi[3], S.phin[1]);
-        }
-    }
-}
-
-static int batch_steps(gpx_batch *b, const BatchPlan &p, int it0, int n, int graph, float *ms)
-{
-    // Work queued on the models' own streams (uploads) completes first.
-    for (gpx_ctx *c : b->ctx) GPX_BTRY(hipStreamSynchronize(c->stream));
-    hipEvent_t e0, e1;
-    GPX_BTRY(hipEventCreate(&e0));
-    GPX_BTRY(hipEventCreate(&e1));
-    hipGraph_t gr = nullptr;
-    hipGraphExec_t ge = nullptr;
-    if (graph) {
-        GPX_BTRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        for (int s = 0; s < n; ++s)
-            hipLaunchKernelGGL(p.k, dim3(p.grid), dim3(p.B), p.lds, b->stream, batch_args(b, p, s, it0 + s));
-        GPX_BTRY(hipStreamEndCapture(b->stream, &gr));
-        GPX_BTRY(hipGraphInstantiate(&ge, gr, nullptr, nullptr, 0));
-    }
-    GPX_BTRY(hipEventRecord(e0, b->stream));
-    if (graph) {
-        GPX_BTRY(hipGraphLaunch(ge, b->stream));
-    } else {
-        for (int s = 0; s < n; ++s) {
-            hipLaunchKernelGGL(p.k, dim3(p.grid), dim3(p.B), p.lds, b->stream, batch_args(b, p, s, it0 + s));
-            GPX_BTRY(hipGetLastError());
-        }
-    }
-    GPX_BTRY(hipEventRecord(e1, b->stream));
-    GPX_BTRY(hipEventSynchronize(e1));
-    float t = 0;
-    GPX_BTRY(hipEventElapsedTime(&t, e0, e1));
-    if (ms) *ms = t;
-    if (ge) hipGraphExecDestroy(ge);
-    if (gr) hipGraphDestroy(gr);
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
-    batch_swap(b, n);
-    return 0;
-}
-
-// The H and E passes of every model, as four launches per iteration (H
-// interior, H boundary, E interior, E boundary), each over the items of a group
-// of models: one block per item, the block finding its model in the table.
-// Groups are consecutive models whose state fits together in the 256 MB
+// Groups.  Consecutive models whose state fits together in the 256 MB
 // last-level cache (192 MB budget; a larger model is a group of its own); a
 // group runs all its iterations before the next one starts, so that its state
-// stays cached between passes, as it does when the models run one by one.
+// stays cached, as it does when the models run one by one.  A group whose
+// models share their row kernels takes the two row passes, or the one-launch step
+// where form 4 would; any other (different PML orders mixed, say) four general
+// passes, H interior, H boundary, E interior, E boundary.  One block per item,
+// the block finding its model in the table.
 static const double GROUP_BYTES = 192.0 * 1024 * 1024;
 
 extern "C" int gpx_batch_set_group_bytes(gpx_batch *b, double bytes)
@@ -3087,20 +2909,91 @@ extern "C" int gpx_batch_set_group_bytes(gpx_batch *b, double bytes)
     return 0;
 }
 
-struct PassGroup {
+struct BatchGroup {
     int g0 = 0, gn = 0;
+    enum { GENERAL, PASSES, STEP } kind = GENERAL;
+    int B = 0, nitems_rows = 0;
+    size_t lds_rows[2] = {0, 0};        // of the E pass or the step, of the H pass
+    size_t off_rows = 0;                // of the group's item0 table in ditem0
     int nitems[4] = {0, 0, 0, 0}, grid[4] = {0, 0, 0, 0};
     size_t lds[4] = {0, 0, 0, 0};
     size_t item_off[4] = {0, 0, 0, 0};  // of the group's item0 table in dpitem
 };
 
-struct PassPlan {
+struct BatchPlan {
     many_kernel k[4] = {nullptr, nullptr, nullptr, nullptr};
-    std::vector<PassGroup> groups;
+    std::vector<BatchGroup> groups;
     int B = 256;
+    int xc = 0;                          // of the last group with one launch per iteration
 };
 
-static int batch_prepare_passes(gpx_batch *b, PassPlan &p)
+// A group of one model (a model larger than the group budget, or the last one
+// left) shares its launches with nothing, so it runs as a plain solve of
+// that model instead: run_steps with the model's own step form, on the
+// model's stream, ordered after the batch stream's earlier work and before its
+// later work.  The step forms give the same bits as the passes.
+static bool group_alone(const BatchGroup &g) { return g.gn == 1; }
+
+// Tiles and chunks of a group's models for the one-launch step (blocks of `tile`
+// cells, 0: chosen) or the row passes, with chunks of xchunk planes (0: chosen).
+static int batch_plan_rows(gpx_batch *b, int tile, int xchunk, BatchGroup &g, std::vector<RowModel> &models, int &xc)
+{
+    int cus = 256;
+    for (int t = g.g0; t < g.g0 + g.gn; ++t) {
+        gpx_ctx *c = b->ctx[t];
+        if (g.kind == BatchGroup::STEP)
+            if (int rc = ensure_next_state(c)) return bfail(b, rc, "gpx_batch: " + c->err);
+        if (int rc = ensure_row(c)) return bfail(b, rc, "gpx_batch: " + c->err);
+        models[t] = c->rowh;
+        if (c->cur) {  // launch parity 0 reads the current state
+            std::swap(models[t].F[0], models[t].F[1]);
+            std::swap(models[t].phiH[0], models[t].phiH[1]);
+        }
+        if (c->cus > 0) cus = c->cus;
+    }
+    if (g.kind == BatchGroup::PASSES) {
+        g.B = 256;
+        xc = xchunk ? xchunk : pass_chunk(b->ctx[g.g0]);
+        for (;; --xc) {
+            g.nitems_rows = 0;
+            for (int t = g.g0; t < g.g0 + g.gn; ++t) {
+                pass_items(b->ctx[t], g.B, xc, models[t]);
+                g.nitems_rows += models[t].pitems;
+            }
+            if (xchunk || xc <= 1 || g.nitems_rows >= pass_fill(b->ctx[g.g0])) break;
+        }
+        for (int f = 0; f < 2; ++f)
+            for (int t = g.g0; t < g.g0 + g.gn; ++t) g.lds_rows[f] = std::max(g.lds_rows[f], pass_lds(b->ctx[t], f));
+        return 0;
+    }
+    int B = tile ? tile / NC : ROW_BLOCK_MAX;
+    auto fits = [&](int block) {
+        for (int t = g.g0; t < g.g0 + g.gn; ++t)
+            if (step_lds(b->ctx[t], block) > (size_t)MAX_LDS_BYTES) return false;
+        return true;
+    };
+    while (!tile && B > 128 && !fits(B)) B /= 2;
+    auto items = [&](int block, int chunk) {
+        int n = 0;
+        for (int t = g.g0; t < g.g0 + g.gn; ++t) {
+            row_tiles(b->ctx[t], block, chunk, models[t]);
+            n += models[t].nitems;
+        }
+        return n;
+    };
+    xc = xchunk ? xchunk : 4;
+    int n = items(B, xc);
+    while (!tile && B > 128 && n < 2 * cus) n = items(B /= 2, xc);
+    while (!xchunk && xc > 2 && n < 2 * cus) n = items(B, --xc);
+    g.B = B;
+    g.nitems_rows = n;
+    for (int t = g.g0; t < g.g0 + g.gn; ++t) g.lds_rows[0] = std::max(g.lds_rows[0], step_lds(b->ctx[t], B));
+    return 0;
+}
+
+// Launch tables.  tile 0: groups; else one group of every model with blocks
+// of `tile` cells.
+static int batch_prepare(gpx_batch *b, int tile, int xchunk, BatchPlan &p)
 {
     const int n = (int)b->ctx.size();
     for (int kind = 0; kind < 4; ++kind)
@@ -3111,9 +3004,9 @@ static int batch_prepare_passes(gpx_batch *b, PassPlan &p)
     double acc = 0;
     for (int t = 0; t < n; ++t) {
         const gpx_ctx *c = b->ctx[t];
-        const double bytes = (double)(c->bytes - c->next_bytes);  // the second copies are not used
-        if (p.groups.empty() || acc + bytes > b->group_bytes) {
-            p.groups.push_back(PassGroup());
+        const double bytes = (double)(c->bytes - c->next_bytes);
+        if (p.groups.empty() || (!tile && acc + bytes > b->group_bytes)) {
+            p.groups.push_back(BatchGroup());
             p.groups.back().g0 = t;
             acc = 0;
         }
@@ -3122,9 +3015,22 @@ static int batch_prepare_passes(gpx_batch *b, PassPlan &p)
     }
     const int G = (int)p.groups.size();
     std::vector<StepArgs> args(4 * (size_t)n);
-    std::vector<int> item0(4 * (size_t)(n + G), 0);
+    std::vector<RowModel> models(n);
+    std::vector<int> item0(4 * (size_t)(n + G), 0), ritem0((size_t)n + G, 0);
+    hipSetDevice(b->device);
     for (int gi = 0; gi < G; ++gi) {
-        PassGroup &g = p.groups[gi];
+        BatchGroup &g = p.groups[gi];
+        if (!tile && group_alone(g)) continue;
+        if (batch_rows(b, g.g0, g.gn) && (tile || batch_plain(b, g.g0, g.gn))) g.kind = BatchGroup::STEP;
+        else if (batch_passes(b, g.g0, g.gn)) g.kind = BatchGroup::PASSES;
+        if (g.kind != BatchGroup::GENERAL) {
+            if (int rc = batch_plan_rows(b, tile, xchunk, g, models, p.xc)) return rc;
+            g.off_rows = (size_t)g.g0 + gi;
+            for (int t = 0; t < g.gn; ++t)
+                ritem0[g.off_rows + t + 1] = ritem0[g.off_rows + t] + (g.kind == BatchGroup::STEP ? models[g.g0 + t].nitems
+                                                                                                  : models[g.g0 + t].pitems);
+            continue;
+        }
         for (int kind = 0; kind < 4; ++kind) {
             const int field = kind < 2 ? 1 : 0;
             const bool bnd = kind & 1;
@@ -3136,7 +3042,7 @@ static int batch_prepare_passes(gpx_batch *b, PassPlan &p)
                 int block, grid;
                 size_t lds;
                 base_args(c, field, a, block, lds);
-                plan(c, bnd, 0, p.B, a, grid);
+                plan(c, bnd, p.B, a, grid);
                 const int f = field == 1 ? h_flags(c) : e_flags(c);
                 a.flags = bnd ? f : f & ~F_PML_ALL;
                 a.it = 0;
@@ -3147,16 +3053,35 @@ static int batch_prepare_passes(gpx_batch *b, PassPlan &p)
             g.grid[kind] = (g.nitems[kind] + 7) / 8 * 8;
         }
     }
-    hipSetDevice(b->device);
     GPX_BTRY(hipMemcpyAsync(b->dpass, args.data(), args.size() * sizeof(StepArgs), hipMemcpyHostToDevice, b->stream));
     GPX_BTRY(hipMemcpyAsync(b->dpitem, item0.data(), item0.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
+    GPX_BTRY(hipMemcpyAsync(b->dmodels, models.data(), models.size() * sizeof(RowModel), hipMemcpyHostToDevice, b->stream));
+    GPX_BTRY(hipMemcpyAsync(b->ditem0, ritem0.data(), ritem0.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
     GPX_BTRY(hipStreamSynchronize(b->stream));
     return 0;
 }
 
-static void batch_pass_launch(const gpx_batch *b, const PassPlan &p, const PassGroup &g, int it)
+// Step s (0, 1, ...) of a run, iteration it, of one group.
+static void batch_launch(const gpx_batch *b, const BatchPlan &p, const BatchGroup &g, int s, int it)
 {
     const int n = (int)b->ctx.size();
+    if (g.kind != BatchGroup::GENERAL) {
+        const RowKernels k = row_kernels(b->ctx[g.g0]);
+        RowArgs a;
+        a.item0 = b->ditem0 + g.off_rows;
+        a.ntr = g.gn;
+        a.nitems = g.nitems_rows;
+        a.per_xcd = (g.nitems_rows + 7) / 8;
+        a.flip = g.kind == BatchGroup::STEP ? s & 1 : 0;
+        a.it = it;
+        auto launch = [&](row_kernel f, size_t lds) {
+            hipLaunchKernelGGL(f, dim3(8 * a.per_xcd), dim3(g.B), lds, b->stream, b->dmodels + g.g0, a);
+        };
+        if (g.kind == BatchGroup::STEP) return launch(k.step, g.lds_rows[0]);
+        launch(k.h, g.lds_rows[1]);
+        launch(k.e, g.lds_rows[0]);
+        return;
+    }
     for (int kind = 0; kind < 4; ++kind) {
         if (!g.nitems[kind]) continue;
         PassMany m;
@@ -3170,16 +3095,9 @@ static void batch_pass_launch(const gpx_batch *b, const PassPlan &p, const PassG
     }
 }
 
-// A group of one model (a model larger than the group budget, or the last
-// one left) shares its launches with nothing, so it runs as a plain solve of
-// that model instead: run_steps with the model's own step form (timed on its
-// first long run, as gpx_run does), on the model's stream, ordered after the
-// batch stream's earlier work and before its later work.  The step forms
-// give the same bits as the passes.
-static bool group_alone(const PassGroup &g) { return g.gn == 1; }
-
-static int batch_pass_steps(gpx_batch *b, const PassPlan &p, int it0, int n, int graph, float *ms)
+static int batch_steps(gpx_batch *b, const BatchPlan &p, int it0, int n, int graph, float *ms)
 {
+    // Work queued on the models' own streams (uploads) completes first.
     for (gpx_ctx *c : b->ctx) GPX_BTRY(hipStreamSynchronize(c->stream));
     hipEvent_t e0, e1, eb, ec;
     GPX_BTRY(hipEventCreate(&e0));
@@ -3189,9 +3107,10 @@ static int batch_pass_steps(gpx_batch *b, const PassPlan &p, int it0, int n, int
     std::vector<hipGraph_t> gr;
     std::vector<hipGraphExec_t> ge;
     int rc = 0;
+    auto alone = [&](const BatchGroup &g) { return group_alone(g) && g.kind == BatchGroup::GENERAL; };
     if (graph) {
-        for (const PassGroup &g : p.groups) {
-            if (group_alone(g)) {
+        for (const BatchGroup &g : p.groups) {
+            if (alone(g)) {
                 gr.push_back(nullptr);
                 ge.push_back(nullptr);
                 continue;
@@ -3200,7 +3119,7 @@ static int batch_pass_steps(gpx_batch *b, const PassPlan &p, int it0, int n, int
             hipGraphExec_t x = nullptr;
             hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
             if (e == hipSuccess) {
-                for (int s = 0; s < n; ++s) batch_pass_launch(b, p, g, it0 + s);
+                for (int s = 0; s < n; ++s) batch_launch(b, p, g, s, it0 + s);
                 e = hipStreamEndCapture(b->stream, &h);
             }
             if (e == hipSuccess) gr.push_back(h);
@@ -3215,8 +3134,9 @@ static int batch_pass_steps(gpx_batch *b, const PassPlan &p, int it0, int n, int
     if (!rc) {
         hipError_t e = hipEventRecord(e0, b->stream);
         for (size_t gi = 0; e == hipSuccess && !rc && gi < p.groups.size(); ++gi) {
-            if (group_alone(p.groups[gi])) {
-                gpx_ctx *c = b->ctx[p.groups[gi].g0];
+            const BatchGroup &g = p.groups[gi];
+            if (alone(g)) {
+                gpx_ctx *c = b->ctx[g.g0];
                 e = hipEventRecord(eb, b->stream);
                 if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, eb, 0);
                 if (e != hipSuccess) break;
@@ -3226,14 +3146,18 @@ static int batch_pass_steps(gpx_batch *b, const PassPlan &p, int it0, int n, int
                 }
                 e = hipEventRecord(ec, c->stream);
                 if (e == hipSuccess) e = hipStreamWaitEvent(b->stream, ec, 0);
-            } else if (graph) {
+                continue;
+            }
+            if (graph) {
                 e = hipGraphLaunch(ge[gi], b->stream);
             } else {
                 for (int s = 0; e == hipSuccess && s < n; ++s) {
-                    batch_pass_launch(b, p, p.groups[gi], it0 + s);
+                    batch_launch(b, p, g, s, it0 + s);
                     e = hipGetLastError();
                 }
             }
+            if (g.kind == BatchGroup::STEP && (n & 1))
+                for (int t = g.g0; t < g.g0 + g.gn; ++t) b->ctx[t]->cur ^= 1;
         }
         if (!rc) {
             if (e == hipSuccess) e = hipEventRecord(e1, b->stream);
@@ -3261,11 +3185,6 @@ extern "C" int gpx_batch_run(gpx_batch *b, int it0, int n, int graph, float *ms)
     if (!b || it0 < 0 || n < 1 || it0 + n > b->ctx[0]->desc.iterations)
         return bfail(b, GPX_EARG, "gpx_batch_run: bad argument");
     hipSetDevice(b->device);
-    if (!b->tile) {
-        PassPlan p;
-        if (int rc = batch_prepare_passes(b, p)) return rc;
-        return batch_pass_steps(b, p, it0, n, graph, ms);
-    }
     BatchPlan p;
     if (int rc = batch_prepare(b, b->tile, b->xchunk, p)) return rc;
     return batch_steps(b, p, it0, n, graph, ms);
@@ -3279,13 +3198,8 @@ static int zero_state(gpx_ctx *ctx)
     hipStream_t s = c->stream;
     for (float *m : c->Fmem)
         if (m) GPX_TRY(hipMemsetAsync(m, 0, (size_t)6 * c->fstride * 4, s));
-    for (const Slab &S : c->slabs) {
-        for (int q = 0; q < 4; ++q)
-            GPX_TRY(hipMemsetAsync(S.phi[q], 0, (size_t)S.order * S.dims[q][0] * S.dims[q][1] * S.dims[q][2] * 4, s));
-        for (int q = 0; q < 2; ++q)
-            if (S.phin[q])
-                GPX_TRY(hipMemsetAsync(S.phin[q], 0, (size_t)S.order * S.dims[q + 2][0] * S.dims[q + 2][1] * S.dims[q + 2][2] * 4, s));
-    }
+    for (float *m : {c->phiE, c->phiH[0], c->phiH[1]})
+        if (m) GPX_TRY(hipMemsetAsync(m, 0, phi_bytes(c), s));
     if (c->desc.maxpoles > 0)
         for (int q = 0; q < 3; ++q)
             if (c->T[q])
@@ -3304,33 +3218,30 @@ extern "C" int gpx_batch_tune(gpx_batch *b, int steps, int *tile_cells, int *xch
     int bt = 0, bx = 0;
     bool all_alone = true;
     {
-        PassPlan p;
-        if (int rc = batch_prepare_passes(b, p)) return rc;
+        BatchPlan p;
+        if (int rc = batch_prepare(b, 0, 0, p)) return rc;
         float ms = 0;
-        if (int rc = batch_pass_steps(b, p, 0, 1, 0, nullptr)) return rc;  // first launch
-        if (int rc = batch_pass_steps(b, p, 0, steps, 0, &ms)) return rc;
+        if (int rc = batch_steps(b, p, 0, 1, 0, nullptr)) return rc;  // first launch
+        if (int rc = batch_prepare(b, 0, 0, p)) return rc;
+        if (int rc = batch_steps(b, p, 0, steps, 0, &ms)) return rc;
         best = ms / steps;
-        for (const PassGroup &g : p.groups) all_alone = all_alone && group_alone(g);
+        for (const BatchGroup &g : p.groups) all_alone = all_alone && group_alone(g);
     }
     // Models too large to share a group each fill the GPU on their own and
-    // run as plain solves; the fused step over all models is not timed for
-    // them (it trails the plain forms of such models by a third).
-    for (int tc : all_alone ? std::vector<int>() : batch_tiles(b)) {
+    // run as plain solves; models that take the passes are slower in one launch
+    // whatever its tiles (one_launch).
+    for (int tc : all_alone || !batch_plain(b, 0, (int)b->ctx.size()) ? std::vector<int>() : batch_tiles(b)) {
         BatchPlan p;
         if (int rc = batch_prepare(b, tc, 0, p)) return rc;
-        const int base = p.xc;
-        for (int xc : {base, 2 * base, (base + 1) / 2}) {
-            if (xc < 2) continue;
-            if (int rc = batch_prepare(b, tc, xc, p)) return rc;
-            float ms = 0;
-            if (int rc = batch_steps(b, p, 0, 1, 0, nullptr)) return rc;  // first launch of a shape
-            if (int rc = batch_steps(b, p, 0, steps, 0, &ms)) return rc;
-            ms /= steps;
-            if (best < 0 || ms < best) {
-                best = ms;
-                bt = tc;
-                bx = xc;
-            }
+        float ms = 0;
+        if (int rc = batch_steps(b, p, 0, 1, 0, nullptr)) return rc;  // first launch of a shape
+        if (int rc = batch_prepare(b, tc, 0, p)) return rc;
+        if (int rc = batch_steps(b, p, 0, steps, 0, &ms)) return rc;
+        ms /= steps;
+        if (best < 0 || ms < best) {
+            best = ms;
+            bt = tc;
+            bx = p.xc;
         }
     }
     for (gpx_ctx *c : b->ctx)

@@ -1,10 +1,10 @@
-// Fused time-step kernels for models with MRIPML, one CFS term (one translation unit
-// per PML form, compiled in parallel).
-#include "gpx_step.h"
+// Row kernels for models with MRIPML, one CFS term (one translation unit per PML form,
+// compiled in parallel).
+#include "gpx_rows.h"
 
 namespace gpx {
-StepKernels step_kernel_mri1(int id_bytes, int P, bool C)
+RowKernels row_kernel_mri1(int P, bool C, bool hu)
 {
-    return step_kernel_table<1, 1>(id_bytes, P, C);
+    return row_kernel_table<1, 1>(P, C, hu);
 }
 }  // namespace gpx

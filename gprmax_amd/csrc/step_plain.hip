@@ -1,10 +1,11 @@
-// Fused time-step kernels for models with no PML slabs (one translation unit
-// per PML form, compiled in parallel).
-#include "gpx_step.h"
+// Row kernels for models without PML slabs (one translation unit per PML form,
+// compiled in parallel).
+#include "gpx_rows.h"
 
 namespace gpx {
-StepKernels step_kernel_plain(int id_bytes, int P, bool C)
+RowKernels row_kernel_plain(int P, bool C, bool hu)
 {
-    return step_kernel_table<0, 0>(id_bytes, P, C);
+    return row_kernel_table<0, 0>(P, C, hu);
 }
+
 }  // namespace gpx

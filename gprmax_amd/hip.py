@@ -193,31 +193,26 @@ class HipSolver:
         self._check(self.lib.gpx_set_launch(self.ctx, xchunk, block))
 
     def set_step(self, fused=4, tile_cells=0):
-        """Step form of gpx_run: 0 the H and E passes, 1 the fused step, 2 the
-        passes with interior and boundary kernels side by side, 3 the split
-        step, 5 the split step with the H boundary pass beside the interior
-        kernel, 6 the passes as one launch each over every cell, 7 the split
-        step with the H boundary pass inside the interior kernel's launch, 4
-        (the library's default) the fastest of 7, 6, 2, 5, 3 and 0 (of 6, 2
-        and 0 where the split step does not apply), timed on the first run of
-        at least 26 iterations.  All give the same bits."""
+        """Step form of gpx_run: 0 and 6 the H and E row passes, 1 the whole
+        step in one launch, 2 the general passes with interior and boundary
+        kernels side by side, 3, 5, 7 and 4 (the default) by rule: the one
+        launch for 3-D models without slabs and poles, the passes otherwise.
+        All give the same bits."""
         self._check(self.lib.gpx_set_step(self.ctx, int(fused), int(tile_cells)))
 
     def step_kind(self):
-        """Cells per fused block, or 0 when another form runs."""
+        """Cells per block of the one-launch step, or 0 when another form runs."""
         return int(self.lib.gpx_step_kind(self.ctx))
 
     def step_form(self):
-        """The form gpx_run uses: 0 passes, 1 fused, 2 side by side, 3 split,
-        5 split with the H boundary pass beside the interior kernel, 6 merged
-        passes, 7 split with the H boundary pass in the interior launch."""
+        """The form gpx_run uses: 0 and 6 passes, 1 one launch, 2 side by side,
+        3, 5, 7 by rule (the default reports 3 until its first long run, then 6
+        for the passes or 7 for the one launch)."""
         return int(self.lib.gpx_step_form(self.ctx))
 
     def step_choice(self):
-        """The default form's choice: -1 not timed yet, 0 passes, 1 split,
-        2 split with the H boundary pass beside, 3 passes side by side, 4
-        merged passes, 5 split with the H boundary pass in the interior
-        launch."""
+        """The default form's choice, made on the first run of at least 26
+        iterations: -1 not yet, 4 the passes, 5 the one launch."""
         return int(self.lib.gpx_step_choice(self.ctx))
 
     def run(self, it0=0, n=None):
@@ -233,9 +228,9 @@ class HipSolver:
         return t.value, h.value, e.value
 
     def run_profiled(self, it0, n):
-        """Mean ms per iteration of each kernel: (H interior, H boundary, E
-        interior, E boundary) for the passes; (interior, H boundary, 0, E
-        boundary) for the split step; (step, 0, 0, 0) for the fused step."""
+        """Mean ms per iteration of each kernel: (H, 0, E, 0) for the row
+        passes, (step, 0, 0, 0) for the one launch, (H interior, H boundary, E
+        interior, E boundary) for the general passes."""
         ms = (ctypes.c_float * 4)()
         self._check(self.lib.gpx_run_profiled(self.ctx, it0, n, ms))
         return tuple(ms)
@@ -326,10 +321,10 @@ def device_info(device=0):
 
 
 class HipBatch:
-    """Several HipSolver models advanced together: per iteration, four launches
-    (the H and E passes, interior and boundary) each over all models, or one
-    launch of the fused step over all models; optionally all iterations in one
-    HIP graph."""
+    """Several HipSolver models advanced together: per iteration, the H and E
+    row passes each over all models, or one launch of the whole step over all
+    models (models that share no row kernels: four general passes); optionally
+    all iterations in one HIP graph."""
 
     def __init__(self, solvers):
         self.lib = library()
@@ -363,7 +358,8 @@ class HipBatch:
         self.close()
 
     def set_shape(self, tile_cells=0, xchunk=0):
-        """tile_cells 0: the H and E passes; 256, 512, 1024: the fused step."""
+        """tile_cells 0: by the rule of the default step form; 256, 512, 1024:
+        the one-launch step with that many cells per block."""
         self._check(self.lib.gpx_batch_set_shape(self.b, int(tile_cells), int(xchunk)))
 
     def set_group_bytes(self, nbytes=0):
@@ -373,7 +369,7 @@ class HipBatch:
 
     def tune(self, steps=3):
         """Pick the fastest launch shape; returns (tile_cells, xchunk, ms per
-        iteration), tile_cells 0 for the passes.  Leaves every model at the
+        iteration), tile_cells 0 for the rule's.  Leaves every model at the
         zero state."""
         t, x, ms = ctypes.c_int(), ctypes.c_int(), ctypes.c_float()
         self._check(self.lib.gpx_batch_tune(self.b, int(steps), ctypes.byref(t), ctypes.byref(x), ctypes.byref(ms)))

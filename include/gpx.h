@@ -130,8 +130,7 @@ int gpx_add_snapshot(gpx_ctx *ctx, int xs, int ys, int zs, int dx, int dy, int d
 /* The time loop: iterations [it0, it0 + n), every sub-step of an iteration
  * inside the kernels of the step form set by gpx_set_step (replaces
  * model_build_run.py:590-696).  Enqueued on the ctx stream; returns without
- * waiting, except that under the default form the first run of at least 26
- * iterations waits once, after its 14th iteration, to read its timing. */
+ * waiting. */
 int gpx_run(gpx_ctx *ctx, int it0, int n);
 
 /* As gpx_run, and reports the elapsed device time measured with HIP events
@@ -141,13 +140,11 @@ int gpx_run_timed(gpx_ctx *ctx, int it0, int n, int per_kernel, float *ms_total,
                   float *ms_h, float *ms_e);
 
 /* As gpx_run, with HIP events around every kernel; ms4 receives the mean
- * duration in ms of each kernel of an iteration: the fused step kernel in
- * ms4[0] (ms4[1..3] = 0); the split step's interior kernel, H boundary and E
- * boundary passes in ms4[0], ms4[1], ms4[3] (ms4[2] = 0); or with the
- * two-pass form H interior, H boundary, E interior, E boundary (interior =
- * cells away from the faces and PML slabs, boundary = the rest).  The form 4
- * choice is not timed here: a profiled run uses the split step until a
- * gpx_run has made the choice.  Waits once, at the end. */
+ * duration in ms of each kernel of an iteration: the one-launch step in
+ * ms4[0]; the row passes, H in ms4[0] and E in ms4[2]; or the general passes,
+ * H interior, H boundary, E interior, E boundary (interior = cells away from
+ * the faces and PML slabs, boundary = the rest).  Slots not named are 0.  Makes
+ * no form 4 choice.  Waits once, at the end. */
 int gpx_run_profiled(gpx_ctx *ctx, int it0, int n, float *ms4);
 
 /* Cells of the interior box (the rest are boundary cells), and the box
@@ -162,44 +159,30 @@ int gpx_part(gpx_ctx *ctx, int part, int arg, int it);
  * threads per block of the H and E passes (64, 128, 256, 512 or 1024; 0 = auto). */
 int gpx_set_launch(gpx_ctx *ctx, int xchunk, int block);
 
-/* Step form of gpx_run.  fused = 1: one kernel per iteration that does the
- * H and the E update with the state double-buffered on the device; fused = 0:
- * an H pass and an E pass per iteration; fused = 2: the passes with their
- * interior and boundary kernels running side by side on two streams, one
- * block per item each (gpx_run_profiled always runs them one after the
- * other); fused = 3: the
- * split step, one kernel doing H and E for the interior and the H and E
- * boundary passes around it, double-buffered; fused = 5: the split step with
- * the H boundary pass running beside the interior kernel on a second stream
- * (gpx_run_profiled runs them one after the other); fused = 6: the passes,
- * each as one launch over every cell, the interior and boundary items of
- * each x chunk next to each other; fused = 7: the split step with the H
- * boundary pass's items inside the interior kernel's launch, likewise
- * interleaved; fused = 4 (default): the first gpx_run of at least 26
- * iterations times forms 7, 6, 2, 5, the split step and the passes (forms 6,
- * 2 and the passes where the split step does not apply) on four iterations
- * each and keeps the fastest (gpx_step_choice).  tile_cells = cells per fused block (256, 512 or 1024;
- * 0 = auto).  All forms give identical results; the
- * fused form needs a tile of at least twice nz+1 cells within the LDS budget,
- * the split step a model without dispersive poles, and the passes run when
- * the chosen form does not apply (form 5 as the split step). */
+/* Step form of gpx_run.  fused = 0 and 6: the row passes, H and E as one launch
+ * each over every cell, in place; fused = 1: the whole step in one launch, the
+ * state double-buffered; fused = 2: the general passes with their interior
+ * and boundary kernels side by side on two streams (gpx_run_profiled runs them
+ * one after the other); fused = 3, 5, 7 and 4 (default): by rule, the one
+ * launch for 3-D models without slabs and dispersive poles, the passes
+ * otherwise.  tile_cells = cells per block of form 1 (256, 512 or 1024; 0 =
+ * auto).  All forms give identical results; models the row kernels do not take
+ * (slabs of different orders, in another order or overlapping, more than 32
+ * bits of byte offsets, tables past the LDS) run the general passes. */
 int gpx_set_step(gpx_ctx *ctx, int fused, int tile_cells);
 
-/* Cells per block of the fused step that gpx_run will use, or 0 when it will
+/* Cells per block of the one-launch step under form 1, or 0 when gpx_run will
  * run another form. */
 int gpx_step_kind(const gpx_ctx *ctx);
 
-/* The form gpx_run will use: 0 passes, 1 fused step, 2 passes side by side,
- * 3 split step, 5 split step with the H boundary pass beside the interior
- * kernel, 6 merged passes, 7 split step with the H boundary pass in the
- * interior kernel's launch.  gpx_run_profiled reports the split step's
- * interior kernel in ms4[0] and its boundary passes in ms4[1] and ms4[3]
- * (form 7: the merged launch in ms4[0], ms4[1] = 0), and the merged passes'
- * H and E launches in ms4[0] and ms4[2]. */
+/* The form gpx_run will use: 1 the one launch, 2 side by side, 6 the passes, 3,
+ * 5, 7 the rule's on 3-D models without poles (0: elsewhere, and the passes).
+ * Form 4 reports 3 or 0 until it has chosen, then 6 for the passes, 7 for the
+ * one launch. */
 int gpx_step_form(const gpx_ctx *ctx);
 
-/* Form 4's choice: -1 not timed yet, 0 the passes, 1 the split step, 2 form 5,
- * 3 form 2, 4 form 6, 5 form 7. */
+/* Form 4's choice, made on the first gpx_run of at least 26 iterations: -1 not
+ * yet, 4 form 6 (the passes), 5 form 7 (the one launch). */
 int gpx_step_choice(const gpx_ctx *ctx);
 
 int gpx_synchronize(gpx_ctx *ctx);
@@ -228,11 +211,11 @@ size_t gpx_memory_bytes(const gpx_ctx *ctx);
  * re-runs run_model and so a whole solve_gpu (gprMax/gprMax.py:222-232 with
  * gprMax/model_build_run.py:84-406); here the traces stay separate gpx_ctx
  * models, each built and uploaded as usual.  Each iteration of the batch is
- * either four launches (H interior, H boundary, E interior, E boundary), each
- * over the work of every model (tile 0, the default), or one launch of the
- * fused step over every model (tile > 0).  Requirements: one device, the same
+ * the row passes, or the one-launch step, each launch over the work of every
+ * model (tile 0, the default: by form 4's rule; tile > 0: the one launch), or
+ * for models that share no row kernels four general passes.  Requirements: one device, the same
  * iteration count, no snapshots, and the same kernel (index width, poles and
- * their kind, PML formulation) for every model; the fused step also needs one
+ * their kind, PML formulation) for every model; the one launch also needs one
  * PML order for all slabs of all models.  The contexts must outlive the
  * batch; results are read from each context (gpx_download_rx, ...). */
 typedef struct gpx_batch gpx_batch;
@@ -241,13 +224,12 @@ int gpx_batch_create(gpx_ctx *const *ctxs, int n, gpx_batch **out);
 int gpx_batch_destroy(gpx_batch *b);
 /* Message of the last failure (NULL: of the last gpx_batch_create). */
 const char *gpx_batch_last_error(const gpx_batch *b);
-/* tile_cells 0: the H and E passes; 256, 512 or 1024: the fused step with
- * that many cells per block and `xchunk` planes per x chunk (0 = chosen for
- * the batch). */
+/* tile_cells 0: by rule; 256, 512 or 1024: the one-launch step with that many
+ * cells per block.  `xchunk` planes per x chunk (0 = chosen for the batch). */
 int gpx_batch_set_shape(gpx_batch *b, int tile_cells, int xchunk);
-/* Autotuner: times `steps` iterations of the passes and of the fused step for
- * each usable tile size and three chunk lengths around the planned one, keeps
- * the fastest (*tile_cells 0 for the passes), reports it and its time per
+/* Autotuner: times `steps` iterations of the rule's kernels and, for models
+ * without slabs and poles, of the one-launch step with each usable tile size,
+ * keeps the fastest (*tile_cells 0 for the rule's), reports it and its time per
  * iteration, then resets every model to the zero state (fields, Phi, T,
  * receiver buffer).  Call before stepping. */
 int gpx_batch_tune(gpx_batch *b, int steps, int *tile_cells, int *xchunk, float *ms_per_step);

@@ -1,0 +1,67 @@
+"""Edges of the row kernels (csrc/gpx_rows.h) against the CPU oracle from a
+random state: row lengths around the lanes' two cells and the rows' padding,
+rows longer than a wave, slabs of one cell, slabs that meet or overlap (the
+general passes), values of every magnitude down to the subnormal ones (the
+slabs' division), materials with different H coefficients.
+
+Both sides round every operation the same way, so the expected agreement is
+bit for bit.
+"""
+
+import numpy as np
+import pytest
+
+import oracle
+from oracle import solver as osolver
+from gpu_models import randomise_tables, rich_model
+from test_gpu_parity import COMPS, _assert_state_equal, _hip, _push_state, _random_state
+
+pytestmark = pytest.mark.gpu
+
+FACES = {'x0': 3, 'y0': 2, 'z0': 4, 'xmax': 1, 'ymax': 4, 'zmax': 3}
+MEET = {'x0': 4, 'y0': 4, 'z0': 4, 'xmax': 4, 'ymax': 4, 'zmax': 4}
+
+
+def _check(G, form, xchunk, scale=None):
+    _random_state(G, 9)
+    if scale is not None:
+        rng = np.random.default_rng(3)
+        arrays = [getattr(G, c) for c in COMPS]
+        for pml in G.pmls:
+            arrays += [pml.EPhi1, pml.EPhi2, pml.HPhi1, pml.HPhi2]
+        for a in arrays:
+            a *= np.exp2(-rng.integers(0, scale, a.shape)).astype(np.float32)
+    lib = oracle.load(np.float32)
+    with _hip()(G) as s:
+        s.set_step(form)
+        s.set_launch(xchunk, 0)
+        _push_state(s, G)
+        s.run(0, 4)
+        for it in range(4):
+            osolver.step(lib, G, it, 8)
+        _assert_state_equal(s, G, 'form {}'.format(form))
+
+
+@pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
+@pytest.mark.parametrize('shape', [(13, 14, 12), (12, 15, 13), (14, 13, 14), (15, 12, 15), (12, 13, 127), (13, 12, 131)],
+                         ids=str)
+@pytest.mark.parametrize('order,formulation', [(1, 'HORIPML'), (2, 'HORIPML'), (1, 'MRIPML'), (2, 'MRIPML')])
+def test_row_lengths(order, formulation, shape, form):
+    G = rich_model(seed=50, shape=shape, iterations=8, snapshots=False, pml=FACES, order=order, formulation=formulation)
+    _check(G, form, 3)
+
+
+@pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
+@pytest.mark.parametrize('magnetic', [False, True])
+def test_values_of_every_magnitude(magnetic, form):
+    G = rich_model(seed=51, shape=(13, 14, 15), iterations=8, snapshots=False, pml=FACES)
+    if magnetic:
+        randomise_tables(G, 52, scaled=True)
+    _check(G, form, 0, scale=145)
+
+
+@pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
+@pytest.mark.parametrize('shape', [(10, 12, 12), (12, 10, 12), (12, 12, 9), (12, 12, 10)], ids=str)
+def test_slabs_close_to_the_opposite_one(shape, form):
+    G = rich_model(seed=53, shape=shape, iterations=8, snapshots=False, pml=MEET)
+    _check(G, form, 0)
