@@ -23,26 +23,29 @@
 //   B: T_p = T_p - zt_p E^{n+1}
 // so T^{n+1}_p = eqt_p T^n_p + zt_p (E^n - E^{n+1}).  Its reverse, with lT_p
 // = dL/dT^{n+1}_p: the adjoint of E^{n+1} seen by the E update is
-// lE* = lE - sum_p zt_p lT_p (k_adj_disp, before the gathers, which then
-// use lE*); then lE^n = CA lE* + sum_p zt_p lT_p, lT^n_p = eqt_p lT_p -
+// lE* = lE - sum_p zt_p lT_p (which the gathers use); then lE^n = CA lE* + sum_p zt_p lT_p, lT^n_p = eqt_p lT_p -
 // IEA ee_p lE*, and dL/dIEA gains -lE* phi^n (phi^n saved by the recompute).
 //
 // Iteration n maps the state s^n = (E^n, H^n, PhiE^n, PhiH^n) to s^{n+1}
 // linearly.  Its adjoint, applied from n = N-1 down to 0 to the adjoint state
 // (lE, lH, mE, mH) = dL/ds^{n+1}, is two gather kernels:
-//   k_adj_e : lH += (dE^{n+1}/dH^{n+1})^T lE  (curl and E-PML terms); gradients
-//             from lE and the stored E^n and curl H^{n+1}; mE = (dE/dPhiE)^T lE + RE mE;
-//             lE = CA lE
-//   k_adj_h : lE += (dH^{n+1}/dE^n)^T lH      (curl and H-PML terms);
-//             mH = (dH/dPhiH)^T lH + RE mH; lH = DA lH = lH; and the
-//             receiver residual of iteration n is added to lEz at each
-//             receiver (the thread of the point adds it after its update).
-// lE, mE and mH
-// are double-buffered (read one copy, write the other), so each kernel's
-// gathers see the values of the previous sub-step only.  Forward states
-// come from checkpoints every K iterations; each segment is recomputed
-// forward, storing E^n and curl H^{n+1} for every iteration of it, before the
-// adjoint sweeps back over it.
+//   E half: lH += (dE^{n+1}/dH^{n+1})^T lE  (curl and E-PML terms); gradients
+//           from lE and the stored E^n and curl H^{n+1}; mE = (dE/dPhiE)^T lE + RE mE;
+//   H half: lE = CA lE + (dH^{n+1}/dE^n)^T lH  (curl and H-PML terms);
+//           mH = (dH/dPhiH)^T lH + RE mH (lH = DA lH = lH); and the receiver
+//           residual of iteration n is added to lEz at each receiver.
+// Each half gathers from one field and updates the other in place; mE and mH are
+// double-buffered (read one copy, write the other).  With poles the H half
+// also leaves lE* of the next iteration down, so the array holds lE*.
+// Forward states come from checkpoints every K iterations; each segment is
+// recomputed forward, storing E^n and curl H^{n+1} for every iteration of it,
+// before the adjoint sweeps back over it.  E^n is not copied: the E pass
+// reads it from its slot of the store and writes E^{n+1} into the next.
+//
+// The row kernels (inv_rows.h) run models whose slabs they can place: at most one
+// per direction, in the order x0, y0, z0, xmax, ymax, zmax, the ones of an
+// axis apart; the kernels here, one point a thread and a loop over the slabs, run
+// any other.
 
 #include <hip/hip_runtime.h>
 
@@ -54,6 +57,9 @@
 #include <vector>
 
 #include "gpx.h"
+#include "inv_rows.h"
+
+using namespace gpx;
 
 namespace {
 
@@ -79,48 +85,18 @@ struct InvSlab {
     int gE_lo[3], gE_hi[3], gH_lo[3], gH_hi[3];
 };
 
+// Arrays hold one float per grid point, rows of kp floats (InvStep has them by
+// component), parameters and gradients too (0 where a point is no cell).
 struct InvArgs {
-    int nx, ny, nz;
-    long long ntot;
-    float d, DB, cH;                     // cell size; DB = dt/(mu0 d); cH = dt/mu0
-    float *E[3], *H[3];                  // fields (forward) or adjoint fields
-    // Adjoint fields, one float4 per grid point: lE of the sub-step (read),
-    // lE^n (written by the E half, completed by the H half) and lH.  The w of
-    // lE and lE^n is CB of the point's cell, that of lH its CA (0 where the
-    // point is no cell), carried along so that the E gather's CB lE terms and
-    // CA come with the loads it makes anyway.
-    float4 *lE, *lEn, *lH;
-    float *EC;                           // forward: where to save, per point, E^n (3 floats)
-                                         // then the curl of H^{n+1} (3), as three float2
-                                         // (or null); adjoint: the saved values
-    const float *CA, *CB, *IEA;          // per cell [nx][ny][nz]
-    float2 *gCAB;                        // gradient accumulators (adjoint): dL/dCA, dL/dCB per cell
-    float *gIEA;                         // and dL/dIEA
+    int nx, ny, nz, kp;
+    long long n;                         // floats of one component
+    float d;
+    InvStep b;
     int nslab;
     InvSlab slab[INV_MAX_SLABS];
-    int si, sj, sk;                      // source edge (Ez), -1 when none
-    float sfac;                          // dl / (dx dy dz)
-    const float *waves;                  // [iterations]
-    int it, iterations;
-    long long ncell;
     int P;                               // Debye poles (0: none)
-    const float *dc;                     // [3][P][ncell]: ee, eqt, zt of every cell and pole
-    float *T[3];                         // forward: T of E component c, [P][ntot]; adjoint: lT
-    float *Ps[3];                        // forward: where to save phi^n (or null); adjoint: phi^n
-    int nrx;
-    const int *rxc;                      // [nrx][3]
-    const uint8_t *rxrow;                // adjoint: per (i, j) row of points, 1 when a receiver is on it
-    float *traces;                       // [nrx][iterations]
-    const float *resid;                  // [nrx][iterations], dL/d(trace)
-    // Grid points [fast[0], fast[1]) x [fast[2], fast[3]) x [fast[4], fast[5])
-    // have every neighbour of the adjoint gathers inside the grid and updated,
-    // and no PML term: the adjoint kernels take a short path there.
-    int fast[6];
-    int shell[6][6];                     // [lo x, y, z, hi x, y, z] of the shell boxes
-    int mix_nf, mix_ns, mix_gf[2], mix_gs;  // block counts and grid sizes of the mixed launches
-    // Launches over every grid point: all_gk blocks of 128 points along k per
-    // (j, i) row, all_blocks blocks, padded to a multiple of 8 (all_per_xcd x 8).
-    int all_gk, all_blocks, all_per_xcd;
+    const uint8_t *rxrow;                // per (i, j) row of points, 1 when a receiver is on it
+    int all_gk, all_blocks, all_per_xcd; // all_gk blocks of 128 points along k per (j, i) row
 };
 
 // One-dimensional launches: the hardware deals block b to XCD b mod 8, so block
@@ -146,20 +122,10 @@ __device__ __forceinline__ bool all_point(const InvArgs &a, int &i, int &j, int 
     return true;
 }
 
-// Component c (0, 1, 2) of an adjoint field's float4.
-__device__ __forceinline__ float comp3(const float4 &v, int c)
-{
-    return c == 0 ? v.x : (c == 1 ? v.y : v.z);
-}
-
 // Grid offsets are 32-bit: gpx_inv_create requires fewer than 2^31 points.
 __device__ __forceinline__ int fidx(const InvArgs &a, int i, int j, int k)
 {
-    return (i * (a.ny + 1) + j) * (a.nz + 1) + k;
-}
-__device__ __forceinline__ int cidx(const InvArgs &a, int i, int j, int k)
-{
-    return (i * a.ny + j) * a.nz + k;
+    return (i * (a.ny + 1) + j) * a.kp + k;
 }
 __device__ __forceinline__ bool in_box3(const int *lo, const int *hi, int i, int j, int k)
 {
@@ -228,150 +194,118 @@ __device__ __forceinline__ int axis_of(const InvSlab &s, int i, int j, int k)
     return s.axis == 0 ? i : (s.axis == 1 ? j : k);
 }
 
+// Component c of a point of an array.
+__device__ __forceinline__ float at3(const InvArgs &a, const float *f, int c, int o) { return f[c * a.n + o]; }
+
 // ------------------------------------------------------------------ forward
-// H update and H-PML of one iteration; one thread per grid point.
+// Receiver samples, H update and H-PML of one iteration; one thread per grid point.
 __global__ void k_inv_h(InvArgs a)
 {
-    {
-        int i, j, k;
-        if (!all_point(a, i, j, k) || k > a.nz) return;
-        const int g = fidx(a, i, j, k);
-        const int o = g, oi = fidx(a, i + 1, j, k), oj = fidx(a, i, j + 1, k), ok = o + 1;
-        float h[3] = {a.H[0][o], a.H[1][o], a.H[2][o]};
-        if (h_upd(a, 0, i, j, k))
-            h[0] = 1.0f * h[0] - a.DB * (a.E[2][oj] - a.E[2][o]) + a.DB * (a.E[1][ok] - a.E[1][o]);
-        if (h_upd(a, 1, i, j, k))
-            h[1] = 1.0f * h[1] - a.DB * (a.E[0][ok] - a.E[0][o]) + a.DB * (a.E[2][oi] - a.E[2][o]);
-        if (h_upd(a, 2, i, j, k))
-            h[2] = 1.0f * h[2] - a.DB * (a.E[1][oi] - a.E[1][o]) + a.DB * (a.E[0][oj] - a.E[0][o]);
-        for (int s = 0; s < a.nslab; ++s) {
-            const InvSlab &S = a.slab[s];
-            if (!in_h(S, i, j, k)) continue;
-            int p;
-            int q[2];
-            pidx(S, false, i, j, k, p, q[0], q[1]);
-            const float RA01 = S.RH[p] - 1.0f, RB0 = S.RH[S.t + p], RE0 = S.RH[2 * S.t + p],
-                        RF0 = S.RH[3 * S.t + p];
-            const int on = S.axis == 0 ? oi : (S.axis == 1 ? oj : ok);
-            const float ph2[2] = {S.PH1[q[0]], S.PH2[q[1]]};  // both loads before either store
-            for (int w = 0; w < 2; ++w) {
-                int comp, src, sign;
-                h_pair(S.axis, w, comp, src, sign);
-                float *Phi = w == 0 ? S.PH1 : S.PH2;
-                const float dd = (a.E[src][on] - a.E[src][o]) / a.d;
-                const float ph = ph2[w];
-                const float corr = a.cH * (RA01 * dd + RB0 * ph);
-                Phi[q[w]] = RE0 * ph - RF0 * dd;
-                h[comp] = sign > 0 ? h[comp] + corr : h[comp] - corr;
-            }
+    int i, j, k;
+    if (!all_point(a, i, j, k) || k > a.nz) return;
+    const InvStep &b = a.b;
+    const int o = fidx(a, i, j, k), oi = fidx(a, i + 1, j, k), oj = fidx(a, i, j + 1, k), ok = o + 1;
+    if (a.rxrow[i * (a.ny + 1) + j])
+        for (int r = 0; r < b.nrx; ++r)
+            if (b.rxc[3 * r] == i && b.rxc[3 * r + 1] == j && b.rxc[3 * r + 2] == k)
+                b.traces[(long long)r * b.iterations + b.it] = at3(a, b.E, 2, o);
+    auto E = [&](int c, int at) { return at3(a, b.E, c, at); };
+    float h[3] = {at3(a, b.H, 0, o), at3(a, b.H, 1, o), at3(a, b.H, 2, o)};
+    if (h_upd(a, 0, i, j, k)) h[0] = 1.0f * h[0] - b.DB * (E(2, oj) - E(2, o)) + b.DB * (E(1, ok) - E(1, o));
+    if (h_upd(a, 1, i, j, k)) h[1] = 1.0f * h[1] - b.DB * (E(0, ok) - E(0, o)) + b.DB * (E(2, oi) - E(2, o));
+    if (h_upd(a, 2, i, j, k)) h[2] = 1.0f * h[2] - b.DB * (E(1, oi) - E(1, o)) + b.DB * (E(0, oj) - E(0, o));
+    for (int s = 0; s < a.nslab; ++s) {
+        const InvSlab &S = a.slab[s];
+        if (!in_h(S, i, j, k)) continue;
+        int p;
+        int q[2];
+        pidx(S, false, i, j, k, p, q[0], q[1]);
+        const float RA01 = S.RH[p] - 1.0f, RB0 = S.RH[S.t + p], RE0 = S.RH[2 * S.t + p], RF0 = S.RH[3 * S.t + p];
+        const int on = S.axis == 0 ? oi : (S.axis == 1 ? oj : ok);
+        for (int w = 0; w < 2; ++w) {
+            int comp, src, sign;
+            h_pair(S.axis, w, comp, src, sign);
+            float *Phi = w == 0 ? S.PH1 : S.PH2;
+            const float dd = (E(src, on) - E(src, o)) / a.d;
+            const float ph = Phi[q[w]];
+            const float corr = b.cH * (RA01 * dd + RB0 * ph);
+            Phi[q[w]] = RE0 * ph - RF0 * dd;
+            h[comp] = sign > 0 ? h[comp] + corr : h[comp] - corr;
         }
-        a.H[0][o] = h[0];
-        a.H[1][o] = h[1];
-        a.H[2][o] = h[2];
     }
+    for (int c = 0; c < 3; ++c) b.H[c * a.n + o] = h[c];
 }
 
-// Receiver samples of iteration it (the state before its H update).
-__global__ void k_inv_rx(InvArgs a)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= a.nrx) return;
-    const int *c = a.rxc + 3 * r;
-    a.traces[(long long)r * a.iterations + a.it] = a.E[2][fidx(a, c[0], c[1], c[2])];
-}
-
-// E update, E-PML and the Hertzian dipole of one iteration.
+// E update with the poles, E-PML and the Hertzian dipole of one iteration.
 __global__ void k_inv_e(InvArgs a)
 {
-    {
-        int i, j, k;
-        if (!all_point(a, i, j, k) || k > a.nz) return;
-        const int g = fidx(a, i, j, k);
-        const int o = g;
-        const int om[3] = {i > 0 ? fidx(a, i - 1, j, k) : o, j > 0 ? fidx(a, i, j - 1, k) : o, k > 0 ? o - 1 : o};
-        float e[3] = {a.E[0][o], a.E[1][o], a.E[2][o]};
-        const float en[3] = {e[0], e[1], e[2]};  // E^n, saved at the end (stores after every load)
-        // The differences of H^{n+1} of the E update (om clamps to the point
-        // itself at the low faces, so every load is inside the grid).
-        const float h0 = a.H[0][o], h1 = a.H[1][o], h2 = a.H[2][o];
-        const float d2y = h2 - a.H[2][om[1]], d1z = h1 - a.H[1][om[2]];
-        const float d0z = h0 - a.H[0][om[2]], d2x = h2 - a.H[2][om[0]];
-        const float d1x = h1 - a.H[1][om[0]], d0y = h0 - a.H[0][om[1]];
-        const bool cell = i < a.nx && j < a.ny && k < a.nz;
-        const int oc = cell ? cidx(a, i, j, k) : 0;
-        const float CA = cell ? a.CA[oc] : 0.f, CB = cell ? a.CB[oc] : 0.f, IEA = cell ? a.IEA[oc] : 0.f;
-        const bool upd[3] = {e_upd(a, 0, i, j, k), e_upd(a, 1, i, j, k), e_upd(a, 2, i, j, k)};
-        // dispersive part A: phi from T^n, then T advanced with E^n
-        float phi[3] = {0.f, 0.f, 0.f}, tv[3][INV_MAX_POLES];
-        const bool disp = a.P > 0 && cell;
-        if (disp) {
-            for (int c = 0; c < 3; ++c) {
-                if (!upd[c]) continue;
-                float ph = 0.f;
-                for (int p = 0; p < a.P; ++p) {
-                    const float ee = a.dc[(long long)p * a.ncell + oc];
-                    const float eq = a.dc[(long long)(a.P + p) * a.ncell + oc];
-                    const float zt = a.dc[(long long)(2 * a.P + p) * a.ncell + oc];
-                    const float t = a.T[c][(long long)p * a.ntot + o];
-                    ph = ph + ee * t;
-                    tv[c][p] = eq * t + zt * e[c];
-                }
-                phi[c] = ph;
-            }
+    int i, j, k;
+    if (!all_point(a, i, j, k) || k > a.nz) return;
+    const InvStep &b = a.b;
+    const int o = fidx(a, i, j, k);
+    const int om[3] = {i > 0 ? fidx(a, i - 1, j, k) : o, j > 0 ? fidx(a, i, j - 1, k) : o, k > 0 ? o - 1 : o};
+    auto dH = [&](int c, int axis) { return at3(a, b.H, c, o) - at3(a, b.H, c, om[axis]); };
+    float e[3] = {at3(a, b.E, 0, o), at3(a, b.E, 1, o), at3(a, b.E, 2, o)};
+    // (om clamps to the point itself at the low faces, so every load is inside
+    // the grid)
+    const float d2y = dH(2, 1), d1z = dH(1, 2), d0z = dH(0, 2), d2x = dH(2, 0), d1x = dH(1, 0), d0y = dH(0, 1);
+    const bool cell = i < a.nx && j < a.ny && k < a.nz;
+    const float CA = b.mat[o], CB = b.mat[a.n + o], IEA = b.mat[2 * a.n + o];
+    const bool upd[3] = {e_upd(a, 0, i, j, k), e_upd(a, 1, i, j, k), e_upd(a, 2, i, j, k)};
+    // dispersive part A: phi from T^n, then T advanced with E^n
+    float phi[3] = {0.f, 0.f, 0.f}, tv[3][INV_MAX_POLES];
+    const bool disp = a.P > 0 && cell;
+    for (int c = 0; c < 3; ++c) {
+        if (!disp || !upd[c]) continue;
+        float ph = 0.f;
+        for (int p = 0; p < a.P; ++p) {
+            const float ee = b.dc[p * a.n + o], eq = b.dc[(a.P + p) * a.n + o], zt = b.dc[(2 * a.P + p) * a.n + o];
+            const float t = b.T[(c * a.P + p) * a.n + o];
+            ph = ph + ee * t;
+            tv[c][p] = eq * t + zt * e[c];
         }
-        if (upd[0]) e[0] = CA * e[0] + CB * d2y - CB * d1z;
-        if (upd[1]) e[1] = CA * e[1] + CB * d0z - CB * d2x;
-        if (upd[2]) e[2] = CA * e[2] + CB * d1x - CB * d0y;
-        if (disp)
-            for (int c = 0; c < 3; ++c)
-                if (upd[c]) e[c] = e[c] - IEA * phi[c];
-        for (int s = 0; s < a.nslab; ++s) {
-            const InvSlab &S = a.slab[s];
-            if (!in_e(S, i, j, k)) continue;
-            int p;
-            int q[2];
-            pidx(S, true, i, j, k, p, q[0], q[1]);
-            const float RA01 = S.RE[p] - 1.0f, RB0 = S.RE[S.t + p], RE0 = S.RE[2 * S.t + p],
-                        RF0 = S.RE[3 * S.t + p];
-            const float ph2[2] = {S.PE1[q[0]], S.PE2[q[1]]};  // both loads before either store
-            for (int w = 0; w < 2; ++w) {
-                int comp, src, sign;
-                e_pair(S.axis, w, comp, src, sign);
-                float *Phi = w == 0 ? S.PE1 : S.PE2;
-                const float dd = (a.H[src][o] - a.H[src][om[S.axis]]) / a.d;
-                const float ph = ph2[w];
-                const float corr = IEA * (RA01 * dd + RB0 * ph);
-                Phi[q[w]] = RE0 * ph - RF0 * dd;
-                e[comp] = sign > 0 ? e[comp] + corr : e[comp] - corr;
-            }
+        phi[c] = ph;
+    }
+    if (upd[0]) e[0] = CA * e[0] + CB * d2y - CB * d1z;
+    if (upd[1]) e[1] = CA * e[1] + CB * d0z - CB * d2x;
+    if (upd[2]) e[2] = CA * e[2] + CB * d1x - CB * d0y;
+    if (disp)
+        for (int c = 0; c < 3; ++c)
+            if (upd[c]) e[c] = e[c] - IEA * phi[c];
+    for (int s = 0; s < a.nslab; ++s) {
+        const InvSlab &S = a.slab[s];
+        if (!in_e(S, i, j, k)) continue;
+        int p;
+        int q[2];
+        pidx(S, true, i, j, k, p, q[0], q[1]);
+        const float RA01 = S.RE[p] - 1.0f, RB0 = S.RE[S.t + p], RE0 = S.RE[2 * S.t + p], RF0 = S.RE[3 * S.t + p];
+        for (int w = 0; w < 2; ++w) {
+            int comp, src, sign;
+            e_pair(S.axis, w, comp, src, sign);
+            float *Phi = w == 0 ? S.PE1 : S.PE2;
+            const float dd = dH(src, S.axis) / a.d;
+            const float ph = Phi[q[w]];
+            const float corr = IEA * (RA01 * dd + RB0 * ph);
+            Phi[q[w]] = RE0 * ph - RF0 * dd;
+            e[comp] = sign > 0 ? e[comp] + corr : e[comp] - corr;
         }
-        if (i == a.si && j == a.sj && k == a.sk)
-            e[2] = e[2] - IEA * a.waves[a.it] * a.sfac;
-        if (disp)  // dispersive part B
-            for (int c = 0; c < 3; ++c) {
-                if (!upd[c]) continue;
-                for (int p = 0; p < a.P; ++p) {
-                    const float zt = a.dc[(long long)(2 * a.P + p) * a.ncell + oc];
-                    a.T[c][(long long)p * a.ntot + o] = tv[c][p] - zt * e[c];
-                }
-            }
-        a.E[0][o] = e[0];
-        a.E[1][o] = e[1];
-        a.E[2][o] = e[2];
-        if (a.EC) {  // E^n, then the curl of H^{n+1} in the form dL/dCB reads it
-            float2 *q = reinterpret_cast<float2 *>(a.EC) + 3 * (size_t)o;
-            q[0] = make_float2(en[0], en[1]);
-            q[1] = make_float2(en[2], d2y - d1z);
-            q[2] = make_float2(d0z - d2x, d1x - d0y);
-        }
-        if (disp && a.Ps[0])
-            for (int c = 0; c < 3; ++c) a.Ps[c][o] = phi[c];
+    }
+    if (i == b.si && j == b.sj && k == b.sk) e[2] = e[2] - IEA * b.w * b.sfac;
+    for (int c = 0; c < 3; ++c) {
+        if (disp && upd[c])  // dispersive part B
+            for (int p = 0; p < a.P; ++p)
+                b.T[(c * a.P + p) * a.n + o] = tv[c][p] - b.dc[(2 * a.P + p) * a.n + o] * e[c];
+        b.En[c * a.n + o] = e[c];
+    }
+    if (b.curl) {  // the curl of H^{n+1} in the form dL/dCB reads it, and phi^n
+        b.curl[o] = d2y - d1z;
+        b.curl[a.n + o] = d0z - d2x;
+        b.curl[2 * a.n + o] = d1x - d0y;
+        for (int c = 0; c < 3 && a.P; ++c) b.phi[c * a.n + o] = phi[c];
     }
 }
 
 // ------------------------------------------------------------------ adjoint
-// lE, lH, mE, mH live in a.E, a.H and the slab Phi pointers.
-
 // dL/d(dd) of one E-PML term at E edge (comp of the pair w) of slab S; zero
 // outside the slab's E box.
 __device__ __forceinline__ float e_pml_ldd(const InvArgs &a, const InvSlab &S, int w, int i, int j, int k)
@@ -383,10 +317,10 @@ __device__ __forceinline__ float e_pml_ldd(const InvArgs &a, const InvSlab &S, i
     int q[2];
     pidx(S, true, i, j, k, p, q[0], q[1]);
     const float RA01 = S.RE[p] - 1.0f, RF0 = S.RE[3 * S.t + p];
-    const float IEA = (i < a.nx && j < a.ny && k < a.nz) ? a.IEA[cidx(a, i, j, k)] : 0.f;
-    const float lF = comp3(a.lE[fidx(a, i, j, k)], comp);
+    const int o = fidx(a, i, j, k);
+    const float lF = at3(a, a.b.lE, comp, o);
     const float mu = (w == 0 ? S.PE1 : S.PE2)[q[w]];
-    return (float)sign * IEA * RA01 * lF - RF0 * mu;
+    return (float)sign * at3(a, a.b.mat, 2, o) * RA01 * lF - RF0 * mu;
 }
 
 __device__ __forceinline__ float h_pml_ldd(const InvArgs &a, const InvSlab &S, int w, int i, int j, int k)
@@ -398,419 +332,180 @@ __device__ __forceinline__ float h_pml_ldd(const InvArgs &a, const InvSlab &S, i
     int q[2];
     pidx(S, false, i, j, k, p, q[0], q[1]);
     const float RA01 = S.RH[p] - 1.0f, RF0 = S.RH[3 * S.t + p];
-    const float lF = comp3(a.lH[fidx(a, i, j, k)], comp);
+    const float lF = at3(a, a.b.H, comp, fidx(a, i, j, k));
     const float mu = (w == 0 ? S.PH1 : S.PH2)[q[w]];
-    return (float)sign * a.cH * RA01 * lF - RF0 * mu;
+    return (float)sign * a.b.cH * RA01 * lF - RF0 * mu;
 }
 
-// Reverse of the dispersive parts of updated E edge (c, o) of cell oc, given
-// lE* = dL/dE^{n+1} with the B part folded in (k_adj_disp): lE^n gains
-// sum_p zt_p lT_p, lT_p becomes eqt_p lT_p - IEA ee_p lE*, and dL/dIEA
-// gains -lE* phi^n.
-__device__ __forceinline__ void disp_reverse(const InvArgs &a, int c, int o, int oc, float IEA, float lEs,
-                                             float &out, float &giea)
-{
-    float add = 0.f;
-    for (int p = 0; p < a.P; ++p) {
-        const float ee = a.dc[(long long)p * a.ncell + oc];
-        const float eq = a.dc[(long long)(a.P + p) * a.ncell + oc];
-        const float zt = a.dc[(long long)(2 * a.P + p) * a.ncell + oc];
-        float *lt = a.T[c] + (long long)p * a.ntot + o;
-        const float l = *lt;
-        add = add + zt * l;
-        *lt = eq * l - IEA * ee * lEs;
-    }
-    out = out + add;
-    giea += -lEs * a.Ps[c][o];
-}
-
-// lE* = lE - sum_p zt_p lT_p on the updated E edges of cells with poles: the
-// adjoint of E^{n+1} as the E update sees it (B subtracts zt_p E^{n+1} from
-// T^{n+1}).  Runs before the E gathers of the same iteration.
-__global__ void k_adj_disp(InvArgs a)
-{
-    int i, j, k;
-    if (!all_point(a, i, j, k) || k >= a.nz || j >= a.ny || i >= a.nx) return;
-    const int o = fidx(a, i, j, k), oc = cidx(a, i, j, k);
-    const float4 v = a.lE[o];
-    float l3[3] = {v.x, v.y, v.z};
-    for (int c = 0; c < 3; ++c) {
-        if (!e_upd(a, c, i, j, k)) continue;
-        float l = l3[c];
-        for (int p = 0; p < a.P; ++p)
-            l = l - a.dc[(long long)(2 * a.P + p) * a.ncell + oc] * a.T[c][(long long)p * a.ntot + o];
-        l3[c] = l;
-    }
-    a.lE[o] = make_float4(l3[0], l3[1], l3[2], v.w);
-}
-
-// The adjoint fields at the start of the backward: zero, with CB of the
-// point's cell in the w of both lE copies and its CA in the w of lH (0 where
-// the point is no cell).
-__global__ void k_adj_init(InvArgs a)
-{
-    int i, j, k;
-    if (!all_point(a, i, j, k) || k > a.nz) return;
-    const int o = fidx(a, i, j, k);
-    const bool cell = i < a.nx && j < a.ny && k < a.nz;
-    const float cb = cell ? a.CB[cidx(a, i, j, k)] : 0.f, ca = cell ? a.CA[cidx(a, i, j, k)] : 0.f;
-    a.lE[o] = make_float4(0.f, 0.f, 0.f, cb);
-    a.lEn[o] = make_float4(0.f, 0.f, 0.f, cb);
-    a.lH[o] = make_float4(0.f, 0.f, 0.f, ca);
-}
-
-// lEz^n at point (i, j, k) after the H half: v plus dL/d(trace sample of
-// iteration it) of every receiver on the point, in receiver order.
-__device__ __forceinline__ float adj_rx_add(const InvArgs &a, int i, int j, int k, float v)
-{
-    if (!a.rxrow[i * (a.ny + 1) + j]) return v;
-    for (int r = 0; r < a.nrx; ++r) {
-        const int *c = a.rxc + 3 * r;
-        if (c[0] == i && c[1] == j && c[2] == k) v += a.resid[(long long)r * a.iterations + a.it];
-    }
-    return v;
-}
-
-// CB of the cell of E edge (i, j, k) times lE_c there, when that edge is updated.
+// CB of the cell of E edge (i, j, k) times lE_c there, when that edge is
+// updated; DB times lH_c at H cell (i, j, k), likewise.
 __device__ __forceinline__ float xi(const InvArgs &a, int c, int i, int j, int k)
 {
     if (!e_upd(a, c, i, j, k)) return 0.f;
-    const float4 v = a.lE[fidx(a, i, j, k)];  // w: CB of the cell
-    return v.w * comp3(v, c);
+    const int o = fidx(a, i, j, k);
+    return at3(a, a.b.mat, 1, o) * at3(a, a.b.lE, c, o);
 }
-
-// Reverse of the E half of iteration n, one thread per grid point:
-//   lH    += (dE^{n+1}/dH^{n+1})^T lE^{n+1}      (curl and E-PML terms, a gather)
-//   lE^n   = CA lE^{n+1} on updated edges (else unchanged), into En
-//   mE^n   = RE mE^{n+1} + (dE^{n+1}/dPhiE^n)^T lE^{n+1}, into the Q arrays
-//   gradients of the cell from lE^{n+1}, the saved E^n and curl H^{n+1}.
-// lE^{n+1} and mE^{n+1} are only read, so neighbours see consistent values.
-// FAST = true runs over the points of the fast box only (every lane of a wave
-// takes the short path); FAST = false over all other points.
-template <bool FAST>
-__device__ __forceinline__ void adj_e_point(const InvArgs &a, int bx, int by)
-{
-    {
-        // launched over (segments of a (j, k) plane, i) of the fast box (FAST),
-        // every lane a point of the plane, or over the shell boxes
-        int i, j, k;
-        if (FAST) {
-            const int fz = a.fast[5] - a.fast[4], t = bx * blockDim.x + threadIdx.x;
-            if (t >= (a.fast[3] - a.fast[2]) * fz) return;
-            k = a.fast[4] + t % fz;
-            j = a.fast[2] + t / fz;
-            i = a.fast[0] + by;
-        } else {
-            // the shell around the fast box, as up to six disjoint boxes
-            // (blockIdx.y), each enumerated flat so every lane has a point
-            const int *lo = a.shell[by], *hi = a.shell[by] + 3;
-            const int sx = hi[0] - lo[0], sy = hi[1] - lo[1], sz = hi[2] - lo[2];
-            const int t = bx * blockDim.x + threadIdx.x;
-            if (sx <= 0 || sy <= 0 || sz <= 0 || t >= sx * sy * sz) return;
-            k = lo[2] + t % sz;
-            j = lo[1] + (t / sz) % sy;
-            i = lo[0] + t / (sz * sy);
-        }
-        const int g = fidx(a, i, j, k);
-        if (FAST) {
-            // The same arithmetic with direct offsets: every edge involved is
-            // updated and no PML term exists here.
-            const int o = g;
-            const int NZ1 = a.nz + 1, PL = (a.ny + 1) * NZ1;
-            const int oc = cidx(a, i, j, k);
-            // CB lE at the point and at its k+1, j+1 and i+1 neighbours (the
-            // w of each is CB of that point's cell).
-            // Every load comes before the first store: the compiler cannot
-            // move a load above a store through these pointers, and a load
-            // after a store costs the point a second memory round trip.
-            const float4 q0 = a.lE[o], qk = a.lE[o + 1], qj = a.lE[o + NZ1], qi = a.lE[o + PL];
-            const float dh0 = q0.w * q0.y - qk.w * qk.y - q0.w * q0.z + qj.w * qj.z;
-            const float dh1 = q0.w * q0.z - qi.w * qi.z - q0.w * q0.x + qk.w * qk.x;
-            const float dh2 = q0.w * q0.x - qj.w * qj.x - q0.w * q0.y + qi.w * qi.y;
-            const float lE[3] = {q0.x, q0.y, q0.z};
-            const float4 hq = a.lH[o];  // w: CA of the cell
-            const float CA = hq.w;
-            const float2 *sq = reinterpret_cast<const float2 *>(a.EC) + 3 * (size_t)o;
-            const float2 s0 = sq[0], s1 = sq[1], s2 = sq[2];
-            const float En[3] = {s0.x, s0.y, s1.x}, curl[3] = {s1.y, s2.x, s2.y};
-            float gca = 0.f, gcb = 0.f;
-            for (int c = 0; c < 3; ++c) {
-                gca += lE[c] * En[c];
-                gcb += lE[c] * curl[c];
-            }
-            const float2 gab = a.gCAB[oc];
-            const float gca0 = gab.x, gcb0 = gab.y;
-            a.lH[o] = make_float4(hq.x + dh0, hq.y + dh1, hq.z + dh2, hq.w);
-            a.gCAB[oc] = make_float2(gca0 + gca, gcb0 + gcb);
-            float giea = 0.f;
-            if (i == a.si && j == a.sj && k == a.sk) giea += -lE[2] * a.waves[a.it] * a.sfac;
-            float out[3] = {CA * lE[0], CA * lE[1], CA * lE[2]};
-            if (a.P > 0) {
-                const float IEA = a.IEA[oc];
-                for (int c = 0; c < 3; ++c) disp_reverse(a, c, o, oc, IEA, lE[c], out[c], giea);
-            }
-            if (giea != 0.f) a.gIEA[oc] += giea;
-            a.lEn[o] = make_float4(out[0], out[1], out[2], q0.w);
-            return;
-        }
-        // Ex(i,j,k) = ... + CB (Hz(i,j,k) - Hz(i,j-1,k)) - CB (Hy(i,j,k) - Hy(i,j,k-1))
-        // Ey(i,j,k) = ... + CB (Hx(i,j,k) - Hx(i,j,k-1)) - CB (Hz(i,j,k) - Hz(i-1,j,k))
-        // Ez(i,j,k) = ... + CB (Hy(i,j,k) - Hy(i-1,j,k)) - CB (Hx(i,j,k) - Hx(i,j-1,k))
-        float dh[3];
-        if (i >= 1 && i + 2 <= a.nx && j >= 1 && j + 2 <= a.ny && k >= 1 && k + 2 <= a.nz) {
-            // every edge the curl terms read is updated: xi without its range
-            // checks, as on the fast path (same terms, same order)
-            const int o = g, NZ1 = a.nz + 1, PL = (a.ny + 1) * NZ1;
-            const float4 q0 = a.lE[o], qk = a.lE[o + 1], qj = a.lE[o + NZ1], qi = a.lE[o + PL];
-            dh[0] = q0.w * q0.y - qk.w * qk.y - q0.w * q0.z + qj.w * qj.z;
-            dh[1] = q0.w * q0.z - qi.w * qi.z - q0.w * q0.x + qk.w * qk.x;
-            dh[2] = q0.w * q0.x - qj.w * qj.x - q0.w * q0.y + qi.w * qi.y;
-        } else {
-            dh[0] = xi(a, 1, i, j, k) - xi(a, 1, i, j, k + 1) - xi(a, 2, i, j, k) + xi(a, 2, i, j + 1, k);
-            dh[1] = xi(a, 2, i, j, k) - xi(a, 2, i + 1, j, k) - xi(a, 0, i, j, k) + xi(a, 0, i, j, k + 1);
-            dh[2] = xi(a, 0, i, j, k) - xi(a, 0, i, j + 1, k) - xi(a, 1, i, j, k) + xi(a, 1, i + 1, j, k);
-        }
-        const int o = g;
-        // Loads first (see the fast path), then the stores.
-        const float4 le = a.lE[o];
-        float lE[3] = {le.x, le.y, le.z};
-        float out[3] = {lE[0], lE[1], lE[2]};
-        const float4 hq = a.lH[o];  // w: CA of the cell (0 where the point is no cell)
-        const bool cell = i < a.nx && j < a.ny && k < a.nz;
-        float gca = 0.f, gcb = 0.f, gca0 = 0.f, gcb0 = 0.f;
-        int oc = 0;
-        float CA = 0.f, IEA = 0.f;
-        if (cell) {
-            oc = cidx(a, i, j, k);
-            const int om[3] = {i > 0 ? fidx(a, i - 1, j, k) : o, j > 0 ? fidx(a, i, j - 1, k) : o,
-                                     k > 0 ? o - 1 : o};
-            CA = hq.w;
-            IEA = a.IEA[oc];
-            const float2 *sq = reinterpret_cast<const float2 *>(a.EC) + 3 * (size_t)o;
-            const float2 s0 = sq[0], s1 = sq[1], s2 = sq[2];
-            const float En[3] = {s0.x, s0.y, s1.x}, curl[3] = {s1.y, s2.x, s2.y};
-            for (int c = 0; c < 3; ++c) {
-                if (!e_upd(a, c, i, j, k)) continue;
-                gca += lE[c] * En[c];
-                gcb += lE[c] * curl[c];
-            }
-            const float2 gab = a.gCAB[oc];
-            gca0 = gab.x;
-            gcb0 = gab.y;
-        }
-        // E-PML: dd = (S(e) - S(e - axis)) / d uses H at the edge and at edge - axis,
-        // so H here feeds the edge here (+) and the edge one step up the axis (-).
-        // The edge's own term (e_pml_ldd of the edge, with its lE and IEA, 0
-        // outside the cells) shares the slab index, profile values and Phi
-        // adjoints with the update of the Phi adjoints, mE^n = RE mE^{n+1} +
-        // (dE/dPhiE)^T lE, written into the Q arrays (edges of cells only;
-        // edges outside the cells are never updated).
-        for (int s = 0; s < a.nslab; ++s) {
-            const InvSlab &S = a.slab[s];
-            if (!in_box3(S.gE_lo, S.gE_hi, i, j, k)) continue;
-            const bool own = in_e(S, i, j, k);
-            int p = 0;
-            int q[2] = {0, 0};
-            float mu[2] = {0.f, 0.f}, RA01 = 0.f, RB0 = 0.f, RE0 = 0.f, RF0 = 0.f;
-            if (own) {
-                pidx(S, true, i, j, k, p, q[0], q[1]);
-                RA01 = S.RE[p] - 1.0f;
-                RB0 = S.RE[S.t + p];
-                RE0 = S.RE[2 * S.t + p];
-                RF0 = S.RE[3 * S.t + p];
-                mu[0] = S.PE1[q[0]];
-                mu[1] = S.PE2[q[1]];
-            }
-            const int ip = i + (S.axis == 0), jp = j + (S.axis == 1), kp = k + (S.axis == 2);
-            for (int w = 0; w < 2; ++w) {
-                int comp, src, sign;
-                e_pair(S.axis, w, comp, src, sign);
-                const float ldd = own ? (float)sign * IEA * RA01 * lE[comp] - RF0 * mu[w] : 0.f;
-                dh[src] += (ldd - e_pml_ldd(a, S, w, ip, jp, kp)) / a.d;
-                if (own && cell) (w == 0 ? S.QE1 : S.QE2)[q[w]] = RE0 * mu[w] + (float)sign * IEA * RB0 * lE[comp];
-            }
-        }
-        a.lH[o] = make_float4(hq.x + dh[0], hq.y + dh[1], hq.z + dh[2], hq.w);
-        if (cell) {  // edges outside the cells are never updated
-            float giea = 0.f;
-            for (int c = 0; c < 3; ++c) {
-                if (!e_upd(a, c, i, j, k)) continue;
-                out[c] = CA * lE[c];
-                if (a.P > 0) disp_reverse(a, c, o, oc, IEA, lE[c], out[c], giea);
-            }
-            if (i == a.si && j == a.sj && k == a.sk) giea += -lE[2] * a.waves[a.it] * a.sfac;
-            a.gCAB[oc] = make_float2(gca0 + gca, gcb0 + gcb);
-            if (giea != 0.f) a.gIEA[oc] += giea;
-        }
-        a.lEn[o] = make_float4(out[0], out[1], out[2], le.w);
-    }
-}
-
-template <bool FAST>
-__global__ void k_adj_e(InvArgs a)
-{
-    adj_e_point<FAST>(a, blockIdx.x, blockIdx.y);
-}
-
-// DB times lH_c at H cell (i, j, k), when that cell is updated.
 __device__ __forceinline__ float eta(const InvArgs &a, int c, int i, int j, int k)
 {
     if (!h_upd(a, c, i, j, k)) return 0.f;
-    return a.DB * comp3(a.lH[fidx(a, i, j, k)], c);
+    return a.b.DB * at3(a, a.b.H, c, fidx(a, i, j, k));
+}
+
+// Reverse of the E half of iteration n, one thread per grid point:
+//   lH    += (dE^{n+1}/dH^{n+1})^T lE*      (curl and E-PML terms, a gather)
+//   mE^n   = RE mE^{n+1} + (dE^{n+1}/dPhiE^n)^T lE*, into the Q arrays
+//   gradients of the cell from lE*, the saved E^n and curl H^{n+1}.
+__global__ void k_adj_e(InvArgs a)
+{
+    int i, j, k;
+    if (!all_point(a, i, j, k) || k > a.nz) return;
+    const InvStep &b = a.b;
+    const int o = fidx(a, i, j, k);
+    // Ex(i,j,k) = ... + CB (Hz(i,j,k) - Hz(i,j-1,k)) - CB (Hy(i,j,k) - Hy(i,j,k-1))
+    // Ey(i,j,k) = ... + CB (Hx(i,j,k) - Hx(i,j,k-1)) - CB (Hz(i,j,k) - Hz(i-1,j,k))
+    // Ez(i,j,k) = ... + CB (Hy(i,j,k) - Hy(i-1,j,k)) - CB (Hx(i,j,k) - Hx(i,j-1,k))
+    float dh[3];
+    dh[0] = xi(a, 1, i, j, k) - xi(a, 1, i, j, k + 1) - xi(a, 2, i, j, k) + xi(a, 2, i, j + 1, k);
+    dh[1] = xi(a, 2, i, j, k) - xi(a, 2, i + 1, j, k) - xi(a, 0, i, j, k) + xi(a, 0, i, j, k + 1);
+    dh[2] = xi(a, 0, i, j, k) - xi(a, 0, i, j + 1, k) - xi(a, 1, i, j, k) + xi(a, 1, i + 1, j, k);
+    const float lE[3] = {at3(a, b.lE, 0, o), at3(a, b.lE, 1, o), at3(a, b.lE, 2, o)};
+    const bool cell = i < a.nx && j < a.ny && k < a.nz;
+    const float IEA = b.mat[2 * a.n + o];
+    // E-PML: dd = (S(e) - S(e - axis)) / d uses H at the edge and at edge - axis,
+    // so H here feeds the edge here (+) and the edge one step up the axis (-).
+    for (int s = 0; s < a.nslab; ++s) {
+        const InvSlab &S = a.slab[s];
+        if (!in_box3(S.gE_lo, S.gE_hi, i, j, k)) continue;
+        const bool own = in_e(S, i, j, k);
+        int p = 0;
+        int q[2] = {0, 0};
+        if (own) pidx(S, true, i, j, k, p, q[0], q[1]);
+        const int ip = i + (S.axis == 0), jp = j + (S.axis == 1), kp = k + (S.axis == 2);
+        for (int w = 0; w < 2; ++w) {
+            int comp, src, sign;
+            e_pair(S.axis, w, comp, src, sign);
+            dh[src] += (e_pml_ldd(a, S, w, i, j, k) - e_pml_ldd(a, S, w, ip, jp, kp)) / a.d;
+            if (own && cell)
+                (w == 0 ? S.QE1 : S.QE2)[q[w]] = S.RE[2 * S.t + p] * (w == 0 ? S.PE1 : S.PE2)[q[w]] +
+                                                 (float)sign * IEA * S.RE[S.t + p] * lE[comp];
+        }
+    }
+    for (int c = 0; c < 3; ++c) b.H[c * a.n + o] += dh[c];
+    if (!cell) return;
+    float gca = 0.f, gcb = 0.f, giea = 0.f;
+    for (int c = 0; c < 3; ++c) {
+        if (!e_upd(a, c, i, j, k)) continue;
+        gca += lE[c] * at3(a, b.E, c, o);
+        gcb += lE[c] * at3(a, b.curl, c, o);
+    }
+    if (i == b.si && j == b.sj && k == b.sk) giea += -lE[2] * b.w * b.sfac;
+    for (int c = 0; c < 3 && a.P; ++c)
+        if (e_upd(a, c, i, j, k)) giea += -lE[c] * at3(a, b.phi, c, o);
+    b.grad[o] += gca;
+    b.grad[a.n + o] += gcb;
+    if (giea != 0.f) b.grad[2 * a.n + o] += giea;
 }
 
 // Reverse of the H half of iteration n (lH = dL/dH^{n+1}, complete):
-//   lE^n  += (dH^{n+1}/dE^n)^T lH                  (curl and H-PML terms, a gather)
+//   lE^n   = CA lE* (+ the poles) on updated edges + (dH^{n+1}/dE^n)^T lH (a gather)
 //   mH^n   = RE mH^{n+1} + (dH^{n+1}/dPhiH^n)^T lH, into the Q arrays
-// and lH^n = DA lH = lH.
-// FAST = true runs over the points of the fast box only (every lane of a wave
-// takes the short path); FAST = false over all other points.
-template <bool FAST>
-__device__ __forceinline__ void adj_h_point(const InvArgs &a, int bx, int by)
+//   lT one iteration back, and lE* of iteration n-1 from it.
+__global__ void k_adj_h(InvArgs a)
 {
-    {
-        // launched over (segments of a (j, k) plane, i) of the fast box (FAST),
-        // every lane a point of the plane, or over the shell boxes
-        int i, j, k;
-        if (FAST) {
-            const int fz = a.fast[5] - a.fast[4], t = bx * blockDim.x + threadIdx.x;
-            if (t >= (a.fast[3] - a.fast[2]) * fz) return;
-            k = a.fast[4] + t % fz;
-            j = a.fast[2] + t / fz;
-            i = a.fast[0] + by;
-        } else {
-            // the shell around the fast box, as up to six disjoint boxes
-            // (blockIdx.y), each enumerated flat so every lane has a point
-            const int *lo = a.shell[by], *hi = a.shell[by] + 3;
-            const int sx = hi[0] - lo[0], sy = hi[1] - lo[1], sz = hi[2] - lo[2];
-            const int t = bx * blockDim.x + threadIdx.x;
-            if (sx <= 0 || sy <= 0 || sz <= 0 || t >= sx * sy * sz) return;
-            k = lo[2] + t % sz;
-            j = lo[1] + (t / sz) % sy;
-            i = lo[0] + t / (sz * sy);
+    int i, j, k;
+    if (!all_point(a, i, j, k) || k > a.nz) return;
+    const InvStep &b = a.b;
+    const int o = fidx(a, i, j, k);
+    // Hx(i,j,k) = Hx - DB (Ez(i,j+1,k) - Ez(i,j,k)) + DB (Ey(i,j,k+1) - Ey(i,j,k))
+    // Hy(i,j,k) = Hy - DB (Ex(i,j,k+1) - Ex(i,j,k)) + DB (Ez(i+1,j,k) - Ez(i,j,k))
+    // Hz(i,j,k) = Hz - DB (Ey(i+1,j,k) - Ey(i,j,k)) + DB (Ex(i,j+1,k) - Ex(i,j,k))
+    float de[3];
+    de[0] = eta(a, 1, i, j, k) - eta(a, 1, i, j, k - 1) - eta(a, 2, i, j, k) + eta(a, 2, i, j - 1, k);
+    de[1] = eta(a, 2, i, j, k) - eta(a, 2, i - 1, j, k) - eta(a, 0, i, j, k) + eta(a, 0, i, j, k - 1);
+    de[2] = eta(a, 0, i, j, k) - eta(a, 0, i, j - 1, k) - eta(a, 1, i, j, k) + eta(a, 1, i - 1, j, k);
+    const float lH[3] = {at3(a, b.H, 0, o), at3(a, b.H, 1, o), at3(a, b.H, 2, o)};
+    // H-PML: dd = (S(h + axis) - S(h)) / d, so E here feeds the cell here (-)
+    // and the cell one step down the axis (+).
+    for (int s = 0; s < a.nslab; ++s) {
+        const InvSlab &S = a.slab[s];
+        if (!in_box3(S.gH_lo, S.gH_hi, i, j, k)) continue;
+        const bool own = in_h(S, i, j, k);
+        int p = 0;
+        int q[2] = {0, 0};
+        if (own) pidx(S, false, i, j, k, p, q[0], q[1]);
+        const int im = i - (S.axis == 0), jm = j - (S.axis == 1), km = k - (S.axis == 2);
+        for (int w = 0; w < 2; ++w) {
+            int comp, src, sign;
+            h_pair(S.axis, w, comp, src, sign);
+            de[src] += (h_pml_ldd(a, S, w, im, jm, km) - h_pml_ldd(a, S, w, i, j, k)) / a.d;
+            if (own)
+                (w == 0 ? S.QH1 : S.QH2)[q[w]] = S.RH[2 * S.t + p] * (w == 0 ? S.PH1 : S.PH2)[q[w]] +
+                                                 (float)sign * b.cH * S.RH[S.t + p] * lH[comp];
         }
-        const int g = fidx(a, i, j, k);
-        if (FAST) {
-            const int o = g;
-            const int NZ1 = a.nz + 1, PL = (a.ny + 1) * NZ1;
-            // DB lH at the point and at its k-1, j-1 and i-1 neighbours
-            const float4 h0 = a.lH[o], hk = a.lH[o - 1], hj = a.lH[o - NZ1], hi = a.lH[o - PL];
-            const float DB = a.DB;
-            const float de0 = DB * h0.y - DB * hk.y - DB * h0.z + DB * hj.z;
-            const float de1 = DB * h0.z - DB * hi.z - DB * h0.x + DB * hk.x;
-            const float de2 = DB * h0.x - DB * hj.x - DB * h0.y + DB * hi.y;
-            const float4 e = a.lE[o];
-            a.lE[o] = make_float4(e.x + de0, e.y + de1, adj_rx_add(a, i, j, k, e.z + de2), e.w);
-            return;
-        }
-        // Hx(i,j,k) = Hx - DB (Ez(i,j+1,k) - Ez(i,j,k)) + DB (Ey(i,j,k+1) - Ey(i,j,k))
-        // Hy(i,j,k) = Hy - DB (Ex(i,j,k+1) - Ex(i,j,k)) + DB (Ez(i+1,j,k) - Ez(i,j,k))
-        // Hz(i,j,k) = Hz - DB (Ey(i+1,j,k) - Ey(i,j,k)) + DB (Ex(i,j+1,k) - Ex(i,j,k))
-        float de[3];
-        if (i >= 1 && i + 1 <= a.nx && j >= 1 && j + 1 <= a.ny && k >= 1 && k + 1 <= a.nz) {
-            // every cell the curl terms read is updated: eta without its range
-            // checks, as on the fast path (same terms, same order)
-            const int o = g, NZ1 = a.nz + 1, PL = (a.ny + 1) * NZ1;
-            const float4 h0 = a.lH[o], hk = a.lH[o - 1], hj = a.lH[o - NZ1], hi = a.lH[o - PL];
-            const float DB = a.DB;
-            de[0] = DB * h0.y - DB * hk.y - DB * h0.z + DB * hj.z;
-            de[1] = DB * h0.z - DB * hi.z - DB * h0.x + DB * hk.x;
-            de[2] = DB * h0.x - DB * hj.x - DB * h0.y + DB * hi.y;
-        } else {
-            de[0] = eta(a, 1, i, j, k) - eta(a, 1, i, j, k - 1) - eta(a, 2, i, j, k) + eta(a, 2, i, j - 1, k);
-            de[1] = eta(a, 2, i, j, k) - eta(a, 2, i - 1, j, k) - eta(a, 0, i, j, k) + eta(a, 0, i, j, k - 1);
-            de[2] = eta(a, 0, i, j, k) - eta(a, 0, i, j - 1, k) - eta(a, 1, i, j, k) + eta(a, 1, i - 1, j, k);
-        }
-        // Loads first (lH here and lE for the update), then the stores.
-        const float4 lh = a.lH[g];
-        const float lH[3] = {lh.x, lh.y, lh.z};
-        const float4 ev = a.lE[g];
-        // H-PML: dd = (S(h + axis) - S(h)) / d, so E here feeds the cell here (-)
-        // and the cell one step down the axis (+).  The cell's own term
-        // (h_pml_ldd of the cell, with its lH) shares the slab index, profile
-        // values and Phi adjoints with the update of the Phi adjoints, mH^n =
-        // RE mH^{n+1} + (dH/dPhiH)^T lH, written into the Q arrays.
-        for (int s = 0; s < a.nslab; ++s) {
-            const InvSlab &S = a.slab[s];
-            if (!in_box3(S.gH_lo, S.gH_hi, i, j, k)) continue;
-            const bool own = in_h(S, i, j, k);
-            int p = 0;
-            int q[2] = {0, 0};
-            float mu[2] = {0.f, 0.f}, RA01 = 0.f, RB0 = 0.f, RE0 = 0.f, RF0 = 0.f;
-            if (own) {
-                pidx(S, false, i, j, k, p, q[0], q[1]);
-                RA01 = S.RH[p] - 1.0f;
-                RB0 = S.RH[S.t + p];
-                RE0 = S.RH[2 * S.t + p];
-                RF0 = S.RH[3 * S.t + p];
-                mu[0] = S.PH1[q[0]];
-                mu[1] = S.PH2[q[1]];
+    }
+    const float CA = b.mat[o], IEA = b.mat[2 * a.n + o];
+    for (int c = 0; c < 3; ++c) {
+        const float l = at3(a, b.lE, c, o);
+        float out = l;
+        const bool upd = e_upd(a, c, i, j, k);
+        if (upd) {
+            float add = 0.f;
+            for (int p = 0; p < a.P; ++p) {
+                const float ee = b.dc[p * a.n + o], eq = b.dc[(a.P + p) * a.n + o], zt = b.dc[(2 * a.P + p) * a.n + o];
+                float *lt = b.T + (c * a.P + p) * a.n + o;
+                add = add + zt * *lt;
+                *lt = eq * *lt - IEA * ee * l;
             }
-            const int im = i - (S.axis == 0), jm = j - (S.axis == 1), km = k - (S.axis == 2);
-            for (int w = 0; w < 2; ++w) {
-                int comp, src, sign;
-                h_pair(S.axis, w, comp, src, sign);
-                const float ldd = own ? (float)sign * a.cH * RA01 * lH[comp] - RF0 * mu[w] : 0.f;
-                de[src] += (h_pml_ldd(a, S, w, im, jm, km) - ldd) / a.d;
-                if (own) (w == 0 ? S.QH1 : S.QH2)[q[w]] = RE0 * mu[w] + (float)sign * a.cH * RB0 * lH[comp];
-            }
+            out = CA * l;
+            if (a.P) out = out + add;
         }
-        a.lE[g] = make_float4(ev.x + de[0], ev.y + de[1], adj_rx_add(a, i, j, k, ev.z + de[2]), ev.w);
+        out = out + de[c];
+        if (c == 2 && a.rxrow[i * (a.ny + 1) + j])
+            for (int r = 0; r < b.nrx; ++r)
+                if (b.rxc[3 * r] == i && b.rxc[3 * r + 1] == j && b.rxc[3 * r + 2] == k)
+                    out += b.resid[(long long)r * b.iterations + b.it];
+        for (int p = 0; p < a.P && upd; ++p)
+            out = out - b.dc[(2 * a.P + p) * a.n + o] * b.T[(c * a.P + p) * a.n + o];
+        b.lE[c * a.n + o] = out;
     }
 }
 
-template <bool FAST>
-__global__ void k_adj_h(InvArgs a)
+// Cells [nx][ny][nz] of a dense array to points (0 where a point is no cell),
+// and back.
+__global__ void k_inv_to_points(InvArgs a, const float *cells, float *points)
 {
-    adj_h_point<FAST>(a, blockIdx.x, blockIdx.y);
+    int i, j, k;
+    if (!all_point(a, i, j, k) || k >= a.kp) return;
+    const bool cell = i < a.nx && j < a.ny && k < a.nz;
+    points[fidx(a, i, j, k)] = cell ? cells[((long long)i * a.ny + j) * a.nz + k] : 0.f;
 }
-
-// The fast-box and shell blocks of one half-step in one launch: the shell
-// blocks (latency-bound gathers) are spread evenly among the fast ones
-// (bandwidth-bound) so that the two kinds run side by side.  Block b is a
-// shell block when floor((b+1) ns / (nf+ns)) > floor(b ns / (nf+ns)).
-__device__ __forceinline__ bool mix_shell(const InvArgs &a, int b, int &idx)
+__global__ void k_inv_to_cells(InvArgs a, const float *points, float *cells)
 {
-    const long long tot = (long long)a.mix_nf + a.mix_ns;
-    const long long c0 = (long long)b * a.mix_ns / tot, c1 = (long long)(b + 1) * a.mix_ns / tot;
-    idx = c1 > c0 ? (int)c0 : (int)(b - c1);
-    return c1 > c0;
+    int i, j, k;
+    if (!all_point(a, i, j, k) || i >= a.nx || j >= a.ny || k >= a.nz) return;
+    cells[((long long)i * a.ny + j) * a.nz + k] = points[fidx(a, i, j, k)];
 }
-
-__global__ void k_adj_e_mix(InvArgs a)
-{
-    int q;
-    if (mix_shell(a, blockIdx.x, q)) adj_e_point<false>(a, q % a.mix_gs, q / a.mix_gs);
-    else adj_e_point<true>(a, q % a.mix_gf[0], q / a.mix_gf[0]);
-}
-
-__global__ void k_adj_h_mix(InvArgs a)
-{
-    int q;
-    if (mix_shell(a, blockIdx.x, q)) adj_h_point<false>(a, q % a.mix_gs, q / a.mix_gs);
-    else adj_h_point<true>(a, q % a.mix_gf[0], q / a.mix_gf[0]);
-}
-
 
 }  // namespace
 
 // ====================================================================== host
 struct gpx_inv {
     gpx_inv_desc desc;
-    long long ntot = 0, ncell = 0;
+    int kp = 0;                    // floats per row of points
+    long long n = 0, ncell = 0;    // floats of one component (every row of points, rounded up to 64)
     hipStream_t stream = nullptr;
-    float *F = nullptr;            // E, H: 6 x ntot
-    float4 *LE[2] = {nullptr, nullptr};  // adjoint lE, two copies, and lH: one float4
-    float4 *LH = nullptr;                // per grid point each (InvArgs::lE, lH)
-    float *ck = nullptr;           // checkpoints: nck x (6 ntot + phi)
-    float *seg = nullptr;          // segment store: K x 6 x ntot
-    float *par = nullptr;          // CA, CB, IEA: 3 x ncell
-    float *grad = nullptr;         // (gCA, gCB) interleaved per cell, then gIEA: 3 x ncell
-    float *waves = nullptr;
+    float *F = nullptr;            // E, H: 6 n
+    float *L = nullptr;            // adjoint lE, lH: 6 n
+    float *ck = nullptr;           // checkpoints: nck x ck_stride
+    float *seg = nullptr;          // segment store: K x seg_stride
+    float *par = nullptr;          // CA, CB, IEA: 3 n
+    float *grad = nullptr;         // gCA, gCB, gIEA: 3 n
+    float *dense = nullptr;        // ncell: a parameter or gradient as the caller has it
     int P = 0;                     // Debye poles
-    float *dc = nullptr;           // ee, eqt, zt: 3 x P x ncell
-    float *T = nullptr;            // T of Ex, Ey, Ez: 3 x P x ntot
+    float *dc = nullptr;           // ee, eqt, zt: 3 P n
+    float *T = nullptr;            // T of Ex, Ey, Ez: 3 P n
     float *LT = nullptr;           // its adjoint
+    std::vector<float> waves;
     int *rxc = nullptr;
     uint8_t *rxrow = nullptr;      // [nx+1][ny+1]: 1 on the rows of points that hold a receiver
     float *traces = nullptr, *resid = nullptr;
@@ -819,17 +514,28 @@ struct gpx_inv {
     bool have_model = false, have_forward = false;
     struct Slab {
         InvSlab s;
+        int dir;
+        std::vector<float> R[2];         // E, H profiles: RA, RB, RE, RF
         long long n[4] = {0, 0, 0, 0};   // Phi sizes
         float *phi[4] = {nullptr, nullptr, nullptr, nullptr};
         float *mu[4] = {nullptr, nullptr, nullptr, nullptr};
         float *mu2[4] = {nullptr, nullptr, nullptr, nullptr};  // second copies
-        float *R = nullptr;              // E then H tables, 8 t floats
+        float *dR = nullptr;             // E then H tables, 8 t floats
     };
     std::vector<Slab> slabs;
-    long long phi_total = 0;
-    int fast[6] = {0, 0, 0, 0, 0, 0};  // see InvArgs
-    int shell[6][6] = {};              // see InvArgs
-    int shell_max = 0;                 // points of the largest shell box
+    // Which kernels run the model, decided when its slabs or poles have changed
+    // (prepare).  Row kernels: their description, and the Phi of all slabs, per
+    // field 2 x np floats (term 1, term 2).
+    bool dirty = true, rows = false;
+    RowModel *row = nullptr;
+    float *img = nullptr;          // its tables (row_stage)
+    uint32_t *planeflag = nullptr; // [nx + 1]
+    std::vector<uint32_t> slabflag;
+    int items = 0;
+    size_t lds[2] = {0, 0};        // of the E and the H passes
+    long long np = 0;
+    float *phi[2] = {nullptr, nullptr}, *mu[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [E, H], [copy]
+    long long phi_total = 0;       // floats of the forward's Phi
     float ms_fwd = 0, ms_bwd = 0;
     // Segments whose stored states the forward keeps (gpx_inv_set_keep): the
     // last nkeep segments, each K x seg_stride floats, in `keep`; the backward
@@ -861,43 +567,11 @@ extern "C" const char *gpx_inv_last_error(const gpx_inv *v)
     return v ? v->err.c_str() : g_inv_err.c_str();
 }
 
-// The box of grid points where the adjoint kernels need no range check and
-// no PML term: points 1..n-2 on every axis, shrunk past every slab's E box
-// and the edges one below it, and its H box and the cells one above it.
-static void update_fast(gpx_inv *v)
+template <class T>
+static void ifree(T *&p)
 {
-    const int n[3] = {v->desc.nx, v->desc.ny, v->desc.nz};
-    int lo[3] = {1, 1, 1}, hi[3] = {n[0] - 1, n[1] - 1, n[2] - 1};
-    for (const auto &S : v->slabs) {
-        const InvSlab &s = S.s;
-        const int ax = s.axis;
-        if (s.minus) {
-            const int end = s.hiE[ax] > s.hiH[ax] + 1 ? s.hiE[ax] : s.hiH[ax] + 1;
-            if (end > lo[ax]) lo[ax] = end;
-        } else {
-            const int start = s.loE[ax] - 1 < s.loH[ax] ? s.loE[ax] - 1 : s.loH[ax];
-            if (start < hi[ax]) hi[ax] = start;
-        }
-    }
-    for (int q = 0; q < 3; ++q) {
-        v->fast[2 * q] = lo[q];
-        v->fast[2 * q + 1] = hi[q] > lo[q] ? hi[q] : lo[q];
-    }
-    // The grid points [0, n] minus the fast box: below / above it in x (all
-    // y, z), then in y within its x range (all z), then in z within its x
-    // and y ranges.
-    const int N[3] = {n[0] + 1, n[1] + 1, n[2] + 1};
-    const int *f = v->fast;
-    const int boxes[6][6] = {
-        {0, 0, 0, f[0], N[1], N[2]},          {f[1], 0, 0, N[0], N[1], N[2]},
-        {f[0], 0, 0, f[1], f[2], N[2]},       {f[0], f[3], 0, f[1], N[1], N[2]},
-        {f[0], f[2], 0, f[1], f[3], f[4]},    {f[0], f[2], f[5], f[1], f[3], N[2]}};
-    memcpy(v->shell, boxes, sizeof(boxes));
-    v->shell_max = 0;
-    for (auto &b : boxes) {
-        const long long vol = (long long)(b[3] - b[0]) * (b[4] - b[1]) * (b[5] - b[2]);
-        if (vol > v->shell_max) v->shell_max = (int)vol;
-    }
+    if (p) hipFree(p);
+    p = nullptr;
 }
 
 extern "C" int gpx_inv_create(const gpx_inv_desc *d, gpx_inv **out)
@@ -908,28 +582,46 @@ extern "C" int gpx_inv_create(const gpx_inv_desc *d, gpx_inv **out)
         return ifail(nullptr, GPX_EARG, "gpx_inv_create: bad descriptor");
     if (d->nx + 1 > 65535 || d->ny + 1 > 65535)
         return ifail(nullptr, GPX_ELIMIT, "gpx_inv_create: at most 65534 cells along x and y");
-    if ((double)(d->nx + 1) * (d->ny + 1) * (d->nz + 1) >= 2147483647.0)
+    const double rows = (double)(d->nx + 1) * (d->ny + 1);
+    if (rows * (d->nz + 1) >= 2147483647.0)
         return ifail(nullptr, GPX_ELIMIT, "gpx_inv_create: at most 2^31 grid points");
     if (hipSetDevice(d->device) != hipSuccess) return ifail(nullptr, GPX_EARG, "gpx_inv_create: bad device");
     gpx_inv *v = new gpx_inv();
     v->desc = *d;
-    v->ntot = (long long)(d->nx + 1) * (d->ny + 1) * (d->nz + 1);
+    v->kp = (d->nz + 4) & ~3;
+    if (rows * v->kp >= 2147483647.0) v->kp = d->nz + 1;
+    v->n = ((long long)(d->nx + 1) * (d->ny + 1) * v->kp + 63) / 64 * 64;
     v->ncell = (long long)d->nx * d->ny * d->nz;
+    const size_t b = (size_t)v->n * 4;
     hipError_t e = hipStreamCreateWithFlags(&v->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc((void **)&v->F, 6 * v->ntot * 4);
-    for (float4 **p : {&v->LE[0], &v->LE[1], &v->LH})
-        if (e == hipSuccess) e = hipMalloc((void **)p, v->ntot * 16);
-    if (e == hipSuccess) e = hipMalloc((void **)&v->seg, (size_t)d->K * ((6 * v->ntot + 3) / 4 * 4) * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&v->par, 3 * v->ncell * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&v->grad, 3 * v->ncell * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&v->waves, (size_t)d->iterations * 4);
+    if (e == hipSuccess) e = hipMalloc((void **)&v->F, 6 * b);
+    if (e == hipSuccess) e = hipMalloc((void **)&v->L, 6 * b);
+    if (e == hipSuccess) e = hipMalloc((void **)&v->seg, (size_t)d->K * 6 * b);
+    if (e == hipSuccess) e = hipMalloc((void **)&v->par, 3 * b);
+    if (e == hipSuccess) e = hipMalloc((void **)&v->grad, 3 * b);
+    if (e == hipSuccess) e = hipMalloc((void **)&v->dense, v->ncell * 4);
     if (e != hipSuccess) {
         gpx_inv_destroy(v);
         return ifail(nullptr, (int)e, std::string("gpx_inv_create: ") + hipGetErrorString(e));
     }
-    update_fast(v);
     *out = v;
     return 0;
+}
+
+// Phi and its adjoints of both layouts.
+static void free_phi(gpx_inv *v)
+{
+    for (auto &S : v->slabs)
+        for (int q = 0; q < 4; ++q) {
+            ifree(S.phi[q]);
+            ifree(S.mu[q]);
+            ifree(S.mu2[q]);
+        }
+    for (int f = 0; f < 2; ++f) {
+        ifree(v->phi[f]);
+        ifree(v->mu[f][0]);
+        ifree(v->mu[f][1]);
+    }
 }
 
 extern "C" int gpx_inv_destroy(gpx_inv *v)
@@ -937,19 +629,15 @@ extern "C" int gpx_inv_destroy(gpx_inv *v)
     if (!v) return 0;
     hipSetDevice(v->desc.device);
     if (v->stream) hipStreamSynchronize(v->stream);
-    for (float4 *p : {v->LE[0], v->LE[1], v->LH})
+    for (float *p : {v->F, v->L, v->ck, v->seg, v->par, v->grad, v->dense, v->traces, v->resid, v->dc, v->T, v->LT,
+                     v->keep, v->img})
         if (p) hipFree(p);
-    for (float *p : {v->F, v->ck, v->seg, v->par, v->grad, v->waves, v->traces, v->resid, v->dc,
-                     v->T, v->LT, v->keep})
-        if (p) hipFree(p);
-    if (v->rxc) hipFree(v->rxc);
-    if (v->rxrow) hipFree(v->rxrow);
-    for (auto &S : v->slabs) {
-        for (float *p : S.phi) if (p) hipFree(p);
-        for (float *p : S.mu) if (p) hipFree(p);
-        for (float *p : S.mu2) if (p) hipFree(p);
-        if (S.R) hipFree(S.R);
-    }
+    ifree(v->rxc);
+    ifree(v->rxrow);
+    ifree(v->row);
+    ifree(v->planeflag);
+    free_phi(v);
+    for (auto &S : v->slabs) ifree(S.dR);
     if (v->stream) hipStreamDestroy(v->stream);
     delete v;
     return 0;
@@ -970,6 +658,7 @@ extern "C" int gpx_inv_add_pml(gpx_inv *v, int dir, int xs, int xf, int ys, int 
     const int axis = dir % 3, minus = dir < 3;
     const int st[3] = {xs, ys, zs}, en[3] = {xf, yf, zf};
     const int t = en[axis] - st[axis];
+    S.dir = dir;
     s.axis = axis;
     s.minus = minus;
     s.t = t;
@@ -978,8 +667,7 @@ extern "C" int gpx_inv_add_pml(gpx_inv *v, int dir, int xs, int xf, int ys, int 
         s.hiE[n] = s.hiH[n] = en[n];
         s.org[n] = st[n];
     }
-    if (false) {
-    } else if (minus) {  // E cells f - p, H cells f - (p + 1)
+    if (minus) {  // E cells f - p, H cells f - (p + 1)
         s.loE[axis] = en[axis] - t + 1;
         s.hiE[axis] = en[axis] + 1;
         s.pendE = en[axis];
@@ -1016,25 +704,38 @@ extern "C" int gpx_inv_add_pml(gpx_inv *v, int dir, int xs, int xf, int ys, int 
         s.dH1[n] = dims[2][n];
         s.dH2[n] = dims[3][n];
     }
-    for (int q = 0; q < 4; ++q) {
-        S.n[q] = (long long)dims[q][0] * dims[q][1] * dims[q][2];
-        INV_TRY(hipMalloc((void **)&S.phi[q], S.n[q] * 4));
-        INV_TRY(hipMalloc((void **)&S.mu[q], S.n[q] * 4));
-        INV_TRY(hipMalloc((void **)&S.mu2[q], S.n[q] * 4));
-        v->phi_total += S.n[q];
+    for (int q = 0; q < 4; ++q) S.n[q] = (long long)dims[q][0] * dims[q][1] * dims[q][2];
+    S.R[0].assign(eR, eR + 4 * t);
+    S.R[1].assign(hR, hR + 4 * t);
+    INV_TRY(hipMalloc((void **)&S.dR, (size_t)8 * t * 4));
+    hipError_t e = hipMemcpy(S.dR, eR, (size_t)4 * t * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(S.dR + 4 * t, hR, (size_t)4 * t * 4, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        ifree(S.dR);
+        return ifail(v, (int)e, std::string("gpx_inv_add_pml: ") + hipGetErrorString(e));
     }
-    INV_TRY(hipMalloc((void **)&S.R, (size_t)8 * t * 4));
-    INV_TRY(hipMemcpy(S.R, eR, (size_t)4 * t * 4, hipMemcpyHostToDevice));
-    INV_TRY(hipMemcpy(S.R + 4 * t, hR, (size_t)4 * t * 4, hipMemcpyHostToDevice));
-    s.RE = S.R;
-    s.RH = S.R + 4 * t;
+    s.RE = S.dR;
+    s.RH = S.dR + 4 * t;
     v->slabs.push_back(S);
-    update_fast(v);
-    if (v->ck) {  // checkpoint layout depends on the Phi sizes
-        hipFree(v->ck);
-        v->ck = nullptr;
-    }
+    v->dirty = true;
     v->have_forward = false;
+    return 0;
+}
+
+static InvArgs inv_args(const gpx_inv *v);
+static dim3 grid_all(const gpx_inv *v)
+{
+    return dim3((unsigned)(8 * inv_args(v).all_per_xcd));
+}
+
+// `count` arrays of cells from the host to points (the caller waits).
+static int upload_cells(gpx_inv *v, const float *src, int count, float *dst)
+{
+    for (int q = 0; q < count; ++q) {
+        INV_TRY(hipMemcpyAsync(v->dense, src + q * v->ncell, (size_t)v->ncell * 4, hipMemcpyHostToDevice, v->stream));
+        hipLaunchKernelGGL(k_inv_to_points, grid_all(v), dim3(128), 0, v->stream, inv_args(v), v->dense, dst + q * v->n);
+        INV_TRY(hipGetLastError());
+    }
     return 0;
 }
 
@@ -1042,9 +743,10 @@ extern "C" int gpx_inv_set_model(gpx_inv *v, const float *CA, const float *CB, c
 {
     if (!v || !CA || !CB || !IEA) return ifail(v, GPX_EARG, "gpx_inv_set_model: null argument");
     hipSetDevice(v->desc.device);
-    INV_TRY(hipMemcpy(v->par, CA, v->ncell * 4, hipMemcpyHostToDevice));
-    INV_TRY(hipMemcpy(v->par + v->ncell, CB, v->ncell * 4, hipMemcpyHostToDevice));
-    INV_TRY(hipMemcpy(v->par + 2 * v->ncell, IEA, v->ncell * 4, hipMemcpyHostToDevice));
+    const float *src[3] = {CA, CB, IEA};
+    for (int q = 0; q < 3; ++q)
+        if (int rc = upload_cells(v, src[q], 1, v->par + q * v->n)) return rc;
+    INV_TRY(hipStreamSynchronize(v->stream));
     v->have_model = true;
     v->have_forward = false;
     return 0;
@@ -1055,155 +757,261 @@ extern "C" int gpx_inv_set_dispersive(gpx_inv *v, int P, const float *ee, const 
     if (!v || P < 0 || P > INV_MAX_POLES || (P > 0 && (!ee || !eqt || !zt)))
         return ifail(v, GPX_EARG, "gpx_inv_set_dispersive: bad argument (at most 4 poles)");
     hipSetDevice(v->desc.device);
+    const size_t b = (size_t)v->n * 4;
     if (P != v->P) {
-        for (float **p : {&v->dc, &v->T, &v->LT, &v->ck, &v->seg}) {
-            if (*p) hipFree(*p);
-            *p = nullptr;
-        }
+        for (float **p : {&v->dc, &v->T, &v->LT, &v->ck, &v->seg}) ifree(*p);
         v->P = P;
+        v->dirty = true;
         // the segment store keeps phi^n of the three E components beside E^n, curl H^{n+1}
-        INV_TRY(hipMalloc((void **)&v->seg, (size_t)v->desc.K * (((P ? 9 : 6) * v->ntot + 3) / 4 * 4) * 4));
-        if (P) {
-            INV_TRY(hipMalloc((void **)&v->dc, (size_t)3 * P * v->ncell * 4));
-            INV_TRY(hipMalloc((void **)&v->T, (size_t)3 * P * v->ntot * 4));
-            INV_TRY(hipMalloc((void **)&v->LT, (size_t)3 * P * v->ntot * 4));
-        }
+        INV_TRY(hipMalloc((void **)&v->seg, (size_t)v->desc.K * (P ? 9 : 6) * b));
+        if (P)
+            for (float **p : {&v->dc, &v->T, &v->LT}) INV_TRY(hipMalloc((void **)p, (size_t)3 * P * b));
     }
-    const size_t b = (size_t)P * v->ncell * 4;
-    if (P) {
-        INV_TRY(hipMemcpy(v->dc, ee, b, hipMemcpyHostToDevice));
-        INV_TRY(hipMemcpy(v->dc + (size_t)P * v->ncell, eqt, b, hipMemcpyHostToDevice));
-        INV_TRY(hipMemcpy(v->dc + (size_t)2 * P * v->ncell, zt, b, hipMemcpyHostToDevice));
-    }
+    const float *src[3] = {ee, eqt, zt};
+    for (int q = 0; q < 3 && P; ++q)
+        if (int rc = upload_cells(v, src[q], P, v->dc + (size_t)q * P * v->n)) return rc;
+    INV_TRY(hipStreamSynchronize(v->stream));
     v->have_forward = false;
     return 0;
 }
 
 static int n_checkpoints(const gpx_inv *v) { return (v->desc.iterations + v->desc.K - 1) / v->desc.K; }
-static long long ck_stride(const gpx_inv *v) { return 6 * v->ntot + 3 * v->P * v->ntot + v->phi_total; }
-// Floats per iteration in the segment store: E^n and curl H^{n+1} interleaved
-// (6 per point), then phi^n of the three E components with poles; rounded up
-// to 4 floats so that every slot is 16-byte aligned.
-static long long seg_stride(const gpx_inv *v) { return ((v->P ? 9 : 6) * v->ntot + 3) / 4 * 4; }
+static long long ck_stride(const gpx_inv *v) { return 6 * v->n + 3 * v->P * v->n + v->phi_total; }
+// Floats per iteration in the segment store: E^n, curl H^{n+1} and, with poles,
+// phi^n, three components each.
+static long long seg_stride(const gpx_inv *v) { return (v->P ? 9 : 6) * v->n; }
 
-static int all_gk(const gpx_inv *v);
-static int all_blocks(const gpx_inv *v);
+// Whether the row kernels can run the model: whole lanes, slabs in direction
+// order with the two of an axis at least four cells apart (so that a lane and
+// its neighbours see one of them), a cell size row_quot takes, 32-bit byte
+// offsets into arrays of three components (three per pole) and into a Phi array.
+static bool inv_rows_ok(const gpx_inv *v)
+{
+    const gpx_inv_desc &g = v->desc;
+    if (v->kp % 4 != 0 || !(g.d > 1e-12f && g.d < 1.6e7f)) return false;
+    if ((double)v->n * 12.0 * (v->P > 1 ? v->P : 1) >= 4294967295.0) return false;
+    int before = -1, end[3] = {-4, -4, -4};
+    double np = 0;
+    for (const auto &S : v->slabs) {
+        const InvSlab &s = S.s;
+        const int ax = s.axis, lo = s.loE[ax] < s.loH[ax] ? s.loE[ax] : s.loH[ax];
+        if (S.dir <= before || lo - end[ax] < 4) return false;
+        before = S.dir;
+        end[ax] = s.hiE[ax] > s.hiH[ax] ? s.hiE[ax] : s.hiH[ax];
+        np += ((double)s.hiE[0] - s.loE[0]) * ((double)s.hiE[1] - s.loE[1]) * ((double)s.hiE[2] - s.loE[2] + 8);
+    }
+    return np * 8.0 < 2147483647.0;
+}
 
-static InvArgs inv_args(const gpx_inv *v, bool adjoint, int it)
+// Settles the kernels of a model whose slabs or poles have changed, and lays
+// the Phi arrays out for them.
+static int prepare(gpx_inv *v)
+{
+    if (!v->dirty) return 0;
+    const gpx_inv_desc &g = v->desc;
+    INV_TRY(hipStreamSynchronize(v->stream));
+    free_phi(v);
+    ifree(v->ck);
+    v->rows = inv_rows_ok(v);
+    v->phi_total = 0;
+    if (!v->rows) {
+        for (auto &S : v->slabs)
+            for (int q = 0; q < 4; ++q) {
+                for (float **p : {&S.phi[q], &S.mu[q], &S.mu2[q]}) INV_TRY(hipMalloc((void **)p, S.n[q] * 4));
+                v->phi_total += S.n[q];
+            }
+        v->dirty = false;
+        return 0;
+    }
+    RowModel m;
+    memset(&m, 0, sizeof(m));
+    m.nx = g.nx; m.ny = g.ny; m.nz = g.nz;
+    m.kp = v->kp;
+    m.plane = (g.ny + 1) * v->kp;
+    m.cs = (uint32_t)(v->n * 4);
+    const double mu0 = 1.25663706127e-6;
+    m.h[0] = 1.0f;
+    m.h[1] = m.h[2] = m.h[3] = (float)((1.0 / g.d) * (g.dt / mu0));
+    m.h[4] = (float)(g.dt / mu0);
+    int nRT = 0;
+    for (const auto &S : v->slabs) nRT += 4 * S.s.t;
+    const int nI = row_image(0, nRT, 0);
+    std::vector<float> img((size_t)2 * nI + 4, 0.f);
+    v->slabflag.assign(g.nx + 1, 0u);
+    long long np = 0;
+    int first = 0;
+    for (const auto &S : v->slabs) {
+        const InvSlab &s = S.s;
+        int ext[3];
+        for (int q = 0; q < 3; ++q) ext[q] = s.hiE[q] - s.loE[q];
+        const int aE = s.loE[2] & ~3, aH = s.loH[2] & ~3;   // cell k at k mod 4
+        const int nk = ((s.hiE[2] - aE > s.hiH[2] - aH ? s.hiE[2] - aE : s.hiH[2] - aH) + 3) & ~3;
+        for (int f = 0; f < 2; ++f) {
+            RowSlab d;
+            memset(&d, 0, sizeof(d));
+            d.t = s.t;
+            d.pend = f ? s.pendH : s.pendE;
+            d.sign = s.minus ? -1 : 1;
+            for (int q = 0; q < 3; ++q) {
+                d.lo[q] = f ? s.loH[q] : s.loE[q];
+                d.hi[q] = f ? s.hiH[q] : s.hiE[q];
+            }
+            d.sy = nk;
+            d.sx = ext[1] * nk;
+            d.off = (int)(np - (long long)d.lo[0] * d.sx - (long long)d.lo[1] * d.sy - (d.lo[2] & ~3));
+            d.rt = first;
+            d.d = g.d;
+            d.rd = (float)(1.0 / (double)g.d);
+            d.rl = (float)(1.0 / (double)g.d - (double)d.rd);
+            float *rt = img.data() + f * nI, *sl = rt + nRT;
+            for (int p = 0; p < s.t; ++p) {
+                float *e = rt + first + 4 * p;
+                const float *R = S.R[f].data();
+                e[0] = R[p] - 1.0f;
+                e[1] = R[s.t + p];
+                e[2] = R[2 * s.t + p];
+                e[3] = R[3 * s.t + p];
+            }
+            memcpy(sl + S.dir * (sizeof(RowSlab) / 4), &d, sizeof(d));
+            const RowAt w = {d.lo[1], d.hi[1], d.lo[2], d.hi[2], d.off, d.sx, d.sy, 0};
+            (f ? m.atH : m.atE)[S.dir] = w;
+            for (int i = d.lo[0]; i < d.hi[0] && i <= g.nx; ++i)
+                v->slabflag[i] |= 1u << ((f ? PF_SLAB_H : PF_SLAB_E) + S.dir);
+        }
+        first += 4 * s.t;
+        np += (long long)ext[0] * ext[1] * nk;
+    }
+    v->np = np;
+    v->phi_total = 4 * np;
+    for (int f = 0; f < 2 && np; ++f)
+        for (float **p : {&v->phi[f], &v->mu[f][0], &v->mu[f][1]}) INV_TRY(hipMalloc((void **)p, (size_t)2 * np * 4 + 16));
+    ifree(v->img);
+    INV_TRY(hipMalloc((void **)&v->img, img.size() * 4));
+    INV_TRY(hipMemcpy(v->img, img.data(), img.size() * 4, hipMemcpyHostToDevice));
+    m.img = reinterpret_cast<const float4 *>(v->img);
+    m.n4E = m.n4H = nI / 4;
+    m.nRT = nRT;
+    m.np4 = (uint32_t)(np * 4);
+    if (!v->planeflag) INV_TRY(hipMalloc((void **)&v->planeflag, (size_t)(g.nx + 1) * 4));
+    m.planeflag = v->planeflag;
+    // launch shape, as the solver's row passes (pass_items there)
+    const int lanes = (g.ny + 1) * (v->kp / NC);
+    m.pseg = (lanes + 255) / 256;
+    for (m.pxc = 2;; --m.pxc) {
+        m.pitems = m.pseg * ((g.nx + m.pxc) / m.pxc);
+        if (m.pxc == 1 || m.pitems >= 1024) break;
+    }
+    v->items = m.pitems;
+    v->lds[0] = v->lds[1] = (size_t)nI * 4 + 16;
+    if (!v->row) INV_TRY(hipMalloc((void **)&v->row, sizeof(RowModel)));
+    INV_TRY(hipMemcpy(v->row, &m, sizeof(m), hipMemcpyHostToDevice));
+    v->dirty = false;
+    return 0;
+}
+
+// What every launch of a kernel has in common.
+static InvArgs inv_args(const gpx_inv *v)
 {
     InvArgs a;
     memset(&a, 0, sizeof(a));
     const gpx_inv_desc &g = v->desc;
     a.nx = g.nx; a.ny = g.ny; a.nz = g.nz;
-    a.ntot = v->ntot;
+    a.kp = v->kp;
+    a.n = v->n;
     a.d = g.d;
     const double mu0 = 1.25663706127e-6;
-    a.DB = (float)((1.0 / g.d) * (g.dt / mu0));
-    a.cH = (float)(g.dt / mu0);
-    for (int c = 0; c < 3 && !adjoint; ++c) {  // the adjoint fields are set by the backward
-        a.E[c] = v->F + c * v->ntot;
-        a.H[c] = v->F + (3 + c) * v->ntot;
-    }
-    a.CA = v->par;
-    a.CB = v->par + v->ncell;
-    a.IEA = v->par + 2 * v->ncell;
-    a.gCAB = reinterpret_cast<float2 *>(v->grad);
-    a.gIEA = v->grad + 2 * v->ncell;
+    InvStep &b = a.b;
+    b.DB = (float)((1.0 / g.d) * (g.dt / mu0));
+    b.cH = (float)(g.dt / mu0);
+    b.mat = v->par;
+    b.dc = v->dc;
+    b.grad = v->grad;
+    b.rxc = v->rxc;
+    b.resid = v->resid;
+    b.traces = v->traces;
+    b.nrx = v->nrx;
+    b.iterations = g.iterations;
+    b.si = v->si; b.sj = v->sj; b.sk = v->sk;
+    b.sfac = v->sfac;
+    b.nitems = v->items;
+    b.per_xcd = (v->items + 7) / 8;
+    a.P = v->P;
+    a.rxrow = v->rxrow;
     a.nslab = (int)v->slabs.size();
+    for (int s = 0; s < a.nslab; ++s) a.slab[s] = v->slabs[s].s;
+    a.all_gk = (g.nz + 1 + 127) / 128;
+    a.all_blocks = a.all_gk * (g.ny + 1) * (g.nx + 1);
+    a.all_per_xcd = (a.all_blocks + 7) / 8;
+    return a;
+}
+
+// Copies the state (fields, T and Phi) to or from checkpoint c.
+static int checkpoint(gpx_inv *v, int c, bool save)
+{
+    float *at = v->ck + (long long)c * ck_stride(v);
+    auto cp = [&](float *live, long long n) {
+        float *ckp = at;
+        at += n;
+        return save ? hipMemcpyAsync(ckp, live, n * 4, hipMemcpyDeviceToDevice, v->stream)
+                    : hipMemcpyAsync(live, ckp, n * 4, hipMemcpyDeviceToDevice, v->stream);
+    };
+    INV_TRY(cp(v->F, 6 * v->n));
+    if (v->P) INV_TRY(cp(v->T, 3 * v->P * v->n));
+    for (int f = 0; f < 2 && v->rows && v->np; ++f) INV_TRY(cp(v->phi[f], 2 * v->np));
+    for (auto &S : v->slabs)
+        for (int q = 0; q < 4 && !v->rows; ++q) INV_TRY(cp(S.phi[q], S.n[q]));
+    return 0;
+}
+
+static InvKernels inv_kernels_of(const gpx_inv *v)
+{
+    return v->slabs.empty() ? inv_kernels<0>(v->P) : inv_kernels<1>(v->P);
+}
+
+// Forward iterations [n0, n1), one segment or the head of one.  With `store`
+// they leave E^n, curl H^{n+1} (and phi^n) of each in its slot there: E^n is in
+// slot n (copied there for the first) and E^{n+1} goes to slot n+1, after the
+// last one back to the fields.
+static int forward_steps(gpx_inv *v, int n0, int n1, float *store)
+{
+    InvArgs a = inv_args(v);
+    InvStep &b = a.b;
+    const InvKernels k = inv_kernels_of(v);
     for (int s = 0; s < a.nslab; ++s) {
-        a.slab[s] = v->slabs[s].s;
-        float *const *P = adjoint ? v->slabs[s].mu : v->slabs[s].phi;
+        float *const *P = v->slabs[s].phi;
         a.slab[s].PE1 = P[0];
         a.slab[s].PE2 = P[1];
         a.slab[s].PH1 = P[2];
         a.slab[s].PH2 = P[3];
     }
-    a.si = v->si; a.sj = v->sj; a.sk = v->sk;
-    a.sfac = v->sfac;
-    a.waves = v->waves;
-    a.it = it;
-    a.iterations = g.iterations;
-    a.nrx = v->nrx;
-    a.rxc = v->rxc;
-    a.rxrow = v->rxrow;
-    a.traces = v->traces;
-    a.resid = v->resid;
-    a.ncell = v->ncell;
-    a.P = v->P;
-    a.dc = v->dc;
-    for (int c = 0; c < 3 && v->P; ++c) a.T[c] = (adjoint ? v->LT : v->T) + (size_t)c * v->P * v->ntot;
-    memcpy(a.fast, v->fast, sizeof(a.fast));
-    memcpy(a.shell, v->shell, sizeof(a.shell));
-    a.all_gk = all_gk(v);
-    a.all_blocks = all_blocks(v);
-    a.all_per_xcd = (a.all_blocks + 7) / 8;
-    return a;
-}
-
-// Launch shapes: 128 threads along k, one block row per (j, i).  Launches over
-// every point are one-dimensional (all_point): all_gk blocks per row, the
-// block count padded to a multiple of 8.
-static int all_gk(const gpx_inv *v)
-{
-    return (v->desc.nz + 1 + 127) / 128;
-}
-static int all_blocks(const gpx_inv *v)
-{
-    return all_gk(v) * (v->desc.ny + 1) * (v->desc.nx + 1);
-}
-static dim3 grid_all(const gpx_inv *v)
-{
-    return dim3((unsigned)((all_blocks(v) + 7) / 8 * 8));
-}
-// Threads per block of the adjoint gathers (fast-box and shell blocks).
-constexpr int ADJ_BLOCK = 256;  // 64: 3.06x, 128: 2.99x, 256: 2.91x, 512: 2.98x, 1024: 3.12x (kept segments, 160x160x120)
-static dim3 grid_fast(const gpx_inv *v)
-{
-    const int fx = v->fast[1] - v->fast[0], fy = v->fast[3] - v->fast[2], fz = v->fast[5] - v->fast[4];
-    const long long plane = fy > 0 && fz > 0 ? (long long)fy * fz : 1;
-    return dim3((unsigned)((plane + ADJ_BLOCK - 1) / ADJ_BLOCK), fx > 0 ? fx : 1, 1);
-}
-static dim3 grid_shell(const gpx_inv *v)
-{
-    return dim3(v->shell_max > 0 ? (v->shell_max + ADJ_BLOCK - 1) / ADJ_BLOCK : 1, 6, 1);
-}
-static bool fast_empty(const gpx_inv *v)
-{
-    return v->fast[1] <= v->fast[0] || v->fast[3] <= v->fast[2] || v->fast[5] <= v->fast[4];
-}
-
-// Copies the state (fields and Phi) to or from checkpoint c.
-static int checkpoint(gpx_inv *v, int c, bool save)
-{
-    float *dst = v->ck + (long long)c * ck_stride(v);
-    auto cp = [&](float *ckp, float *live, long long n) {
-        return save ? hipMemcpyAsync(ckp, live, n * 4, hipMemcpyDeviceToDevice, v->stream)
-                    : hipMemcpyAsync(live, ckp, n * 4, hipMemcpyDeviceToDevice, v->stream);
-    };
-    INV_TRY(cp(dst, v->F, 6 * v->ntot));
-    long long off = 6 * v->ntot;
-    if (v->P) {
-        INV_TRY(cp(dst + off, v->T, 3 * v->P * v->ntot));
-        off += 3 * v->P * v->ntot;
-    }
-    for (auto &S : v->slabs)
-        for (int q = 0; q < 4; ++q) {
-            INV_TRY(cp(dst + off, S.phi[q], S.n[q]));
-            off += S.n[q];
+    b.E = b.En = v->F;
+    b.H = v->F + 3 * v->n;
+    b.T = v->T;
+    if (store && n0 < n1) INV_TRY(hipMemcpyAsync(store, v->F, (size_t)3 * v->n * 4, hipMemcpyDeviceToDevice, v->stream));
+    for (int it = n0; it < n1; ++it) {
+        b.it = it;
+        b.w = v->waves[it];
+        if (store) {
+            float *slot = store + (long long)(it - n0) * seg_stride(v);
+            b.E = slot;
+            b.En = it + 1 < n1 ? slot + seg_stride(v) : v->F;
+            b.curl = slot + 3 * v->n;
+            b.phi = slot + 6 * v->n;
         }
+        if (v->rows) {
+            const dim3 G(8 * b.per_xcd);
+            b.P = v->phi[1];
+            hipLaunchKernelGGL(k.h, G, dim3(256), v->lds[1], v->stream, v->row, b);
+            b.P = v->phi[0];
+            hipLaunchKernelGGL(k.e, G, dim3(256), v->lds[0], v->stream, v->row, b);
+        } else {
+            const dim3 G(8 * a.all_per_xcd);
+            hipLaunchKernelGGL(k_inv_h, G, dim3(128), 0, v->stream, a);
+            hipLaunchKernelGGL(k_inv_e, G, dim3(128), 0, v->stream, a);
+        }
+    }
+    INV_TRY(hipGetLastError());
     return 0;
-}
-
-// One forward iteration; with `slot`, the kernels also store E^n, curl H^{n+1}
-// (and phi^n) there, as the recompute does.
-static void forward_step(gpx_inv *v, int it, bool rx, float *slot = nullptr)
-{
-    InvArgs a = inv_args(v, false, it);
-    if (slot) a.EC = slot;
-    for (int q = 0; slot && v->P && q < 3; ++q) a.Ps[q] = slot + (6 + q) * v->ntot;
-    if (rx && v->nrx) hipLaunchKernelGGL(k_inv_rx, dim3((v->nrx + 63) / 64), dim3(64), 0, v->stream, a);
-    hipLaunchKernelGGL(k_inv_h, grid_all(v), dim3(128), 0, v->stream, a);
-    hipLaunchKernelGGL(k_inv_e, grid_all(v), dim3(128), 0, v->stream, a);
 }
 
 extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, const float *waves, int nrx,
@@ -1222,7 +1030,8 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
     hipSetDevice(g.device);
     v->si = si; v->sj = sj; v->sk = sk;
     v->sfac = sfac;
-    INV_TRY(hipMemcpy(v->waves, waves, (size_t)g.iterations * 4, hipMemcpyHostToDevice));
+    v->waves.assign(waves, waves + g.iterations);
+    if (int rc = prepare(v)) return rc;
     if (nrx != v->nrx || !v->rxc) {
         if (v->rxc) hipFree(v->rxc);
         if (v->traces) hipFree(v->traces);
@@ -1235,12 +1044,17 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
         INV_TRY(hipMalloc((void **)&v->resid, (size_t)(nrx > 0 ? nrx : 1) * g.iterations * 4));
     }
     if (nrx) INV_TRY(hipMemcpy(v->rxc, rx, (size_t)nrx * 3 * 4, hipMemcpyHostToDevice));
-    {  // the rows of points that hold a receiver, for the adjoint H half
+    {  // the rows and planes of points that hold a receiver
         const size_t rows = (size_t)(g.nx + 1) * (g.ny + 1);
         if (!v->rxrow) INV_TRY(hipMalloc((void **)&v->rxrow, rows));
         std::vector<uint8_t> flag(rows, 0);
         for (int r = 0; r < nrx; ++r) flag[(size_t)rx[3 * r] * (g.ny + 1) + rx[3 * r + 1]] = 1;
         INV_TRY(hipMemcpy(v->rxrow, flag.data(), rows, hipMemcpyHostToDevice));
+        if (v->rows) {
+            std::vector<uint32_t> pf(v->slabflag);
+            for (int r = 0; r < nrx; ++r) pf[rx[3 * r]] |= PF_RX;
+            INV_TRY(hipMemcpy(v->planeflag, pf.data(), pf.size() * 4, hipMemcpyHostToDevice));
+        }
     }
     if (!v->ck) INV_TRY(hipMalloc((void **)&v->ck, (size_t)n_checkpoints(v) * ck_stride(v) * 4));
     // the segments whose states this forward keeps
@@ -1267,27 +1081,22 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
         }
     }
     v->nkeep = nkeep;
-    INV_TRY(hipMemsetAsync(v->F, 0, 6 * v->ntot * 4, v->stream));
-    if (v->P) INV_TRY(hipMemsetAsync(v->T, 0, (size_t)3 * v->P * v->ntot * 4, v->stream));
+    INV_TRY(hipMemsetAsync(v->F, 0, (size_t)6 * v->n * 4, v->stream));
+    if (v->P) INV_TRY(hipMemsetAsync(v->T, 0, (size_t)3 * v->P * v->n * 4, v->stream));
+    for (int f = 0; f < 2 && v->rows && v->np; ++f) INV_TRY(hipMemsetAsync(v->phi[f], 0, (size_t)2 * v->np * 4, v->stream));
     for (auto &S : v->slabs)
-        for (int q = 0; q < 4; ++q) INV_TRY(hipMemsetAsync(S.phi[q], 0, S.n[q] * 4, v->stream));
+        for (int q = 0; q < 4 && !v->rows; ++q) INV_TRY(hipMemsetAsync(S.phi[q], 0, S.n[q] * 4, v->stream));
     hipEvent_t e0, e1;
     INV_TRY(hipEventCreate(&e0));
     INV_TRY(hipEventCreate(&e1));
     INV_TRY(hipEventRecord(e0, v->stream));
-    for (int it = 0; it < g.iterations; ++it) {
-        const int c = it / g.K;
-        if (c >= nseg - nkeep) {  // a kept segment: its states, no checkpoint
-            float *slot = v->keep + (long long)(c - (nseg - nkeep)) * seg_floats +
-                          (long long)(it - c * g.K) * seg_stride(v);
-            forward_step(v, it, true, slot);
-            continue;
-        }
-        if (it % g.K == 0)
+    for (int c = 0; c < nseg; ++c) {
+        const int n0 = c * g.K, n1 = n0 + g.K < g.iterations ? n0 + g.K : g.iterations;
+        const bool kept = c >= nseg - nkeep;  // its states, no checkpoint
+        if (!kept)
             if (int rc = checkpoint(v, c, true)) return rc;
-        forward_step(v, it, true);
+        if (int rc = forward_steps(v, n0, n1, kept ? v->keep + (long long)(c - (nseg - nkeep)) * seg_floats : nullptr)) return rc;
     }
-    INV_TRY(hipGetLastError());
     INV_TRY(hipEventRecord(e1, v->stream));
     INV_TRY(hipEventSynchronize(e1));
     INV_TRY(hipEventElapsedTime(&v->ms_fwd, e0, e1));
@@ -1305,55 +1114,55 @@ extern "C" int gpx_inv_backward(gpx_inv *v, const float *resid, float *gCA, floa
     const gpx_inv_desc &g = v->desc;
     hipSetDevice(g.device);
     if (v->nrx) INV_TRY(hipMemcpy(v->resid, resid, (size_t)v->nrx * g.iterations * 4, hipMemcpyHostToDevice));
-    {  // zero adjoint fields, CB and CA of the cells in the w components
-        InvArgs a = inv_args(v, true, 0);
-        a.lE = v->LE[0];
-        a.lEn = v->LE[1];
-        a.lH = v->LH;
-        hipLaunchKernelGGL(k_adj_init, grid_all(v), dim3(128), 0, v->stream, a);
-        INV_TRY(hipGetLastError());
-    }
-    INV_TRY(hipMemsetAsync(v->grad, 0, 3 * v->ncell * 4, v->stream));
-    if (v->P) INV_TRY(hipMemsetAsync(v->LT, 0, (size_t)3 * v->P * v->ntot * 4, v->stream));
+    INV_TRY(hipMemsetAsync(v->L, 0, (size_t)6 * v->n * 4, v->stream));
+    INV_TRY(hipMemsetAsync(v->grad, 0, (size_t)3 * v->n * 4, v->stream));
+    if (v->P) INV_TRY(hipMemsetAsync(v->LT, 0, (size_t)3 * v->P * v->n * 4, v->stream));
+    for (int f = 0; f < 2 && v->rows && v->np; ++f)
+        for (float *p : v->mu[f]) INV_TRY(hipMemsetAsync(p, 0, (size_t)2 * v->np * 4, v->stream));
     for (auto &S : v->slabs)
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 4 && !v->rows; ++q) {
             INV_TRY(hipMemsetAsync(S.mu[q], 0, S.n[q] * 4, v->stream));
             INV_TRY(hipMemsetAsync(S.mu2[q], 0, S.n[q] * 4, v->stream));
         }
-    float4 *lEb[2] = {v->LE[0], v->LE[1]};  // current and next copy of lE
+    InvArgs a = inv_args(v);
+    InvStep &b = a.b;
+    const InvKernels k = inv_kernels_of(v);
+    b.lE = v->L;
+    b.H = v->L + 3 * v->n;
+    b.T = v->LT;
     int cur = 0;
     hipEvent_t e0, e1;
     INV_TRY(hipEventCreate(&e0));
     INV_TRY(hipEventCreate(&e1));
     INV_TRY(hipEventRecord(e0, v->stream));
-    const dim3 G = grid_all(v), GF = grid_fast(v), GS = grid_shell(v);
-    const bool nofast = fast_empty(v);
     const int nseg = n_checkpoints(v);
     for (int c = nseg - 1; c >= 0; --c) {
         const int n0 = c * g.K, n1 = n0 + g.K < g.iterations ? n0 + g.K : g.iterations;
         const bool kept = c >= nseg - v->nkeep;
         float *base = kept ? v->keep + (long long)(c - (nseg - v->nkeep)) * g.K * seg_stride(v) : v->seg;
         // recompute the segment, storing E^n and curl H^{n+1} (kept segments have them)
-        if (!kept)
+        if (!kept) {
             if (int rc = checkpoint(v, c, false)) return rc;
-        for (int it = n0; it < n1 && !kept; ++it) {
-            float *slot = base + (long long)(it - n0) * seg_stride(v);
-            InvArgs a = inv_args(v, false, it);
-            a.EC = slot;  // the kernels save E^n, curl H^{n+1} (and phi^n) here
-            for (int q = 0; v->P && q < 3; ++q) a.Ps[q] = slot + (6 + q) * v->ntot;
-            hipLaunchKernelGGL(k_inv_h, G, dim3(128), 0, v->stream, a);
-            hipLaunchKernelGGL(k_inv_e, G, dim3(128), 0, v->stream, a);
+            if (int rc = forward_steps(v, n0, n1, base)) return rc;
         }
         // adjoint sweep over the segment
-        for (int it = n1 - 1; it >= n0; --it) {
+        for (int it = n1 - 1; it >= n0; --it, cur ^= 1) {
             float *slot = base + (long long)(it - n0) * seg_stride(v);
-            InvArgs a = inv_args(v, true, it);
-            a.EC = slot;
-            for (int q = 0; v->P && q < 3; ++q) a.Ps[q] = slot + (6 + q) * v->ntot;
-            a.lE = lEb[cur];
-            a.lEn = lEb[cur ^ 1];
-            a.lH = v->LH;
-            if (v->P) hipLaunchKernelGGL(k_adj_disp, G, dim3(128), 0, v->stream, a);
+            b.it = it;
+            b.w = v->waves[it];
+            b.E = slot;
+            b.curl = slot + 3 * v->n;
+            b.phi = slot + 6 * v->n;
+            if (v->rows) {
+                const dim3 G(8 * b.per_xcd);
+                b.P = v->mu[0][cur];
+                b.Q = v->mu[0][cur ^ 1];
+                hipLaunchKernelGGL(k.adj_e, G, dim3(256), v->lds[0], v->stream, v->row, b);
+                b.P = v->mu[1][cur];
+                b.Q = v->mu[1][cur ^ 1];
+                hipLaunchKernelGGL(k.adj_h, G, dim3(256), v->lds[1], v->stream, v->row, b);
+                continue;
+            }
             for (int s = 0; s < a.nslab; ++s) {
                 const auto &S = v->slabs[s];
                 float *const *P = cur == 0 ? S.mu : S.mu2;
@@ -1361,22 +1170,9 @@ extern "C" int gpx_inv_backward(gpx_inv *v, const float *resid, float *gCA, floa
                 a.slab[s].PE1 = P[0]; a.slab[s].PE2 = P[1]; a.slab[s].PH1 = P[2]; a.slab[s].PH2 = P[3];
                 a.slab[s].QE1 = Q[0]; a.slab[s].QE2 = Q[1]; a.slab[s].QH1 = Q[2]; a.slab[s].QH2 = Q[3];
             }
-            if (nofast) {
-                hipLaunchKernelGGL(k_adj_e<false>, GS, dim3(ADJ_BLOCK), 0, v->stream, a);
-                a.lE = a.lEn;  // lE^n, completed by the H half
-                hipLaunchKernelGGL(k_adj_h<false>, GS, dim3(ADJ_BLOCK), 0, v->stream, a);
-            } else {
-                a.mix_nf = (int)(GF.x * GF.y * GF.z);
-                a.mix_ns = (int)(GS.x * GS.y);
-                a.mix_gf[0] = (int)GF.x;
-                a.mix_gf[1] = (int)GF.y;
-                a.mix_gs = (int)GS.x;
-                const dim3 GM(a.mix_nf + a.mix_ns);
-                hipLaunchKernelGGL(k_adj_e_mix, GM, dim3(ADJ_BLOCK), 0, v->stream, a);
-                a.lE = a.lEn;  // lE^n, completed by the H half
-                hipLaunchKernelGGL(k_adj_h_mix, GM, dim3(ADJ_BLOCK), 0, v->stream, a);
-            }
-            cur ^= 1;
+            const dim3 G(8 * a.all_per_xcd);
+            hipLaunchKernelGGL(k_adj_e, G, dim3(128), 0, v->stream, a);
+            hipLaunchKernelGGL(k_adj_h, G, dim3(128), 0, v->stream, a);
         }
         INV_TRY(hipGetLastError());
     }
@@ -1385,13 +1181,13 @@ extern "C" int gpx_inv_backward(gpx_inv *v, const float *resid, float *gCA, floa
     INV_TRY(hipEventElapsedTime(&v->ms_bwd, e0, e1));
     hipEventDestroy(e0);
     hipEventDestroy(e1);
-    std::vector<float> ab((size_t)2 * v->ncell);
-    INV_TRY(hipMemcpy(ab.data(), v->grad, (size_t)2 * v->ncell * 4, hipMemcpyDeviceToHost));
-    for (long long c = 0; c < v->ncell; ++c) {
-        gCA[c] = ab[2 * c];
-        gCB[c] = ab[2 * c + 1];
+    float *out[3] = {gCA, gCB, gIEA};
+    for (int q = 0; q < 3; ++q) {
+        hipLaunchKernelGGL(k_inv_to_cells, grid_all(v), dim3(128), 0, v->stream, a, v->grad + q * v->n, v->dense);
+        INV_TRY(hipGetLastError());
+        INV_TRY(hipMemcpyAsync(out[q], v->dense, (size_t)v->ncell * 4, hipMemcpyDeviceToHost, v->stream));
+        INV_TRY(hipStreamSynchronize(v->stream));
     }
-    INV_TRY(hipMemcpy(gIEA, v->grad + 2 * v->ncell, v->ncell * 4, hipMemcpyDeviceToHost));
     return 0;
 }
 

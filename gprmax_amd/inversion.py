@@ -241,9 +241,10 @@ class InversionGrid(InversionGeometry):
 
     def keep_bytes_all(self):
         """Device bytes that keep every segment: per iteration 6 (9 with
-        poles) floats per grid point, rounded up to a multiple of 4 floats."""
+        poles) arrays of the grid points, their rows padded to 4 floats and
+        each array to 64."""
         per = 9 if self.debye is not None else 6
-        floats = (per * (self.nx + 1) * (self.ny + 1) * (self.nz + 1) + 3) // 4 * 4
+        floats = per * (-(-(self.nx + 1) * (self.ny + 1) * (-(-(self.nz + 1) // 4) * 4) // 64) * 64)
         return 4.0 * floats * self.K * (-(-self.iterations // self.K))
 
     def timings(self):
