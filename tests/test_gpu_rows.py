@@ -65,3 +65,27 @@ def test_values_of_every_magnitude(magnetic, form):
 def test_slabs_close_to_the_opposite_one(shape, form):
     G = rich_model(seed=53, shape=shape, iterations=8, snapshots=False, pml=MEET)
     _check(G, form, 0)
+
+
+def test_indices_of_several_pieces_are_checked_to_the_last():
+    """129 x 119 x 181 points x 6 indices are two pieces of the upload; an
+    index past the tables is refused wherever it is, the first one named, and
+    the model then takes good indices and keeps them when more bad ones come."""
+    from gprmax_amd.grid import ModelBuilder
+    from gprmax_amd.utilities import GeneralError
+    G = ModelBuilder(128, 118, 180, 1e-3, 1e-3, 1e-3, 4, pml_cells=4).finalise()
+    good = G.ID.copy()
+    for at in ((0, 0, 0, 0), (2, 64, 7, 180), (5, 128, 118, 180)):
+        G.ID = good.copy()
+        G.ID[at] = 60000 + at[0]
+        G.ID[5, 128, 118, 180] = max(60001, G.ID[5, 128, 118, 180])
+        with pytest.raises(GeneralError, match='material index {} '.format(G.ID[at])):
+            _hip()(G)
+    G.ID = good
+    with _hip()(G) as s:
+        bad = good.copy()
+        bad[3, 2, 1, 0] = 70000
+        with pytest.raises(GeneralError, match='material index 70000 '):
+            s._check(s.lib.gpx_upload_id(s.ctx, np.ascontiguousarray(bad, dtype=np.uint32).ctypes.data))
+        s.run(0, 4)
+        assert not np.any(s.download_fields())
