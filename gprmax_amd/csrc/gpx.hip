@@ -24,6 +24,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <limits.h>
+#include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <string.h>
@@ -2203,6 +2205,8 @@ static RowArgs row_args(const gpx_ctx *ctx, int nitems, int it)
     b.per_xcd = (nitems + 7) / 8;
     b.flip = ctx->cur;
     b.it = it;
+    b.p0 = 0;
+    b.p1 = ctx->desc.nx + 1;
     return b;
 }
 
@@ -2216,10 +2220,13 @@ static hipError_t launch_row_step(gpx_ctx *ctx, int it)
     return hipGetLastError();
 }
 
-// The H (field 1) or E pass in one launch.
-static hipError_t launch_row_pass(const gpx_ctx *ctx, int field, int it)
+// The H (field 1) or E pass over planes [p0, p1), in one launch.
+static hipError_t launch_row_pass(const gpx_ctx *ctx, int field, int it, int p0, int p1)
 {
-    const RowArgs b = row_args(ctx, ctx->rowh.pitems, it);
+    const RowModel &m = ctx->rowh;
+    RowArgs b = row_args(ctx, m.pseg * ((p1 - p0 + m.pxc - 1) / m.pxc), it);
+    b.p0 = p0;
+    b.p1 = p1;
     const RowKernels k = row_kernels(ctx);
     hipLaunchKernelGGL(field == 1 ? k.h : k.e, dim3(8 * b.per_xcd), dim3(pass_block(ctx)), pass_lds(ctx, field),
                        ctx->stream, ctx->row, b);
@@ -2377,6 +2384,59 @@ static int e_flags(const gpx_ctx *ctx)
     return f;
 }
 
+// Bytes that an iteration of the row passes goes over, each array once.
+static double pass_bytes(const gpx_ctx *ctx)
+{
+    double b = (double)ctx->fstride * 24.0 + (double)ctx->ntot * 2.0 * (ctx->hu ? 3 : 6);
+    if (!ctx->slabs.empty()) b += 2.0 * (double)phi_bytes(ctx);
+    if (ctx->desc.maxpoles > 0) {
+        b += (double)ctx->ntot * 12.0;
+        for (int c = 0; c < 3; ++c) b += (double)ctx->tn[c] * ctx->desc.maxpoles * (ctx->disp_complex ? 8 : 4);
+    }
+    return b;
+}
+
+// Blocks of planes of run_wave: as few as keep a block within WAVE_BYTES, every
+// one more being a launch of 5 us per pass beside its bytes.  The last-level
+// cache has 256 MB; past about 200 a block evicts itself between the passes.  us per
+// iteration in 1, 2, 3, ... blocks (MB of a block in brackets where fastest):
+// 300x300x200 348, 335, 296, 275 (at 3: 199), 283 ...; 250x220x180 179, 146 (168), 161;
+// 611x407x45 247, 226, 200 (146), 209; 420x400x200 612, 629, 606, 604, 567, 519
+// (182), 520 at 7, 570 at 13; 240x240x180 with 3 poles 320, 323, 294 (199), 299.
+static const double WAVE_BYTES = 200.0 * 1024 * 1024;
+// Iterations a block is taken through: 300x300x200 takes 357 us an iteration at
+// 1, 316 at 2, 290 at 4, 280 at 8, 276 at 16 and 278 at 32.  At one iteration whole passes
+// are the faster ones (347).
+static const int WAVE_ITS = 16;
+static int wave_blocks(const gpx_ctx *ctx)
+{
+    const double n = ceil(pass_bytes(ctx) / WAVE_BYTES);
+    return n < (double)(ctx->desc.nx + 1) ? (int)n : ctx->desc.nx + 1;
+}
+
+// The row passes of iterations [it, it + n) in blocks of planes, each block
+// taken through all of them before the next one is begun, so that what its
+// first pass brings into the last-level cache serves the others too.  A block's
+// planes move down by one with each iteration: iteration s of the block that
+// begins at plane a covers planes [a - s, a - s + w).  New H at plane i needs E
+// of the iteration before at i and i + 1, which the block has just made up to
+// a - s + w; new E at i needs this iteration's H at i and i - 1, and the block
+// before ended at a - s - 1.  Every cell sees the same values in the same order
+// as in whole passes.  On grids past the cache whole passes run at the rate of
+// the memory (4.7 of about 5 TB/s), the blocks at that of the cache (6.5 of 8).
+static int run_wave(gpx_ctx *ctx, int it, int n, int blocks)
+{
+    const int nx1 = ctx->desc.nx + 1, w = (nx1 + n - 1 + blocks - 1) / blocks;
+    for (int a = 0; a < nx1 + n - 1; a += w)
+        for (int s = 0; s < n; ++s) {
+            const int p0 = std::max(a - s, 0), p1 = std::min(a - s + w, nx1);
+            if (p0 >= p1) continue;
+            GPX_TRY(launch_row_pass(ctx, 1, it + s, p0, p1));
+            GPX_TRY(launch_row_pass(ctx, 0, it + s, p0, p1));
+        }
+    return 0;
+}
+
 // Timing events, destroyed when the set goes out of scope.
 struct EventSet {
     std::vector<hipEvent_t> e;
@@ -2406,6 +2466,7 @@ static int run_steps(gpx_ctx *ctx, int it0, int n, float *ms4)
         if (int rc = ensure_next_state(ctx)) return rc;
     if (n > 0 && rows)
         if (int rc = ensure_row(ctx)) return rc;
+    const int waves = kind == RUN_PASSES && !ms4 && ctx->tls.empty() ? wave_blocks(ctx) : 1;
     // With ms4, six events per iteration are recorded around the kernels and
     // read once at the end, so the host never waits between iterations and
     // the gaps between events are the kernels' own.
@@ -2425,15 +2486,24 @@ static int run_steps(gpx_ctx *ctx, int it0, int n, float *ms4)
             if (ev) GPX_TRY(hipEventRecord(ev[1], ctx->stream));
             continue;
         }
+        if (waves > 1) {
+            // up to the next iteration that a snapshot is taken before
+            int end = std::min(it0 + n, it + WAVE_ITS);
+            for (const Snap &S : ctx->snaps)
+                if (S.time - 1 > it && S.time - 1 < end) end = S.time - 1;
+            if (int rc = run_wave(ctx, it, end - it, end - it > 1 ? waves : 1)) return rc;
+            it = end - 1;
+            continue;
+        }
         if (kind == RUN_PASSES) {
             // events: the H pass between ev[0] and ev[1], the E pass between
             // ev[3] and ev[4]
             if (ev) GPX_TRY(hipEventRecord(ev[0], ctx->stream));
-            GPX_TRY(launch_row_pass(ctx, 1, it));
+            GPX_TRY(launch_row_pass(ctx, 1, it, 0, ctx->desc.nx + 1));
             if (ev) GPX_TRY(hipEventRecord(ev[1], ctx->stream));
             GPX_TRY(launch_tl(ctx, 1, it));
             if (ev) GPX_TRY(hipEventRecord(ev[3], ctx->stream));
-            GPX_TRY(launch_row_pass(ctx, 0, it));
+            GPX_TRY(launch_row_pass(ctx, 0, it, 0, ctx->desc.nx + 1));
             if (ev) GPX_TRY(hipEventRecord(ev[4], ctx->stream));
             GPX_TRY(launch_tl(ctx, 0, it));
             continue;
@@ -3135,6 +3205,8 @@ static void batch_launch(const gpx_batch *b, const BatchPlan &p, const BatchGrou
         a.per_xcd = (g.nitems_rows + 7) / 8;
         a.flip = g.kind == BatchGroup::STEP ? s & 1 : 0;
         a.it = it;
+        a.p0 = 0;
+        a.p1 = INT_MAX;
         auto launch = [&](row_kernel f, size_t lds) {
             hipLaunchKernelGGL(f, dim3(8 * a.per_xcd), dim3(g.B), lds, b->stream, b->dmodels + g.g0, a);
         };

@@ -45,11 +45,14 @@
 // on the host with the same operations, and the division by the cell size is
 // the correctly rounded quotient (row_quot).
 //
+// Grids past the last-level cache go through the passes in blocks of planes, several
+// iterations a block (run_wave in gpx.hip).
+//
 // Measured, us per iteration, two passes here and four (interior and boundary
 // apart, one cell per lane) or two with one merged step before:
 //   120x105 (2-D)  8.6 from 16.7     100x100x100   22.5 from 40.8
-//   157x131x97 MRIPML order 2  45 from 72        300x300x200  349 from 425
-//   611x407x45  248 from 375      240x240x180, 3 poles  326 from 478
+//   157x131x97 MRIPML order 2  45 from 72        300x300x200  276 from 425
+//   611x407x45  200 from 375      240x240x180, 3 poles  294 from 478
 #ifndef GPX_ROWS_H
 #define GPX_ROWS_H
 
@@ -116,6 +119,7 @@ struct RowArgs {
     const int *item0;                // [ntr + 1]: first item of each model (unused with one)
     int ntr, nitems, per_xcd;
     int flip, it;
+    int p0, p1;                      // the passes' planes (p1 past the last one: to the model's end)
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -893,12 +897,13 @@ __global__ void __launch_bounds__(ROW_BLOCK_MAX) __attribute__((amdgpu_waves_per
 }
 
 // ---------------------------------------------------------------- passes
-// The lane of pass item `item`: segment of the plane's lanes, x chunk.
+// The lane of pass item `item`: segment of the plane's lanes, x chunk of the
+// launch's planes.
 struct RowLane {
     int j, kl, xa, xb;
     bool live;
 };
-__device__ __forceinline__ RowLane row_lane(const RowModel &a, int item)
+__device__ __forceinline__ RowLane row_lane(const RowModel &a, int item, int p0, int p1)
 {
     RowLane q;
     const int seg = item % a.pseg, ch = item / a.pseg, lpr = a.kp / NC;
@@ -906,8 +911,8 @@ __device__ __forceinline__ RowLane row_lane(const RowModel &a, int item)
     q.live = t < (a.ny + 1) * lpr;
     q.j = q.live ? t / lpr : 0;
     q.kl = q.live ? NC * (t - q.j * lpr) : 0;
-    q.xa = ch * a.pxc;
-    q.xb = min(q.xa + a.pxc, a.nx + 1);
+    q.xa = p0 + ch * a.pxc;
+    q.xb = min(min(q.xa + a.pxc, p1), a.nx + 1);
     return q;
 }
 
@@ -923,7 +928,7 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_row_h
     if (g >= b.nitems) return;
     int first;
     const RowModel &a = models[row_model_of(b, g, first)];
-    const RowLane q = row_lane(a, g - first);
+    const RowLane q = row_lane(a, g - first, b.p0, b.p1);
     const int j = q.j, kl = q.kl, it = b.it, lane = threadIdx.x & 63;
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t toj = j < a.ny ? to + 4u * (uint32_t)a.kp : to;
@@ -997,7 +1002,7 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
     if (g >= b.nitems) return;
     int first;
     const RowModel &a = models[row_model_of(b, g, first)];
-    const RowLane q = row_lane(a, g - first);
+    const RowLane q = row_lane(a, g - first, b.p0, b.p1);
     const int j = q.j, kl = q.kl, it = b.it, lane = threadIdx.x & 63;
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t tob = j > 0 ? to - 4u * (uint32_t)a.kp : to;

@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_inv_r
     const int g = logical_block(b.per_xcd);
     if (g >= b.nitems) return;
     const RowModel &a = *models;
-    const RowLane q = row_lane(a, g);
+    const RowLane q = row_lane(a, g, 0, a.nx + 1);
     const int j = q.j, kl = q.kl, lane = threadIdx.x & 63;
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t toj = j < a.ny ? to + 4u * (uint32_t)a.kp : to;
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(P > 0 ? 2 : 0, OR
     const int g = logical_block(b.per_xcd);
     if (g >= b.nitems) return;
     const RowModel &a = *models;
-    const RowLane q = row_lane(a, g);
+    const RowLane q = row_lane(a, g, 0, a.nx + 1);
     const int j = q.j, kl = q.kl, lane = threadIdx.x & 63;
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t tob = j > 0 ? to - 4u * (uint32_t)a.kp : to;
@@ -398,7 +398,7 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(2, ORDER) k_inv_a
     const int g = logical_block(b.per_xcd);
     if (g >= b.nitems) return;
     const RowModel &a = *models;
-    const RowLane q = row_lane(a, g);
+    const RowLane q = row_lane(a, g, 0, a.nx + 1);
     const int j = q.j, kl = q.kl, lane = threadIdx.x & 63;
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t toj = j < a.ny ? to + 4u * (uint32_t)a.kp : to;
@@ -609,7 +609,7 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(P > 0 ? 2 : 1, OR
     const int g = logical_block(b.per_xcd);
     if (g >= b.nitems) return;
     const RowModel &a = *models;
-    const RowLane q = row_lane(a, g);
+    const RowLane q = row_lane(a, g, 0, a.nx + 1);
     const int j = q.j, kl = q.kl, lane = threadIdx.x & 63;
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t tob = j > 0 ? to - 4u * (uint32_t)a.kp : to;

@@ -89,3 +89,30 @@ def test_indices_of_several_pieces_are_checked_to_the_last():
             s._check(s.lib.gpx_upload_id(s.ctx, np.ascontiguousarray(bad, dtype=np.uint32).ctypes.data))
         s.run(0, 4)
         assert not np.any(s.download_fields())
+
+
+@pytest.mark.parametrize('shape,poles,magnetic', [((60, 360, 340), 0, False), ((61, 330, 300), 2, True), ((12, 870, 701), 0, True)],
+                         ids=str)
+def test_blocks_of_planes(shape, poles, magnetic):
+    """Grids past the last-level cache go through the passes in blocks of planes
+    that move with the iterations, fewer planes than iterations too; sources,
+    receivers, snapshots between and runs of one iteration: as whole general
+    passes give it, bit for bit."""
+    G = rich_model(seed=54, shape=shape, iterations=40, pml=FACES, poles=poles)
+    if magnetic:
+        randomise_tables(G, 55, scaled=True)
+    for n, s in enumerate(G.snapshots):
+        s.time = 5 + 14 * n
+    rng = np.random.default_rng(56)
+    F = rng.standard_normal((6,) + tuple(n + 1 for n in shape), dtype=np.float32)
+    got = []
+    for form in (4, 2):
+        with _hip()(G) as s:
+            s.set_step(form)
+            s.upload_fields(F)
+            for it, n in ((0, 23), (23, 1), (24, 2), (26, 9)):
+                s.run(it, n)
+            got.append([s.download_fields(), s.download_rx()] + [s.download_phi(p, w) for p in range(6) for w in range(4)]
+                       + [s.download_snapshot(n) for n in range(len(G.snapshots))] + ([s.download_T()] if poles else []))
+    for n, (a, b) in enumerate(zip(*got)):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), n
