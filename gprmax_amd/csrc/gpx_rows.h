@@ -203,7 +203,8 @@ __device__ __forceinline__ uint32_t row_quot(fN x, const RowSlab &S, fN &q)
     for (int u = 0; u < NC; ++u) {
         const float v = __builtin_fmaf(x[u], S.rd, x[u] * S.rl);
         q[u] = __builtin_fmaf(__builtin_fmaf(-v, S.d, x[u]), S.rd, v);
-        const uint32_t b = __builtin_bit_cast(uint32_t, x[u]) * 2u - 1u;  // zero wraps to the largest
+        const float xu = x[u];  // bit_cast of the element itself reads element 0
+        const uint32_t b = __builtin_bit_cast(uint32_t, xu) * 2u - 1u;  // zero wraps to the largest
         least = b < least ? b : least;
     }
     return least;

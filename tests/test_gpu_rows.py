@@ -61,6 +61,29 @@ def test_values_of_every_magnitude(magnetic, form):
 
 
 @pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
+@pytest.mark.parametrize('cell', [0, 1])
+def test_tiny_values_in_one_cell_of_a_lane(cell, form):
+    """Fields of 2^-126 to 2^-148 in one of a lane's two cells and zero in the
+    other: the slabs' quotient of either cell is that of the division."""
+    G = rich_model(seed=52, shape=(13, 14, 15), iterations=8, snapshots=False, pml=FACES)
+    _random_state(G, 9)
+    for c in COMPS:
+        a = getattr(G, c)
+        a *= np.exp2(-np.random.default_rng(4).integers(126, 149, a.shape).astype(np.float32))
+        a[:, :, 1 - cell::2] = 0
+    for pml in G.pmls:
+        for a in (pml.EPhi1, pml.EPhi2, pml.HPhi1, pml.HPhi2):
+            a[:] = 0
+    lib = oracle.load(np.float32)
+    with _hip()(G) as s:
+        s.set_step(form)
+        _push_state(s, G)
+        s.run(0, 1)
+        osolver.step(lib, G, 0, 8)
+        _assert_state_equal(s, G, 'form {}'.format(form))
+
+
+@pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
 @pytest.mark.parametrize('shape', [(10, 12, 12), (12, 10, 12), (12, 12, 9), (12, 12, 10)], ids=str)
 def test_slabs_close_to_the_opposite_one(shape, form):
     G = rich_model(seed=53, shape=shape, iterations=8, snapshots=False, pml=MEET)
