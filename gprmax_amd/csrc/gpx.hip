@@ -747,13 +747,13 @@ struct gpx_ctx {
     // second copy is allocated when it first runs), `cur` the current one; E
     // Phi once.  ntot counts padded points.
     float *Fmem[2] = {nullptr, nullptr};    // 6 x fstride floats: Ex, Ey, Ez, Hx, Hy, Hz
-    float *phiH[2] = {nullptr, nullptr}, *phiE = nullptr;
-    int cur = 0;
+    float *phiH[2] = {nullptr, nullptr}, *phiE[2] = {nullptr, nullptr};
+    int cur = 0, curE = 0;    // current copy of the fields and H Phi, of E Phi
     float *field(int c) const { return Fmem[cur] + c * fstride; }
     long long np = 0;         // floats of one (order, term) block of Phi
     int phi_orders = 0;       // orders the Phi arrays hold
     bool phi_dirty = false;   // slabs were added since the Phi arrays were laid out
-    size_t next_bytes = 0;    // bytes of the second state and of the second H Phi
+    size_t next_bytes = 0;    // bytes of the second state and of the second Phi
     long long fstride = 0;    // floats between components: ntot rounded up to 64, and a row more
     uint16_t *ID = nullptr;   // [6][ntot] (nmat < 2^16, see gpx_create)
     std::vector<float> hostE, hostH, hostdisp;  // coefficients and pole tables, for the row kernels' tables
@@ -761,6 +761,7 @@ struct gpx_ctx {
     int nimg = 0;
     RowModel *row = nullptr;  // the model as the row kernels see it
     RowModel rowh;            // its host copy
+    bool state_given = false; // fields or Phi have been uploaded
     bool row_dirty = true;    // something in it changed
     bool planes_dirty = true; // slabs, sources or receivers changed since the planes' flags went up
     bool hu = false;          // every material has the same H coefficients
@@ -946,7 +947,8 @@ extern "C" int gpx_destroy(gpx_ctx *ctx)
     if (ctx->disp) hipFree(ctx->disp);
     if (ctx->dispflag) hipFree(ctx->dispflag);
     for (auto &p : ctx->phiH) if (p) hipFree(p);
-    if (ctx->phiE) hipFree(ctx->phiE);
+    for (float *m : ctx->phiE)
+        if (m) hipFree(m);
     if (ctx->img) hipFree(ctx->img);
     if (ctx->row) hipFree(ctx->row);
     for (auto &s : ctx->src) {
@@ -998,7 +1000,7 @@ static int ensure_phi(gpx_ctx *ctx)
     hipSetDevice(ctx->desc.device);
     std::vector<std::vector<float>> keep;
     std::vector<Slab> now = ctx->slabs;
-    if (ctx->phiE) {  // values of the slabs that were there, in the old layout
+    if (ctx->phiE[ctx->curE]) {  // values of the slabs that were there, in the old layout
         long long acc = 0;
         size_t n = 0;
         while (n < ctx->slabs.size() && acc < ctx->np) acc += (long long)now[n].ni * now[n].nj * now[n].nkp, ++n;
@@ -1010,12 +1012,14 @@ static int ensure_phi(gpx_ctx *ctx)
                 if (int rc = phi_transfer(ctx, (int)s, w, keep.back().data(), false)) return rc;
             }
         GPX_TRY(hipStreamSynchronize(ctx->stream));
-        ctx->bytes -= phi_bytes(ctx) * (ctx->phiH[1] ? 3 : 2);
-        if (ctx->phiH[1]) ctx->next_bytes -= phi_bytes(ctx);
-        for (float **p : {&ctx->phiE, &ctx->phiH[0], &ctx->phiH[1]}) {
+        const int next = (ctx->phiH[1] != nullptr) + (ctx->phiE[1] != nullptr);
+        ctx->bytes -= phi_bytes(ctx) * (2 + next);
+        ctx->next_bytes -= phi_bytes(ctx) * next;
+        for (float **p : {&ctx->phiE[0], &ctx->phiE[1], &ctx->phiH[0], &ctx->phiH[1]}) {
             if (*p) hipFree(*p);
             *p = nullptr;
         }
+        ctx->curE = 0;
     }
     ctx->np = 0;
     ctx->phi_orders = 0;
@@ -1024,7 +1028,7 @@ static int ensure_phi(gpx_ctx *ctx)
         ctx->np += (long long)S.ni * S.nj * S.nkp;
         if (S.order > ctx->phi_orders) ctx->phi_orders = S.order;
     }
-    GPX_TRY(dalloc(ctx, (void **)&ctx->phiE, phi_bytes(ctx)));
+    GPX_TRY(dalloc(ctx, (void **)&ctx->phiE[0], phi_bytes(ctx)));
     const bool two = ctx->Fmem[1] != nullptr;
     for (int q = 0; q < (two ? 2 : 1); ++q) {
         GPX_TRY(dalloc(ctx, (void **)&ctx->phiH[q], phi_bytes(ctx)));
@@ -1058,6 +1062,19 @@ static int ensure_next_state(gpx_ctx *ctx)
         ctx->next_bytes += b;
         GPX_TRY(hipMemcpyAsync(ctx->phiH[1], ctx->phiH[0], b, hipMemcpyDeviceToDevice, ctx->stream));
     }
+    ctx->row_dirty = true;
+    return 0;
+}
+
+// The 2-D kernel writes the next E Phi into a second copy too.
+static int ensure_next_plane(gpx_ctx *ctx)
+{
+    if (int rc = ensure_next_state(ctx)) return rc;
+    if (!ctx->phiE[0] || ctx->phiE[1]) return 0;
+    const size_t b = phi_bytes(ctx);   // the current one is phiE[0]
+    GPX_TRY(dalloc(ctx, (void **)&ctx->phiE[1], b, false));
+    ctx->next_bytes += b;
+    GPX_TRY(hipMemcpyAsync(ctx->phiE[1], ctx->phiE[0], b, hipMemcpyDeviceToDevice, ctx->stream));
     ctx->row_dirty = true;
     return 0;
 }
@@ -1615,7 +1632,7 @@ static void fill_slab_args(const gpx_ctx *ctx, int field, int s, SlabArgs &a)
     a.t = S.t;
     a.order = S.order;
     a.d = S.d;
-    a.phi1 = field == 0 ? ctx->phiE : ctx->phiH[ctx->cur];
+    a.phi1 = field == 0 ? ctx->phiE[ctx->curE] : ctx->phiH[ctx->cur];
     a.phi2 = a.phi1 ? a.phi1 + ctx->np : nullptr;
     a.roff = S.roff;
 }
@@ -2182,7 +2199,8 @@ static int ensure_row(gpx_ctx *ctx)
     m.nmat = g.nmat;
     for (int n = 0; n < 5 && ctx->hu; ++n) m.h[n] = ctx->hostH[n];
     m.nRT = nRT;
-    m.phiE = ctx->phiE;
+    m.phiE[0] = ctx->phiE[0];
+    m.phiE[1] = ctx->phiE[1];
     m.phiH[0] = ctx->phiH[0];
     m.phiH[1] = ctx->phiH[1];
     m.np4 = (uint32_t)(ctx->np * 4);
@@ -2204,6 +2222,7 @@ static RowArgs row_args(const gpx_ctx *ctx, int nitems, int it)
     b.nitems = nitems;
     b.per_xcd = (nitems + 7) / 8;
     b.flip = ctx->cur;
+    b.flipE = ctx->curE;
     b.it = it;
     b.p0 = 0;
     b.p1 = ctx->desc.nx + 1;
@@ -2230,6 +2249,95 @@ static hipError_t launch_row_pass(const gpx_ctx *ctx, int field, int it, int p0,
     const RowKernels k = row_kernels(ctx);
     hipLaunchKernelGGL(field == 1 ? k.h : k.e, dim3(8 * b.per_xcd), dim3(pass_block(ctx)), pass_lds(ctx, field),
                        ctx->stream, ctx->row, b);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------- 2-D models
+// Tiles of the 2-D kernel (gpx_plane.h); w: the axis of one cell, -1 when it
+// cannot run the model.
+struct PlaneShape {
+    int w, tp, tq, halo;
+};
+
+// The axis of one cell, when the 2-D kernel can run the model: what it leaves out
+// is zero and stays so.  No state has been uploaded, sources lie on the
+// plane's cells and drive its components, slabs lie across the two long axes
+// and every coefficient is finite.  -1 otherwise.
+static int plane_axis(const gpx_ctx *ctx)
+{
+    const gpx_desc &g = ctx->desc;
+    const int dim[3] = {g.nx, g.ny, g.nz};
+    int w = -1;
+    for (int q = 0; q < 3; ++q)
+        if (dim[q] == 1) {
+            if (w >= 0) return -1;
+            w = q;
+        }
+    if (w < 0 || g.maxpoles > 0 || ctx->state_given || !ctx->tls.empty() || !rows_ok(ctx)) return -1;
+    auto finite = [](const std::vector<float> &x) {
+        return std::all_of(x.begin(), x.end(), [](float v) { return isfinite(v); });
+    };
+    if (!finite(ctx->hostE) || !finite(ctx->hostH)) return -1;
+    for (const Slab &S : ctx->slabs)
+        if (S.dir % 3 == w || !finite(S.R[0]) || !finite(S.R[1])) return -1;
+    for (int kind : {GPX_SRC_MAGNETIC, GPX_SRC_VOLTAGE, GPX_SRC_HERTZIAN})
+        for (int s = 0; s < ctx->src[kind].n; ++s) {
+            const int *in = &ctx->src[kind].host[6 * s];
+            if (in[w] != 0 || ((in[3] & 3) == w) != (kind != GPX_SRC_MAGNETIC)) return -1;
+        }
+    return w;
+}
+
+// Tiles for a run of n iterations: the shape that takes the least time by what
+// launches of several shapes took, 5.5 us + 0.7 us for each wave a SIMD is
+// given + for each iteration 0.25 us a wave, 0.5 at the least.  Measured, us per iteration
+// (columns of a tile, halo): 120x105 2.09 (16x16, 4), 1.75 (16x32, 6), 1.88 (32x32,
+// 8), the passes 8.6; 250x180 2.60, 3.00, 1.92, 9.5; 500x500 7.4, 9.0, 6.7, 5.2
+// (32x32, 4), 17.9; 1200x1000 28, 35, 24, 18.3 (32x32, 4), 57.
+static PlaneShape plane_shape(const gpx_ctx *ctx, int n)
+{
+    PlaneShape best = {plane_axis(ctx), 0, 0, 0};
+    if (best.w < 0) return best;
+    const gpx_desc &g = ctx->desc;
+    const int np = best.w == 0 ? g.ny : g.nx, nq = best.w == 2 ? g.ny : g.nz, cus = ctx->cus > 0 ? ctx->cus : 256;
+    const int tiles[3][2] = {{16, 16}, {16, 32}, {32, 32}};
+    double least = 0;
+    for (auto &t : tiles)
+        for (int h = 1; 2 * h + 4 <= t[0] && (h <= n || h == 1); ++h) {
+            const int op = t[0] - 2 * h, oq = t[1] - 2 * h;
+            const double blocks = (double)((np + op) / op) * ((nq + oq) / oq);
+            const double waves = ceil(blocks / cus) * t[0] * t[1] / 256;
+            const double us = (5.5 + 0.7 * waves + h * std::max(0.5, 0.25 * waves)) / h;
+            if (best.halo && us >= least) continue;
+            least = us;
+            best = {best.w, t[0], t[1], h};
+        }
+    return best;
+}
+
+// Iterations [it, it + n), n at most the halo, in one launch.
+static hipError_t launch_plane(gpx_ctx *ctx, const PlaneShape &s, int it, int n)
+{
+    const gpx_desc &g = ctx->desc;
+    PlaneArgs b;
+    b.flip = ctx->cur;
+    b.flipE = ctx->curE;
+    b.it = it;
+    b.n = n;
+    b.w = s.w;
+    b.tp = s.tp;
+    b.tq = s.tq;
+    b.halo = s.halo;
+    b.hu = ctx->hu;
+    const int op = s.tp - 2 * s.halo, oq = s.tq - 2 * s.halo;
+    const int np = s.w == 0 ? g.ny : g.nx, nq = s.w == 2 ? g.ny : g.nz;
+    b.ntq = (nq + oq) / oq;
+    b.nitems = (np + op) / op * b.ntq;
+    b.per_xcd = (b.nitems + 7) / 8;
+    const int B = s.tp * s.tq;
+    hipLaunchKernelGGL(row_kernels(ctx).plane, dim3(8 * b.per_xcd), dim3(B), (size_t)B * 12, ctx->stream, ctx->row, b);
+    ctx->cur ^= 1;
+    ctx->curE ^= ctx->slabs.empty() ? 0 : 1;
     return hipGetLastError();
 }
 
@@ -2278,8 +2386,9 @@ static bool one_launch(const gpx_ctx *ctx)
 }
 
 // What gpx_run does with the model: STEP (one launch), PASSES (two row
-// passes), GENERAL (the general passes), BESIDE (form 2).
-enum RunKind { RUN_STEP, RUN_PASSES, RUN_GENERAL, RUN_BESIDE };
+// passes), PLANE (several iterations of a 2-D model a launch), GENERAL (the
+// general passes), BESIDE (form 2).
+enum RunKind { RUN_STEP, RUN_PASSES, RUN_PLANE, RUN_GENERAL, RUN_BESIDE };
 
 static RunKind run_kind(const gpx_ctx *ctx)
 {
@@ -2288,7 +2397,7 @@ static RunKind run_kind(const gpx_ctx *ctx)
     case 1: return step_block(ctx) ? RUN_STEP : passes;
     case 2: return RUN_BESIDE;
     case 0: case 6: return passes;
-    default: return one_launch(ctx) ? RUN_STEP : passes;   // 3, 5, 7 and 4
+    default: return plane_axis(ctx) >= 0 ? RUN_PLANE : (one_launch(ctx) ? RUN_STEP : passes);   // 3, 5, 7 and 4
     }
 }
 
@@ -2460,10 +2569,14 @@ static int run_steps(gpx_ctx *ctx, int it0, int n, float *ms4)
     if (!ms4 && ctx->fused == 4 && ctx->choice == -1 && n >= CHOOSE_ITS)
         ctx->choice = one_launch(ctx) ? 5 : 4;
     const int hf = h_flags(ctx), ef = e_flags(ctx);
-    const RunKind kind = run_kind(ctx);
-    const bool rows = kind == RUN_STEP || kind == RUN_PASSES;
+    RunKind kind = run_kind(ctx);
+    if (ms4 && kind == RUN_PLANE) kind = RUN_PASSES;   // the kernels of each iteration are timed
+    const bool rows = kind == RUN_STEP || kind == RUN_PASSES || kind == RUN_PLANE;
     if (n > 0 && kind == RUN_STEP)
         if (int rc = ensure_next_state(ctx)) return rc;
+    if (n > 0 && kind == RUN_PLANE)
+        if (int rc = ensure_next_plane(ctx)) return rc;
+    const PlaneShape shape = kind == RUN_PLANE ? plane_shape(ctx, n) : PlaneShape{-1, 0, 0, 0};
     if (n > 0 && rows)
         if (int rc = ensure_row(ctx)) return rc;
     const int waves = kind == RUN_PASSES && !ms4 && ctx->tls.empty() ? wave_blocks(ctx) : 1;
@@ -2486,12 +2599,13 @@ static int run_steps(gpx_ctx *ctx, int it0, int n, float *ms4)
             if (ev) GPX_TRY(hipEventRecord(ev[1], ctx->stream));
             continue;
         }
-        if (waves > 1) {
+        if (waves > 1 || kind == RUN_PLANE) {
             // up to the next iteration that a snapshot is taken before
-            int end = std::min(it0 + n, it + WAVE_ITS);
+            int end = std::min(it0 + n, it + (kind == RUN_PLANE ? shape.halo : WAVE_ITS));
             for (const Snap &S : ctx->snaps)
                 if (S.time - 1 > it && S.time - 1 < end) end = S.time - 1;
-            if (int rc = run_wave(ctx, it, end - it, end - it > 1 ? waves : 1)) return rc;
+            if (kind == RUN_PLANE) GPX_TRY(launch_plane(ctx, shape, it, end - it));
+            else if (int rc = run_wave(ctx, it, end - it, end - it > 1 ? waves : 1)) return rc;
             it = end - 1;
             continue;
         }
@@ -2690,6 +2804,7 @@ extern "C" int gpx_upload_fields(gpx_ctx *ctx, const float *in6)
     if (!ctx || !in6) return fail(ctx, GPX_EARG, "gpx_upload_fields: null argument");
     const gpx_desc &g = ctx->desc;
     const size_t pts = (size_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
+    ctx->state_given = true;
     // Both states, where there are two: cells that no update touches keep
     // their value in either.
     for (int c = 0; c < 6; ++c)
@@ -2712,8 +2827,8 @@ static int phi_transfer(gpx_ctx *ctx, int slab, int which, float *host, bool up)
     const long long *d = S.dims[which];
     const size_t block = (size_t)S.ni * S.nj * S.nkp;
     std::vector<float> t(block);
-    float *arrays[2] = {field == 0 ? ctx->phiE : ctx->phiH[ctx->cur], nullptr};
-    if (up && field == 1) arrays[1] = ctx->phiH[ctx->cur ^ 1];
+    float *arrays[2] = {field == 0 ? ctx->phiE[ctx->curE] : ctx->phiH[ctx->cur], nullptr};
+    if (up) arrays[1] = field == 0 ? ctx->phiE[ctx->curE ^ 1] : ctx->phiH[ctx->cur ^ 1];
     for (int o = 0; o < S.order; ++o) {
         const size_t at = (size_t)(2 * o + w) * ctx->np + S.base;
         if (int rc = copy_out(ctx, t.data(), arrays[0] + at, block * 4)) return rc;
@@ -2752,6 +2867,7 @@ extern "C" int gpx_upload_pml_phi(gpx_ctx *ctx, int slab, int which, const float
 {
     if (!ctx || !in) return fail(ctx, GPX_EARG, "gpx_upload_pml_phi: null argument");
     if (int rc = phi_check(ctx, slab, which)) return rc;
+    ctx->state_given = true;
     return phi_transfer(ctx, slab, which, const_cast<float *>(in), true);
 }
 
@@ -3078,6 +3194,7 @@ static int batch_plan_rows(gpx_batch *b, int tile, int xchunk, BatchGroup &g, st
             std::swap(models[t].F[0], models[t].F[1]);
             std::swap(models[t].phiH[0], models[t].phiH[1]);
         }
+        if (c->curE) std::swap(models[t].phiE[0], models[t].phiE[1]);
         if (c->cus > 0) cus = c->cus;
     }
     if (g.kind == BatchGroup::PASSES) {
@@ -3204,6 +3321,7 @@ static void batch_launch(const gpx_batch *b, const BatchPlan &p, const BatchGrou
         a.nitems = g.nitems_rows;
         a.per_xcd = (g.nitems_rows + 7) / 8;
         a.flip = g.kind == BatchGroup::STEP ? s & 1 : 0;
+        a.flipE = 0;
         a.it = it;
         a.p0 = 0;
         a.p1 = INT_MAX;
@@ -3331,7 +3449,7 @@ static int zero_state(gpx_ctx *ctx)
     hipStream_t s = c->stream;
     for (float *m : c->Fmem)
         if (m) GPX_TRY(hipMemsetAsync(m, 0, (size_t)6 * c->fstride * 4, s));
-    for (float *m : {c->phiE, c->phiH[0], c->phiH[1]})
+    for (float *m : {c->phiE[0], c->phiE[1], c->phiH[0], c->phiH[1]})
         if (m) GPX_TRY(hipMemsetAsync(m, 0, phi_bytes(c), s));
     if (c->desc.maxpoles > 0)
         for (int q = 0; q < 3; ++q)

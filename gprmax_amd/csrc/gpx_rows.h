@@ -90,7 +90,8 @@ typedef int RowAt __attribute__((ext_vector_type(8)));  // of a slab: lo[1], hi[
 constexpr int row_entry(int form, int order) { return order == 2 ? (form == 0 ? 12 : 8) : 4; }
 
 // A model as the row kernels see it; in device memory, read through the scalar
-// cache.  State and H Phi twice: launch argument `flip` says which is current.
+// cache.  State and Phi twice: launch arguments `flip` (E Phi:
+// `flipE`) say which is current.
 struct RowModel {
     int nx, ny, nz, kp, plane;       // kp: floats per row; plane = (ny + 1) kp
     int LT, LTo, hk, R, Ro, hj;      // lanes of a tile (own: LTo, halo: hk), rows (own: Ro, halo: hj)
@@ -107,7 +108,7 @@ struct RowModel {
     float h[5];                      // the H coefficients when every material has the same
     int nRT;                         // floats of a field's profile table
     RowAt atE[6], atH[6];            // the slabs by direction
-    float *phiE, *phiH[2];
+    float *phiE[2], *phiH[2];
     uint32_t np4;                    // bytes of one (order, term) block of Phi
     TArgs T;
     int iterations;
@@ -118,7 +119,7 @@ struct RowModel {
 struct RowArgs {
     const int *item0;                // [ntr + 1]: first item of each model (unused with one)
     int ntr, nitems, per_xcd;
-    int flip, it;
+    int flip, flipE, it;
     int p0, p1;                      // the passes' planes (p1 past the last one: to the model's end)
 };
 
@@ -759,7 +760,7 @@ __device__ __forceinline__ RowPlace row_place(const RowModel &a, int tk, int t)
 }
 
 template <int P, bool CPLX, int FORM, int ORDER, bool HU>
-__device__ __forceinline__ void row_step_item(const RowModel &a, const RowLds &S, int item, int flip, int it)
+__device__ __forceinline__ void row_step_item(const RowModel &a, const RowLds &S, int item, int flip, int flipE, int it)
 {
     const int tk = item % a.ntk, r1 = item / a.ntk;
     const int tj = r1 % a.ntj, ch = r1 / a.ntj;
@@ -775,7 +776,7 @@ __device__ __forceinline__ void row_step_item(const RowModel &a, const RowLds &S
     const uint32_t ti = to >> 1;
     const int xa = ch * a.xc, xb = min(xa + a.xc, a.nx + 1), xs = xa > 0 ? xa - 1 : 0;
     const rsrc_t rF = rsrc(a.F[flip]), wF = rsrc(a.F[flip ^ 1]), rI = rsrc(a.ID);
-    const rsrc_t rP = rsrc(a.phiH[flip]), wP = rsrc(a.phiH[flip ^ 1]), rPE = rsrc(a.phiE);
+    const rsrc_t rP = rsrc(a.phiH[flip]), wP = rsrc(a.phiH[flip ^ 1]), rPE = rsrc(a.phiE[flipE]);
     const uint32_t P4 = (uint32_t)a.plane * 4u, Pi = (uint32_t)a.plane * 2u, cs = a.cs, ci = a.ci;
     const uint32_t np4 = __builtin_amdgcn_readfirstlane(a.np4);
     // the next lane of the wave holds E at k+1, except where the row goes on
@@ -894,7 +895,7 @@ __global__ void __launch_bounds__(ROW_BLOCK_MAX) __attribute__((amdgpu_waves_per
     const RowModel &a = models[row_model_of(b, g, first)];
     const RowLds S = row_stage<ORDER, HU, true, true>(lds4, a);
     __syncthreads();
-    row_step_item<P, CPLX, FORM, ORDER, HU>(a, S, g - first, b.flip, b.it);
+    row_step_item<P, CPLX, FORM, ORDER, HU>(a, S, g - first, b.flip, b.flipE, b.it);
 }
 
 // ---------------------------------------------------------------- passes
@@ -1008,7 +1009,7 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t tob = j > 0 ? to - 4u * (uint32_t)a.kp : to;
     const uint32_t ti = to >> 1;
-    const rsrc_t rF = rsrc(a.F[b.flip]), rI = rsrc(a.ID), rP = rsrc(a.phiE);
+    const rsrc_t rF = rsrc(a.F[b.flip]), rI = rsrc(a.ID), rP = rsrc(a.phiE[b.flipE]);
     const uint32_t P4 = (uint32_t)a.plane * 4u, Pi = (uint32_t)a.plane * 2u, cs = a.cs, ci = a.ci;
     const uint32_t np4 = __builtin_amdgcn_readfirstlane(a.np4);
     const bool patch = q.live && lane == 0 && kl > 0;
@@ -1072,11 +1073,20 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
     }
 }
 
-typedef void (*row_kernel)(const RowModel *, RowArgs);
+}  // namespace gpx
 
-// The kernels of one model: the whole step, the H pass, the E pass.
+#include "gpx_plane.h"
+
+namespace gpx {
+
+typedef void (*row_kernel)(const RowModel *, RowArgs);
+typedef void (*plane_kernel)(const RowModel *, PlaneArgs);
+
+// The kernels of one model: the whole step, the H pass, the E pass, several
+// iterations of a 2-D model (without poles).
 struct RowKernels {
     row_kernel step, h, e;
+    plane_kernel plane;
 };
 
 template <int FORM, int ORDER>
@@ -1084,7 +1094,8 @@ RowKernels row_kernel_table(int P, bool C, bool hu)
 {
 #define GPX_RK(PP, CC)                                                                                       \
     RowKernels{hu ? k_row_step<PP, CC, FORM, ORDER, true> : k_row_step<PP, CC, FORM, ORDER, false>,          \
-               hu ? k_row_h<FORM, ORDER, true> : k_row_h<FORM, ORDER, false>, k_row_e<PP, CC, FORM, ORDER>}
+               hu ? k_row_h<FORM, ORDER, true> : k_row_h<FORM, ORDER, false>, k_row_e<PP, CC, FORM, ORDER>, \
+               PP == 0 ? k_plane<FORM, ORDER> : nullptr}
     switch (P) {
     case 0: return GPX_RK(0, false);
     case 1: return C ? GPX_RK(1, true) : GPX_RK(1, false);

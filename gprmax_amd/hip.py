@@ -196,8 +196,9 @@ class HipSolver:
         """Step form of gpx_run: 0 and 6 the H and E row passes, 1 the whole
         step in one launch, 2 the general passes with interior and boundary
         kernels side by side, 3, 5, 7 and 4 (the default) by rule: the one
-        launch for 3-D models without slabs and poles, the passes otherwise.
-        All give the same bits."""
+        launch for 3-D models without slabs and poles, several iterations a
+        launch for 2-D models without poles, the passes otherwise.  All give
+        the same bits."""
         self._check(self.lib.gpx_set_step(self.ctx, int(fused), int(tile_cells)))
 
     def step_kind(self):

@@ -164,9 +164,10 @@ int gpx_set_launch(gpx_ctx *ctx, int xchunk, int block);
  * state double-buffered; fused = 2: the general passes with their interior
  * and boundary kernels side by side on two streams (gpx_run_profiled runs them
  * one after the other); fused = 3, 5, 7 and 4 (default): by rule, the one
- * launch for 3-D models without slabs and dispersive poles, the passes
- * otherwise.  tile_cells = cells per block of form 1 (256, 512 or 1024; 0 =
- * auto).  All forms give identical results; models the row kernels do not take
+ * launch for 3-D models without slabs and dispersive poles, several iterations
+ * a launch for 2-D models without poles (reported as the passes, which
+ * gpx_run_profiled times), the passes otherwise.  tile_cells = cells per block
+ * of form 1 (256, 512 or 1024; 0 = auto).  All forms give identical results; models the row kernels do not take
  * (slabs of different orders, in another order or overlapping, more than 32
  * bits of byte offsets, tables past the LDS) run the general passes. */
 int gpx_set_step(gpx_ctx *ctx, int fused, int tile_cells);

@@ -13,7 +13,7 @@ import pytest
 
 import oracle
 from oracle import solver as osolver
-from gpu_models import randomise_tables, rich_model
+from gpu_models import plane_model, randomise_tables, rich_model
 from test_gpu_parity import COMPS, _assert_state_equal, _hip, _push_state, _random_state
 
 pytestmark = pytest.mark.gpu
@@ -139,3 +139,38 @@ def test_blocks_of_planes(shape, poles, magnetic):
                        + [s.download_snapshot(n) for n in range(len(G.snapshots))] + ([s.download_T()] if poles else []))
     for n, (a, b) in enumerate(zip(*got)):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), n
+
+
+@pytest.mark.parametrize('n', [1, 7, 31], ids=['n1', 'n7', 'n31'])
+@pytest.mark.parametrize('size', [(14, 17), (25, 24), (57, 90), (300, 211)], ids=str)
+@pytest.mark.parametrize('axis', [0, 1, 2], ids=['TMx', 'TMy', 'TMz'])
+def test_2d_tiles(axis, size, n):
+    """Several iterations of a 2-D model in one launch, planes smaller and
+    larger than a tile, sources on one edge and several receivers at one point,
+    between snapshots and in stretches of n; as the passes give it, bit for bit."""
+    G = plane_model(seed=60 + n, axis=axis, size=size, iterations=62, order=1 + n % 2,
+                    formulation='MRIPML' if n == 7 else 'HORIPML')
+    G.rxs = G.rxs + G.rxs[:1] + G.rxs[-1:]
+    G.hertziandipoles = G.hertziandipoles + G.hertziandipoles[:1]
+    got = []
+    for form in (4, 6):
+        with _hip()(G) as s:
+            s.set_step(form)
+            for it in range(0, 62, n):
+                s.run(it, min(n, 62 - it))
+            got.append([s.download_fields(), s.download_rx(), s.download_snapshot(0)]
+                       + [s.download_phi(p, w) for p in range(len(G.pmls)) for w in range(4)])
+    assert np.abs(got[0][0]).max() > 0
+    for q, (a, b) in enumerate(zip(*got)):
+        assert np.array_equal(a, b), q
+    # what the tiles' kernel leaves out may not be zero: the passes run
+    F = np.random.default_rng(61).standard_normal(got[0][0].shape).astype(np.float32)
+    out = []
+    for form in (4, 6):
+        with _hip()(G) as s:
+            s.set_step(form)
+            s.run(0, 9)
+            s.upload_fields(F)
+            s.run(9, 3)
+            out.append(s.download_fields())
+    assert np.array_equal(*out)
