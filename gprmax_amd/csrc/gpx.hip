@@ -774,6 +774,7 @@ struct gpx_ctx {
     uint8_t *dispflag = nullptr;
     float *T[3] = {nullptr, nullptr, nullptr};  // compacted: [P][tn[c]] (x2 complex)
     uint32_t *tslot[3] = {nullptr, nullptr, nullptr};  // [ntot]: place of an edge with poles
+    uint32_t *tmasks = nullptr;      // the same as the row passes read it
     long long tn[3] = {0, 0, 0};     // edges with poles per component
     bool tslot_dirty = true;         // ID or dispersive tables changed since the slots were built
     bool have_id = false, have_coeffs = false, have_disp = false;
@@ -940,6 +941,7 @@ extern "C" int gpx_destroy(gpx_ctx *ctx)
     for (auto &p : ctx->Fmem) if (p) hipFree(p);
     for (auto &p : ctx->T) if (p) hipFree(p);
     for (auto &p : ctx->tslot) if (p) hipFree(p);
+    if (ctx->tmasks) hipFree(ctx->tmasks);
     if (ctx->ID) hipFree(ctx->ID);
     if (ctx->cE) hipFree(ctx->cE);
     if (ctx->cH) hipFree(ctx->cH);
@@ -1117,6 +1119,29 @@ __global__ void __launch_bounds__(1024) k_tslot_fill(const IDT *ID, const uint8_
     if (e < ntot) slot[e] = f ? boff[blockIdx.x] + (uint32_t)(off + before) : 0xffffffffu;
 }
 
+// The slots as the passes read them (row_slots_of): a wave for each group of
+// 64 lanes of a plane (128 cells of `plane`, fewer at its end) and each component.
+__global__ void k_tslot_masks(const uint32_t *slot, uint32_t *masks, int c, int plane, int groups, int n)
+{
+    const int g = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (g >= n) return;
+    const int i = g / groups, q = (g - i * groups) * 128 + 2 * lane;
+    const uint32_t *s = slot + (size_t)i * plane;
+    const uint32_t s0 = q < plane ? s[q] : T_NOSLOT, s1 = q + 1 < plane ? s[q + 1] : T_NOSLOT;
+    const unsigned long long even = __ballot(s0 != T_NOSLOT), odd = __ballot(s1 != T_NOSLOT), any = even | odd;
+    const uint32_t mine = s0 != T_NOSLOT ? s0 : s1;
+    const uint32_t first = any ? __shfl(mine, __ffsll(any) - 1) : 0u;
+    if (lane == 0) {
+        uint32_t *m = masks + (size_t)g * 16;
+        m[4 * c] = (uint32_t)even;
+        m[4 * c + 1] = (uint32_t)(even >> 32);
+        m[4 * c + 2] = (uint32_t)odd;
+        m[4 * c + 3] = (uint32_t)(odd >> 32);
+        m[12 + c] = first;
+    }
+}
+static int tslot_groups(const gpx_ctx *ctx) { return (ctx->plane + 127) / 128; }
+
 static int ensure_tslots(gpx_ctx *ctx);
 
 static void fill_targs(const gpx_ctx *ctx, TArgs &t)
@@ -1126,6 +1151,8 @@ static void fill_targs(const gpx_ctx *ctx, TArgs &t)
         t.slot[c] = ctx->tslot[c];
         t.n[c] = ctx->tn[c];
     }
+    t.masks = ctx->tmasks;
+    t.groups = tslot_groups(ctx);
 }
 
 // Builds the slots and the compacted auxiliary arrays (zeroed) once the
@@ -1139,6 +1166,8 @@ static int ensure_tslots(gpx_ctx *ctx)
     if (N >= 0xffffffffLL) return fail(ctx, GPX_ELIMIT, "dispersive models need fewer than 2^32 points");
     hipSetDevice(ctx->desc.device);
     const int nb = (int)((N + 1023) / 1024);
+    const int ng = (ctx->desc.nx + 1) * tslot_groups(ctx);
+    if (!ctx->tmasks) GPX_TRY(dalloc(ctx, (void **)&ctx->tmasks, (size_t)ng * 64, false));
     uint32_t *boff = nullptr;
     GPX_TRY(dalloc(ctx, (void **)&boff, (size_t)nb * 4, false));
     std::vector<uint32_t> h(nb);
@@ -1160,12 +1189,15 @@ static int ensure_tslots(gpx_ctx *ctx)
         if ((rc = copy_in(ctx, boff, h.data(), (size_t)nb * 4))) break;
         hipLaunchKernelGGL(k_tslot_fill<uint16_t>, dim3(nb), dim3(1024), 0, ctx->stream,
                            ctx->ID + (size_t)c * N, ctx->dispflag, N, boff, ctx->tslot[c]);
+        hipLaunchKernelGGL(k_tslot_masks, dim3((ng + 3) / 4), dim3(256), 0, ctx->stream, ctx->tslot[c], ctx->tmasks, c,
+                           ctx->plane, tslot_groups(ctx), ng);
         hipError_t e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) { rc = fail_hip(ctx, e, "slot build"); break; }
         ctx->tn[c] = (long long)acc;
         if (ctx->T[c]) { hipFree(ctx->T[c]); ctx->T[c] = nullptr; }
         ctx->row_dirty = true;
-        const size_t tb = (size_t)P * (size_t)(acc > 0 ? acc : 1) * 4 * (ctx->disp_complex ? 2 : 1);
+        // a pair's load at the last slot goes one value further
+        const size_t tb = ((size_t)P * (size_t)(acc > 0 ? acc : 1) + 1) * 4 * (ctx->disp_complex ? 2 : 1);
         e = dalloc(ctx, (void **)&ctx->T[c], tb);
         if (e != hipSuccess) { rc = fail_hip(ctx, e, "auxiliary values"); break; }
     }
@@ -2499,7 +2531,7 @@ static double pass_bytes(const gpx_ctx *ctx)
     double b = (double)ctx->fstride * 24.0 + (double)ctx->ntot * 2.0 * (ctx->hu ? 3 : 6);
     if (!ctx->slabs.empty()) b += 2.0 * (double)phi_bytes(ctx);
     if (ctx->desc.maxpoles > 0) {
-        b += (double)ctx->ntot * 12.0;
+        b += (double)ctx->ntot / 2;
         for (int c = 0; c < 3; ++c) b += (double)ctx->tn[c] * ctx->desc.maxpoles * (ctx->disp_complex ? 8 : 4);
     }
     return b;

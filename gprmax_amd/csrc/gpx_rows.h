@@ -52,7 +52,7 @@
 // apart, one cell per lane) or two with one merged step before:
 //   120x105 (2-D)  8.6 from 16.7     100x100x100   22.5 from 40.8
 //   157x131x97 MRIPML order 2  45 from 72        300x300x200  276 from 425
-//   611x407x45  200 from 375      240x240x180, 3 poles  294 from 478
+//   611x407x45  200 from 375      240x240x180, 3 poles  269 from 478
 #ifndef GPX_ROWS_H
 #define GPX_ROWS_H
 
@@ -485,7 +485,8 @@ __device__ __forceinline__ void row_h(const RowModel &a, const RowLds &S, uint32
 {
     const fN dEz_y = ezj - ez, dEy_z = eyk - ey, dEx_z = exk - ex;
     const fN dEz_x = ez1 - ez, dEy_x = ey1 - ey, dEx_y = exj - ex;
-    const bool bx = i >= 1 && j < a.ny, by = i < a.nx && j >= 1, bz = i < a.nx && j < a.ny;
+    const int nx = a.nx, ny = a.ny, nz = a.nz;   // read once, and no branches
+    const bool bx = (i >= 1) & (j < ny), by = (i < nx) & (j >= 1), bz = (i < nx) & (j < ny);
     float4 ux, uy, uz;
     if (HU) ux = uy = uz = make_float4(a.h[0], a.h[1], a.h[2], a.h[3]);
 #pragma unroll
@@ -499,9 +500,9 @@ __device__ __forceinline__ void row_h(const RowModel &a, const RowLds &S, uint32
         const float nx_ = ux.x * hx[u] - ux.z * dEz_y[u] + ux.w * dEy_z[u];
         const float ny_ = uy.x * hy[u] - uy.w * dEx_z[u] + uy.y * dEz_x[u];
         const float nz_ = uz.x * hz[u] - uz.y * dEy_x[u] + uz.z * dEx_y[u];
-        hx[u] = bx && k < a.nz ? nx_ : hx[u];
-        hy[u] = by && k < a.nz ? ny_ : hy[u];
-        hz[u] = bz && k >= 1 && k <= a.nz ? nz_ : hz[u];
+        hx[u] = bx & (k < nz) ? nx_ : hx[u];
+        hy[u] = by & (k < nz) ? ny_ : hy[u];
+        hz[u] = bz & (k >= 1) & (k <= nz) ? nz_ : hz[u];
     }
     auto c3 = [&](int u) { return HU ? a.h[4] : S.sH[id_of(m3, u)]; };
     auto c4 = [&](int u) { return HU ? a.h[4] : S.sH[id_of(m4, u)]; };
@@ -566,22 +567,131 @@ __device__ __forceinline__ void row_rx(const RowModel &a, int i, int j, int kl, 
 template <int P, bool CPLX>
 struct RowT {
     uN s;                // slots, T_NOSLOT for edges without poles or outside the range
-    float r[NC][P > 0 ? P : 1], i[NC][P > 0 && CPLX ? P : 1];
+    fN r[P > 0 ? P : 1], i[P > 0 && CPLX ? P : 1];   // of the lane's cells
 };
 
+// Calls f for poles (or cells) 0 to P - 1, each a constant (with a loop the values are
+// indexed before it is unrolled and end up in scratch memory).
+template <int P, class Fn>
+__device__ __forceinline__ void row_poles(const Fn &f)
+{
+    if constexpr (P > 0) {
+        row_poles<P - 1>(f);
+        f(std::integral_constant<int, P - 1>{});
+    }
+}
+
+// The values of pole p of component c.  A lane without any loads and stores at
+// T_NONE, past the resource's end, where the hardware drops the access: no branch
+// splits the plane's loads, which a wait for each component's would follow.
+constexpr uint32_t T_NONE = 0xfffffff0u;
+template <bool CPLX>
+__device__ __forceinline__ rsrc_t row_t_at(const TArgs &T, int c, int p)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(T.T[c] + (size_t)p * (size_t)T.n[c] * (CPLX ? 2 : 1), 0, 0xffffff00u, 0x00020000);
+}
+
+// Neighbouring edges with poles have neighbouring slots, so one load a pole
+// brings both cells' values, or a value and what lies after it (after the
+// last slot: the array's padding); row_t_settle gives the second cell its own
+// where the values are first used.
 template <int P, bool CPLX>
 __device__ __forceinline__ void row_t_load(const TArgs &T, int c, RowT<P, CPLX> &t)
 {
-#pragma unroll
-    for (int u = 0; u < NC; ++u)
-        if (t.s[u] != T_NOSLOT) {
-            if (CPLX) {
-                t_load_at<P, CPLX>(T, c, t.s[u], t.r[u], t.i[u]);
-            } else {
-                float none[P > 0 ? P : 1];
-                t_load_at<P, CPLX>(T, c, t.s[u], t.r[u], none);
-            }
+    const uint32_t q0 = t.s[0], q1 = t.s[1], s = q0 != T_NOSLOT ? q0 : q1;
+    const uint32_t q = s != T_NOSLOT ? s * (CPLX ? 8u : 4u) : T_NONE;
+    row_poles<P>([&](auto pole) {
+        constexpr int p = decltype(pole)::value;
+        const rsrc_t r = row_t_at<CPLX>(T, c, p);
+        if constexpr (CPLX) {
+            const float4 v = bits<float4>(__builtin_amdgcn_raw_buffer_load_b128(r, q, 0, 0));
+            t.r[p] = (fN){v.x, v.z};
+            t.i[p] = (fN){v.y, v.w};
+        } else {
+            t.r[p] = bldN(r, q, 0);
         }
+    });
+}
+template <int P, bool CPLX>
+__device__ __forceinline__ void row_t_settle(RowT<P, CPLX> &t)
+{
+    const bool both = t.s[0] != T_NOSLOT;
+    row_poles<P>([&](auto pole) {
+        constexpr int p = decltype(pole)::value;
+        const float x = t.r[p][0], y = t.r[p][1];
+        t.r[p][1] = both ? y : x;
+        if constexpr (CPLX) {
+            const float v = t.i[p][0], w = t.i[p][1];
+            t.i[p][1] = both ? w : v;
+        }
+    });
+}
+template <int P, bool CPLX>
+__device__ __forceinline__ void row_t_store(const TArgs &T, int c, const RowT<P, CPLX> &t)
+{
+    const uint32_t q0 = t.s[0], q1 = t.s[1], w = CPLX ? 8u : 4u;
+    const bool in0 = q0 != T_NOSLOT, in1 = q1 != T_NOSLOT;
+    const uint32_t two = in0 & in1 ? q0 * w : T_NONE, one = in0 != in1 ? (in0 ? q0 : q1) * w : T_NONE;
+    if (__any(in0 & in1)) row_poles<P>([&](auto pole) {
+        constexpr int p = decltype(pole)::value;
+        const rsrc_t r = row_t_at<CPLX>(T, c, p);
+        if constexpr (CPLX)
+            __builtin_amdgcn_raw_buffer_store_b128(bits<u32x4>(make_float4(t.r[p][0], t.i[p][0], t.r[p][1], t.i[p][1])), r, two, 0, 0);
+        else
+            bstN(r, two, 0, t.r[p]);
+    });
+    if (!__any(in0 != in1)) return;
+    row_poles<P>([&](auto pole) {
+        constexpr int p = decltype(pole)::value;
+        const rsrc_t r = row_t_at<CPLX>(T, c, p);
+        const float r0 = t.r[p][0], r1 = t.r[p][1];
+        if constexpr (CPLX) {
+            const float i0 = t.i[p][0], i1 = t.i[p][1];
+            __builtin_amdgcn_raw_buffer_store_b64(bits<u32x2>(make_float2(in0 ? r0 : r1, in0 ? i0 : i1)), r, one, 0, 0);
+        } else {
+            bst(r, one, 0, in0 ? r0 : r1);
+        }
+    });
+}
+
+// disp_a and disp_b for cell U of a lane.
+template <int U, int P, bool CPLX>
+__device__ __forceinline__ float row_disp_a(const float *D, uint32_t m, RowT<P, CPLX> &t, float e)
+{
+    float phi = 0.f;
+    const float *c = D + (size_t)m * 3 * P * (CPLX ? 2 : 1);
+    row_poles<P>([&](auto pole) {
+        constexpr int p = decltype(pole)::value;
+        const float r = t.r[p][U];
+        if constexpr (CPLX) {
+            const float *k = c + 6 * p;
+            const float i = t.i[p][U];
+            if constexpr (P == 1) phi = k[0] * r;
+            else phi = phi + k[0] * r;
+            t.r[p][U] = (k[2] * r - k[3] * i) + k[4] * e;
+            t.i[p][U] = (k[2] * i + k[3] * r) + k[5] * e;
+        } else {
+            const float *k = c + 3 * p;
+            if constexpr (P == 1) phi = k[0] * r;
+            else phi = phi + k[0] * r;
+            t.r[p][U] = k[1] * r + k[2] * e;
+        }
+    });
+    return phi;
+}
+template <int U, int P, bool CPLX>
+__device__ __forceinline__ void row_disp_b(const float *D, uint32_t m, RowT<P, CPLX> &t, float e)
+{
+    const float *c = D + (size_t)m * 3 * P * (CPLX ? 2 : 1);
+    row_poles<P>([&](auto pole) {
+        constexpr int p = decltype(pole)::value;
+        if constexpr (CPLX) {
+            t.r[p][U] = t.r[p][U] - c[6 * p + 4] * e;
+            t.i[p][U] = t.i[p][U] - c[6 * p + 5] * e;
+        } else {
+            t.r[p][U] = t.r[p][U] - c[3 * p + 2] * e;
+        }
+    });
 }
 
 // E of a lane's cells at plane i: update_electric or dispersive part A
@@ -597,21 +707,26 @@ __device__ __forceinline__ void row_e(const RowModel &a, const RowLds &S, uint32
 {
     const fN dHz_y = hz - hzj, dHy_z = hy - hyk, dHx_z = hx - hxk;
     const fN dHz_x = hz - hzm, dHy_x = hy - hym, dHx_y = hx - hxj;
-    const bool bx = i < a.nx && j >= 1 && j < a.ny, by = i >= 1 && i < a.nx && j < a.ny,
-               bz = i >= 1 && i < a.nx && j >= 1 && j < a.ny;
-#pragma unroll
-    for (int u = 0; u < NC; ++u) {
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const bool ji = (j >= 1) & (j < ny), ii = (i >= 1) & (i < nx);
+    const bool bx = (i < nx) & ji, by = ii & (j < ny), bz = ii & ji;
+    if constexpr (P > 0) {
+        row_t_settle(tx);
+        row_t_settle(ty);
+        row_t_settle(tz);
+    }
+    row_poles<NC>([&](auto cell) {
+        constexpr int u = decltype(cell)::value;
         const int k = kl + u;
         const uint32_t i0 = id_of(m0, u), i1 = id_of(m1, u), i2 = id_of(m2, u);
         const float4 q0 = S.cE[i0], q1 = S.cE[i1], q2 = S.cE[i2];
-        const bool rx_ = bx && k >= 1 && k < a.nz, ry_ = by && k >= 1 && k < a.nz, rz_ = bz && k < a.nz;
+        const bool ki = (k >= 1) & (k < nz), rx_ = bx & ki, ry_ = by & ki, rz_ = bz & (k < nz);
         float vx = q0.x * ex[u] + q0.z * dHz_y[u] - q0.w * dHy_z[u];
         float vy = q1.x * ey[u] + q1.w * dHx_z[u] - q1.y * dHz_x[u];
         float vz = q2.x * ez[u] + q2.y * dHy_x[u] - q2.z * dHx_y[u];
         if (P > 0) {
-            float none[P > 0 ? P : 1];
             auto part_a = [&](RowT<P, CPLX> &t, uint32_t m, float e, float v) {
-                const float phi = t.s[u] != T_NOSLOT ? disp_a<P, CPLX>(S.disp, m, t.r[u], CPLX ? t.i[u] : none, e) : 0.f;
+                const float phi = t.s[u] != T_NOSLOT ? row_disp_a<u, P, CPLX>(S.disp, m, t, e) : 0.f;
                 return v - S.sE[m] * phi;
             };
             vx = part_a(tx, i0, ex[u], vx);
@@ -621,7 +736,7 @@ __device__ __forceinline__ void row_e(const RowModel &a, const RowLds &S, uint32
         ex[u] = rx_ ? vx : ex[u];
         ey[u] = ry_ ? vy : ey[u];
         ez[u] = rz_ ? vz : ez[u];
-    }
+    });
     auto c0 = [&](int u) { return S.sE[id_of(m0, u)]; };
     auto c1 = [&](int u) { return S.sE[id_of(m1, u)]; };
     auto c2 = [&](int u) { return S.sE[id_of(m2, u)]; };
@@ -677,24 +792,42 @@ __device__ __forceinline__ void row_e(const RowModel &a, const RowLds &S, uint32
             }
         }
     }
-    if (P > 0) {
-        float none[P > 0 ? P : 1];
-#pragma unroll
-        for (int u = 0; u < NC; ++u) {
-            auto part_b = [&](RowT<P, CPLX> &t, int c, uint32_t m, float e) {
-                if (t.s[u] == T_NOSLOT) return;
-                disp_b<P, CPLX>(S.disp, m, t.r[u], CPLX ? t.i[u] : none, e);
-                t_store<P, CPLX>(a.T, c, t.s[u], t.r[u], CPLX ? t.i[u] : none);
+    if constexpr (P > 0) {
+        row_poles<NC>([&](auto cell) {
+            constexpr int u = decltype(cell)::value;
+            auto part_b = [&](RowT<P, CPLX> &t, uint32_t m, float e) {
+                if (t.s[u] != T_NOSLOT) row_disp_b<u, P, CPLX>(S.disp, m, t, e);
             };
-            part_b(tx, 0, id_of(m0, u), ex[u]);
-            part_b(ty, 1, id_of(m1, u), ey[u]);
-            part_b(tz, 2, id_of(m2, u), ez[u]);
-        }
+            part_b(tx, id_of(m0, u), ex[u]);
+            part_b(ty, id_of(m1, u), ey[u]);
+            part_b(tz, id_of(m2, u), ez[u]);
+        });
+        row_t_store(a.T, 0, tx);
+        row_t_store(a.T, 1, ty);
+        row_t_store(a.T, 2, tz);
     }
 }
 
-// Slots of a lane's edges at plane i, with the edges outside the update
-// ranges (which hold no auxiliary values in use) marked as without.
+// Edges outside the update ranges (which hold no auxiliary values in use)
+// count as without.
+template <int P, bool CPLX>
+__device__ __forceinline__ void row_slots_in(const RowModel &a, int i, int j, int kl, RowT<P, CPLX> &tx, RowT<P, CPLX> &ty,
+                                             RowT<P, CPLX> &tz)
+{
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const bool ji = (j >= 1) & (j < ny), ii = (i >= 1) & (i < nx);
+    const bool bx = (i < nx) & ji, by = ii & (j < ny), bz = ii & ji;
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int k = kl + u;
+        const bool ki = (k >= 1) & (k < nz);
+        tx.s[u] = bx & ki ? tx.s[u] : T_NOSLOT;
+        ty.s[u] = by & ki ? ty.s[u] : T_NOSLOT;
+        tz.s[u] = bz & (k < nz) ? tz.s[u] : T_NOSLOT;
+    }
+}
+
+// Slots of a lane's edges at plane i, from the arrays of every edge's slot.
 template <int P, bool CPLX>
 __device__ __forceinline__ void row_slots(const RowModel &a, int i, int j, int kl, uint32_t off, RowT<P, CPLX> &tx,
                                           RowT<P, CPLX> &ty, RowT<P, CPLX> &tz)
@@ -708,15 +841,40 @@ __device__ __forceinline__ void row_slots(const RowModel &a, int i, int j, int k
     tx.s = get(0);
     ty.s = get(1);
     tz.s = get(2);
-    const bool bx = i < a.nx && j >= 1 && j < a.ny, by = i >= 1 && i < a.nx && j < a.ny,
-               bz = i >= 1 && i < a.nx && j >= 1 && j < a.ny;
-#pragma unroll
-    for (int u = 0; u < NC; ++u) {
-        const int k = kl + u;
-        if (!(bx && k >= 1 && k < a.nz)) tx.s[u] = T_NOSLOT;
-        if (!(by && k >= 1 && k < a.nz)) ty.s[u] = T_NOSLOT;
-        if (!(bz && k < a.nz)) tz.s[u] = T_NOSLOT;
-    }
+    row_slots_in(a, i, j, kl, tx, ty, tz);
+}
+
+// The same for a wave of a pass, whose lanes hold 128 edges one after the other
+// (group `grp` of the plane): of each component the first slot among them and
+// two masks of the edges with poles, one for each cell of a lane, 64 bytes in
+// all through the scalar cache.  Slots read edge by edge are 12 bytes a cell more to
+// fetch (the E pass of 240x240x180, 30 % of the cells with 3 poles, moves about
+// 85); with a load for each value instead of each pair besides, us per iteration:
+// that grid 296, now 269; 200x150x130 Drude 96, 76; 121x104x90 with two complex poles
+// 44.9, 43.1; 150x140x100, 2 poles in 10 % of the cells, 55.1, 54.7.
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ u32x16 row_masks(const TArgs &T, int i, int grp)
+{
+    typedef __attribute__((address_space(4))) const u32x16 cu32x16;
+    return ((cu32x16 *)T.masks)[(size_t)i * T.groups + grp];
+}
+template <int P, bool CPLX>
+__device__ __forceinline__ void row_slots_of(const RowModel &a, int i, int j, int kl, u32x16 w, bool live, RowT<P, CPLX> &tx,
+                                             RowT<P, CPLX> &ty, RowT<P, CPLX> &tz)
+{
+    const int lane = threadIdx.x & 63;
+    auto get = [&](int c, RowT<P, CPLX> &t) {
+        const uint32_t e0 = w[4 * c], e1 = w[4 * c + 1], o0 = w[4 * c + 2], o1 = w[4 * c + 3];
+        uint32_t n = __builtin_amdgcn_mbcnt_hi(e1, __builtin_amdgcn_mbcnt_lo(e0, w[12 + c]));
+        n = __builtin_amdgcn_mbcnt_hi(o1, __builtin_amdgcn_mbcnt_lo(o0, n));
+        const uint32_t even = ((lane < 32 ? e0 : e1) >> (lane & 31)) & 1u, odd = ((lane < 32 ? o0 : o1) >> (lane & 31)) & 1u;
+        t.s[0] = live && even ? n : T_NOSLOT;
+        t.s[1] = live && odd ? n + even : T_NOSLOT;
+    };
+    get(0, tx);
+    get(1, ty);
+    get(2, tz);
+    row_slots_in(a, i, j, kl, tx, ty, tz);
 }
 
 // ---------------------------------------------------------------- whole step
@@ -1013,6 +1171,11 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
     const uint32_t P4 = (uint32_t)a.plane * 4u, Pi = (uint32_t)a.plane * 2u, cs = a.cs, ci = a.ci;
     const uint32_t np4 = __builtin_amdgcn_readfirstlane(a.np4);
     const bool patch = q.live && lane == 0 && kl > 0;
+    int grp = 0;    // the wave's place in the plane, in groups of 64 lanes; past the plane's end any
+    if (P > 0) {
+        grp = __builtin_amdgcn_readfirstlane(((g - first) % a.pseg * (int)blockDim.x + (int)threadIdx.x) >> 6);
+        grp = min(grp, a.T.groups - 1);
+    }
     RowSlabs L;
     if (ORDER > 0) L = row_slabs(a.atE, j, kl, q.live);
     const uint32_t sm = (uint32_t)(q.xa > 0 ? q.xa - 1 : 0) * P4;
@@ -1026,7 +1189,8 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
     auto load = [&](int i) {
         pf = plane_flags(a, i);
         const uint32_t so = (uint32_t)i * P4, si = (uint32_t)i * Pi;
-        if (P > 0 && q.live) row_slots(a, i, j, kl, to, tx, ty, tz);
+        u32x16 masks = 0u;
+        if (P > 0) masks = row_masks(a.T, i, grp);
         hx = bldN(rF, to, so + 3 * cs);
         hy = bldN(rF, to, so + 4 * cs);
         hz = bldN(rF, to, so + 5 * cs);
@@ -1046,7 +1210,8 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
             m = L.m & (pf >> PF_SLAB_E);
             row_phis(ph, L, m, (pf >> PF_SLAB_E) & 1u, rP, np4, i, j, kl);
         }
-        if (P > 0 && q.live) {
+        if (P > 0) {
+            row_slots_of(a, i, j, kl, masks, q.live, tx, ty, tz);
             row_t_load(a.T, 0, tx);
             row_t_load(a.T, 1, ty);
             row_t_load(a.T, 2, tz);

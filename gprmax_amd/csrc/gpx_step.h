@@ -331,6 +331,8 @@ struct TArgs {
     float *T[3];
     const uint32_t *slot[3];
     long long n[3];
+    const uint32_t *masks;    // [nx + 1][groups] entries of 64 bytes (row_slots_of)
+    int groups;
 };
 
 // Slot of an edge whose material has no poles.

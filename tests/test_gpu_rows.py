@@ -51,6 +51,26 @@ def test_row_lengths(order, formulation, shape, form):
     _check(G, form, 3)
 
 
+@pytest.mark.parametrize('block', [64, 512])
+@pytest.mark.parametrize('shape', [(13, 14, 12), (12, 31, 33), (12, 13, 131)], ids=str)
+@pytest.mark.parametrize('kind,poles', [('debye', 1), ('debye', 2), ('debye', 3), ('drude', 4), ('lorentz', 1), ('lorentz', 2),
+                                        ('lorentz', 3), ('lorentz', 4)])
+def test_auxiliary_values_by_groups(kind, poles, shape, block):
+    """Slots from a wave's masks: planes that end within a group of lanes and
+    blocks that end past the plane; edges with poles in one cell of a lane, in
+    both, in none."""
+    G = rich_model(seed=57, shape=shape, iterations=8, snapshots=False, pml=FACES, poles=poles, kind=kind)
+    _random_state(G, 9)
+    lib = oracle.load(np.float32)
+    with _hip()(G) as s:
+        s.set_launch(3, block)
+        _push_state(s, G)
+        s.run(0, 4)
+        for it in range(4):
+            osolver.step(lib, G, it, 8)
+        _assert_state_equal(s, G, 'block {}'.format(block))
+
+
 @pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
 @pytest.mark.parametrize('magnetic', [False, True])
 def test_values_of_every_magnitude(magnetic, form):
