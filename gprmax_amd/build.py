@@ -4,7 +4,11 @@ Flags:
 * ``-ffp-contract=off`` and ``-fhip-fp32-correctly-rounded-divide-sqrt``: every
   float expression rounds as written, so the kernels reproduce the CPU path's
   float32 arithmetic exactly;
-* ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed FP32 math.
+* ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed FP32 math;
+* ``-mllvm -amdgpu-kernarg-preload-count=16``: a kernel's first 16 dwords of
+  arguments are in registers when it starts, which spares a launch one round
+  trip through the scalar cache (us per iteration of the two passes on 60^3:
+  11.3 without, 11.0 with; 300x300x200: 274.9, 272.7).
 """
 
 import glob
@@ -28,6 +32,7 @@ HIPCC_FLAGS = [
     '-ffp-contract=off',
     '-fhip-fp32-correctly-rounded-divide-sqrt',
     '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
+    '-mllvm', '-amdgpu-kernarg-preload-count=16',
     '-Wall', '-Wno-unused-function',
 ]
 
