@@ -387,6 +387,15 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(P > 0 ? 2 : 0, OR
 }
 
 // ------------------------------------------------------------------ adjoint
+// A load of the stored states, which the sweep reads once, slots one after the
+// other: not to be kept, so that lE, lH and the gradients, which every iteration
+// goes over, stay in the last-level cache (the sweeps and their recompute on
+// 160x160x120, 600 iterations: 93.3 ms with ordinary loads, 90.4).
+__device__ __forceinline__ fN bld_stored(rsrc_t r, uint32_t voff, uint32_t soff)
+{
+    return bits<fN>(__builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 2));
+}
+
 // E half of iteration n: lH += (dE^{n+1}/dH^{n+1})^T lE*, the gradients from
 // lE*, E^n and the curl, and the Phi adjoints into b.Q.  lE* (the poles' part B
 // folded in) is left as it is.
@@ -433,12 +442,12 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(2, ORDER) k_inv_a
         hx = bldN(rH, to, so);
         hy = bldN(rH, to, so + cs);
         hz = bldN(rH, to, so + 2 * cs);
-        e0 = bldN(rE, to, so);
-        e1 = bldN(rE, to, so + cs);
-        e2 = bldN(rE, to, so + 2 * cs);
-        c0 = bldN(rC, to, so);
-        c1 = bldN(rC, to, so + cs);
-        c2 = bldN(rC, to, so + 2 * cs);
+        e0 = bld_stored(rE, to, so);
+        e1 = bld_stored(rE, to, so + cs);
+        e2 = bld_stored(rE, to, so + 2 * cs);
+        c0 = bld_stored(rC, to, so);
+        c1 = bld_stored(rC, to, so + cs);
+        c2 = bld_stored(rC, to, so + 2 * cs);
         gA = bldN(rG, to, so);
         gB = bldN(rG, to, so + cs);
         if (ORDER > 0) {
