@@ -368,7 +368,7 @@ def main():
                     help='headline workload: also run the B-scan and adjoint workloads and report them (1) or not (0)')
     ap.add_argument('--forms-traces', type=int, default=16, help='B-scan traces of that report')
     ap.add_argument('--bscan-its', type=int, default=1500, help='iterations per B-scan trace')
-    ap.add_argument('--bscan-graph', type=int, default=1, help='B-scan batch: iterations in HIP graphs (1) or launched directly (0)')
+    ap.add_argument('--bscan-graph', type=int, default=1, help='passed to the B-scan batch, where it makes no difference')
     ap.add_argument('--adj-its', type=int, default=2000, help='iterations of the adjoint workload')
     ap.add_argument('--fd-cells', type=int, default=0, help='finite-difference check cells (adjoint workload)')
     ap.add_argument('--adj-keep', type=int, default=1,

@@ -324,8 +324,7 @@ def device_info(device=0):
 class HipBatch:
     """Several HipSolver models advanced together: per iteration, the H and E
     row passes each over all models, or one launch of the whole step over all
-    models (models that share no row kernels: four general passes); optionally
-    all iterations in one HIP graph."""
+    models (models that share no row kernels: four general passes)."""
 
     def __init__(self, solvers):
         self.lib = library()
@@ -377,7 +376,9 @@ class HipBatch:
         return t.value, x.value, ms.value
 
     def run(self, it0, n, graph=True):
-        """Advance every model by n iterations from it0; returns device ms."""
+        """Advance every model by n iterations from it0; returns device ms.
+        ``graph`` makes no difference: a graph of one run costs more to make
+        than it saves."""
         ms = ctypes.c_float()
         self._check(self.lib.gpx_batch_run(self.b, int(it0), int(n), int(bool(graph)), ctypes.byref(ms)))
         return ms.value
@@ -413,7 +414,7 @@ def solve_bscan(grids, device=0, graph=True, group_bytes=0, tune_steps=3):
 
     Consecutive models form groups as the batch forms them (state bytes up to
     ``group_bytes``, 0: 192 MiB): a group of several runs as one HipBatch
-    (tuned, shared launches, ``graph``), a group of one as that model's plain
+    (tuned, shared launches), a group of one as that model's plain
     solve with its own step form.  While a group runs, a second host thread
     builds and uploads the next one, so each group's set-up hides behind the
     device work of the group before it; a group's models are freed once their

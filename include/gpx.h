@@ -239,8 +239,8 @@ int gpx_batch_tune(gpx_batch *b, int steps, int *tile_cells, int *xchunk, float 
  * the 256 MB last-level cache; a larger model forms its own group); each group
  * runs all its iterations before the next starts. */
 int gpx_batch_set_group_bytes(gpx_batch *b, double bytes);
-/* Iterations [it0, it0 + n) of every model; graph != 0 captures the n
- * launches in one HIP graph and launches that.  Waits; *ms (optional) is the
+/* Iterations [it0, it0 + n) of every model, launched on the batch's stream
+ * whatever `graph` says (a graph of one run costs more to make than it saves).  Waits; *ms (optional) is the
  * device time measured with HIP events around the launches. */
 int gpx_batch_run(gpx_batch *b, int it0, int n, int graph, float *ms);
 
