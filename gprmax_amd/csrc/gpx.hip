@@ -2539,19 +2539,22 @@ static double pass_bytes(const gpx_ctx *ctx)
 
 // Blocks of planes of run_wave: as few as keep a block within WAVE_BYTES, every
 // one more being a launch of 5 us per pass beside its bytes.  The last-level
-// cache has 256 MB; past about 200 a block evicts itself between the passes.  us per
-// iteration in 1, 2, 3, ... blocks (MB of a block in brackets where fastest):
+// cache has 256 MB; a block moves through the planes, and past about 200 it evicts itself
+// between the passes.  A grid that fits whole, up to WHOLE_BYTES, is not divided.  us per
+// iteration in 1, 2, 3, ... blocks (MiB of a block in brackets where fastest):
 // 300x300x200 348, 335, 296, 275 (at 3: 199), 283 ...; 250x220x180 179, 146 (168), 161;
 // 611x407x45 247, 226, 200 (146), 209; 420x400x200 612, 629, 606, 604, 567, 519
 // (182), 520 at 7, 570 at 13; 240x240x180 with 3 poles 320, 323, 294 (199), 299.
-static const double WAVE_BYTES = 200.0 * 1024 * 1024;
+// Around the whole cache: 196 MiB 76, 91; 216 82, 96; 236 90, 105; 248 119, 109; 256
+// 124, 110; 315 159, 132.
+static const double WAVE_BYTES = 200.0 * 1024 * 1024, WHOLE_BYTES = 240.0 * 1024 * 1024;
 // Iterations a block is taken through: 300x300x200 takes 357 us an iteration at
 // 1, 316 at 2, 290 at 4, 280 at 8, 276 at 16 and 278 at 32.  At one iteration whole passes
 // are the faster ones (347).
 static const int WAVE_ITS = 16;
 static int wave_blocks(const gpx_ctx *ctx)
 {
-    const double n = ceil(pass_bytes(ctx) / WAVE_BYTES);
+    const double bytes = pass_bytes(ctx), n = bytes <= WHOLE_BYTES ? 1.0 : ceil(bytes / WAVE_BYTES);
     return n < (double)(ctx->desc.nx + 1) ? (int)n : ctx->desc.nx + 1;
 }
 

@@ -134,7 +134,7 @@ def test_indices_of_several_pieces_are_checked_to_the_last():
         assert not np.any(s.download_fields())
 
 
-@pytest.mark.parametrize('shape,poles,magnetic', [((60, 360, 340), 0, False), ((61, 330, 300), 2, True), ((12, 870, 701), 0, True)],
+@pytest.mark.parametrize('shape,poles,magnetic', [((60, 380, 362), 0, False), ((61, 330, 300), 2, True), ((12, 870, 701), 0, True)],
                          ids=str)
 def test_blocks_of_planes(shape, poles, magnetic):
     """Grids past the last-level cache go through the passes in blocks of planes
