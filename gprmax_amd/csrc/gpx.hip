@@ -761,7 +761,7 @@ struct gpx_ctx {
     int nimg = 0;
     RowModel *row = nullptr;  // the model as the row kernels see it
     RowModel rowh;            // its host copy
-    bool state_given = false; // fields or Phi have been uploaded
+    bool state_given = false; // fields or Phi have been uploaded, or see note_state
     bool row_dirty = true;    // something in it changed
     bool planes_dirty = true; // slabs, sources or receivers changed since the planes' flags went up
     bool hu = false;          // every material has the same H coefficients
@@ -2292,7 +2292,7 @@ struct PlaneShape {
 };
 
 // The axis of one cell, when the 2-D kernel can run the model: what it leaves out
-// is zero and stays so.  No state has been uploaded, sources lie on the
+// is zero and stays so.  No state has been uploaded, sources lie (and lay) on the
 // plane's cells and drive its components, slabs lie across the two long axes
 // and every coefficient is finite.  -1 otherwise.
 static int plane_axis(const gpx_ctx *ctx)
@@ -2499,6 +2499,16 @@ static int check_tls(gpx_ctx *ctx)
     return 0;
 }
 
+static int plane_axis(const gpx_ctx *ctx);
+
+// Called before anything steps a model: once a 2-D model is stepped with what the
+// 2-D kernel leaves out (a source of another component, say), that may stay
+// behind in the state, and later runs take the passes too.
+static void note_state(gpx_ctx *ctx)
+{
+    if (plane_axis(ctx) < 0) ctx->state_given = true;
+}
+
 static int check_ready(gpx_ctx *ctx)
 {
     if (!ctx->have_id || !ctx->have_coeffs)
@@ -2508,6 +2518,7 @@ static int check_ready(gpx_ctx *ctx)
     if (int rc = ensure_tslots(ctx)) return rc;
     if (int rc = ensure_planes(ctx)) return rc;
     if (int rc = ensure_phi(ctx)) return rc;
+    note_state(ctx);
     return check_tls(ctx);
 }
 
@@ -3300,7 +3311,10 @@ static int batch_prepare(gpx_batch *b, int tile, int xchunk, BatchPlan &p)
     std::vector<int> item0(4 * (size_t)(n + G), 0), ritem0((size_t)n + G, 0);
     hipSetDevice(b->device);
     for (gpx_ctx *c : b->ctx)   // sources or receivers may be new since the batch was made
+    {
         if (int rc = ensure_planes(c)) return bfail(b, rc, "gpx_batch: " + c->err);
+        note_state(c);
+    }
     for (int gi = 0; gi < G; ++gi) {
         BatchGroup &g = p.groups[gi];
         if (!tile && group_alone(g)) continue;

@@ -194,3 +194,24 @@ def test_2d_tiles(axis, size, n):
             s.run(9, 3)
             out.append(s.download_fields())
     assert np.array_equal(*out)
+
+
+def test_2d_source_of_another_component_stays_in_the_state():
+    """A 2-D run with a source off the plane's components, then without it: the
+    later run goes on from what the source left, as the passes do."""
+    import ctypes
+    G = plane_model(seed=62, axis=2, size=(40, 33), iterations=40, snapshots=False)
+    out = []
+    for form in (4, 6):
+        with _hip()(G) as s:
+            s.set_step(form)
+            info = np.array([[5, 16, 0, 2, 0, 39], [20, 16, 0, 2, 0, 39]], np.int32)        # along z
+            fac, waves = np.full((2, 2), 3.0, np.float32), np.ones((2, 40), np.float32)
+            ptr = [a.ctypes.data_as(ctypes.c_void_p) for a in (info, fac, waves)]
+            s._check(s.lib.gpx_set_sources(s.ctx, 1, 2, *ptr))
+            s.run(0, 11)
+            s._check(s.lib.gpx_set_sources(s.ctx, 1, 0, None, None, None))
+            s.run(11, 20)
+            out.append(s.download_fields())
+    assert np.abs(out[0][2]).max() > 0 and np.abs(out[0][5]).max() > 0
+    assert np.array_equal(*out)
