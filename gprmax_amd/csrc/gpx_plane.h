@@ -104,7 +104,8 @@ __device__ __forceinline__ float plane_corr(PlaneSlab<FORM, ORDER> &s, float c, 
 {
     const float v = __builtin_fmaf(x, s.rd, x * s.rl);
     float q = __builtin_fmaf(__builtin_fmaf(-v, s.d, x), s.rd, v);
-    if (__builtin_bit_cast(uint32_t, x) * 2u - 1u < ROW_TINY) q = x / s.d;
+    const RowOdd odd = {__builtin_bit_cast(uint32_t, x) * 2u - 1u, q != q};
+    if (odd.any()) q = x / s.d;
     float none = 0.f;
     return row_corr<FORM, ORDER>(s.e, c, q, s.p[0], ORDER == 2 ? s.p[ORDER - 1] : none);
 }

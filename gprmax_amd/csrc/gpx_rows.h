@@ -194,23 +194,29 @@ __device__ __forceinline__ float from_prev(float edge, float v)
 // place, and from there one step with the exact remainder (fma) gives the
 // rounded quotient (Markstein's theorem).  That holds while |x| is zero or at
 // least 2^-100 (d being a cell size, 2^-40 < d < 2^24): no quotient is then
-// subnormal and every remainder is exact.  True when a cell has a smaller x, for
-// which the division itself is needed.  Four operations instead of the
+// subnormal and every remainder is exact; and while the quotient is finite: for an
+// infinite x, or one whose quotient overflows, the remainder is the difference
+// of two infinities and q comes out as NaN.  `odd` collects what a cell had of
+// either, for which the division itself is needed.  Four operations instead of the
 // division's twelve.
-__device__ __forceinline__ uint32_t row_quot(fN x, const RowSlab &S, fN &q)
+struct RowOdd {
+    uint32_t least = ~0u;    // twice the bits of the least x but zero, less one
+    bool nan = false;        // a q is NaN
+    __device__ __forceinline__ bool any() const { return (least < 27u << 24) | nan; }  // exponent field below 27
+};
+__device__ __forceinline__ void row_quot(fN x, const RowSlab &S, fN &q, RowOdd &odd)
 {
-    uint32_t least = ~0u;
 #pragma unroll
     for (int u = 0; u < NC; ++u) {
         const float v = __builtin_fmaf(x[u], S.rd, x[u] * S.rl);
         q[u] = __builtin_fmaf(__builtin_fmaf(-v, S.d, x[u]), S.rd, v);
         const float xu = x[u];  // bit_cast of the element itself reads element 0
         const uint32_t b = __builtin_bit_cast(uint32_t, xu) * 2u - 1u;  // zero wraps to the largest
-        least = b < least ? b : least;
+        odd.least = b < odd.least ? b : odd.least;
     }
-    return least;
+    static_assert(NC == 2, "one comparison for a lane's two cells");
+    odd.nan |= __builtin_isunordered(q[0], q[1]);
 }
-constexpr uint32_t ROW_TINY = 27u << 24;  // of row_quot's result: exponent field below 27
 
 // Makes the compiler forget how a value was computed, so that what is derived
 // from it again later is computed again instead of being kept in registers.
@@ -309,8 +315,10 @@ __device__ __forceinline__ void row_slab(const RowSlab &S, const float *RT, int 
     const int klo = S.lo[2], khi = S.hi[2], at = S.rt + S.sign * ((ALONGK ? kl : c) - S.pend) * NE;
     const int step = ALONGK ? S.sign * NE : 0;
     fN Q1, Q2;
-    const uint32_t t1 = row_quot(D1, S, Q1), t2 = row_quot(D2, S, Q2);
-    if ((t1 < t2 ? t1 : t2) < ROW_TINY) {
+    RowOdd odd;
+    row_quot(D1, S, Q1, odd);
+    row_quot(D2, S, Q2, odd);
+    if (odd.any()) {
 #pragma unroll
         for (int u = 0; u < NC; ++u) {
             Q1[u] = D1[u] / S.d;

@@ -83,7 +83,9 @@ __device__ __forceinline__ InvSlabs inv_slabs(const RowAt *at, int j, int kl, bo
 __device__ __forceinline__ fN inv_quot(fN a, const RowSlab &S)
 {
     fN q;
-    if (row_quot(a, S, q) < ROW_TINY) {
+    RowOdd odd;
+    row_quot(a, S, q, odd);
+    if (odd.any()) {
 #pragma unroll
         for (int u = 0; u < NC; ++u) q[u] = a[u] / S.d;
     }

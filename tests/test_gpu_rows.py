@@ -104,6 +104,55 @@ def test_tiny_values_in_one_cell_of_a_lane(cell, form):
 
 
 @pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
+@pytest.mark.parametrize('value', [np.inf, -np.inf, np.nan, 3e38, -2e36], ids=str)
+def test_quotients_that_overflow(value, form):
+    """Fields with a few infinities, or values whose quotient by the cell size
+    overflows, in either cell of a lane: infinities and NaN are where the
+    division leaves them."""
+    G = rich_model(seed=58, shape=(13, 14, 15), iterations=8, snapshots=False, pml=FACES)
+    _random_state(G, 9)
+    rng = np.random.default_rng(5)
+    for c in COMPS:
+        a = getattr(G, c)
+        a[rng.random(a.shape) < 0.02] = value
+    lib = oracle.load(np.float32)
+    with _hip()(G) as s:
+        s.set_step(form)
+        _push_state(s, G)
+        s.run(0, 1)
+        osolver.step(lib, G, 0, 8)
+        F = s.download_fields()
+        for n, c in enumerate(COMPS):
+            assert np.array_equal(F[n], getattr(G, c), equal_nan=True), c
+        for n, pml in enumerate(G.pmls):
+            for w, name in enumerate(('EPhi1', 'EPhi2', 'HPhi1', 'HPhi2')):
+                assert np.array_equal(s.download_phi(n, w), getattr(pml, name), equal_nan=True), (pml.ID, name)
+        assert np.isinf(F).any() or np.isnan(value)
+
+
+@pytest.mark.parametrize('axis', [0, 1, 2], ids=['TMx', 'TMy', 'TMz'])
+def test_2d_quotients_that_overflow(axis):
+    """The same for the 2-D kernel, from sources in and beside the slabs, against
+    the general passes."""
+    G = plane_model(seed=63, axis=axis, size=(25, 24), iterations=30, snapshots=False)
+    cells = np.zeros((6, 6), np.int32)
+    u, v = (a for a in range(3) if a != axis)
+    cells[:, u], cells[:, v] = (1, 2, 5, 12, 21, 23), (12, 3, 20, 4, 9, 21)
+    cells[:, 3], cells[:, 5] = axis, 29
+    fac, waves = np.ones((6, 2), np.float32), np.zeros((6, 30), np.float32)
+    waves[:, 3] = (3e38, -3e38, 1e36, np.inf, -1e37, 2e38)
+    got = []
+    for form in (4, 2):
+        with _hip()(G) as s:
+            s.set_step(form)
+            s._check(s.lib.gpx_set_sources(s.ctx, 0, 6, cells.ctypes.data, fac.ctypes.data, waves.ctypes.data))
+            s.run(0, 5)
+            got.append(s.download_fields())
+    assert np.isinf(got[0]).any()
+    assert np.array_equal(got[0], got[1], equal_nan=True)
+
+
+@pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
 @pytest.mark.parametrize('shape', [(10, 12, 12), (12, 10, 12), (12, 12, 9), (12, 12, 10)], ids=str)
 def test_slabs_close_to_the_opposite_one(shape, form):
     G = rich_model(seed=53, shape=shape, iterations=8, snapshots=False, pml=MEET)
