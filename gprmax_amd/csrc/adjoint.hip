@@ -547,7 +547,7 @@ struct gpx_inv {
     std::string err;
 };
 
-static std::string g_inv_err;
+static thread_local std::string g_inv_err;   // as g_err in gpx.hip
 
 static int ifail(gpx_inv *v, int code, const std::string &m)
 {

@@ -174,7 +174,7 @@ __global__ void k_edges_scatter(EdgeArgs a)
     }
 }
 
-std::string g_edge_err;
+thread_local std::string g_edge_err;
 
 // ---------------------------------------------------------------- no-allocation variant
 // gpx_edges_static keeps its hash tables in one file-scope device array per

@@ -806,7 +806,8 @@ struct gpx_ctx {
     std::string err;
 };
 
-static std::string g_err;
+// Of the last failure without a context, per thread: models are made on several at a time.
+static thread_local std::string g_err;
 static int update_planeflags(gpx_ctx *ctx);
 static int ensure_planes(gpx_ctx *ctx);
 

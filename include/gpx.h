@@ -20,7 +20,7 @@
  * Every function returns 0 on success, a positive hipError_t for a HIP
  * failure or a negative GPX_E* code for a bad argument or state; the message
  * is available from gpx_last_error(ctx) (or gpx_last_error(NULL) for
- * gpx_create failures).  Nothing throws across the ABI.  A ctx is used from
+ * gpx_create failures, on the thread that failed).  Nothing throws across the ABI.  A ctx is used from
  * one host thread at a time; all its work goes to one HIP stream.
  */
 #ifndef GPX_H

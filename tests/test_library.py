@@ -106,3 +106,39 @@ def test_bscan_groups_follow_the_state_budget():
     assert bscan_groups(grids, group_bytes=80e6) == [[0, 1], [2], [3], [4, 5], [6], [7]]
     assert bscan_groups(grids, group_bytes=1) == [[n] for n in range(8)]
     assert bscan_groups([]) == []
+
+
+def test_errors_without_a_context_belong_to_the_thread():
+    """Models are made on several threads at a time: a failure on one leaves
+    the message of another as it is."""
+    import threading
+    from gprmax_amd.hip import GpxDesc, library
+    from gprmax_amd.inversion import GpxInvDesc, SIGNATURES as INV
+    lib = library()
+    for name, (args, res) in INV.items():
+        getattr(lib, name).argtypes, getattr(lib, name).restype = args, res
+    barrier = threading.Barrier(8)
+    said = [None] * 8
+
+    def work(n):
+        ctx = ctypes.c_void_p()
+        mine = []
+        for _ in range(50):
+            lib.gpx_create(ctypes.byref(GpxDesc(4095, 4095, 63 + n, 5, 2, 0, 0, 0)), ctypes.byref(ctx))
+            if n % 2:
+                lib.gpx_inv_create(None, None)
+            else:
+                lib.gpx_inv_create(ctypes.byref(GpxInvDesc(0, 1, 1, 1, 1, 0, 1e-3, 1e-12)), ctypes.byref(ctx))
+            barrier.wait()   # every thread has failed
+            mine.append((lib.gpx_last_error(None).decode(), lib.gpx_inv_last_error(None).decode()))
+            barrier.wait()
+        said[n] = mine
+    threads = [threading.Thread(target=work, args=(n,)) for n in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for n in range(8):
+        for message, inv in said[n]:
+            assert str(4096 * 4096 * (64 + n)) in message
+            assert ('null argument' if n % 2 else 'bad descriptor') in inv
