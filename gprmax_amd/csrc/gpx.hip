@@ -716,7 +716,7 @@ struct Slab {
     // (1, 2) the slabs one after the other, each [ni][nj][nkp] in ascending
     // cell order (the reference runs the profile axis of the minus slabs
     // backwards), rows padded so that cell k sits at k mod 4 as in the fields.
-    long long base;        // of the slab within a block of one order and term
+    long long base = 0;    // of the slab within a block of one order and term
     int ni, nj, nkp;
     std::vector<float> R[2];  // E, H profile tables RA, RB, RE, RF, each [order][t]
 };
@@ -2172,6 +2172,7 @@ static int pass_fill(const gpx_ctx *ctx) { return 4 * (ctx->cus > 0 ? ctx->cus :
 // changed).
 static int ensure_row(gpx_ctx *ctx)
 {
+    if (ctx->phi_dirty) return fail(ctx, GPX_ESTATE, "slabs without Phi arrays");   // check_ready lays them out
     if (ctx->rare_dirty || !ctx->rare) GPX_TRY(upload_rare(ctx));
     if (!ctx->row_dirty) return 0;
     const gpx_desc &g = ctx->desc;
@@ -3311,11 +3312,8 @@ static int batch_prepare(gpx_batch *b, int tile, int xchunk, BatchPlan &p)
     std::vector<RowModel> models(n);
     std::vector<int> item0(4 * (size_t)(n + G), 0), ritem0((size_t)n + G, 0);
     hipSetDevice(b->device);
-    for (gpx_ctx *c : b->ctx)   // sources or receivers may be new since the batch was made
-    {
-        if (int rc = ensure_planes(c)) return bfail(b, rc, "gpx_batch: " + c->err);
-        note_state(c);
-    }
+    for (gpx_ctx *c : b->ctx)   // slabs, sources, receivers or tables may be new since the batch was made
+        if (int rc = check_ready(c)) return bfail(b, rc, "gpx_batch: " + c->err);
     for (int gi = 0; gi < G; ++gi) {
         BatchGroup &g = p.groups[gi];
         if (!tile && group_alone(g)) continue;

@@ -264,3 +264,43 @@ def test_2d_source_of_another_component_stays_in_the_state():
             out.append(s.download_fields())
     assert np.abs(out[0][2]).max() > 0 and np.abs(out[0][5]).max() > 0
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize('group_bytes', [0, 1], ids=['one-group', 'each-alone'])
+def test_slabs_added_after_the_batch_was_made(group_bytes):
+    """A model of a batch that gets its slabs after the batch was made, between
+    runs of it too, ends as one that is run alone."""
+    from gprmax_amd.hip import HipBatch
+    from gprmax_amd.pml import DIRECTION_CODE
+    models = [rich_model(seed=64 + n, shape=(14, 13, 15), iterations=12, snapshots=False, pml=3) for n in range(2)]
+
+    def add(s, p):
+        R = [np.ascontiguousarray(np.stack([getattr(p, f + q) for q in ('RA', 'RB', 'RE', 'RF')]), np.float32) for f in 'EH']
+        s._check(s.lib.gpx_add_pml(s.ctx, DIRECTION_CODE[p.direction], p.xs, p.xf, p.ys, p.yf, p.zs, p.zf, len(p.CFS),
+                                   float(p.d), R[0].ctypes.data, R[1].ctypes.data, None))
+    slabs = models[1].pmls
+    out = []
+    for batch in (False, True):
+        models[1].pmls = []
+        ss = [_hip()(G) for G in models]
+        models[1].pmls = slabs
+        b = HipBatch(ss) if batch else None
+        if batch:
+            b.set_group_bytes(group_bytes)
+        for first, n, new in ((0, 5, slabs[:2]), (5, 7, slabs[2:])):
+            for p in new:
+                add(ss[1], p)
+            if batch:
+                b.run(first, n)
+            else:
+                for s in ss:
+                    s.run(first, n)
+        out.append([(s.download_fields(), s.download_rx()) for s in ss]
+                   + [[ss[1].download_phi(p, w) for p in range(6) for w in range(4)]])
+        if batch:
+            b.close()
+        for s in ss:
+            s.close()
+    for a, c in zip(*out):
+        for x, y in zip(a, c):
+            assert np.abs(x).max() > 0 and np.array_equal(x, y)

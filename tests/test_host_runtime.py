@@ -1,0 +1,70 @@
+"""Host code of the library against a HIP runtime made of host memory
+(fake_hip.cpp): what it allocates, launches and reports, without a GPU.  Each test
+runs in a process of its own, in which the runtime's functions are loaded before
+the library's."""
+
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+HEAD = '''
+import ctypes, sys
+import numpy as np
+sys.path[:0] = [{root!r}, {here!r}]
+fake = ctypes.CDLL({lib!r}, mode=ctypes.RTLD_GLOBAL)
+fake.fake_most_lds.restype = fake.fake_live_bytes.restype = ctypes.c_size_t
+fake.fake_launches.restype = fake.fake_allocations.restype = ctypes.c_long
+from gpu_models import plane_model, rich_model
+from gprmax_amd.hip import HipBatch, HipSolver
+from gprmax_amd.utilities import GeneralError
+def add_pml(s, p):
+    eR = np.ascontiguousarray(np.stack([p.ERA, p.ERB, p.ERE, p.ERF]), dtype=np.float32)
+    hR = np.ascontiguousarray(np.stack([p.HRA, p.HRB, p.HRE, p.HRF]), dtype=np.float32)
+    from gprmax_amd.pml import DIRECTION_CODE
+    s._check(s.lib.gpx_add_pml(s.ctx, DIRECTION_CODE[p.direction], p.xs, p.xf, p.ys, p.yf, p.zs, p.zf, len(p.CFS),
+                               float(p.d), eR.ctypes.data, hR.ctypes.data, None))
+'''
+
+
+@pytest.fixture(scope='module')
+def runtime(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp('fake_hip') / 'libfake_hip.so')
+    subprocess.run(['g++', '-std=c++17', '-O1', '-w', '-fPIC', '-shared', '-D__HIP_PLATFORM_AMD__', '-I/opt/rocm/include',
+                    os.path.join(HERE, 'fake_hip.cpp'), '-o', lib], check=True)
+    head = HEAD.format(root=os.path.dirname(HERE), here=HERE, lib=lib)
+
+    def run(code):
+        r = subprocess.run([sys.executable, '-c', head + textwrap.dedent(code)], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+    return run
+
+
+def test_slabs_added_to_a_model_of_a_batch_get_their_phi(runtime):
+    """A model that has its slabs when the batch is made, and one that gets them
+    afterwards, hold the same arrays when the batch runs."""
+    runtime('''
+        for shape, pml in (((12, 13, 14), 3), ((12, 13, 14), {'x0': 3, 'zmax': 2})):
+            G = [rich_model(seed=n, shape=shape, pml=pml, snapshots=False) for n in range(2)]
+            for group in (0, 1):
+                held = []
+                for late in (False, True):
+                    slabs = list(G[1].pmls)
+                    G[1].pmls = [] if late else slabs
+                    ss = [HipSolver(g) for g in G]
+                    with HipBatch(ss) as b:
+                        b.set_group_bytes(group)
+                        for p in slabs if late else []:
+                            add_pml(ss[1], p)
+                        b.run(0, 4)
+                        held.append(fake.fake_live_bytes())
+                    for s in ss:
+                        s.close()
+                    G[1].pmls = slabs
+                assert held[0] == held[1], held
+    ''')
