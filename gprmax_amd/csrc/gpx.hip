@@ -716,7 +716,7 @@ struct Slab {
     // (1, 2) the slabs one after the other, each [ni][nj][nkp] in ascending
     // cell order (the reference runs the profile axis of the minus slabs
     // backwards), rows padded so that cell k sits at k mod 4 as in the fields.
-    long long base = 0;    // of the slab within a block of one order and term
+    long long base = -1;   // of the slab within a block of one order and term (-1: not laid out yet)
     int ni, nj, nkp;
     std::vector<float> R[2];  // E, H profile tables RA, RB, RE, RF, each [order][t]
 };
@@ -993,7 +993,23 @@ static int copy_out(gpx_ctx *ctx, void *dst, const void *src, size_t bytes)
 // ---------------------------------------------------------------- Phi arrays
 static size_t phi_bytes(const gpx_ctx *ctx) { return (size_t)ctx->phi_orders * 2 * ctx->np * 4 + 16; }
 
-static int phi_transfer(gpx_ctx *ctx, int slab, int which, float *host, bool up);
+// Several arrays, all of them or none.
+static int dalloc_all(gpx_ctx *ctx, int n, float **p, const size_t *bytes, bool zero)
+{
+    for (int q = 0; q < n; ++q) p[q] = nullptr;
+    for (int q = 0; q < n; ++q) {
+        const hipError_t e = dalloc(ctx, (void **)&p[q], bytes[q], zero);
+        if (e == hipSuccess) continue;
+        for (int f = 0; f <= q; ++f) {
+            if (!p[f]) continue;
+            hipFree(p[f]);
+            ctx->bytes -= bytes[f];
+            p[f] = nullptr;
+        }
+        return fail_hip(ctx, e, "hipMalloc");
+    }
+    return 0;
+}
 
 // Lays the Phi arrays out once slabs are there; slabs added later keep the
 // values of the ones before.
@@ -1001,46 +1017,49 @@ static int ensure_phi(gpx_ctx *ctx)
 {
     if (!ctx->phi_dirty) return 0;
     hipSetDevice(ctx->desc.device);
-    std::vector<std::vector<float>> keep;
-    std::vector<Slab> now = ctx->slabs;
-    if (ctx->phiE[ctx->curE]) {  // values of the slabs that were there, in the old layout
-        long long acc = 0;
-        size_t n = 0;
-        while (n < ctx->slabs.size() && acc < ctx->np) acc += (long long)now[n].ni * now[n].nj * now[n].nkp, ++n;
-        ctx->phi_dirty = false;
-        for (size_t s = 0; s < n; ++s)
-            for (int w = 0; w < 4; ++w) {
-                const Slab &S = ctx->slabs[s];
-                keep.emplace_back((size_t)S.order * S.dims[w][0] * S.dims[w][1] * S.dims[w][2]);
-                if (int rc = phi_transfer(ctx, (int)s, w, keep.back().data(), false)) return rc;
-            }
+    long long np = 0;
+    int orders = 0;
+    std::vector<long long> base;
+    for (const Slab &S : ctx->slabs) {
+        base.push_back(np);
+        np += (long long)S.ni * S.nj * S.nkp;
+        if (S.order > orders) orders = S.order;
+    }
+    const size_t nb = (size_t)orders * 2 * np * 4 + 16, bytes[3] = {nb, nb, nb};
+    const bool two = ctx->Fmem[1] != nullptr;
+    float *p[3];   // E, H and H of the second state
+    if (int rc = dalloc_all(ctx, two ? 3 : 2, p, bytes, true)) return rc;
+    if (ctx->phiE[ctx->curE]) {  // values of the slabs that were there, laid out the same in themselves
+        for (size_t s = 0; s < ctx->slabs.size() && ctx->slabs[s].base >= 0; ++s) {
+            const Slab &S = ctx->slabs[s];
+            for (int q = 0; q < 2 * S.order; ++q)
+                for (int f = 0; f < (two ? 3 : 2); ++f) {
+                    const float *old = (f ? ctx->phiH[ctx->cur] : ctx->phiE[ctx->curE]) + (size_t)q * ctx->np + S.base;
+                    GPX_TRY(hipMemcpyAsync(p[f] + (size_t)q * np + base[s], old, (size_t)S.ni * S.nj * S.nkp * 4,
+                                           hipMemcpyDeviceToDevice, ctx->stream));
+                }
+        }
         GPX_TRY(hipStreamSynchronize(ctx->stream));
         const int next = (ctx->phiH[1] != nullptr) + (ctx->phiE[1] != nullptr);
         ctx->bytes -= phi_bytes(ctx) * (2 + next);
         ctx->next_bytes -= phi_bytes(ctx) * next;
-        for (float **p : {&ctx->phiE[0], &ctx->phiE[1], &ctx->phiH[0], &ctx->phiH[1]}) {
-            if (*p) hipFree(*p);
-            *p = nullptr;
+        for (float **q : {&ctx->phiE[0], &ctx->phiE[1], &ctx->phiH[0], &ctx->phiH[1]}) {
+            if (*q) hipFree(*q);
+            *q = nullptr;
         }
-        ctx->curE = 0;
     }
-    ctx->np = 0;
-    ctx->phi_orders = 0;
-    for (Slab &S : ctx->slabs) {
-        S.base = ctx->np;
-        ctx->np += (long long)S.ni * S.nj * S.nkp;
-        if (S.order > ctx->phi_orders) ctx->phi_orders = S.order;
-    }
-    GPX_TRY(dalloc(ctx, (void **)&ctx->phiE[0], phi_bytes(ctx)));
-    const bool two = ctx->Fmem[1] != nullptr;
-    for (int q = 0; q < (two ? 2 : 1); ++q) {
-        GPX_TRY(dalloc(ctx, (void **)&ctx->phiH[q], phi_bytes(ctx)));
-        if (q) ctx->next_bytes += phi_bytes(ctx);
+    ctx->np = np;
+    ctx->phi_orders = orders;
+    for (size_t s = 0; s < base.size(); ++s) ctx->slabs[s].base = base[s];
+    ctx->curE = 0;
+    ctx->phiE[0] = p[0];
+    ctx->phiH[0] = p[1];
+    if (two) {
+        ctx->phiH[1] = p[2];
+        ctx->next_bytes += nb;
     }
     ctx->phi_dirty = false;
     ctx->row_dirty = true;
-    for (size_t n = 0; n < keep.size(); ++n)
-        if (int rc = phi_transfer(ctx, (int)n / 4, (int)n % 4, keep[n].data(), true)) return rc;
     return 0;
 }
 
@@ -1053,19 +1072,19 @@ static int ensure_next_state(gpx_ctx *ctx)
 {
     if (ctx->Fmem[1]) return 0;
     // Without a second state the current one is Fmem[0].
-    const size_t fb = (size_t)6 * ctx->fstride * 4;
-    float *m = nullptr;
-    GPX_TRY(dalloc(ctx, (void **)&m, fb, false));
-    ctx->Fmem[1] = m;
-    ctx->next_bytes += fb;
-    GPX_TRY(hipMemcpyAsync(m, ctx->Fmem[0], fb, hipMemcpyDeviceToDevice, ctx->stream));
-    if (ctx->phiH[0]) {
-        const size_t b = phi_bytes(ctx);
-        GPX_TRY(dalloc(ctx, (void **)&ctx->phiH[1], b, false));
-        ctx->next_bytes += b;
-        GPX_TRY(hipMemcpyAsync(ctx->phiH[1], ctx->phiH[0], b, hipMemcpyDeviceToDevice, ctx->stream));
+    const size_t bytes[2] = {(size_t)6 * ctx->fstride * 4, phi_bytes(ctx)};
+    const int n = ctx->phiH[0] ? 2 : 1;
+    float *p[2];
+    if (int rc = dalloc_all(ctx, n, p, bytes, false)) return rc;
+    ctx->Fmem[1] = p[0];
+    ctx->next_bytes += bytes[0];
+    if (n == 2) {
+        ctx->phiH[1] = p[1];
+        ctx->next_bytes += bytes[1];
     }
     ctx->row_dirty = true;
+    GPX_TRY(hipMemcpyAsync(p[0], ctx->Fmem[0], bytes[0], hipMemcpyDeviceToDevice, ctx->stream));
+    if (n == 2) GPX_TRY(hipMemcpyAsync(p[1], ctx->phiH[0], bytes[1], hipMemcpyDeviceToDevice, ctx->stream));
     return 0;
 }
 
@@ -1075,10 +1094,12 @@ static int ensure_next_plane(gpx_ctx *ctx)
     if (int rc = ensure_next_state(ctx)) return rc;
     if (!ctx->phiE[0] || ctx->phiE[1]) return 0;
     const size_t b = phi_bytes(ctx);   // the current one is phiE[0]
-    GPX_TRY(dalloc(ctx, (void **)&ctx->phiE[1], b, false));
+    float *p;
+    if (int rc = dalloc_all(ctx, 1, &p, &b, false)) return rc;
+    ctx->phiE[1] = p;
     ctx->next_bytes += b;
-    GPX_TRY(hipMemcpyAsync(ctx->phiE[1], ctx->phiE[0], b, hipMemcpyDeviceToDevice, ctx->stream));
     ctx->row_dirty = true;
+    GPX_TRY(hipMemcpyAsync(p, ctx->phiE[0], b, hipMemcpyDeviceToDevice, ctx->stream));
     return 0;
 }
 

@@ -68,3 +68,46 @@ def test_slabs_added_to_a_model_of_a_batch_get_their_phi(runtime):
                     G[1].pmls = slabs
                 assert held[0] == held[1], held
     ''')
+
+
+def test_an_allocation_that_fails_leaves_the_model_whole(runtime):
+    """Every device allocation of a run fails once, on models that hold one or two
+    states and on ones that get slabs between runs: the run reports it, and the
+    next one holds what a model has whose allocations never failed."""
+    runtime('''
+        def models():
+            yield rich_model(seed=1, shape=(12, 13, 14), pml=3, snapshots=False), 1
+            yield rich_model(seed=2, shape=(12, 13, 14), pml=0, snapshots=False), 4
+            yield plane_model(seed=3, axis=2, snapshots=False), 4
+            yield rich_model(seed=4, shape=(12, 13, 14), poles=2, pml=3, snapshots=False), 4
+        for G, form in models():
+            slabs = list(G.pmls)
+            for first in (slabs, slabs[:1], []):
+                G.pmls = first
+                def go(fail):
+                    with HipSolver(G) as s:
+                        s.set_step(form)
+                        for phase in range(2):
+                            if phase:
+                                for p in slabs[len(first):]:
+                                    add_pml(s, p)
+                            fake.fake_fail_at(fail[phase])
+                            if fail[phase]:
+                                try:
+                                    s.run(0, 3)
+                                    raise SystemExit('no error')
+                                except GeneralError as e:
+                                    assert 'memory' in str(e), e
+                            fake.fake_fail_at(0)
+                            s.run(0, 3)
+                            made[phase] = fake.fake_allocations()
+                        return fake.fake_live_bytes()
+                made = [0, 0]
+                held, counts = go([0, 0]), list(made)
+                assert counts[0] > 0
+                for phase in range(2):
+                    for n in range(1, counts[phase] + 1):
+                        fail = [0, 0]
+                        fail[phase] = n
+                        assert go(fail) == held, (form, len(first), fail)
+    ''')
