@@ -781,10 +781,20 @@ static long long ck_stride(const gpx_inv *v) { return 6 * v->n + 3 * v->P * v->n
 // phi^n, three components each.
 static long long seg_stride(const gpx_inv *v) { return (v->P ? 9 : 6) * v->n; }
 
+// Floats of one field's tables (row_stage).
+static int inv_image(const gpx_inv *v)
+{
+    int nRT = 0;
+    for (const auto &S : v->slabs) nRT += 4 * S.s.t;
+    return row_image(0, nRT, 0);
+}
+static size_t inv_lds(const gpx_inv *v) { return (size_t)inv_image(v) * 4 + 16; }
+
 // Whether the row kernels can run the model: whole lanes, slabs in direction
 // order with the two of an axis at least four cells apart (so that a lane and
 // its neighbours see one of them), a cell size row_quot takes, 32-bit byte
-// offsets into arrays of three components (three per pole) and into a Phi array.
+// offsets into arrays of three components (three per pole) and into a Phi array,
+// and profiles that fit the LDS.
 static bool inv_rows_ok(const gpx_inv *v)
 {
     const gpx_inv_desc &g = v->desc;
@@ -800,7 +810,7 @@ static bool inv_rows_ok(const gpx_inv *v)
         end[ax] = s.hiE[ax] > s.hiH[ax] ? s.hiE[ax] : s.hiH[ax];
         np += ((double)s.hiE[0] - s.loE[0]) * ((double)s.hiE[1] - s.loE[1]) * ((double)s.hiE[2] - s.loE[2] + 8);
     }
-    return np * 8.0 < 2147483647.0;
+    return np * 8.0 < 2147483647.0 && inv_lds(v) <= (size_t)MAX_LDS_BYTES;
 }
 
 // Settles the kernels of a model whose slabs or poles have changed, and lays
@@ -833,9 +843,9 @@ static int prepare(gpx_inv *v)
     m.h[0] = 1.0f;
     m.h[1] = m.h[2] = m.h[3] = (float)((1.0 / g.d) * (g.dt / mu0));
     m.h[4] = (float)(g.dt / mu0);
+    const int nI = inv_image(v);
     int nRT = 0;
     for (const auto &S : v->slabs) nRT += 4 * S.s.t;
-    const int nI = row_image(0, nRT, 0);
     std::vector<float> img((size_t)2 * nI + 4, 0.f);
     v->slabflag.assign(g.nx + 1, 0u);
     long long np = 0;
@@ -902,7 +912,7 @@ static int prepare(gpx_inv *v)
         if (m.pxc == 1 || m.pitems >= 1024) break;
     }
     v->items = m.pitems;
-    v->lds[0] = v->lds[1] = (size_t)nI * 4 + 16;
+    v->lds[0] = v->lds[1] = inv_lds(v);
     if (!v->row) INV_TRY(hipMalloc((void **)&v->row, sizeof(RowModel)));
     INV_TRY(hipMemcpy(v->row, &m, sizeof(m), hipMemcpyHostToDevice));
     v->dirty = false;

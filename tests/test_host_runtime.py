@@ -111,3 +111,25 @@ def test_an_allocation_that_fails_leaves_the_model_whole(runtime):
                         fail[phase] = n
                         assert go(fail) == held, (form, len(first), fail)
     ''')
+
+
+@pytest.mark.parametrize('thick,rows', [(2000, True), (2100, False)])
+def test_inversion_profiles_past_the_lds_take_the_general_kernels(thick, rows, runtime):
+    """Slabs of 2 x 2100 cells have 67 KB of profile entries a field, more than the
+    64 KB a block's tables may take; of 2 x 2000, 64 000 B."""
+    runtime('''
+        from gprmax_amd.inversion import InversionGeometry, InversionGrid
+        init = InversionGeometry.__init__
+        def only_x(self, *a, **k):
+            init(self, *a, **k)
+            self.slabs = [p for p in self.slabs if p.direction[0] == 'x']
+        InversionGeometry.__init__ = only_x
+        shape = ({n}, 8, 8)
+        g = InversionGrid(shape, 2e-3, 2, pml={thick}, er_pml=6.0, K=1)
+        g.set_model(np.full(shape, 6.0), np.zeros(shape))
+        tr = g.forward(({n} // 2, 4, 4), [({n} // 2, 4, 5)], np.ones(2, np.float32))
+        g.backward(tr)
+        assert fake.fake_most_lds() <= 65536, fake.fake_most_lds()
+        assert (fake.fake_launches(b'k_inv_row_h') > 0) is {rows}
+        assert (fake.fake_launches(b'k_inv_h') > 0) is not {rows}
+    '''.format(n=2 * thick + 20, thick=thick, rows=rows))
