@@ -95,7 +95,6 @@ struct InvArgs {
     int nslab;
     InvSlab slab[INV_MAX_SLABS];
     int P;                               // Debye poles (0: none)
-    const uint8_t *rxrow;                // per (i, j) row of points, 1 when a receiver is on it
     int all_gk, all_blocks, all_per_xcd; // all_gk blocks of 128 points along k per (j, i) row
 };
 
@@ -205,10 +204,9 @@ __global__ void k_inv_h(InvArgs a)
     if (!all_point(a, i, j, k) || k > a.nz) return;
     const InvStep &b = a.b;
     const int o = fidx(a, i, j, k), oi = fidx(a, i + 1, j, k), oj = fidx(a, i, j + 1, k), ok = o + 1;
-    if (a.rxrow[i * (a.ny + 1) + j])
-        for (int r = 0; r < b.nrx; ++r)
-            if (b.rxc[3 * r] == i && b.rxc[3 * r + 1] == j && b.rxc[3 * r + 2] == k)
-                b.traces[(long long)r * b.iterations + b.it] = at3(a, b.E, 2, o);
+    const int row = i * (a.ny + 1) + j;
+    for (int r = b.rxfirst[row]; r < b.rxfirst[row + 1]; ++r)
+        if (b.rxat[2 * r] == k) b.traces[(long long)b.rxat[2 * r + 1] * b.iterations + b.it] = at3(a, b.E, 2, o);
     auto E = [&](int c, int at) { return at3(a, b.E, c, at); };
     float h[3] = {at3(a, b.H, 0, o), at3(a, b.H, 1, o), at3(a, b.H, 2, o)};
     if (h_upd(a, 0, i, j, k)) h[0] = 1.0f * h[0] - b.DB * (E(2, oj) - E(2, o)) + b.DB * (E(1, ok) - E(1, o));
@@ -460,10 +458,9 @@ __global__ void k_adj_h(InvArgs a)
             if (a.P) out = out + add;
         }
         out = out + de[c];
-        if (c == 2 && a.rxrow[i * (a.ny + 1) + j])
-            for (int r = 0; r < b.nrx; ++r)
-                if (b.rxc[3 * r] == i && b.rxc[3 * r + 1] == j && b.rxc[3 * r + 2] == k)
-                    out += b.resid[(long long)r * b.iterations + b.it];
+        const int row = i * (a.ny + 1) + j;
+        for (int r = b.rxfirst[row]; c == 2 && r < b.rxfirst[row + 1]; ++r)
+            if (b.rxat[2 * r] == k) out += b.resid[(long long)b.rxat[2 * r + 1] * b.iterations + b.it];
         for (int p = 0; p < a.P && upd; ++p)
             out = out - b.dc[(2 * a.P + p) * a.n + o] * b.T[(c * a.P + p) * a.n + o];
         b.lE[c * a.n + o] = out;
@@ -506,8 +503,7 @@ struct gpx_inv {
     float *T = nullptr;            // T of Ex, Ey, Ez: 3 P n
     float *LT = nullptr;           // its adjoint
     std::vector<float> waves;
-    int *rxc = nullptr;
-    uint8_t *rxrow = nullptr;      // [nx+1][ny+1]: 1 on the rows of points that hold a receiver
+    int *rxtab = nullptr;          // InvStep's rxfirst, then rxat
     float *traces = nullptr, *resid = nullptr;
     int nrx = 0, si = -1, sj = -1, sk = -1;
     float sfac = 0;
@@ -632,8 +628,7 @@ extern "C" int gpx_inv_destroy(gpx_inv *v)
     for (float *p : {v->F, v->L, v->ck, v->seg, v->par, v->grad, v->dense, v->traces, v->resid, v->dc, v->T, v->LT,
                      v->keep, v->img})
         if (p) hipFree(p);
-    ifree(v->rxc);
-    ifree(v->rxrow);
+    ifree(v->rxtab);
     ifree(v->row);
     ifree(v->planeflag);
     free_phi(v);
@@ -936,17 +931,16 @@ static InvArgs inv_args(const gpx_inv *v)
     b.mat = v->par;
     b.dc = v->dc;
     b.grad = v->grad;
-    b.rxc = v->rxc;
+    b.rxfirst = v->rxtab;
+    b.rxat = v->rxtab + (size_t)(g.nx + 1) * (g.ny + 1) + 1;
     b.resid = v->resid;
     b.traces = v->traces;
-    b.nrx = v->nrx;
     b.iterations = g.iterations;
     b.si = v->si; b.sj = v->sj; b.sk = v->sk;
     b.sfac = v->sfac;
     b.nitems = v->items;
     b.per_xcd = (v->items + 7) / 8;
     a.P = v->P;
-    a.rxrow = v->rxrow;
     a.nslab = (int)v->slabs.size();
     for (int s = 0; s < a.nslab; ++s) a.slab[s] = v->slabs[s].s;
     a.all_gk = (g.nz + 1 + 127) / 128;
@@ -1042,24 +1036,28 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
     v->sfac = sfac;
     v->waves.assign(waves, waves + g.iterations);
     if (int rc = prepare(v)) return rc;
-    if (nrx != v->nrx || !v->rxc) {
-        if (v->rxc) hipFree(v->rxc);
-        if (v->traces) hipFree(v->traces);
-        if (v->resid) hipFree(v->resid);
-        v->rxc = nullptr;
-        v->traces = v->resid = nullptr;
+    const size_t rows = (size_t)(g.nx + 1) * (g.ny + 1);
+    if (nrx != v->nrx || !v->rxtab) {
+        ifree(v->rxtab);
+        ifree(v->traces);
+        ifree(v->resid);
         v->nrx = nrx;
-        INV_TRY(hipMalloc((void **)&v->rxc, (size_t)(nrx > 0 ? nrx : 1) * 3 * 4));
+        INV_TRY(hipMalloc((void **)&v->rxtab, (rows + 1 + 2 * (size_t)nrx) * 4));
         INV_TRY(hipMalloc((void **)&v->traces, (size_t)(nrx > 0 ? nrx : 1) * g.iterations * 4));
         INV_TRY(hipMalloc((void **)&v->resid, (size_t)(nrx > 0 ? nrx : 1) * g.iterations * 4));
     }
-    if (nrx) INV_TRY(hipMemcpy(v->rxc, rx, (size_t)nrx * 3 * 4, hipMemcpyHostToDevice));
-    {  // the rows and planes of points that hold a receiver
-        const size_t rows = (size_t)(g.nx + 1) * (g.ny + 1);
-        if (!v->rxrow) INV_TRY(hipMalloc((void **)&v->rxrow, rows));
-        std::vector<uint8_t> flag(rows, 0);
-        for (int r = 0; r < nrx; ++r) flag[(size_t)rx[3 * r] * (g.ny + 1) + rx[3 * r + 1]] = 1;
-        INV_TRY(hipMemcpy(v->rxrow, flag.data(), rows, hipMemcpyHostToDevice));
+    {  // the receivers by rows of points, those of a row in their order, and their planes
+        std::vector<int> tab(rows + 1 + 2 * (size_t)nrx, 0);
+        auto row = [&](int r) { return (size_t)rx[3 * r] * (g.ny + 1) + rx[3 * r + 1]; };
+        for (int r = 0; r < nrx; ++r) ++tab[row(r) + 1];
+        for (size_t q = 0; q < rows; ++q) tab[q + 1] += tab[q];
+        std::vector<int> next(tab.begin(), tab.begin() + rows);
+        for (int r = 0; r < nrx; ++r) {
+            int *at = &tab[rows + 1 + 2 * (size_t)next[row(r)]++];
+            at[0] = rx[3 * r + 2];
+            at[1] = r;
+        }
+        INV_TRY(hipMemcpy(v->rxtab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
         if (v->rows) {
             std::vector<uint32_t> pf(v->slabflag);
             for (int r = 0; r < nrx; ++r) pf[rx[3 * r]] |= PF_RX;

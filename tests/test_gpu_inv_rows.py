@@ -69,3 +69,50 @@ def test_gradient_at_the_edges_of_the_rows(shape, pml, poles, monkeypatch):
     assert abs(L - Lg) <= 1e-4 * Lg
     for ours, ref in ((ger, gerg), (gse, gseg)):
         assert np.linalg.norm(ours - ref) < 1e-4 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize('reverse', [False, True], ids=['rows', 'general'])
+def test_many_receivers(reverse, monkeypatch):
+    """300 receivers, several on a row and at a point, against one at a time: the
+    same traces; a gradient against the float64 reference; and a forward of them
+    takes no longer than three of one."""
+    import time
+    from gprmax_amd.inversion import InversionGrid
+    shape, its = (40, 38, 39), 40
+    rng = np.random.default_rng(62)
+    init = InversionGeometry.__init__
+
+    def reversed_init(self, *a, **k):
+        init(self, *a, **k)
+        self.slabs = self.slabs[::-1]
+    if reverse:
+        monkeypatch.setattr(InversionGeometry, '__init__', reversed_init)
+    grid = InversionGrid(shape, 2e-3, its, pml=4, er_pml=7.0, K=16)
+    monkeypatch.undo()
+    geo = InversionGeometry(shape, 2e-3, its, pml=4, er_pml=7.0, K=16)
+    waves = geo.waveform(freq=4e9)
+    er, se = 4 + 6 * rng.random(shape), 1e-3 + 1.9e-2 * rng.random(shape)
+    src = tuple(n // 2 for n in shape)
+    rx = rng.integers(src[0] - 4, src[0] + 5, (300, 3))
+    rx[:80, :2] = src[:2]
+    rx[250:] = rx[200:250]
+    grid.set_model(er, se)
+    one = [grid.forward(src, rx[n:n + 1], waves)[0] for n in (0, 40, 79, 199, 225, 275, 299)]
+    tr = grid.forward(src, rx, waves)
+    for n, t in zip((0, 40, 79, 199, 225, 275, 299), one):
+        assert np.array_equal(tr[n], t) and np.abs(t).max() > 0
+    ger, gse = grid.backward(tr)
+    _, ger_ref, gse_ref = _autograd(geo, waves, er, se, [src], [tuple(r) for r in rx], [np.zeros((300, its))])
+    m = geo.interior
+    for ours, ref in ((ger, ger_ref), (gse, gse_ref)):
+        assert np.linalg.norm((ours - ref)[m]) < 1e-3 * np.linalg.norm(ref[m])
+
+    def took(n):
+        best = 1e9
+        for _ in range(10):
+            t = time.perf_counter()
+            grid.forward(src, rx[:n], waves)
+            best = min(best, time.perf_counter() - t)
+        return best
+    assert took(300) < 3 * took(1)
+    grid.close()
