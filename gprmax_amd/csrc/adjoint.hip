@@ -467,25 +467,29 @@ __global__ void k_adj_h(InvArgs a)
     }
 }
 
-// Cells [nx][ny][nz] of a dense array to points (0 where a point is no cell),
-// and back.
-__global__ void k_inv_to_points(InvArgs a, const float *cells, float *points)
+// Cells [nx][ny][nz] of `count` dense arrays to points (0 where a point is no
+// cell), and back.
+__global__ void k_inv_to_points(InvArgs a, const float *cells, float *points, int count)
 {
     int i, j, k;
     if (!all_point(a, i, j, k) || k >= a.kp) return;
     const bool cell = i < a.nx && j < a.ny && k < a.nz;
-    points[fidx(a, i, j, k)] = cell ? cells[((long long)i * a.ny + j) * a.nz + k] : 0.f;
+    const long long all = (long long)a.nx * a.ny * a.nz, at = ((long long)i * a.ny + j) * a.nz + k;
+    for (int q = 0; q < count; ++q) points[q * a.n + fidx(a, i, j, k)] = cell ? cells[q * all + at] : 0.f;
 }
-__global__ void k_inv_to_cells(InvArgs a, const float *points, float *cells)
+__global__ void k_inv_to_cells(InvArgs a, const float *points, float *cells, int count)
 {
     int i, j, k;
     if (!all_point(a, i, j, k) || i >= a.nx || j >= a.ny || k >= a.nz) return;
-    cells[((long long)i * a.ny + j) * a.nz + k] = points[fidx(a, i, j, k)];
+    const long long all = (long long)a.nx * a.ny * a.nz, at = ((long long)i * a.ny + j) * a.nz + k;
+    for (int q = 0; q < count; ++q) cells[q * all + at] = points[q * a.n + fidx(a, i, j, k)];
 }
 
 }  // namespace
 
 // ====================================================================== host
+constexpr int INV_DENSE = 3;
+
 struct gpx_inv {
     gpx_inv_desc desc;
     int kp = 0;                    // floats per row of points
@@ -497,7 +501,7 @@ struct gpx_inv {
     float *seg = nullptr;          // segment store: K x seg_stride
     float *par = nullptr;          // CA, CB, IEA: 3 n
     float *grad = nullptr;         // gCA, gCB, gIEA: 3 n
-    float *dense = nullptr;        // ncell: a parameter or gradient as the caller has it
+    float *dense = nullptr;        // INV_DENSE x ncell: parameters or gradients as the caller has them
     int P = 0;                     // Debye poles
     float *dc = nullptr;           // ee, eqt, zt: 3 P n
     float *T = nullptr;            // T of Ex, Ey, Ez: 3 P n
@@ -595,7 +599,7 @@ extern "C" int gpx_inv_create(const gpx_inv_desc *d, gpx_inv **out)
     if (e == hipSuccess) e = hipMalloc((void **)&v->seg, (size_t)d->K * 6 * b);
     if (e == hipSuccess) e = hipMalloc((void **)&v->par, 3 * b);
     if (e == hipSuccess) e = hipMalloc((void **)&v->grad, 3 * b);
-    if (e == hipSuccess) e = hipMalloc((void **)&v->dense, v->ncell * 4);
+    if (e == hipSuccess) e = hipMalloc((void **)&v->dense, INV_DENSE * v->ncell * 4);
     if (e != hipSuccess) {
         gpx_inv_destroy(v);
         return ifail(nullptr, (int)e, std::string("gpx_inv_create: ") + hipGetErrorString(e));
@@ -723,12 +727,15 @@ static dim3 grid_all(const gpx_inv *v)
     return dim3((unsigned)(8 * inv_args(v).all_per_xcd));
 }
 
-// `count` arrays of cells from the host to points (the caller waits).
-static int upload_cells(gpx_inv *v, const float *src, int count, float *dst)
+// `count` arrays of cells from the host to points (the caller waits).  All that
+// `dense` holds go over in one launch.
+static int upload_cells(gpx_inv *v, const float *const *src, int count, float *dst)
 {
-    for (int q = 0; q < count; ++q) {
-        INV_TRY(hipMemcpyAsync(v->dense, src + q * v->ncell, (size_t)v->ncell * 4, hipMemcpyHostToDevice, v->stream));
-        hipLaunchKernelGGL(k_inv_to_points, grid_all(v), dim3(128), 0, v->stream, inv_args(v), v->dense, dst + q * v->n);
+    for (int q = 0; q < count; q += INV_DENSE) {
+        const int m = count - q < INV_DENSE ? count - q : INV_DENSE;
+        for (int p = 0; p < m; ++p)
+            INV_TRY(hipMemcpyAsync(v->dense + p * v->ncell, src[q + p], (size_t)v->ncell * 4, hipMemcpyHostToDevice, v->stream));
+        hipLaunchKernelGGL(k_inv_to_points, grid_all(v), dim3(128), 0, v->stream, inv_args(v), v->dense, dst + q * v->n, m);
         INV_TRY(hipGetLastError());
     }
     return 0;
@@ -739,8 +746,7 @@ extern "C" int gpx_inv_set_model(gpx_inv *v, const float *CA, const float *CB, c
     if (!v || !CA || !CB || !IEA) return ifail(v, GPX_EARG, "gpx_inv_set_model: null argument");
     hipSetDevice(v->desc.device);
     const float *src[3] = {CA, CB, IEA};
-    for (int q = 0; q < 3; ++q)
-        if (int rc = upload_cells(v, src[q], 1, v->par + q * v->n)) return rc;
+    if (int rc = upload_cells(v, src, 3, v->par)) return rc;
     INV_TRY(hipStreamSynchronize(v->stream));
     v->have_model = true;
     v->have_forward = false;
@@ -762,9 +768,9 @@ extern "C" int gpx_inv_set_dispersive(gpx_inv *v, int P, const float *ee, const 
         if (P)
             for (float **p : {&v->dc, &v->T, &v->LT}) INV_TRY(hipMalloc((void **)p, (size_t)3 * P * b));
     }
-    const float *src[3] = {ee, eqt, zt};
-    for (int q = 0; q < 3 && P; ++q)
-        if (int rc = upload_cells(v, src[q], P, v->dc + (size_t)q * P * v->n)) return rc;
+    const float *src[3 * INV_MAX_POLES];
+    for (int q = 0; q < 3 * P; ++q) src[q] = (q < P ? ee : (q < 2 * P ? eqt : zt)) + q % P * v->ncell;
+    if (int rc = upload_cells(v, src, 3 * P, v->dc)) return rc;
     INV_TRY(hipStreamSynchronize(v->stream));
     v->have_forward = false;
     return 0;
@@ -1190,12 +1196,11 @@ extern "C" int gpx_inv_backward(gpx_inv *v, const float *resid, float *gCA, floa
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     float *out[3] = {gCA, gCB, gIEA};
-    for (int q = 0; q < 3; ++q) {
-        hipLaunchKernelGGL(k_inv_to_cells, grid_all(v), dim3(128), 0, v->stream, a, v->grad + q * v->n, v->dense);
-        INV_TRY(hipGetLastError());
-        INV_TRY(hipMemcpyAsync(out[q], v->dense, (size_t)v->ncell * 4, hipMemcpyDeviceToHost, v->stream));
-        INV_TRY(hipStreamSynchronize(v->stream));
-    }
+    hipLaunchKernelGGL(k_inv_to_cells, grid_all(v), dim3(128), 0, v->stream, a, v->grad, v->dense, 3);
+    INV_TRY(hipGetLastError());
+    for (int q = 0; q < 3; ++q)
+        INV_TRY(hipMemcpyAsync(out[q], v->dense + q * v->ncell, (size_t)v->ncell * 4, hipMemcpyDeviceToHost, v->stream));
+    INV_TRY(hipStreamSynchronize(v->stream));
     return 0;
 }
 
