@@ -759,20 +759,27 @@ extern "C" int gpx_inv_set_dispersive(gpx_inv *v, int P, const float *ee, const 
         return ifail(v, GPX_EARG, "gpx_inv_set_dispersive: bad argument (at most 4 poles)");
     hipSetDevice(v->desc.device);
     const size_t b = (size_t)v->n * 4;
-    if (P != v->P) {
-        for (float **p : {&v->dc, &v->T, &v->LT, &v->ck, &v->seg}) ifree(*p);
+    v->have_forward = false;
+    if (P != v->P || !v->seg) {
+        auto drop = [&] {
+            for (float **p : {&v->dc, &v->T, &v->LT, &v->ck, &v->seg}) ifree(*p);
+        };
+        drop();
         v->P = P;
         v->dirty = true;
         // the segment store keeps phi^n of the three E components beside E^n, curl H^{n+1}
-        INV_TRY(hipMalloc((void **)&v->seg, (size_t)v->desc.K * (P ? 9 : 6) * b));
-        if (P)
-            for (float **p : {&v->dc, &v->T, &v->LT}) INV_TRY(hipMalloc((void **)p, (size_t)3 * P * b));
+        hipError_t e = hipMalloc((void **)&v->seg, (size_t)v->desc.K * (P ? 9 : 6) * b);
+        for (float **p : {&v->dc, &v->T, &v->LT})
+            if (e == hipSuccess && P) e = hipMalloc((void **)p, (size_t)3 * P * b);
+        if (e != hipSuccess) {   // none of them: no forward until this has succeeded
+            drop();
+            return ifail(v, (int)e, std::string("gpx_inv_set_dispersive: ") + hipGetErrorString(e));
+        }
     }
     const float *src[3 * INV_MAX_POLES];
     for (int q = 0; q < 3 * P; ++q) src[q] = (q < P ? ee : (q < 2 * P ? eqt : zt)) + q % P * v->ncell;
     if (int rc = upload_cells(v, src, 3 * P, v->dc)) return rc;
     INV_TRY(hipStreamSynchronize(v->stream));
-    v->have_forward = false;
     return 0;
 }
 
@@ -1030,6 +1037,7 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
     if (!v || !waves || nrx < 0 || (nrx > 0 && (!rx || !traces)))
         return ifail(v, GPX_EARG, "gpx_inv_forward: bad argument");
     if (!v->have_model) return ifail(v, GPX_ESTATE, "gpx_inv_forward: no model uploaded");
+    if (!v->seg) return ifail(v, GPX_ESTATE, "gpx_inv_forward: the poles of the last gpx_inv_set_dispersive were not set");
     const gpx_inv_desc &g = v->desc;
     if (si < 1 || si >= g.nx || sj < 1 || sj >= g.ny || sk < 0 || sk >= g.nz)
         return ifail(v, GPX_EARG, "gpx_inv_forward: source edge outside the updated Ez range");
@@ -1038,19 +1046,28 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
             rx[3 * r + 2] > g.nz)
             return ifail(v, GPX_EARG, "gpx_inv_forward: receiver outside the grid");
     hipSetDevice(g.device);
+    v->have_forward = false;
     v->si = si; v->sj = sj; v->sk = sk;
     v->sfac = sfac;
     v->waves.assign(waves, waves + g.iterations);
     if (int rc = prepare(v)) return rc;
     const size_t rows = (size_t)(g.nx + 1) * (g.ny + 1);
     if (nrx != v->nrx || !v->rxtab) {
-        ifree(v->rxtab);
-        ifree(v->traces);
-        ifree(v->resid);
+        auto drop = [&] {
+            ifree(v->rxtab);
+            ifree(v->traces);
+            ifree(v->resid);
+        };
+        drop();
         v->nrx = nrx;
-        INV_TRY(hipMalloc((void **)&v->rxtab, (rows + 1 + 2 * (size_t)nrx) * 4));
-        INV_TRY(hipMalloc((void **)&v->traces, (size_t)(nrx > 0 ? nrx : 1) * g.iterations * 4));
-        INV_TRY(hipMalloc((void **)&v->resid, (size_t)(nrx > 0 ? nrx : 1) * g.iterations * 4));
+        const size_t tb = (size_t)(nrx > 0 ? nrx : 1) * g.iterations * 4;
+        hipError_t e = hipMalloc((void **)&v->rxtab, (rows + 1 + 2 * (size_t)nrx) * 4);
+        if (e == hipSuccess) e = hipMalloc((void **)&v->traces, tb);
+        if (e == hipSuccess) e = hipMalloc((void **)&v->resid, tb);
+        if (e != hipSuccess) {
+            drop();
+            return ifail(v, (int)e, std::string("gpx_inv_forward: ") + hipGetErrorString(e));
+        }
     }
     {  // the receivers by rows of points, those of a row in their order, and their planes
         std::vector<int> tab(rows + 1 + 2 * (size_t)nrx, 0);

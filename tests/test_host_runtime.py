@@ -133,3 +133,53 @@ def test_inversion_profiles_past_the_lds_take_the_general_kernels(thick, rows, r
         assert (fake.fake_launches(b'k_inv_row_h') > 0) is {rows}
         assert (fake.fake_launches(b'k_inv_h') > 0) is not {rows}
     '''.format(n=2 * thick + 20, thick=thick, rows=rows))
+
+
+def test_an_allocation_that_fails_leaves_the_inversion_whole(runtime):
+    """The same for the differentiable solver: poles set, a forward with other
+    receivers, and a backward, which needs a forward that succeeded."""
+    runtime('''
+        from gprmax_amd.inversion import InversionGrid
+        shape, w = (12, 13, 14), np.ones(6, np.float32)
+        rx = [(5, 6, 7), (6, 6, 7)]
+        debye = np.full((2,) + shape, 1.0), np.full((2,) + shape, 1e-10)
+        base = fake.fake_live_bytes()
+        def go(phase, n):
+            g = InversionGrid(shape, 2e-3, 6, pml=3, er_pml=6.0, K=2)
+            g.set_model(np.full(shape, 6.0), np.zeros(shape))
+            g.set_keep(g.keep_bytes_all() / 3)
+            def attempt(k, f):
+                if k == phase and n:
+                    fake.fake_fail_at(n)
+                    try:
+                        f()
+                        raise SystemExit('no error')
+                    except GeneralError as e:
+                        assert 'memory' in str(e) or 'allocate' in str(e), e
+                    fake.fake_fail_at(0)
+                    try:
+                        g.backward(np.zeros((2, 6)))
+                        raise SystemExit('a backward without its forward')
+                    except GeneralError as e:
+                        assert 'gpx_inv_forward first' in str(e), e
+                fake.fake_fail_at(0)
+                f()
+                if k == phase:
+                    made[0] = fake.fake_allocations()
+            attempt(0, lambda: g.forward((6, 6, 6), rx, w))
+            attempt(1, lambda: g.set_debye(*debye))
+            attempt(2, lambda: g.forward((6, 6, 6), rx, w))
+            attempt(3, lambda: g.forward((6, 6, 6), rx[:1], w))
+            g.backward(np.zeros((1, 6)))
+            held = fake.fake_live_bytes()
+            g.close()
+            assert fake.fake_live_bytes() == base
+            return held
+        for phase in range(4):
+            made = [0]
+            held = go(phase, 0)
+            counts = made[0]
+            assert counts > 0
+            for n in range(1, counts + 1):
+                assert go(phase, n) == held, (phase, n)
+    ''')
