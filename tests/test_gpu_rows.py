@@ -245,6 +245,61 @@ def test_2d_tiles(axis, size, n):
     assert np.array_equal(*out)
 
 
+@pytest.mark.parametrize('order', [1, 2])
+def test_states_of_several_pieces(order):
+    """Fields and Phi larger than a piece of their transfers, rows with and without
+    padding: what went up comes down, and one iteration from it is that of
+    whole general passes."""
+    from gprmax_amd.grid import ModelBuilder
+    from gprmax_amd.pml import CFS
+    cfs = [CFS() for _ in range(order)]
+    for nz in (62, 63):
+        b = ModelBuilder(220, 170, nz, 1e-3, 1e-3, 1e-3, 4, pml_cells={'x0': 29, 'zmax': 25}, cfs=cfs)
+        G = b.finalise()
+        rng = np.random.default_rng(65)
+        F = rng.standard_normal((6, 221, 171, nz + 1), dtype=np.float32)
+        out = []
+        for form in (4, 2):
+            with _hip()(G) as s:
+                s.set_step(form)
+                s.run(0, 1)
+                P = {(p, w): rng.standard_normal(s.download_phi(p, w).shape, dtype=np.float32) for p in range(2) for w in range(4)}
+                if out:
+                    P = phi
+                phi = P
+                s.upload_fields(F)
+                for k, v in P.items():
+                    s.upload_phi(*k, v)
+                assert np.array_equal(s.download_fields(), F)
+                for k, v in P.items():
+                    assert np.array_equal(s.download_phi(*k), v), k
+                s.run(1, 2)
+                out.append([s.download_fields()] + [s.download_phi(*k) for k in P])
+        for a, c in zip(*out):
+            assert np.array_equal(a, c)
+
+
+def test_padded_rows_transfer_as_fast_as_whole_ones():
+    """Rows of 182 points, padded on the device, against rows of 184: the fields
+    take at most twice as long either way."""
+    import time
+    from gprmax_amd.grid import ModelBuilder
+    took = []
+    for nz in (181, 183):
+        G = ModelBuilder(90, 90, nz, 1e-3, 1e-3, 1e-3, 4, pml_cells=4).finalise()
+        with _hip()(G) as s:
+            F = s.download_fields()
+            down = up = 1e9
+            for _ in range(8):
+                t = time.perf_counter()
+                s._check(s.lib.gpx_download_fields(s.ctx, F.ctypes.data))
+                u = time.perf_counter()
+                s._check(s.lib.gpx_upload_fields(s.ctx, F.ctypes.data))
+                down, up = min(down, u - t), min(up, time.perf_counter() - u)
+            took.append((down, up))
+    assert took[0][0] < 2 * took[1][0] and took[0][1] < 2 * took[1][1], took
+
+
 def test_2d_source_of_another_component_stays_in_the_state():
     """A 2-D run with a source off the plane's components, then without it: the
     later run goes on from what the source left, as the passes do."""
