@@ -3029,16 +3029,17 @@ extern "C" int gpx_download_dispersive_T(gpx_ctx *ctx, float *out)
         std::vector<float> t((size_t)P * (n ? n : 1) * w);
         if (int rc = copy_out(ctx, slot.data(), ctx->tslot[c], N * 4)) return rc;
         if (int rc = copy_out(ctx, t.data(), ctx->T[c], t.size() * 4)) return rc;
-        for (size_t e = 0; e < N; ++e) {
-            const uint32_t s = slot[e];
-            if (s == 0xffffffffu || e % kp >= nk) continue;  // no poles, or padding
-            const size_t h = e / kp * nk + e % kp;
-            for (int p = 0; p < P; ++p) {
-                float *o = out + (((size_t)c * P + p) * pts + h) * 2;
-                o[0] = t[((size_t)p * n + s) * w];
-                if (w == 2) o[1] = t[((size_t)p * n + s) * w + 1];
+        for (size_t r = 0; r < N / kp; ++r)
+            for (size_t k = 0; k < nk; ++k) {   // (a row's padding left out)
+                const uint32_t s = slot[r * kp + k];
+                if (s == 0xffffffffu) continue;  // no poles
+                const size_t h = r * nk + k;
+                for (int p = 0; p < P; ++p) {
+                    float *o = out + (((size_t)c * P + p) * pts + h) * 2;
+                    o[0] = t[((size_t)p * n + s) * w];
+                    if (w == 2) o[1] = t[((size_t)p * n + s) * w + 1];
+                }
             }
-        }
     }
     return 0;
 }
@@ -3058,18 +3059,19 @@ extern "C" int gpx_upload_dispersive_T(gpx_ctx *ctx, const float *in)
         const size_t n = (size_t)ctx->tn[c];
         std::vector<float> t((size_t)P * (n ? n : 1) * w, 0.0f);
         if (int rc = copy_out(ctx, slot.data(), ctx->tslot[c], N * 4)) return rc;
-        for (size_t e = 0; e < N; ++e) {
-            const uint32_t s = slot[e];
-            if (s == 0xffffffffu || e % kp >= nk) continue;  // no poles, or padding
-            const size_t h = e / kp * nk + e % kp;
-            for (int p = 0; p < P; ++p) {
-                const float *v = in + (((size_t)c * P + p) * pts + h) * 2;
-                if (w == 1 && v[1] != 0.0f)
-                    return fail(ctx, GPX_EARG, "gpx_upload_dispersive_T: imaginary part in a real-pole model");
-                t[((size_t)p * n + s) * w] = v[0];
-                if (w == 2) t[((size_t)p * n + s) * w + 1] = v[1];
+        for (size_t r = 0; r < N / kp; ++r)
+            for (size_t k = 0; k < nk; ++k) {
+                const uint32_t s = slot[r * kp + k];
+                if (s == 0xffffffffu) continue;
+                const size_t h = r * nk + k;
+                for (int p = 0; p < P; ++p) {
+                    const float *v = in + (((size_t)c * P + p) * pts + h) * 2;
+                    if (w == 1 && v[1] != 0.0f)
+                        return fail(ctx, GPX_EARG, "gpx_upload_dispersive_T: imaginary part in a real-pole model");
+                    t[((size_t)p * n + s) * w] = v[0];
+                    if (w == 2) t[((size_t)p * n + s) * w + 1] = v[1];
+                }
             }
-        }
         if (int rc = copy_in(ctx, ctx->T[c], t.data(), t.size() * 4)) return rc;
     }
     return 0;
