@@ -741,7 +741,7 @@ struct SrcSet {
 struct gpx_ctx {
     gpx_desc desc;
     long long ntot = 0;
-    int kp = 0, plane = 0;    // floats per field row (nz + 1 rounded up to 4 where that fits); (ny + 1) kp
+    int kp = 0, plane = 0;    // floats per field row (nz + 1, padded: see gpx_create); (ny + 1) kp
     hipStream_t stream = nullptr;
     // The state: fields and H Phi, twice for the double-buffered step (the
     // second copy is allocated when it first runs), `cur` the current one; E
@@ -898,9 +898,11 @@ extern "C" int gpx_create(const gpx_desc *d, gpx_ctx **out)
         ctx->cus = prop.multiProcessorCount;
     }
     // Rows padded to four floats, so that the row kernels load and store whole
-    // lanes; unpadded where the padding alone would pass the 32-bit offsets
+    // lanes.  Not rows of two floats, a 2-D model's, which are a lane as they are
+    // and would be twice as long (1500x1500 with a pole, us an iteration: 134
+    // padded, 68 not); nor where the padding alone would pass the 32-bit offsets
     // (such a grid takes the general passes).
-    ctx->kp = (d->nz + 1 + 3) / 4 * 4;
+    ctx->kp = d->nz == 1 ? 2 : (d->nz + 1 + 3) / 4 * 4;
     if ((unsigned long long)(d->nx + 1) * (d->ny + 1) * ctx->kp * 4ull > 0xFFFFFFFFull) ctx->kp = d->nz + 1;
     ctx->plane = (d->ny + 1) * ctx->kp;
     ctx->ntot = (long long)(d->nx + 1) * ctx->plane;
@@ -2004,7 +2006,7 @@ static size_t pass_lds(const gpx_ctx *ctx, int field) { return (size_t)image_flo
 static bool rows_ok(const gpx_ctx *ctx)
 {
     const int o = slab_order(ctx);
-    if (ctx->kp % 4 != 0 || o < 0) return false;
+    if (ctx->kp % NC != 0 || o < 0) return false;
     double np = 0;
     int before = -1, end[2][3];
     for (auto &f : end)

@@ -11,7 +11,7 @@
 // round the tables, the plane's fields and the Phi, then the stores.
 //
 // Lanes.  Field rows (fixed i, j; z fastest) are padded to a multiple of four
-// floats, and a lane owns two consecutive cells of a row: half the loads,
+// floats (rows of two, a 2-D model's, are not), and a lane owns two consecutive cells of a row: half the loads,
 // stores and address work of a cell per lane, and registers (under 96 with a
 // slab of order 1) for five waves on a SIMD.  Four cells a lane, with twice the
 // registers, took 367 us where two take 349 (300x300x200) and 38.8 where two

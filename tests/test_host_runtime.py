@@ -183,3 +183,17 @@ def test_an_allocation_that_fails_leaves_the_inversion_whole(runtime):
             for n in range(1, counts + 1):
                 assert go(phase, n) == held, (phase, n)
     ''')
+
+
+@pytest.mark.parametrize('poles', [0, 1])
+def test_rows_of_two_points_are_not_padded(poles, runtime):
+    """A TMz model holds what TMx and TMy models of its size hold, but for its Phi,
+    whose rows of two are padded to eight."""
+    runtime('''
+        held = []
+        for axis in range(3):
+            with HipSolver(plane_model(seed=5, axis=axis, size=(399, 399), iterations=4, poles={poles}, snapshots=False)) as s:
+                s.run(0, 4)
+                held.append(fake.fake_live_bytes())
+        assert max(held) < 1.1 * min(held), held
+    '''.format(poles=poles))
