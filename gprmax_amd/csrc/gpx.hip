@@ -852,6 +852,10 @@ extern "C" const char *gpx_last_error(const gpx_ctx *ctx)
     return ctx ? ctx->err.c_str() : g_err.c_str();
 }
 
+// Whether a whole state of so many points a component passes 32-bit byte offsets
+// (the indices, half as many bytes, then may not).
+static bool past_offsets(double points) { return points * 24.0 >= 4294967295.0; }
+
 extern "C" int gpx_create(const gpx_desc *d, gpx_ctx **out)
 {
     gpx_ctx *ctx = nullptr;
@@ -900,10 +904,13 @@ extern "C" int gpx_create(const gpx_desc *d, gpx_ctx **out)
     // Rows padded to four floats, so that the row kernels load and store whole
     // lanes.  Not rows of two floats, a 2-D model's, which are a lane as they are
     // and would be twice as long (1500x1500 with a pole, us an iteration: 134
-    // padded, 68 not); nor where the padding alone would pass the 32-bit offsets
-    // (such a grid takes the general passes).
+    // padded, 68 not); nor where the row kernels cannot run the model: past the
+    // 32-bit offsets by the padding alone, or with poles by the whole state.
     ctx->kp = d->nz == 1 ? 2 : (d->nz + 1 + 3) / 4 * 4;
-    if ((unsigned long long)(d->nx + 1) * (d->ny + 1) * ctx->kp * 4ull > 0xFFFFFFFFull) ctx->kp = d->nz + 1;
+    {
+        const double points = (double)(d->nx + 1) * (d->ny + 1) * ctx->kp;
+        if (points * 4.0 > 4294967295.0 || (d->maxpoles > 0 && past_offsets(points + 128))) ctx->kp = d->nz + 1;
+    }
     ctx->plane = (d->ny + 1) * ctx->kp;
     ctx->ntot = (long long)(d->nx + 1) * ctx->plane;
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
@@ -1943,12 +1950,14 @@ static hipError_t launch_pass_overlap(gpx_ctx *ctx, int field, int flags, int it
 // ---------------------------------------------------------------- row kernels
 // The row kernels are compiled in step_*.hip, one file per PML form.
 namespace gpx {
-RowKernels row_kernel_plain(int P, bool C, bool hu);
-RowKernels row_kernel_hori1(int P, bool C, bool hu);
-RowKernels row_kernel_hori2(int P, bool C, bool hu);
-RowKernels row_kernel_mri1(int P, bool C, bool hu);
-RowKernels row_kernel_mri2(int P, bool C, bool hu);
+RowKernels row_kernel_plain(int P, bool C, bool hu, bool big);
+RowKernels row_kernel_hori1(int P, bool C, bool hu, bool big);
+RowKernels row_kernel_hori2(int P, bool C, bool hu, bool big);
+RowKernels row_kernel_mri1(int P, bool C, bool hu, bool big);
+RowKernels row_kernel_mri2(int P, bool C, bool hu, bool big);
 }  // namespace gpx
+
+static bool big_state(const gpx_ctx *ctx) { return past_offsets((double)ctx->fstride); }
 
 // PML order shared by every slab, 0 without slabs, -1 when they differ.
 static int slab_order(const gpx_ctx *ctx)
@@ -1964,11 +1973,11 @@ static int slab_order(const gpx_ctx *ctx)
 static RowKernels row_kernels(const gpx_ctx *ctx)
 {
     const int P = ctx->desc.maxpoles;
-    const bool C = ctx->disp_complex != 0, hu = ctx->hu;
+    const bool C = ctx->disp_complex != 0, hu = ctx->hu, big = big_state(ctx);
     const int o = slab_order(ctx);
-    if (o <= 0) return row_kernel_plain(P, C, hu);
-    if (ctx->desc.pml_formulation == 0) return o == 1 ? row_kernel_hori1(P, C, hu) : row_kernel_hori2(P, C, hu);
-    return o == 1 ? row_kernel_mri1(P, C, hu) : row_kernel_mri2(P, C, hu);
+    if (o <= 0) return row_kernel_plain(P, C, hu, big);
+    if (ctx->desc.pml_formulation == 0) return o == 1 ? row_kernel_hori1(P, C, hu, big) : row_kernel_hori2(P, C, hu, big);
+    return o == 1 ? row_kernel_mri1(P, C, hu, big) : row_kernel_mri2(P, C, hu, big);
 }
 
 // Floats of dispersive coefficients and of one field's profile tables.
@@ -2000,13 +2009,13 @@ static size_t pass_lds(const gpx_ctx *ctx, int field) { return (size_t)image_flo
 // Models the row kernels take: rows of whole lanes, one PML order for all
 // slabs, slabs given in the order x0, y0, z0, xmax, ymax, zmax (the kernels
 // apply them so; any may be missing) that do not overlap the one opposite, with
-// cell sizes row_quot takes, 32-bit byte offsets into a whole state, the indices
-// and the Phi arrays, and tables that leave room in LDS.  Others take the
-// general passes.
+// cell sizes row_quot takes, 32-bit byte offsets into the Phi arrays and, with
+// poles, into a whole state, and tables that leave room in LDS.  Others take
+// the general passes.
 static bool rows_ok(const gpx_ctx *ctx)
 {
     const int o = slab_order(ctx);
-    if (ctx->kp % NC != 0 || o < 0) return false;
+    if (ctx->kp % NC != 0 || o < 0 || (big_state(ctx) && ctx->desc.maxpoles > 0)) return false;
     double np = 0;
     int before = -1, end[2][3];
     for (auto &f : end)
@@ -2025,16 +2034,14 @@ static bool rows_ok(const gpx_ctx *ctx)
             e = (a.hi[a.axis] + u - 1) / u;
         }
     }
-    if ((double)ctx->fstride * 24.0 >= 4294967295.0 || (double)ctx->ntot * 12.0 >= 4294967295.0 ||
-        np * 8.0 * (o > 0 ? o : 1) >= 2147483647.0)
-        return false;
+    if (np * 8.0 * (o > 0 ? o : 1) >= 2147483647.0) return false;
     return pass_lds(ctx, 0) <= (size_t)MAX_LDS_BYTES && pass_lds(ctx, 1) <= (size_t)MAX_LDS_BYTES;
 }
 
 // Threads per block of the one-launch step: 0 when it cannot run.
 static int step_block(const gpx_ctx *ctx)
 {
-    if (!rows_ok(ctx) || !ctx->tls.empty()) return 0;
+    if (!rows_ok(ctx) || big_state(ctx) || !ctx->tls.empty()) return 0;
     auto ok = [&](int B) { return B >= 128 && B <= ROW_BLOCK_MAX && step_lds(ctx, B) <= (size_t)MAX_LDS_BYTES; };
     if (ctx->fused == 1 && ctx->tile_cells) return ok(ctx->tile_cells / NC) ? ctx->tile_cells / NC : 0;
     for (int B : {ROW_BLOCK_MAX, 256, 128})
@@ -2253,6 +2260,8 @@ static int ensure_row(gpx_ctx *ctx)
     m.F[1] = ctx->Fmem[1];
     m.cs = (uint32_t)(ctx->fstride * 4);
     m.ci = (uint32_t)(ctx->ntot * 2);
+    m.csl = (size_t)ctx->fstride * 4;
+    m.cil = (size_t)ctx->ntot * 2;
     m.ID = ctx->ID;
     m.img = reinterpret_cast<const float4 *>(ctx->img);
     m.n4E = nE / 4;
@@ -2334,7 +2343,7 @@ static int plane_axis(const gpx_ctx *ctx)
             if (w >= 0) return -1;
             w = q;
         }
-    if (w < 0 || g.maxpoles > 0 || ctx->state_given || !ctx->tls.empty() || !rows_ok(ctx)) return -1;
+    if (w < 0 || g.maxpoles > 0 || ctx->state_given || !ctx->tls.empty() || !rows_ok(ctx) || big_state(ctx)) return -1;
     auto finite = [](const std::vector<float> &x) {
         return std::all_of(x.begin(), x.end(), [](float v) { return isfinite(v); });
     };

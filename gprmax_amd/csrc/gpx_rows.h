@@ -114,6 +114,7 @@ struct RowModel {
     int iterations;
     const StepRare *rare;
     const uint32_t *planeflag;       // [nx + 1], slab bits by direction
+    size_t csl, cil;                 // cs and ci where they pass 32 bits (RowComps)
 };
 
 struct RowArgs {
@@ -148,6 +149,21 @@ __device__ __forceinline__ void bstN(rsrc_t r, uint32_t voff, uint32_t soff, fN 
     if constexpr (N == 4) __builtin_amdgcn_raw_buffer_store_b128(bits<u32x4>(v), r, voff, soff, 0);
     else __builtin_amdgcn_raw_buffer_store_b64(bits<u32x2>(v), r, voff, soff, 0);
 }
+// Components of a state or of the indices.  Offsets are 32-bit, so a state of
+// 4 GiB and more (BIG) has a resource for each component, any other one for all.
+// 620x600x500, us an iteration: 4230 in the general passes, 3060 so.
+template <bool BIG>
+struct RowComps {
+    rsrc_t r[BIG ? 6 : 1];
+    uint32_t cs;
+    __device__ __forceinline__ RowComps(const void *base, uint32_t cs_, size_t csl) : cs(cs_)
+    {
+#pragma unroll
+        for (int c = 0; c < (BIG ? 6 : 1); ++c) r[c] = rsrc(static_cast<const char *>(base) + (size_t)c * csl);
+    }
+    __device__ __forceinline__ rsrc_t at(int c) const { return r[BIG ? c : 0]; }
+    __device__ __forceinline__ uint32_t off(int c, uint32_t so) const { return BIG ? so : so + (uint32_t)c * cs; }
+};
 // Flags of plane i, as a scalar load: no kernel writes them, which the compiler
 // cannot see behind the model's pointer; a vector load in its place would make
 // every plane wait for all its loads before it knew its slabs.
@@ -1088,7 +1104,7 @@ __device__ __forceinline__ RowLane row_lane(const RowModel &a, int item, int p0,
 // The first plane's loads go out before the tables are staged, and the Phi
 // loads with them: on small grids a pass is little more than its chain of
 // dependent memory accesses.
-template <int FORM, int ORDER, bool HU>
+template <int FORM, int ORDER, bool HU, bool BIG = false>
 __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_row_h(const RowModel *__restrict__ models, RowArgs b)
 {
     extern __shared__ float4 lds4[];
@@ -1101,13 +1117,14 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_row_h
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t toj = j < a.ny ? to + 4u * (uint32_t)a.kp : to;
     const uint32_t ti = to >> 1;
-    const rsrc_t rF = rsrc(a.F[b.flip]), rI = rsrc(a.ID), rP = rsrc(a.phiH[b.flip]);
-    const uint32_t P4 = (uint32_t)a.plane * 4u, Pi = (uint32_t)a.plane * 2u, cs = a.cs, ci = a.ci;
+    const RowComps<BIG> F(a.F[b.flip], a.cs, a.csl), I(a.ID, a.ci, a.cil);
+    const rsrc_t rP = rsrc(a.phiH[b.flip]);
+    const uint32_t P4 = (uint32_t)a.plane * 4u, Pi = (uint32_t)a.plane * 2u;
     const uint32_t np4 = __builtin_amdgcn_readfirstlane(a.np4);
     const bool patch = q.live && lane == 63 && kl + NC <= a.nz;
     RowSlabs L;
     if (ORDER > 0) L = row_slabs(a.atH, j, kl, q.live);
-    fN ey = bldN(rF, to, (uint32_t)q.xa * P4 + cs), ez = bldN(rF, to, (uint32_t)q.xa * P4 + 2 * cs);
+    fN ey = bldN(F.at(1), to, F.off(1, (uint32_t)q.xa * P4)), ez = bldN(F.at(2), to, F.off(2, (uint32_t)q.xa * P4));
     fN ex, hx, hy, hz, ezj, exj, ey1, ez1;
     float ykn = 0.f, xkn = 0.f;
     idN m3 = 0u, m4 = 0u, m5 = 0u;
@@ -1116,22 +1133,22 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_row_h
     auto load = [&](int i) {
         pf = plane_flags(a, i);
         const uint32_t so = (uint32_t)i * P4, sn = i < a.nx ? so + P4 : so, si = (uint32_t)i * Pi;
-        ex = bldN(rF, to, so);
-        hx = bldN(rF, to, so + 3 * cs);
-        hy = bldN(rF, to, so + 4 * cs);
-        hz = bldN(rF, to, so + 5 * cs);
-        ezj = bldN(rF, toj, so + 2 * cs);
-        exj = bldN(rF, toj, so);
-        ey1 = bldN(rF, to, sn + cs);
-        ez1 = bldN(rF, to, sn + 2 * cs);
+        ex = bldN(F.at(0), to, F.off(0, so));
+        hx = bldN(F.at(3), to, F.off(3, so));
+        hy = bldN(F.at(4), to, F.off(4, so));
+        hz = bldN(F.at(5), to, F.off(5, so));
+        ezj = bldN(F.at(2), toj, F.off(2, so));
+        exj = bldN(F.at(0), toj, F.off(0, so));
+        ey1 = bldN(F.at(1), to, F.off(1, sn));
+        ez1 = bldN(F.at(2), to, F.off(2, sn));
         if (patch) {
-            ykn = bld(rF, to + 4u * NC, so + cs);
-            xkn = bld(rF, to + 4u * NC, so);
+            ykn = bld(F.at(1), to + 4u * NC, F.off(1, so));
+            xkn = bld(F.at(0), to + 4u * NC, F.off(0, so));
         }
         if (!HU) {
-            m3 = bld_ids(rI, ti, si + 3 * ci);
-            m4 = bld_ids(rI, ti, si + 4 * ci);
-            m5 = bld_ids(rI, ti, si + 5 * ci);
+            m3 = bld_ids(I.at(3), ti, I.off(3, si));
+            m4 = bld_ids(I.at(4), ti, I.off(4, si));
+            m5 = bld_ids(I.at(5), ti, I.off(5, si));
         }
         if (ORDER > 0) {
             m = L.m & (pf >> PF_SLAB_H);
@@ -1149,9 +1166,9 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_row_h
                                hz);
         if (ORDER > 0) row_phis_store(ph, m, rP, np4);
         if (q.live) {
-            bstN(rF, to, so + 3 * cs, hx);
-            bstN(rF, to, so + 4 * cs, hy);
-            bstN(rF, to, so + 5 * cs, hz);
+            bstN(F.at(3), to, F.off(3, so), hx);
+            bstN(F.at(4), to, F.off(4, so), hy);
+            bstN(F.at(5), to, F.off(5, so), hz);
         }
         if (++i == q.xb) break;
         ey = ey1;
@@ -1161,7 +1178,7 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_row_h
 }
 
 // E pass, in place: every lane reads H and its own E and writes its own E.
-template <int P, bool CPLX, int FORM, int ORDER>
+template <int P, bool CPLX, int FORM, int ORDER, bool BIG = false>
 __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(CPLX ? 2 : P, ORDER)
 k_row_e(const RowModel *__restrict__ models, RowArgs b)
 {
@@ -1175,8 +1192,9 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
     const uint32_t to = (uint32_t)(j * a.kp + kl) * 4u;
     const uint32_t tob = j > 0 ? to - 4u * (uint32_t)a.kp : to;
     const uint32_t ti = to >> 1;
-    const rsrc_t rF = rsrc(a.F[b.flip]), rI = rsrc(a.ID), rP = rsrc(a.phiE[b.flipE]);
-    const uint32_t P4 = (uint32_t)a.plane * 4u, Pi = (uint32_t)a.plane * 2u, cs = a.cs, ci = a.ci;
+    const RowComps<BIG> F(a.F[b.flip], a.cs, a.csl), I(a.ID, a.ci, a.cil);
+    const rsrc_t rP = rsrc(a.phiE[b.flipE]);
+    const uint32_t P4 = (uint32_t)a.plane * 4u, Pi = (uint32_t)a.plane * 2u;
     const uint32_t np4 = __builtin_amdgcn_readfirstlane(a.np4);
     const bool patch = q.live && lane == 0 && kl > 0;
     int grp = 0;    // the wave's place in the plane, in groups of 64 lanes; past the plane's end any
@@ -1187,7 +1205,7 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
     RowSlabs L;
     if (ORDER > 0) L = row_slabs(a.atE, j, kl, q.live);
     const uint32_t sm = (uint32_t)(q.xa > 0 ? q.xa - 1 : 0) * P4;
-    fN hym = bldN(rF, to, sm + 4 * cs), hzm = bldN(rF, to, sm + 5 * cs);
+    fN hym = bldN(F.at(4), to, F.off(4, sm)), hzm = bldN(F.at(5), to, F.off(5, sm));
     fN ex, ey, ez, hx, hy, hz, hxj, hzj;
     float hxl = 0.f, hyl = 0.f;
     idN m0, m1, m2;
@@ -1199,21 +1217,21 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
         const uint32_t so = (uint32_t)i * P4, si = (uint32_t)i * Pi;
         u32x16 masks = 0u;
         if (P > 0) masks = row_masks(a.T, i, grp);
-        hx = bldN(rF, to, so + 3 * cs);
-        hy = bldN(rF, to, so + 4 * cs);
-        hz = bldN(rF, to, so + 5 * cs);
-        ex = bldN(rF, to, so);
-        ey = bldN(rF, to, so + cs);
-        ez = bldN(rF, to, so + 2 * cs);
-        hxj = bldN(rF, tob, so + 3 * cs);
-        hzj = bldN(rF, tob, so + 5 * cs);
+        hx = bldN(F.at(3), to, F.off(3, so));
+        hy = bldN(F.at(4), to, F.off(4, so));
+        hz = bldN(F.at(5), to, F.off(5, so));
+        ex = bldN(F.at(0), to, F.off(0, so));
+        ey = bldN(F.at(1), to, F.off(1, so));
+        ez = bldN(F.at(2), to, F.off(2, so));
+        hxj = bldN(F.at(3), tob, F.off(3, so));
+        hzj = bldN(F.at(5), tob, F.off(5, so));
         if (patch) {
-            hxl = bld(rF, to - 4u, so + 3 * cs);
-            hyl = bld(rF, to - 4u, so + 4 * cs);
+            hxl = bld(F.at(3), to - 4u, F.off(3, so));
+            hyl = bld(F.at(4), to - 4u, F.off(4, so));
         }
-        m0 = bld_ids(rI, ti, si);
-        m1 = bld_ids(rI, ti, si + ci);
-        m2 = bld_ids(rI, ti, si + 2 * ci);
+        m0 = bld_ids(I.at(0), ti, I.off(0, si));
+        m1 = bld_ids(I.at(1), ti, I.off(1, si));
+        m2 = bld_ids(I.at(2), ti, I.off(2, si));
         if (ORDER > 0) {
             m = L.m & (pf >> PF_SLAB_E);
             row_phis(ph, L, m, (pf >> PF_SLAB_E) & 1u, rP, np4, i, j, kl);
@@ -1235,9 +1253,9 @@ k_row_e(const RowModel *__restrict__ models, RowArgs b)
             row_e<P, CPLX, FORM, ORDER>(a, S, pf, m, ph, i, j, kl, it, hx, hy, hz, hym, hzm, hxj, hzj, hxk, hyk, m0, m1, m2, tx,
                                         ty, tz, ex, ey, ez);
             if (ORDER > 0) row_phis_store(ph, m, rP, np4);
-            bstN(rF, to, so, ex);
-            bstN(rF, to, so + cs, ey);
-            bstN(rF, to, so + 2 * cs, ez);
+            bstN(F.at(0), to, F.off(0, so), ex);
+            bstN(F.at(1), to, F.off(1, so), ey);
+            bstN(F.at(2), to, F.off(2, so), ez);
         }
         if (++i == q.xb) break;
         hym = hy;
@@ -1256,19 +1274,23 @@ typedef void (*row_kernel)(const RowModel *, RowArgs);
 typedef void (*plane_kernel)(const RowModel *, PlaneArgs);
 
 // The kernels of one model: the whole step, the H pass, the E pass, several
-// iterations of a 2-D model (without poles).
+// iterations of a 2-D model (without poles).  big: a state of 4 GiB and more,
+// which has the passes only, and those without poles.
 struct RowKernels {
     row_kernel step, h, e;
     plane_kernel plane;
 };
 
 template <int FORM, int ORDER>
-RowKernels row_kernel_table(int P, bool C, bool hu)
+RowKernels row_kernel_table(int P, bool C, bool hu, bool big)
 {
 #define GPX_RK(PP, CC)                                                                                       \
     RowKernels{hu ? k_row_step<PP, CC, FORM, ORDER, true> : k_row_step<PP, CC, FORM, ORDER, false>,          \
                hu ? k_row_h<FORM, ORDER, true> : k_row_h<FORM, ORDER, false>, k_row_e<PP, CC, FORM, ORDER>, \
                PP == 0 ? k_plane<FORM, ORDER> : nullptr}
+    if (big)
+        return RowKernels{nullptr, hu ? k_row_h<FORM, ORDER, true, true> : k_row_h<FORM, ORDER, false, true>,
+                          k_row_e<0, false, FORM, ORDER, true>, nullptr};
     switch (P) {
     case 0: return GPX_RK(0, false);
     case 1: return C ? GPX_RK(1, true) : GPX_RK(1, false);

@@ -3,8 +3,8 @@
 #include "gpx_rows.h"
 
 namespace gpx {
-RowKernels row_kernel_hori2(int P, bool C, bool hu)
+RowKernels row_kernel_hori2(int P, bool C, bool hu, bool big)
 {
-    return row_kernel_table<0, 2>(P, C, hu);
+    return row_kernel_table<0, 2>(P, C, hu, big);
 }
 }  // namespace gpx

@@ -3,9 +3,9 @@
 #include "gpx_rows.h"
 
 namespace gpx {
-RowKernels row_kernel_plain(int P, bool C, bool hu)
+RowKernels row_kernel_plain(int P, bool C, bool hu, bool big)
 {
-    return row_kernel_table<0, 0>(P, C, hu);
+    return row_kernel_table<0, 0>(P, C, hu, big);
 }
 
 }  // namespace gpx

@@ -210,6 +210,60 @@ def test_blocks_of_planes(shape, poles, magnetic):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), n
 
 
+@pytest.mark.parametrize('order,formulation,uniform', [(0, 'HORIPML', True), (1, 'HORIPML', True), (2, 'HORIPML', False),
+                                                       (1, 'MRIPML', False), (2, 'MRIPML', True)])
+def test_states_past_4_gib(order, formulation, uniform):
+    """180 million points, whose state 32-bit offsets do not reach across: sources,
+    receivers and slabs at the far end of every component, as whole general
+    passes give it, bit for bit."""
+    from types import SimpleNamespace
+    shape = (700, 640, 401)
+    n = tuple(v + 1 for v in shape)
+    points = n[0] * n[1] * n[2]
+    assert points * 24 > 2 ** 32
+    G = rich_model(seed=66, shape=(24, 23, 22), iterations=40, order=max(order, 1), formulation=formulation,
+                   pml={'xmax': 4, 'ymax': 3, 'zmax': 4} if order else 0, snapshots=False)
+    if not uniform:
+        randomise_tables(G, 67, scaled=True)
+    nmat = len(G.updatecoeffsE)
+    pattern = np.random.default_rng(68).integers(0, nmat, 999983, dtype=np.uint32)
+    move = [a - b for a, b in zip(shape, (24, 23, 22))]
+    slabs = []
+    for p in G.pmls:    # the faces at the far end, as thick as they were
+        q = SimpleNamespace(**{k: getattr(p, k) for k in ('direction', 'd', 'CFS', 'ERA', 'ERB', 'ERE', 'ERF', 'HRA', 'HRB', 'HRE', 'HRF')})
+        a = 'xyz'.index(p.direction[0])
+        for x, name in enumerate('xyz'):
+            lo, hi = getattr(p, name + 's'), getattr(p, name + 'f')
+            setattr(q, name + 's', lo + move[x] if x == a else 0)
+            setattr(q, name + 'f', hi + move[x] if x == a else shape[x])
+        slabs.append(q)
+    big = SimpleNamespace(**{k: getattr(G, k) for k in ('iterations', 'updatecoeffsE', 'updatecoeffsH', 'pmlformulation', 'dx', 'dy',
+                                                        'dz', 'dt')},
+                          nx=shape[0], ny=shape[1], nz=shape[2], floattype=np.float32, maxpoles=0, pmls=slabs,
+                          ID=np.resize(pattern, (6,) + n), hertziandipoles=[], magneticdipoles=[], voltagesources=[],
+                          transmissionlines=[], snapshots=[],
+                          rxs=[SimpleNamespace(xcoord=r.xcoord + move[0], ycoord=r.ycoord + move[1], zcoord=r.zcoord + move[2])
+                               for r in G.rxs])
+    F = np.empty((6,) + n, np.float32)
+    got = []
+    for form in (4, 2):
+        with _hip()(big) as s:
+            s.set_step(form)
+            for kind, pol in ((0, 2), (1, 1), (2, 0)):
+                at = np.array([[700 - 9, 640 - 8, 401 - 9, pol, 0, 39], [12, 11, 10, pol, 0, 39]], np.int32)
+                fac, waves = np.full((2, 2), 2.0, np.float32), np.random.default_rng(69).random((2, 40), dtype=np.float32)
+                s._check(s.lib.gpx_set_sources(s.ctx, kind, 2, at.ctypes.data, fac.ctypes.data, waves.ctypes.data))
+            s.run(0, 27)
+            s._check(s.lib.gpx_download_fields(s.ctx, F.ctypes.data))
+            got.append([F[:, -60:, -60:, -60:].copy(), F[:, :60, :60, :60].copy(), s.download_rx()])
+            if form == 4:
+                F[:, -60:, -60:, -60:] = 0
+                F[:, :60, :60, :60] = 0
+                assert not F.any()
+    for a, b in zip(*got):
+        assert np.abs(a).max() > 0 and np.array_equal(a, b)
+
+
 @pytest.mark.parametrize('n', [1, 7, 31], ids=['n1', 'n7', 'n31'])
 @pytest.mark.parametrize('size', [(14, 17), (25, 24), (57, 90), (300, 211)], ids=str)
 @pytest.mark.parametrize('axis', [0, 1, 2], ids=['TMx', 'TMy', 'TMz'])

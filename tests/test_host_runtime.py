@@ -197,3 +197,28 @@ def test_rows_of_two_points_are_not_padded(poles, runtime):
                 held.append(fake.fake_live_bytes())
         assert max(held) < 1.1 * min(held), held
     '''.format(poles=poles))
+
+
+@pytest.mark.parametrize('shape,poles,rows', [((620, 600, 500), 0, True), ((6000, 6000, 4), 1, False), ((620, 600, 440), 1, True)],
+                         ids=str)
+def test_states_past_4_gib_take_the_row_passes(shape, poles, rows, runtime):
+    """187 million points without poles, 180 million with (their rows of five are
+    then not padded to eight); 164 million are within 32-bit offsets."""
+    runtime('''
+        from types import SimpleNamespace
+        shape, poles = {shape}, {poles}
+        n = tuple(v + 1 for v in shape)
+        table = np.ones((2, 5), np.float32)
+        G = SimpleNamespace(nx=shape[0], ny=shape[1], nz=shape[2], iterations=30, floattype=np.float32, maxpoles=poles,
+                            ID=np.zeros((6,) + n, np.uint32), updatecoeffsE=table, updatecoeffsH=table,
+                            updatecoeffsdispersive=np.zeros((2, 3 * poles), np.complex64), pmlformulation='HORIPML', pmls=[],
+                            hertziandipoles=[], magneticdipoles=[], voltagesources=[], transmissionlines=[], snapshots=[], rxs=[])
+        with HipSolver(G) as s:
+            s.set_step(6)
+            s.run(0, 30)
+            h, general = fake.fake_launches(b'k_row_h'), fake.fake_launches(b'k_h_pass')
+            assert (h > 0, general > 0) == ({rows}, not {rows}), (h, general)
+            points = float(np.prod(n))
+            if poles and not {rows}:
+                assert s.memory_bytes() < 50 * points, s.memory_bytes() / points
+    '''.format(shape=shape, poles=poles, rows=rows))
