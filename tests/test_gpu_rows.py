@@ -71,6 +71,47 @@ def test_auxiliary_values_by_groups(kind, poles, shape, block):
         _assert_state_equal(s, G, 'block {}'.format(block))
 
 
+@pytest.mark.parametrize('tile', [256, 512, 1024])
+@pytest.mark.parametrize('xchunk', [0, 1, 3])
+@pytest.mark.parametrize('pml', [0, FACES], ids=['open', 'slabs'])
+def test_dipoles_on_recomputed_cells(pml, xchunk, tile):
+    """The one-launch step computes H of a tile's halo again: the row below it, the
+    lane before it where rows are split, the plane before each chunk.  Magnetic
+    dipoles along whole lines of every axis, which cross all of these, are in the
+    copies as in the owners' values."""
+    from gprmax_amd.grid import ModelBuilder
+    shape = (11, 29, 141)
+
+    def model():
+        bld = ModelBuilder(*shape, 1e-3, 1e-3, 1e-3, 9, pml_cells=pml)
+        soil = bld.add_material(4.0, 0.005, 1, 0, 'soil')
+        bld.box(0, shape[0], 0, shape[1], 0, shape[2] // 2, soil)
+        bld.add_waveform('ricker', 1, 20e9, 'w')
+        lo, hi = (5, 5, 5), tuple(n - 5 for n in shape)
+        for pol, a in zip('xyzxyz', (0, 1, 2, 1, 2, 0)):
+            for c in range(lo[a], hi[a]):
+                at = [lo[0] + 1, lo[1] + 3, lo[2] + 40]
+                at[a] = c
+                bld.add_magnetic_dipole(pol, tuple(at), 'w')
+        bld.add_hertzian_dipole('z', tuple(n // 2 for n in shape), 'w')
+        for k in (6, 61, 63, 64, 65, 127, 129):
+            bld.add_rx((6, 8, k))
+        return bld.finalise()
+    G, Gc = model(), model()
+    with _hip()(G) as s:
+        s.set_step(1, tile)
+        s.set_launch(xchunk, 0)
+        assert s.step_kind() == tile
+        s.run(0, G.iterations)
+        F, rxb = s.download_fields(), s.download_rx()
+    osolver.solve_cpu(1, 1, Gc, nthreads=8)
+    for n, c in enumerate(COMPS):
+        assert np.abs(F[n]).max() > 0 and np.array_equal(F[n], getattr(Gc, c)), c
+    for r, rx in enumerate(Gc.rxs):
+        for c, name in enumerate(COMPS):
+            assert np.array_equal(rxb[c, :, r], rx.outputs[name]), (r, name)
+
+
 @pytest.mark.parametrize('form', [0, 1], ids=['passes', 'one-launch'])
 @pytest.mark.parametrize('magnetic', [False, True])
 def test_values_of_every_magnitude(magnetic, form):
