@@ -507,7 +507,9 @@ struct gpx_inv {
     float *T = nullptr;            // T of Ex, Ey, Ez: 3 P n
     float *LT = nullptr;           // its adjoint
     std::vector<float> waves;
-    int *rxtab = nullptr;          // InvStep's rxfirst, then rxat
+    int *rxtab = nullptr;          // InvStep's rxat, then rxfirst
+    size_t nrxseg = 0;             // segments of rxfirst
+    bool rowrx = false;            // the device's RowModel points to them
     float *traces = nullptr, *resid = nullptr;
     int nrx = 0, si = -1, sj = -1, sk = -1;
     float sfac = 0;
@@ -532,6 +534,7 @@ struct gpx_inv {
     uint32_t *planeflag = nullptr; // [nx + 1]
     std::vector<uint32_t> slabflag;
     int items = 0;
+    int pseg = 0;                  // segments of a plane
     size_t lds[2] = {0, 0};        // of the E and the H passes
     long long np = 0;
     float *phi[2] = {nullptr, nullptr}, *mu[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [E, H], [copy]
@@ -920,9 +923,11 @@ static int prepare(gpx_inv *v)
         if (m.pxc == 1 || m.pitems >= 1024) break;
     }
     v->items = m.pitems;
+    v->pseg = m.pseg;
     v->lds[0] = v->lds[1] = inv_lds(v);
     if (!v->row) INV_TRY(hipMalloc((void **)&v->row, sizeof(RowModel)));
     INV_TRY(hipMemcpy(v->row, &m, sizeof(m), hipMemcpyHostToDevice));
+    v->rowrx = false;
     v->dirty = false;
     return 0;
 }
@@ -944,8 +949,8 @@ static InvArgs inv_args(const gpx_inv *v)
     b.mat = v->par;
     b.dc = v->dc;
     b.grad = v->grad;
-    b.rxfirst = v->rxtab;
-    b.rxat = v->rxtab + (size_t)(g.nx + 1) * (g.ny + 1) + 1;
+    b.rxat = v->rxtab;
+    b.rxfirst = v->rxtab + 2 * (size_t)v->nrx;
     b.resid = v->resid;
     b.traces = v->traces;
     b.iterations = g.iterations;
@@ -1051,17 +1056,19 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
     v->sfac = sfac;
     v->waves.assign(waves, waves + g.iterations);
     if (int rc = prepare(v)) return rc;
-    const size_t rows = (size_t)(g.nx + 1) * (g.ny + 1);
-    if (nrx != v->nrx || !v->rxtab) {
+    const size_t groups = (size_t)(g.nx + 1) * (v->rows ? v->pseg : g.ny + 1);
+    if (nrx != v->nrx || groups != v->nrxseg || !v->rxtab) {
         auto drop = [&] {
             ifree(v->rxtab);
             ifree(v->traces);
             ifree(v->resid);
+            v->rowrx = false;
         };
         drop();
         v->nrx = nrx;
+        v->nrxseg = groups;
         const size_t tb = (size_t)(nrx > 0 ? nrx : 1) * g.iterations * 4;
-        hipError_t e = hipMalloc((void **)&v->rxtab, (rows + 1 + 2 * (size_t)nrx) * 4);
+        hipError_t e = hipMalloc((void **)&v->rxtab, (2 * (size_t)nrx + groups + 1) * 4);
         if (e == hipSuccess) e = hipMalloc((void **)&v->traces, tb);
         if (e == hipSuccess) e = hipMalloc((void **)&v->resid, tb);
         if (e != hipSuccess) {
@@ -1069,18 +1076,30 @@ extern "C" int gpx_inv_forward(gpx_inv *v, int si, int sj, int sk, float sfac, c
             return ifail(v, (int)e, std::string("gpx_inv_forward: ") + hipGetErrorString(e));
         }
     }
-    {  // the receivers by rows of points, those of a row in their order, and their planes
-        std::vector<int> tab(rows + 1 + 2 * (size_t)nrx, 0);
-        auto row = [&](int r) { return (size_t)rx[3 * r] * (g.ny + 1) + rx[3 * r + 1]; };
-        for (int r = 0; r < nrx; ++r) ++tab[row(r) + 1];
-        for (size_t q = 0; q < rows; ++q) tab[q + 1] += tab[q];
-        std::vector<int> next(tab.begin(), tab.begin() + rows);
+    {  // the receivers by segments, those of one in their order, and their planes
+        std::vector<int> tab(2 * (size_t)nrx + groups + 1, 0);
+        int *first = tab.data() + 2 * (size_t)nrx;
+        auto place = [&](int r, size_t &seg) {
+            const int *x = rx + 3 * r, cell = x[1] * v->kp + x[2];
+            seg = v->rows ? (size_t)x[0] * v->pseg + cell / (256 * NC) : (size_t)x[0] * (g.ny + 1) + x[1];
+            return v->rows ? cell : x[2];
+        };
+        size_t seg;
+        for (int r = 0; r < nrx; ++r) place(r, seg), ++first[seg + 1];
+        for (size_t q = 0; q < groups; ++q) first[q + 1] += first[q];
+        std::vector<int> next(first, first + groups);
         for (int r = 0; r < nrx; ++r) {
-            int *at = &tab[rows + 1 + 2 * (size_t)next[row(r)]++];
-            at[0] = rx[3 * r + 2];
-            at[1] = r;
+            const int at = place(r, seg), n = next[seg]++;
+            tab[2 * (size_t)n] = at;
+            tab[2 * (size_t)n + 1] = r;
         }
         INV_TRY(hipMemcpy(v->rxtab, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
+        if (v->rows && !v->rowrx) {
+            const int *at[2] = {v->rxtab + 2 * (size_t)nrx, v->rxtab};
+            static_assert(offsetof(RowModel, rxat) == offsetof(RowModel, rxfirst) + sizeof(at[0]), "both in one copy");
+            INV_TRY(hipMemcpy(&v->row->rxfirst, at, sizeof(at), hipMemcpyHostToDevice));
+            v->rowrx = true;
+        }
         if (v->rows) {
             std::vector<uint32_t> pf(v->slabflag);
             for (int r = 0; r < nrx; ++r) pf[rx[3 * r]] |= PF_RX;

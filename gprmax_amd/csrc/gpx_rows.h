@@ -115,6 +115,10 @@ struct RowModel {
     const StepRare *rare;
     const uint32_t *planeflag;       // [nx + 1], slab bits by direction
     size_t csl, cil;                 // cs and ci where they pass 32 bits (RowComps)
+    // Of the differentiable solver (inv_rows.h), receivers sorted by segments of planes
+    // (a block's lanes): [segments + 1], a segment's first in rxat; [receivers][2],
+    // point of the plane and number.
+    const int *rxfirst, *rxat;
 };
 
 struct RowArgs {
@@ -1084,13 +1088,13 @@ __global__ void __launch_bounds__(ROW_BLOCK_MAX) __attribute__((amdgpu_waves_per
 // The lane of pass item `item`: segment of the plane's lanes, x chunk of the
 // launch's planes.
 struct RowLane {
-    int j, kl, xa, xb;
+    int seg, j, kl, xa, xb;
     bool live;
 };
 __device__ __forceinline__ RowLane row_lane(const RowModel &a, int item, int p0, int p1)
 {
     RowLane q;
-    const int seg = item % a.pseg, ch = item / a.pseg, lpr = a.kp / NC;
+    const int seg = q.seg = item % a.pseg, ch = item / a.pseg, lpr = a.kp / NC;
     const int t = seg * (int)blockDim.x + (int)threadIdx.x;
     q.live = t < (a.ny + 1) * lpr;
     q.j = q.live ? t / lpr : 0;

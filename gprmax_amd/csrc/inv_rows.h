@@ -39,8 +39,9 @@ struct InvStep {
     float *T;                // T (adjoint: lT) of the three components, each [P]
     float *P, *Q;            // Phi of the pass's field; its adjoint read and written
     float *grad;             // dL/dCA, dL/dCB, dL/dIEA
-    const int *rxfirst;      // [rows of points + 1]: a row's first receiver in rxat
-    const int *rxat;         // [receivers by row][2]: k and number of one
+    // Of the general kernels, receivers sorted by rows of points: [rows + 1], a row's
+    // first in rxat; [receivers][2], k and number.  The row kernels': RowModel.
+    const int *rxfirst, *rxat;
     const float *resid;      // [receivers][iterations]
     float *traces;
     int iterations, it;
@@ -141,26 +142,26 @@ __device__ __forceinline__ fN inv_hmask(const RowModel &a, int i, int j, int kl,
     return v;
 }
 
-// A row's receivers, looked up with the plane's loads on planes that have any:
-// with every receiver looked at by every lane of such a plane 400 of them on 40^3
-// took 76 us an iteration, the whole forward without 11.
-struct InvRx {
-    int r0 = 0, r1 = 0;
-    __device__ __forceinline__ void load(const InvStep &b, const RowModel &a, bool any, int i, int j)
-    {
-        r0 = r1 = 0;
-        if (!any) return;
-        const int row = i * (a.ny + 1) + j;
-        r0 = ld(b.rxfirst, 4u * (uint32_t)row);
-        r1 = ld(b.rxfirst, 4u * (uint32_t)row + 4u);
+// Calls f(u, number) for the receivers on a lane's cells u, on planes that have any:
+// those of the block's segment of the plane, one after the other, the same for all
+// lanes, through the scalar cache.  With every receiver looked at by every lane of
+// such a plane 400 on 40^3 took 45 to 76 us an iteration of the forward, now 14 to 19 (one:
+// 11).  The tables' pointers are the model's, not the launch's: those stay in
+// scalar registers throughout, of which the adjoint's H half had none left (91 reads of
+// spilled ones; 60^3 with 6 receivers 28.2 us an iteration of the backward, now 27.9).
+template <class Fn>
+__device__ __forceinline__ void inv_receivers(const InvStep &b, const RowModel &a, uint32_t pf, int i, int seg, uint32_t to, const Fn &f)
+{
+    if (!(pf & PF_RX)) return;
+    typedef __attribute__((address_space(4))) const int cint;
+    typedef __attribute__((address_space(4))) const u32x2 cu32x2;
+    const int at = i * a.pseg + seg, r1 = ((cint *)a.rxfirst)[at + 1];
+    for (int r = ((cint *)a.rxfirst)[at]; r < r1; ++r) {
+        const u32x2 x = ((cu32x2 *)a.rxat)[r];
+        const uint32_t u = x[0] - to / 4u;
+        if (u < NC) f((int)u, (int)x[1]);
     }
-    // f(k, number) for each
-    template <class Fn>
-    __device__ __forceinline__ void each(const InvStep &b, const Fn &f) const
-    {
-        for (int r = r0; r < r1; ++r) f(ld(b.rxat, 8u * (uint32_t)r), ld(b.rxat, 8u * (uint32_t)r + 4u));
-    }
-};
+}
 
 // H pass of the forward, receivers sampled before it.  38.0 + 4.6 us (the
 // receivers a launch of their own) before, 26.9 now.
@@ -185,12 +186,10 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_inv_r
     fN ex, hx, hy, hz, ezj, exj, ey1, ez1;
     float ykn = 0.f, xkn = 0.f;
     RowPhis<ORDER> ph;
-    InvRx rx;
     uint32_t pf = 0, m = 0;
     auto load = [&](int i) {
         pf = plane_flags(a, i);
         const uint32_t so = (uint32_t)i * P4, sn = i < a.nx ? so + P4 : so;
-        rx.load(b, a, q.live && (pf & PF_RX), i, j);
         ex = bldN(rE, to, so);
         hx = bldN(rH, to, so);
         hy = bldN(rH, to, so + cs);
@@ -214,11 +213,10 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_inv_r
     for (int i = q.xa;;) {
         const uint32_t so = (uint32_t)i * P4;
         const fN eyk = shift_up(ey, from_next(ykn, ey.x)), exk = shift_up(ex, from_next(xkn, ex.x));
-        rx.each(b, [&](int k, int r) {
-#pragma unroll
-            for (int u = 0; u < NC; ++u)
-                if (k == kl + u) b.traces[(size_t)r * b.iterations + b.it] = ez[u];
-        });
+        if (q.live)
+            inv_receivers(b, a, pf, i, q.seg, to, [&](int u, int r) {
+                b.traces[(size_t)r * b.iterations + b.it] = u ? ez[1] : ez[0];
+            });
         const idN none = 0u;
         row_h<0, ORDER, true>(a, S, pf, m, ph, i, j, kl, q.live, b.it, ex, ey, ez, ey1, ez1, exj, ezj, exk, eyk, none, none, none,
                               hx, hy, hz);
@@ -657,12 +655,10 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(P > 0 ? 2 : 1, OR
     RowPhi<1> xo, xn, yo, yn, z;
     InvPoles<P> t[3], ee, eq, zt;
     float hxl = 0.f, hyl = 0.f, za = 0.f, zb = 0.f;
-    InvRx rx;
     uint32_t pf = 0, f = 0, fn = 0, mo = 0, mx = 0, my = 0, mz = 0;
     auto load = [&](int i) {
         const uint32_t so = (uint32_t)i * P4;
         pf = plane_flags(a, i);
-        rx.load(b, a, q.live && (pf & PF_RX), i, j);
         hx = bldN(rH, to, so);
         hy = bldN(rH, to, so + cs);
         hz = bldN(rH, to, so + 2 * cs);
@@ -819,10 +815,10 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(P > 0 ? 2 : 1, OR
                 ly[u] = (inv_eupd<1>(a, i, j, k) ? o1[u] : ly[u]) + d1[u];
                 lz[u] = (inv_eupd<2>(a, i, j, k) ? o2[u] : lz[u]) + d2[u];
             }
-            rx.each(b, [&](int k, int r) {
+            inv_receivers(b, a, pf, i, q.seg, to, [&](int at, int r) {
                 const float v = b.resid[(size_t)r * b.iterations + b.it];
 #pragma unroll
-                for (int u = 0; u < NC; ++u) lz[u] = k == kl + u ? lz[u] + v : lz[u];
+                for (int u = 0; u < NC; ++u) lz[u] = at == u ? lz[u] + v : lz[u];
             });
             if (P > 0) {
                 auto next = [&](const InvPoles<P> &t, fN l) {
