@@ -355,7 +355,7 @@ def main():
     ap.add_argument('--no-cpu-baseline', action='store_true')
     ap.add_argument('--xchunk', type=int, default=0)
     ap.add_argument('--block', type=int, default=0)
-    ap.add_argument('--tile', type=int, default=0, help='cells per fused block (0 = auto)')
+    ap.add_argument('--tile', type=int, default=0, help='cells per block of the one launch (0 = auto)')
     ap.add_argument('--fused', action='store_true', help='the whole step in one launch (form 1)')
     ap.add_argument('--overlap', action='store_true', help='the general passes with interior and boundary side by side (form 2)')
     ap.add_argument('--passes', action='store_true', help='the H and E passes (step form 0)')

@@ -20,8 +20,8 @@ import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
-# gpx.hip holds the host code and the two-pass kernels; each step_*.hip holds
-# the fused kernels of one PML form.  They compile in parallel.
+# gpx.hip holds the host code and the general passes; each step_*.hip holds
+# the row kernels of one PML form.  They compile in parallel.
 SOURCES = sorted(glob.glob(os.path.join(HERE, 'csrc', '*.hip')))
 LIBRARY = os.path.join(HERE, 'libgprmax_hip.so')
 ARCH = os.environ.get('GPX_OFFLOAD_ARCH', 'gfx950')

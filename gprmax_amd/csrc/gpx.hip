@@ -2,13 +2,18 @@
 // corrections, dispersive multipole A/B, point sources, receivers and
 // snapshots.  C ABI declared in include/gpx.h.
 //
-// Work mapping.  Field arrays are [nx+1][ny+1][nz+1], z fastest, so one x-plane
-// is a contiguous run of (ny+1)(nz+1) floats.  A block owns `block` consecutive
+// Kernels.  gpx_rows.h has the row kernels, which run almost every model, and
+// gpx_plane.h the one of 2-D models.  Here are the general passes, for models that
+// those cannot place (rows_ok) and for single sub-steps (gpx_part), and the host code.
+//
+// Work mapping of the general passes.  Field arrays are [nx+1][ny+1][kp], z fastest,
+// kp floats a row (nz+1, padded), so one x-plane is a contiguous run of (ny+1) kp
+// floats.  A block owns `block` consecutive
 // points of that plane and marches along x over a chunk of planes; each thread
 // owns one (j, k) column.  Every load of a plane is therefore one coalesced
 // stream, the x-neighbour is carried in registers from the previous plane (a
 // register queue), and the y/z neighbours are the same stream shifted by
-// (nz+1) or 1 elements and are served by L1/L2.  Blocks are remapped so that
+// kp or 1 elements and are served by L1/L2.  Blocks are remapped so that
 // consecutive plane segments land on the same XCD and share its L2.
 //
 // Fusion.  The H pass applies, per cell and in the reference order: receiver
@@ -743,9 +748,10 @@ struct gpx_ctx {
     long long ntot = 0;
     int kp = 0, plane = 0;    // floats per field row (nz + 1, padded: see gpx_create); (ny + 1) kp
     hipStream_t stream = nullptr;
-    // The state: fields and H Phi, twice for the double-buffered step (the
-    // second copy is allocated when it first runs), `cur` the current one; E
-    // Phi once.  ntot counts padded points.
+    // The state: fields and H Phi, twice for the kernels that write the next state
+    // beside the current one (the one-launch step and the 2-D kernel; the second copy
+    // is allocated when one first runs), `cur` the current one; E Phi twice for the
+    // 2-D kernel.  ntot counts padded points.
     float *Fmem[2] = {nullptr, nullptr};    // 6 x fstride floats: Ex, Ey, Ez, Hx, Hy, Hz
     float *phiH[2] = {nullptr, nullptr}, *phiE[2] = {nullptr, nullptr};
     int cur = 0, curE = 0;    // current copy of the fields and H Phi, of E Phi
@@ -788,7 +794,7 @@ struct gpx_ctx {
     std::vector<TLine> tls;          // transmission lines
     TLDev *tldev = nullptr;          // device copy of their descriptions
     uint32_t *planeflag = nullptr;  // [2][nx+1]: slab bits by slab, by direction
-    StepRare *rare = nullptr;        // device copy of the source/receiver tables for the fused step
+    StepRare *rare = nullptr;        // device copy of the source/receiver tables of the row kernels
     bool rare_dirty = true;
     int box[6] = {0, 0, 0, 0, 0, 0}; // interior box (see StepArgs)
     int *frame = nullptr;            // plane offsets outside the interior rectangle
@@ -796,7 +802,7 @@ struct gpx_ctx {
     bool deep = false;               // the interior box has at least two cells on every axis
     int xchunk = 0, block = 0;
     int fused = 4;                   // step form, see gpx_set_step
-    int choice = -1;                 // form 4: -1 open, 4 form 6, 5 form 7
+    int choice = -1;                 // form 4, as reported: -1 open, 4 form 6, 5 form 7
     hipStream_t stream2 = nullptr;   // second stream of form 2
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int tile_cells = 0;              // cells per block of the one-launch step (0 = auto)
@@ -831,11 +837,6 @@ static int fail_hip(gpx_ctx *ctx, hipError_t e, const char *what)
 {
     std::string msg = std::string(what) + ": " + hipGetErrorString(e);
     return fail(ctx, (int)e, msg);
-}
-
-static int check_hip(gpx_ctx *ctx, hipError_t e)
-{
-    return e == hipSuccess ? 0 : fail_hip(ctx, e, "HIP call of the step-form timing");
 }
 
 static hipError_t dalloc(gpx_ctx *ctx, void **p, size_t bytes, bool zero = true)
@@ -2644,8 +2645,8 @@ struct EventSet {
 // `ms4`, events around every kernel give the mean duration of each kernel of
 // an iteration over the run: the one-launch step in ms4[0] (the rest 0); the
 // row passes in ms4[0] and ms4[2]; or H interior, H boundary, E interior and
-// E boundary of the general passes.  Form 4 settles on its first run of at
-// least CHOOSE_ITS iterations.
+// E boundary of the general passes.  Form 4 reports its rule's form from its
+// first run of at least CHOOSE_ITS iterations on (gpx_step_choice).
 static const int CHOOSE_ITS = 26;
 
 static int run_steps(gpx_ctx *ctx, int it0, int n, float *ms4)
@@ -3144,9 +3145,9 @@ extern "C" size_t gpx_memory_bytes(const gpx_ctx *ctx)
 }
 
 // ====================================================================== batch
-// Many models advanced together: one launch of the one-launch step per
-// iteration covers the work items of every model of a group.  Each model keeps
-// its own gpx_ctx (buffers, sources, receivers); the batch only holds the launch
+// Many models advanced together: each launch of an iteration (the two row passes or
+// the one-launch step) covers the work items of every model of a group.  Each model
+// keeps its own gpx_ctx (buffers, sources, receivers); the batch only holds the launch
 // tables.
 struct gpx_batch {
     std::vector<gpx_ctx *> ctx;

@@ -135,23 +135,17 @@ __device__ __forceinline__ To bits(From v)
 {
     return __builtin_bit_cast(To, v);
 }
-template <int N = NC>
 __device__ __forceinline__ fN bldN(rsrc_t r, uint32_t voff, uint32_t soff)
 {
-    if constexpr (N == 4) return bits<fN>(__builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-    else return bits<fN>(__builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+    return bits<fN>(__builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
 }
-template <int N = NC>
 __device__ __forceinline__ idN bld_ids(rsrc_t r, uint32_t voff, uint32_t soff)
 {
-    if constexpr (N == 4) return bits<idN>(__builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
-    else return bits<idN>(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+    return bits<idN>(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
-template <int N = NC>
 __device__ __forceinline__ void bstN(rsrc_t r, uint32_t voff, uint32_t soff, fN v)
 {
-    if constexpr (N == 4) __builtin_amdgcn_raw_buffer_store_b128(bits<u32x4>(v), r, voff, soff, 0);
-    else __builtin_amdgcn_raw_buffer_store_b64(bits<u32x2>(v), r, voff, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(bits<u32x2>(v), r, voff, soff, 0);
 }
 // Components of a state or of the indices.  Offsets are 32-bit, so a state of
 // 4 GiB and more (BIG) has a resource for each component, any other one for all.

@@ -323,8 +323,9 @@ def device_info(device=0):
 
 class HipBatch:
     """Several HipSolver models advanced together: per iteration, the H and E
-    row passes each over all models, or one launch of the whole step over all
-    models (models that share no row kernels: four general passes)."""
+    row passes each over all models of a group, or one launch of the whole step
+    (models that share no row kernels: four general passes); a model that is a
+    group by itself runs as HipSolver.run does."""
 
     def __init__(self, solvers):
         self.lib = library()
@@ -358,8 +359,9 @@ class HipBatch:
         self.close()
 
     def set_shape(self, tile_cells=0, xchunk=0):
-        """tile_cells 0: by the rule of the default step form; 256, 512, 1024:
-        the one-launch step with that many cells per block."""
+        """tile_cells 0: the passes, or the one launch for models without slabs
+        and poles; 256, 512, 1024: the one-launch step with that many cells per
+        block."""
         self._check(self.lib.gpx_batch_set_shape(self.b, int(tile_cells), int(xchunk)))
 
     def set_group_bytes(self, nbytes=0):

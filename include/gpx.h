@@ -105,7 +105,7 @@ int gpx_set_sources(gpx_ctx *ctx, int kind, int n, const int32_t *info, const fl
  * (calculate_incident_V_I).  After the H pass the line records its antenna
  * voltage and current, then updates its current and takes the current of
  * the H loop around the edge; after the E pass it updates its voltage and
- * sets the edge's E.  Models with transmission lines step in the two-pass
+ * sets the edge's E.  Models with transmission lines step in the passes'
  * form; dispersive models, a magnetic dipole on an H component the line
  * reads, or a Hertzian dipole on its edge are refused at the first step
  * (GPX_EARG).  Returns the line's index through *index. */
@@ -152,10 +152,10 @@ int gpx_run_profiled(gpx_ctx *ctx, int it0, int n, float *ms4);
 long long gpx_interior_cells(const gpx_ctx *ctx);
 int gpx_interior_box(const gpx_ctx *ctx, int *box6);
 
-/* One unfused sub-step (enum gpx_part_id) at iteration it. */
+/* One sub-step (enum gpx_part_id) at iteration it. */
 int gpx_part(gpx_ctx *ctx, int part, int arg, int it);
 
-/* Launch shape: planes per chunk along x (0 = auto, both step forms) and
+/* Launch shape: planes per chunk along x (0 = auto) and
  * threads per block of the H and E passes (64, 128, 256, 512 or 1024; 0 = auto). */
 int gpx_set_launch(gpx_ctx *ctx, int xchunk, int block);
 
@@ -166,10 +166,11 @@ int gpx_set_launch(gpx_ctx *ctx, int xchunk, int block);
  * one after the other); fused = 3, 5, 7 and 4 (default): by rule, the one
  * launch for 3-D models without slabs and dispersive poles, several iterations
  * a launch for 2-D models without poles (reported as the passes, which
- * gpx_run_profiled times), the passes otherwise.  tile_cells = cells per block
- * of form 1 (256, 512 or 1024; 0 = auto).  All forms give identical results; models the row kernels do not take
- * (slabs of different orders, in another order or overlapping, more than 32
- * bits of byte offsets, tables past the LDS) run the general passes. */
+ * gpx_run_profiled times), the passes otherwise; a state of 4 GiB and more has
+ * the passes only.  tile_cells = cells per block of form 1 (256, 512 or 1024;
+ * 0 = auto).  All forms give identical results; models the row kernels do not
+ * take (slabs of different orders, in another order or overlapping, poles in a
+ * state of 4 GiB and more, tables past the LDS) run the general passes. */
 int gpx_set_step(gpx_ctx *ctx, int fused, int tile_cells);
 
 /* Cells per block of the one-launch step under form 1, or 0 when gpx_run will
@@ -212,13 +213,14 @@ size_t gpx_memory_bytes(const gpx_ctx *ctx);
  * re-runs run_model and so a whole solve_gpu (gprMax/gprMax.py:222-232 with
  * gprMax/model_build_run.py:84-406); here the traces stay separate gpx_ctx
  * models, each built and uploaded as usual.  Each iteration of the batch is
- * the row passes, or the one-launch step, each launch over the work of every
- * model (tile 0, the default: by form 4's rule; tile > 0: the one launch), or
- * for models that share no row kernels four general passes.  Requirements: one device, the same
- * iteration count, no snapshots, and the same kernel (index width, poles and
- * their kind, PML formulation) for every model; the one launch also needs one
- * PML order for all slabs of all models.  The contexts must outlive the
- * batch; results are read from each context (gpx_download_rx, ...). */
+ * the row passes, 2-D models' too, each launch over the work of every model of a
+ * group; for a group of models without slabs and poles the one-launch step (tile
+ * > 0: for every model); for models that share no row kernels four general
+ * passes.  A model that is a group by itself runs as gpx_run does.
+ * Requirements: one device, the same iteration count, no snapshots, and the same
+ * kernel (poles and their kind, PML formulation) for every model; the one launch
+ * also needs one PML order for all slabs of all models.  The contexts must
+ * outlive the batch; results are read from each context (gpx_download_rx, ...). */
 typedef struct gpx_batch gpx_batch;
 
 int gpx_batch_create(gpx_ctx *const *ctxs, int n, gpx_batch **out);
@@ -240,8 +242,9 @@ int gpx_batch_tune(gpx_batch *b, int steps, int *tile_cells, int *xchunk, float 
  * runs all its iterations before the next starts. */
 int gpx_batch_set_group_bytes(gpx_batch *b, double bytes);
 /* Iterations [it0, it0 + n) of every model, launched on the batch's stream
- * whatever `graph` says (a graph of one run costs more to make than it saves).  Waits; *ms (optional) is the
- * device time measured with HIP events around the launches. */
+ * whatever `graph` says (a graph of one run costs more to make than it saves).
+ * Waits; *ms (optional) is the device time measured with HIP events around the
+ * launches. */
 int gpx_batch_run(gpx_batch *b, int it0, int n, int graph, float *ms);
 
 /* ---- Differentiable solve: forward with checkpoints and its adjoint.
