@@ -2362,9 +2362,9 @@ static int plane_axis(const gpx_ctx *ctx)
 // Tiles for a run of n iterations: the shape that takes the least time by what
 // launches of several shapes took, 5.5 us + 0.7 us for each wave a SIMD is
 // given + for each iteration 0.25 us a wave, 0.5 at the least.  Measured, us per iteration
-// (columns of a tile, halo): 120x105 2.09 (16x16, 4), 1.75 (16x32, 6), 1.88 (32x32,
-// 8), the passes 8.6; 250x180 2.60, 3.00, 1.92, 9.5; 500x500 7.4, 9.0, 6.7, 5.2
-// (32x32, 4), 17.9; 1200x1000 28, 35, 24, 18.3 (32x32, 4), 57.
+// (columns of a tile, halo): 120x105 1.98 (16x16, 4), 1.75 (16x32, 6), 1.90 (32x32,
+// 8), the passes 9.0; 250x180 2.48, 2.93, 1.90, 9.0; 500x500 7.0, 8.6, 6.5, 4.8
+// (32x32, 4), 11.8; 1200x1000 27, 35, 23, 17.0 (32x32, 4), 35.
 static PlaneShape plane_shape(const gpx_ctx *ctx, int n)
 {
     PlaneShape best = {plane_axis(ctx), 0, 0, 0};

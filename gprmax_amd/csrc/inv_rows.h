@@ -16,8 +16,8 @@
 // The figures at each kernel are us per launch on 160x160x120 with 10 cells of
 // PML; before, a thread had one point, lE and lH were float4 with CB and CA in
 // w, and the points near a slab ran apart from the rest.  A gradient of 600
-// iterations: 216 ms before, 148 now; on 40^3 with 3 poles, 150 iterations:
-// 13.6 and 6.4 ms.
+// iterations: 216 ms before, 141 now; on 40^3 with 3 poles, 150 iterations:
+// 13.6 and 6.3 ms.
 #ifndef GPX_INV_ROWS_H
 #define GPX_INV_ROWS_H
 
@@ -164,7 +164,7 @@ __device__ __forceinline__ void inv_receivers(const InvStep &b, const RowModel &
 }
 
 // H pass of the forward, receivers sampled before it.  38.0 + 4.6 us (the
-// receivers a launch of their own) before, 26.9 now.
+// receivers a launch of their own) before, 24.2 now.
 template <int ORDER>
 __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(0, ORDER) k_inv_row_h(const RowModel *__restrict__ models, InvStep b)
 {
@@ -249,7 +249,7 @@ __device__ __forceinline__ InvPoles<P> inv_poles(rsrc_t r, uint32_t to, uint32_t
 
 // E pass of the forward: E^{n+1} into b.En, with the poles, the slabs and the
 // dipole; the curl (and phi^n) for the adjoint where they are kept.
-// 43.6 us before (half of the launches storing), 32.7 now.
+// 43.6 us before (half of the launches storing), 30.4 now.
 template <int P, int ORDER>
 __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(P > 0 ? 2 : 0, ORDER) k_inv_row_e(const RowModel *__restrict__ models,
                                                                                                  InvStep b)
@@ -420,7 +420,7 @@ __device__ __forceinline__ fN bld_stored(rsrc_t r, uint32_t voff, uint32_t soff)
 // E half of iteration n: lH += (dE^{n+1}/dH^{n+1})^T lE*, the gradients from
 // lE*, E^n and the curl, and the Phi adjoints into b.Q.  lE* (the poles' part B
 // folded in) is left as it is.
-// 95.4 us before, 55.7 now.
+// 95.4 us before, 53.2 now.
 template <int P, int ORDER>
 __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(2, ORDER) k_inv_adj_e(const RowModel *__restrict__ models, InvStep b)
 {
@@ -630,7 +630,7 @@ __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(2, ORDER) k_inv_a
 // updated edges, plus the receivers' residuals, in place; lT one iteration
 // back; then, with poles, lE* of iteration n-1 from both; and the Phi adjoints
 // into b.Q.
-// 56.9 us before (and 5.2 for lE* in a launch of its own on 40^3), 35.5 now.
+// 56.9 us before (and 5.2 for lE* in a launch of its own on 40^3), 28.5 now.
 template <int P, int ORDER>
 __global__ void __launch_bounds__(ROW_PASS_MAX) ROW_PASS_WAVES(P > 0 ? 2 : 1, ORDER) k_inv_adj_h(const RowModel *__restrict__ models,
                                                                                                  InvStep b)
